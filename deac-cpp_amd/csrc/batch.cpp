@@ -4,7 +4,8 @@
 // Host work: validation and model building per distinct problem (identical
 // problems share one device copy of K), the kernel-side layouts (K in MFMA
 // tile order, the remainder rows, the walk and sub-stream jump tables), the
-// initial populations (on host threads, with each instance's own stream),
+// random state at each member's first initial draw (the populations are drawn
+// on the device),
 // launch slicing with per-instance stop and compaction, and the same
 // epilogue as deac_run.
 #include <hip/hip_runtime_api.h>
@@ -17,13 +18,13 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <tuple>
 #include <vector>
 
 #include "batch_kernels.hpp"
 #include "deac_engine.h"
 #include "host_model.hpp"
+#include "init_kernels.hpp"
 #include "ks_layout.hpp"
 
 namespace {
@@ -49,6 +50,10 @@ struct BatchModel {
     double *mterm = nullptr;               // [3][Lpad] first-moment, third-moment and normalization weights,
                                            // when moments or per-generation renormalization are used
     uint64_t *walk_rows = nullptr, *sub_tab = nullptr;
+    double *nterm = nullptr;               // [L] weights of the initial normalization, when used
+    std::vector<uint64_t> skip_tab;        // nibble table of T^L, host side
+    std::vector<size_t> insts;             // instances of this problem
+    size_t init_row = 0, init_inst = 0;    // their part of deac_batch::init_start and init_off
     void *kmix[3] = {nullptr, nullptr, nullptr};  // mixed K tiles by precision, built on first use
     double *kscale = nullptr;                     // 2^ex[t] of the mixed K rows
 };
@@ -111,6 +116,10 @@ struct deac_batch {
     deac::BatchDesc *descs = nullptr;          // device copy of the launch descriptors
     deac::BatchDesc *hdescs = nullptr;         // their host side, pinned (3 per instance)
     long *hstatus = nullptr;                   // pinned host copy of status
+    uint64_t *init_start = nullptr;            // [members of all instances][4], model by model: random state at
+                                               // each member's first initial draw
+    long *init_off = nullptr;                  // instances, model by model: offset of the population in pop
+    size_t init_rows = 0;
     double *scratch = nullptr;                 // this device's statistics scratch (deac_batch_run_noalloc)
     std::vector<long> reached;                 // per instance: generation reached by the last run (absolute)
     std::vector<char> epar_valid;              // per instance: epar holds the current population's model ISF
@@ -337,7 +346,10 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     // Jump tables: T^L by rows for the walk, T^(k*Lsub) by nibbles for the
     // mask sub-streams k = 1..S-1.
     std::vector<uint64_t> rows(256 * 4), tabs(static_cast<size_t>(std::max(b.S - 1, 1)) * 64 * 16 * 4);
-    deac::matrix_rows(deac::transition_power(static_cast<uint64_t>(L)), rows.data());
+    const deac::Gf2Matrix skip = deac::transition_power(static_cast<uint64_t>(L));
+    deac::matrix_rows(skip, rows.data());
+    b.skip_tab.resize(64 * 16 * 4);
+    deac::nibble_table(skip, b.skip_tab.data());
     const deac::Gf2Matrix step = deac::transition_power(static_cast<uint64_t>(b.Lsub));
     deac::Gf2Matrix acc = step;
     for (int k = 1; k < b.S; k++) {
@@ -354,6 +366,7 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     A(b.sig, m.T);
     A(b.walk_rows, rows.size());
     A(b.sub_tab, tabs.size());
+    if (m.normalize) A(b.nterm, m.Kc);
     // moment weights (deac.cpp:628-668, 728-768) and the normalization
     // weights of per-generation renormalization (deac.cpp:1342-1352), zero
     // past L
@@ -378,6 +391,7 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     up(b.sig, m.err.data(), m.T * sizeof(double));
     up(b.walk_rows, rows.data(), rows.size() * sizeof(uint64_t));
     up(b.sub_tab, tabs.data(), tabs.size() * sizeof(uint64_t));
+    if (b.nterm) up(b.nterm, m.nterm.data(), m.Kc * sizeof(double));
     if (b.mterm) up(b.mterm, mt.data(), mt.size() * sizeof(double));
     if (m.bdsf && st == DEAC_OK) {
         // [Lpad][fold_rows]: the timeslices of a position contiguous
@@ -392,23 +406,6 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
         if (b.nfm_dt) up(b.nfm_dt, m.nfm_dt.data(), m.T * sizeof(double));
     }
     return st;
-}
-
-// Runs fn(i) for i < n on up to 16 host threads.
-template <class F>
-void parallel_for(size_t n, F fn)
-{
-    const size_t nt = std::min<size_t>(n, std::clamp<unsigned>(std::thread::hardware_concurrency(), 1u, 16u));
-    if (nt <= 1) {
-        for (size_t i = 0; i < n; i++) fn(i);
-        return;
-    }
-    std::vector<std::thread> th;
-    for (size_t t = 0; t < nt; t++)
-        th.emplace_back([&, t] {
-            for (size_t i = t; i < n; i += nt) fn(i);
-        });
-    for (auto &x : th) x.join();
 }
 
 }  // namespace
@@ -505,6 +502,7 @@ deac_status deac_batch_create(const deac_problem *problems, size_t count, deac_b
         h->pop_off[i] = npop;
         h->mask_off[i] = nmask;
         h->epar_off[i] = nepar;
+        h->models[h->model_of[i]]->insts.push_back(i);
         npop += b.m.P * static_cast<size_t>(b.Lpad);
         nmask += static_cast<size_t>(3) * b.Ppad * 2 * b.Lw;
         nepar += b.m.T * static_cast<size_t>(b.Ppad);
@@ -522,8 +520,18 @@ deac_status deac_batch_create(const deac_problem *problems, size_t count, deac_b
     A(h->status, count * 2);
     A(h->accp, count * deac::kBatchMaxP);
     A(h->epar, nepar);
+    std::vector<long> init_off;
+    for (auto &b : h->models) {
+        b->init_row = h->init_rows;
+        b->init_inst = init_off.size();
+        for (size_t i : b->insts) init_off.push_back(static_cast<long>(h->pop_off[i]));
+        h->init_rows += b->insts.size() * b->m.P;
+    }
+    A(h->init_start, h->init_rows * 4);
+    A(h->init_off, count);
     A(h->descs, 3 * count);  // evolution launches, and the evaluation launches of mixed K.S before and after
     if (st != DEAC_OK) return st;
+    BATCH_HIP(hipMemcpy(h->init_off, init_off.data(), count * sizeof(long), hipMemcpyHostToDevice));
     // pinned host sides of the per-round descriptor upload and status read
     if (hipHostMalloc(reinterpret_cast<void **>(&h->hdescs), 3 * count * sizeof(deac::BatchDesc)) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void **>(&h->hstatus), 2 * count * sizeof(long)) != hipSuccess) {
@@ -611,27 +619,48 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
     h->reached.clear();  // set again when this call completes
     std::vector<uint64_t> rng_host(4 * n);
     if (!resume) {
-        // Initial populations on the host (deac.cpp:430-603), each from its own
+        // Initial populations on the device (deac.cpp:430-603), each from its own
         // stream; the state after them is where the device walk starts.
-        std::vector<double> pop_host(h->pop_off.back() + h->models[h->model_of[n - 1]]->m.P *
-                                                             static_cast<size_t>(h->models[h->model_of[n - 1]]->Lpad),
-                                     0.0);
         std::vector<double> cr_host(n * deac::kBatchMaxP * 2, 0.0), f_host(n * deac::kBatchMaxP * 2, 0.0);
-        parallel_for(n, [&](size_t i) {
-            const BatchModel &b = *h->models[h->model_of[i]];
-            deac::Xoshiro rng{{rng_states[4 * i], rng_states[4 * i + 1], rng_states[4 * i + 2], rng_states[4 * i + 3]}};
-            std::vector<double> pop;
-            deac::initial_population(b.m, rng, pop);
-            for (size_t m = 0; m < b.m.P; m++)
-                std::memcpy(&pop_host[h->pop_off[i] + m * b.Lpad], &pop[m * b.m.Kc], b.m.Kc * sizeof(double));
-            std::memcpy(&rng_host[4 * i], rng.s, sizeof rng.s);
-            for (size_t m = 0; m < b.m.P; m++)
-                for (int sg = 0; sg < 2; sg++) {
-                    cr_host[(i * deac::kBatchMaxP + m) * 2 + sg] = b.m.cr0;  // deac.cpp:990-1032
-                    f_host[(i * deac::kBatchMaxP + m) * 2 + sg] = b.m.f0;
+        std::vector<uint64_t> starts(h->init_rows * 4);
+        for (auto &bp : h->models) {
+            const BatchModel &b = *bp;
+            uint64_t *to = &starts[b.init_row * 4];
+            for (size_t i : b.insts) {
+                uint64_t *st = &rng_host[4 * i];
+                std::memcpy(st, &rng_states[4 * i], 4 * sizeof(uint64_t));
+                for (size_t m = 0; m < b.m.P; m++, to += 4) {
+                    std::memcpy(to, st, 4 * sizeof(uint64_t));
+                    deac::nibble_apply(b.skip_tab.data(), st);
+                    for (int sg = 0; sg < 2; sg++) {
+                        cr_host[(i * deac::kBatchMaxP + m) * 2 + sg] = b.m.cr0;  // deac.cpp:990-1032
+                        f_host[(i * deac::kBatchMaxP + m) * 2 + sg] = b.m.f0;
+                    }
                 }
-        });
-        BATCH_HIP(hipMemcpyAsync(h->pop, pop_host.data(), pop_host.size() * sizeof(double), hipMemcpyHostToDevice, s));
+            }
+        }
+        BATCH_HIP(hipMemcpyAsync(h->init_start, starts.data(), starts.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
+                                 s));
+        for (auto &bp : h->models) {
+            const BatchModel &b = *bp;
+            deac::InitArgs ia{};
+            ia.start = h->init_start + b.init_row * 4;
+            ia.offset = h->init_off + b.init_inst;
+            ia.pop = h->pop;
+            ia.tab = b.sub_tab;
+            ia.nterm = b.nterm;
+            ia.rows = static_cast<long>(b.insts.size() * b.m.P);
+            ia.P = static_cast<int>(b.m.P);
+            ia.G = static_cast<int>(b.m.G);
+            ia.nsign = b.m.nsign;
+            ia.stride = b.Lpad;
+            ia.nsub = b.S;
+            ia.sublen = b.Lsub;
+            ia.tab0 = 1;
+            ia.allow_neg = b.m.allow_negative;
+            ia.zeroth = b.m.zeroth_moment;
+            BATCH_HIP(deac::launch_initial_population(ia, s));
+        }
         BATCH_HIP(hipMemcpyAsync(h->rng, rng_host.data(), rng_host.size() * sizeof(uint64_t), hipMemcpyHostToDevice, s));
         BATCH_HIP(hipMemcpyAsync(h->cr_old, cr_host.data(), cr_host.size() * sizeof(double), hipMemcpyHostToDevice, s));
         BATCH_HIP(hipMemcpyAsync(h->f_old, f_host.data(), f_host.size() * sizeof(double), hipMemcpyHostToDevice, s));

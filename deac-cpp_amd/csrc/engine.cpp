@@ -11,6 +11,7 @@
 
 #include "deac_engine.h"
 #include "host_model.hpp"
+#include "init_kernels.hpp"
 #include "kernels.hpp"
 #include "ks_layout.hpp"
 #include "precision_kernels.hpp"
@@ -47,6 +48,10 @@ struct deac_handle {
     deac::MemberCtl *ctl[2] = {};
     uint64_t *raw[2] = {}, *gen_start[2] = {};
     uint64_t *state = nullptr, *skip_rows = nullptr, *lane_tab = nullptr;
+    uint64_t *init_start = nullptr;     // [P][4]: random state at each member's first initial draw
+    std::vector<uint64_t> skip_tab;     // nibble table of T^Kc, host side
+    double *stats = nullptr;            // statistics histories, kept between runs and grown on demand
+    size_t stats_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // per set: walk start, walk end, mask start, mask end, evolve start,
     // evolve end (draws free), status copied
@@ -112,14 +117,6 @@ namespace {
     } while (0)
 
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
-
-// Device population layout: member-major rows of `stride` doubles, rows for
-// MG*4 members, zero padded.
-void pad_rows(const std::vector<double> &pop, size_t P, size_t Kc, int MG, int stride, std::vector<double> &out)
-{
-    out.assign(static_cast<size_t>(MG) * deac::kChainRows * stride, 0.0);
-    for (size_t i = 0; i < P; i++) std::memcpy(&out[i * stride], &pop[i * Kc], Kc * sizeof(double));
-}
 
 // Contraction operands of the split loop at `precision` (kept until another
 // precision is asked for): the kernel matrix in the contraction's lane order,
@@ -319,6 +316,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
         A(h->gen_start[k], static_cast<size_t>(h->batch) * 4);
     }
     A(h->state, 4);
+    A(h->init_start, static_cast<size_t>(P) * 4);
     A(h->skip_rows, 256 * 4);
     A(h->lane_tab, static_cast<size_t>(64) * 64 * 16 * 4);
     if (!m.nterm.empty()) A(h->nterm, Kc);
@@ -333,7 +331,10 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     // Jump tables: T^(nsign*G) by rows for the walk, T^(l*chunk) by nibbles
     // for the mask generator.
     std::vector<uint64_t> rows(256 * 4), tabs(static_cast<size_t>(64) * 64 * 16 * 4);
-    deac::matrix_rows(deac::transition_power(static_cast<uint64_t>(Kc)), rows.data());
+    const deac::Gf2Matrix skip = deac::transition_power(static_cast<uint64_t>(Kc));
+    deac::matrix_rows(skip, rows.data());
+    h->skip_tab.resize(64 * 16 * 4);
+    deac::nibble_table(skip, h->skip_tab.data());
     const deac::Gf2Matrix step = deac::transition_power(static_cast<uint64_t>(h->chunk));
     deac::Gf2Matrix acc = deac::Gf2Matrix::identity();
     for (int l = 0; l < 64; l++) {
@@ -352,6 +353,11 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     if (h->fterm) up(h->fterm, m.fterm.data(), m.Kc * sizeof(double));
     if (h->tterm) up(h->tterm, m.tterm.data(), m.Kc * sizeof(double));
     if (h->nfm_dt) up(h->nfm_dt, m.nfm_dt.data(), m.T * sizeof(double));
+    // Populations: member-major rows of `stride` doubles for MG*4 members,
+    // zero past Kc and past P.
+    for (double *p : {h->pop0, h->pop1})
+        if (st == DEAC_OK && hipMemsetAsync(p, 0, pop_n * sizeof(double), h->stream) != hipSuccess)
+            st = DEAC_ERR_DEVICE;
     if (st != DEAC_OK) return fail(st);
     *out = h;
     return DEAC_OK;
@@ -395,26 +401,50 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     DEAC_HIP(hipSetDevice(h->device));
     if (split) DEAC_TRY(prepare_split(h, o->ks_precision));
 
-    // Initial population and normalization on the host (deac.cpp:430-603).
+    // Initial population and normalization (deac.cpp:430-603) on the device,
+    // from the random state at each member's first draw; the state after the
+    // last member is where the walk starts.
     deac::Xoshiro rng{{rng_state[0], rng_state[1], rng_state[2], rng_state[3]}};
-    std::vector<double> pop, lay;
-    deac::initial_population(m, rng, pop);
-    pad_rows(pop, P, Kc, h->MG, h->stride, lay);
-    std::vector<double> zeros(lay.size(), 0.0);
+    std::vector<uint64_t> starts(P * 4);
+    for (size_t i = 0; i < P; i++) {
+        std::memcpy(&starts[i * 4], rng.s, sizeof rng.s);
+        deac::nibble_apply(h->skip_tab.data(), rng.s);
+    }
     std::vector<int> cur(P, 0);
     std::vector<double> cr(P * nsign, m.cr0), fw(P * nsign, m.f0);  // deac.cpp:990-1032
 
-    double *stats = nullptr;
     const bool track = o->track_stats != 0;
-    if (track && h->alloc(stats, 3 * N) != DEAC_OK) return DEAC_ERR_OUT_OF_MEMORY;
-    void *stats_alloc = stats;
+    if (track && h->stats_cap < 3 * N) {
+        void *old = h->stats;
+        h->release(old);
+        h->stats = nullptr;
+        h->stats_cap = 0;
+        DEAC_TRY(h->alloc(h->stats, 3 * N));
+        h->stats_cap = 3 * N;
+    }
+    double *const stats = track ? h->stats : nullptr;
 
-    DEAC_HIP(hipMemcpyAsync(h->pop0, lay.data(), lay.size() * sizeof(double), hipMemcpyHostToDevice, s));
-    DEAC_HIP(hipMemcpyAsync(h->pop1, zeros.data(), zeros.size() * sizeof(double), hipMemcpyHostToDevice, s));
+    DEAC_HIP(hipMemcpyAsync(h->init_start, starts.data(), starts.size() * sizeof(uint64_t), hipMemcpyHostToDevice, s));
     DEAC_HIP(hipMemcpyAsync(h->cur, cur.data(), P * sizeof(int), hipMemcpyHostToDevice, s));
     DEAC_HIP(hipMemcpyAsync(h->cr_old, cr.data(), cr.size() * sizeof(double), hipMemcpyHostToDevice, s));
     DEAC_HIP(hipMemcpyAsync(h->f_old, fw.data(), fw.size() * sizeof(double), hipMemcpyHostToDevice, s));
     DEAC_HIP(hipMemcpyAsync(h->state, rng.s, sizeof rng.s, hipMemcpyHostToDevice, s));
+    deac::InitArgs ia{};
+    ia.start = h->init_start;
+    ia.pop = h->pop0;
+    ia.tab = h->lane_tab;
+    ia.nterm = m.normalize ? h->nterm : nullptr;
+    ia.rows = static_cast<long>(P);
+    ia.P = static_cast<int>(P);
+    ia.G = static_cast<int>(m.G);
+    ia.nsign = nsign;
+    ia.stride = h->stride;
+    ia.nsub = 64;
+    ia.sublen = h->chunk;
+    ia.tab0 = 0;
+    ia.allow_neg = m.allow_negative;
+    ia.zeroth = m.zeroth_moment;
+    DEAC_HIP(deac::launch_initial_population(ia, s));
 
     deac::EvoArgs ea{};
     ea.P = static_cast<int>(P);
@@ -777,11 +807,9 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     std::memcpy(rng_state, rng.s, sizeof rng.s);
 
     // Epilogue on the host (deac.cpp:1576-1685).
-    std::vector<double> fit(P), l0(lay.size()), l1(lay.size());
+    std::vector<double> fit(P), row(Kc);
     DEAC_HIP(hipMemcpy(fit.data(), h->fitness, P * sizeof(double), hipMemcpyDeviceToHost));
     DEAC_HIP(hipMemcpy(cur.data(), h->cur, P * sizeof(int), hipMemcpyDeviceToHost));
-    DEAC_HIP(hipMemcpy(l0.data(), h->pop0, l0.size() * sizeof(double), hipMemcpyDeviceToHost));
-    DEAC_HIP(hipMemcpy(l1.data(), h->pop1, l1.size() * sizeof(double), hipMemcpyDeviceToHost));
     size_t generation = stopped_at >= 0 ? static_cast<size_t>(stopped_at) : N - 2;
     size_t best = 0;
     double minimum = fit[0];
@@ -790,8 +818,9 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             minimum = fit[i];
             best = i;
         }
-    const std::vector<double> &lb = cur[best] ? l1 : l0;
-    deac::output_transform(m, &lb[best * h->stride], r->dsf, r->frequency);
+    DEAC_HIP(hipMemcpy(row.data(), (cur[best] ? h->pop1 : h->pop0) + best * h->stride, Kc * sizeof(double),
+                       hipMemcpyDeviceToHost));
+    deac::output_transform(m, row.data(), r->dsf, r->frequency);
 
     if (track) {
         std::vector<double> host_stats(3 * N, 0.0);
@@ -813,10 +842,6 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     r->minimum_fitness = minimum;
     r->best_index = best;
     if (r->final_fitness) std::memcpy(r->final_fitness, fit.data(), P * sizeof(double));
-    if (stats_alloc) {
-        h->allocations.erase(std::find(h->allocations.begin(), h->allocations.end(), stats_alloc));
-        (void)hipFree(stats_alloc);
-    }
     return DEAC_OK;
 }
 

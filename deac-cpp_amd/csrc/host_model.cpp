@@ -126,27 +126,20 @@ void nibble_table(const Gf2Matrix &m, uint64_t *tab)
         }
 }
 
-// ---------------------------------------------------------------- reductions
-// matrix_multiply_MxN_by_Nx1 (deac.cpp:102-108) and squared_mean
-// (deac.cpp:171-177) are inlined into deac() by the reference build and
-// vectorised as in-order reductions: 4-wide blocks of rounded products added
-// one by one, then a 2-wide block, then a fused last odd element
-// (squared_mean: up to three fused scalar elements).
-
-double dot_fold4(double acc, const double *a, const double *b, size_t n)
+void nibble_apply(const uint64_t *tab, uint64_t s[4])
 {
-    size_t i = 0;
-    if (n >= 4)
-        for (; i + 4 <= n; i += 4)
-            for (size_t l = 0; l < 4; l++) acc += a[i + l] * b[i + l];
-    if (n - i >= 2) {
-        acc += a[i] * b[i];
-        acc += a[i + 1] * b[i + 1];
-        i += 2;
+    uint64_t o[4] = {0, 0, 0, 0};
+    for (int n = 0; n < 64; n++) {
+        const uint64_t *e = tab + (static_cast<size_t>(n) * 16 + ((s[n >> 4] >> ((n & 15) * 4)) & 15)) * 4;
+        for (int k = 0; k < 4; k++) o[k] ^= e[k];
     }
-    if (n - i == 1) acc = std::fma(a[i], b[i], acc);
-    return acc;
+    std::memcpy(s, o, sizeof o);
 }
+
+// ---------------------------------------------------------------- reductions
+// squared_mean (deac.cpp:171-177) is inlined into deac() by the reference
+// build and vectorised as an in-order reduction: 4-wide blocks of rounded
+// products added one by one, then up to three fused elements.
 
 double mean_of(const double *a, size_t n)  // deac.cpp:163-169
 {
@@ -395,28 +388,6 @@ Model build_model(const deac_problem &p)
         m.nfm_error = std::sqrt(e);
     }
     return m;
-}
-
-void initial_population(const Model &m, Xoshiro &rng, std::vector<double> &pop)
-{
-    const size_t Kc = m.Kc, G = m.G;
-    pop.assign(m.P * Kc, 0.0);
-    for (size_t i = 0; i < m.P; i++)  // deac.cpp:430-450: + and - draws interleaved per gene
-        for (size_t j = 0; j < G; j++)
-            for (int s = 0; s < m.nsign; s++) {
-                double u = rng.uniform();
-                if (m.allow_negative) u -= 0.5;
-                pop[i * Kc + s * G + j] = u;
-            }
-    if (m.nsign == 2)
-        for (size_t i = 0; i < m.P; i++) pop[i * Kc + G] = pop[i * Kc];  // deac.cpp:451-458
-    if (m.normalize)  // deac.cpp:584-602
-        for (size_t i = 0; i < m.P; i++) {
-            double *x = &pop[i * Kc];
-            double norm = 0.0;
-            for (int s = 0; s < m.nsign; s++) norm = dot_fold4(norm, x + s * G, &m.nterm[s * G], G);
-            for (size_t k = 0; k < Kc; k++) x[k] *= m.zeroth_moment / norm;
-        }
 }
 
 void output_transform(const Model &m, const double *xb, double *dsf, double *freq)

@@ -43,6 +43,8 @@ Gf2Matrix transition_power(uint64_t n);
 void matrix_rows(const Gf2Matrix &m, uint64_t *rows);
 // 4-bit lookup table: tab[n][v] = M * (v << 4n), 64 x 16 x 4 words.
 void nibble_table(const Gf2Matrix &m, uint64_t *tab);
+// M s by a nibble table.
+void nibble_apply(const uint64_t *tab, uint64_t s[4]);
 
 // ---------------------------------------------------------------- model
 struct Model {
@@ -70,12 +72,7 @@ deac_status validate(const deac_problem &p, std::string &message);
 // Builds K (deac.cpp:310-401) and the moment vectors (deac.cpp:489-827).
 Model build_model(const deac_problem &p);
 
-// Initial population [P][Kc] (deac.cpp:430-458) and its normalization
-// (deac.cpp:584-602); advances rng.
-void initial_population(const Model &m, Xoshiro &rng, std::vector<double> &pop);
-
 // In-order reductions of the reference build (see host_model.cpp).
-double dot_fold4(double acc, const double *a, const double *b, size_t n);
 double mean_of(const double *a, size_t n);
 double squared_mean_of(const double *a, size_t n);
 

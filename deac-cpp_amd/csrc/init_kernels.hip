@@ -1,0 +1,96 @@
+// gfx950 kernels of the initial populations (deac.cpp:430-458, 584-602): the
+// draws of every member in parallel, then the normalization.  The host only
+// computes the random state at each member's first draw (one GF(2) jump per
+// member).  Compiled with -ffp-contract=off.
+#include <hip/hip_runtime.h>
+
+#include "device_common.hpp"
+#include "fold_common.hpp"
+#include "init_kernels.hpp"
+
+namespace deac {
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kWave = 64;
+
+// One thread per sub-stream of a member's nsign*G draws: it jumps to its
+// first draw with a nibble table and steps sublen draws.  The draws
+// interleave the signs gene by gene; the negative sign's zero frequency
+// repeats the positive one's.  Bound: the 8-byte stores, which a lane makes
+// at consecutive positions of its own run (the cache lines fill in L2).  On
+// host threads with a pageable upload the same populations took 150 ms for
+// 256 instances of 32 members at G = 4096; here 1 ms.
+__global__ __launch_bounds__(kThreads) void init_draw_kernel(InitArgs a)
+{
+    const long item = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x;
+    const long row = item / a.nsub;
+    const int sub = static_cast<int>(item % a.nsub);
+    if (row >= a.rows) return;
+    const uint64_t *st = a.start + row * 4;
+    uint64_t s[4] = {st[0], st[1], st[2], st[3]};
+    if (sub >= a.tab0) {
+        const uint64_t *tab = a.tab + static_cast<size_t>(sub - a.tab0) * (64 * 16 * 4);
+        uint64_t o[4] = {0, 0, 0, 0};
+#pragma unroll 4
+        for (int n = 0; n < 64; n++) {
+            const int v = static_cast<int>((s[n >> 4] >> ((n & 15) * 4)) & 15);
+            const uint64_t *e = tab + (n * 16 + v) * 4;
+            o[0] ^= e[0];
+            o[1] ^= e[1];
+            o[2] ^= e[2];
+            o[3] ^= e[3];
+        }
+        for (int w = 0; w < 4; w++) s[w] = o[w];
+    }
+    const long inst = row / a.P, member = row % a.P;
+    double *x = a.pop + (a.offset ? a.offset[inst] : 0) + static_cast<size_t>(member) * a.stride;
+    const int Kc = a.nsign * a.G;
+    const int d0 = sub * a.sublen, d1 = min(d0 + a.sublen, Kc);
+    for (int d = d0; d < d1; d++) {
+        double u = to_unit(xnext(s));
+        if (a.allow_neg) u -= 0.5;
+        const int j = a.nsign == 2 ? d >> 1 : d;
+        if (a.nsign == 1 || !(d & 1)) {
+            x[j] = u;
+            if (a.nsign == 2 && j == 0) x[a.G] = u;
+        } else if (j > 0) {
+            x[a.G + j] = u;
+        }
+    }
+    if (sub == a.nsub - 1)
+        for (int k = Kc; k < a.stride; k++) x[k] = 0.0;
+}
+
+// One wavefront per member: the zeroth moment as the reference folds it,
+// then every position scaled.  Bound: the fold's chain of adds.
+__global__ __launch_bounds__(kThreads) void init_normalize_kernel(InitArgs a)
+{
+    __shared__ __attribute__((aligned(16))) double buf[kThreads / kWave][kFoldLds];
+    const int wid = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const long row = static_cast<long>(blockIdx.x) * (kThreads / kWave) + wid;
+    if (row >= a.rows) return;
+    const long inst = row / a.P, member = row % a.P;
+    double *x = a.pop + (a.offset ? a.offset[inst] : 0) + static_cast<size_t>(member) * a.stride;
+    const int Kc = a.nsign * a.G;
+    const double scale = a.zeroth / wave_fold(x, a.nterm, Kc, a.G, buf[wid]);
+    for (int k = lane; k < Kc; k += kWave) x[k] *= scale;
+}
+
+}  // namespace
+
+hipError_t launch_initial_population(const InitArgs &a, hipStream_t s)
+{
+    const long items = a.rows * a.nsub;
+    hipLaunchKernelGGL(init_draw_kernel, dim3(static_cast<unsigned>((items + kThreads - 1) / kThreads)), dim3(kThreads),
+                       0, s, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !a.nterm) return e;
+    constexpr long per = kThreads / kWave;
+    hipLaunchKernelGGL(init_normalize_kernel, dim3(static_cast<unsigned>((a.rows + per - 1) / per)), dim3(kThreads), 0,
+                       s, a);
+    return hipGetLastError();
+}
+
+}  // namespace deac
