@@ -50,7 +50,7 @@ struct BatchModel {
     double *mterm = nullptr;               // [3][Lpad] first-moment, third-moment and normalization weights,
                                            // when moments or per-generation renormalization are used
     uint64_t *walk_rows = nullptr, *sub_tab = nullptr;
-    double *nterm = nullptr;               // [L] weights of the initial normalization, when used
+    double *nterm = nullptr;               // [L + 1] weights of the initial normalization, when used
     std::vector<uint64_t> skip_tab;        // nibble table of T^L, host side
     std::vector<size_t> insts;             // instances of this problem
     size_t init_row = 0, init_inst = 0;    // their part of deac_batch::init_start and init_off
@@ -366,7 +366,7 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     A(b.sig, m.T);
     A(b.walk_rows, rows.size());
     A(b.sub_tab, tabs.size());
-    if (m.normalize) A(b.nterm, m.Kc);
+    if (m.normalize) A(b.nterm, m.Kc + 1);
     // moment weights (deac.cpp:628-668, 728-768) and the normalization
     // weights of per-generation renormalization (deac.cpp:1342-1352), zero
     // past L

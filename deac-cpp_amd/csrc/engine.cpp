@@ -32,10 +32,9 @@ struct deac_handle {
     int device = 0;
     hipStream_t stream = nullptr;       // evolution
     hipStream_t draw_stream = nullptr;  // RNG walk, batches ahead of the evolution
-    int MG = 0, TB = 0, stride = 0, nwg = 0, chunk = 0, batch = 0, maxwg = 0;
-    bool overlap = false;               // walk beside the evolution (a CU is left free for it)
+    int MG = 0, TB = 0, stride = 0, rstride = 0, nwg = 0, chunk = 0, batch = 0;
     std::vector<void *> allocations;
-    double *kmat = nullptr, *nterm = nullptr, *fterm = nullptr, *tterm = nullptr, *obs = nullptr, *sig = nullptr;
+    double *kmat = nullptr, *ktile = nullptr, *nterm = nullptr, *fterm = nullptr, *tterm = nullptr, *obs = nullptr, *sig = nullptr;
     double *nfm_dt = nullptr;           // -1st-moment weights over tau (bdsf), or null
     double *pop0 = nullptr, *pop1 = nullptr, *fitness = nullptr, *cr_old = nullptr, *f_old = nullptr;
     double *emod = nullptr, *mom = nullptr;
@@ -265,39 +264,37 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     h->MG = (P + deac::kChainRows - 1) / deac::kChainRows;
     h->TB = (T + deac::kChainTau - 1) / deac::kChainTau;
     h->stride = round_up(Kc, deac::kChunk);
+    h->rstride = round_up(Kc, 2);
     h->chunk = (Kc + 63) / 64;
     // RNG batch: generations whose mask draws are buffered at once (<= 256 MiB
     // per buffer set).
-    const size_t per_gen = static_cast<size_t>(P) * Kc * sizeof(uint64_t);
+    const size_t per_gen = static_cast<size_t>(P) * h->rstride * sizeof(uint64_t);
     h->batch = static_cast<int>(std::clamp<size_t>((size_t(256) << 20) / per_gen, 1, 1024));
 
     const int maxwg = deac::evolve_max_workgroups(device);
     if (maxwg <= 0) return fail(DEAC_ERR_DEVICE);
-    h->maxwg = maxwg;
-    // At least one workgroup per chain task; beyond that, enough for the
-    // trial and selection phases (one per 512 trial items, 32 to 128: more
-    // cost more at every grid barrier than they save).
-    const size_t trial_items = static_cast<size_t>(P) * h->stride / 2;
-    int nwg = std::max(h->MG * h->TB, static_cast<int>(std::clamp<size_t>(trial_items / 512, 32, 128)));
-    const char *user_nwg = std::getenv("DEAC_EVOLVE_WORKGROUPS");
-    if (user_nwg) nwg = std::atoi(user_nwg);
-    h->nwg = std::clamp(nwg, 1, maxwg);
-    // Leave a CU to the walk when that costs no extra round of chain tasks:
-    // the walk then runs beside the evolution instead of in line.
-    const int tasks = h->MG * h->TB;
-    if (!user_nwg && h->nwg == maxwg && maxwg > 1 &&
-        (tasks + maxwg - 2) / (maxwg - 1) == (tasks + maxwg - 1) / maxwg)
-        h->nwg = maxwg - 1;
-    h->overlap = h->nwg < maxwg;
+    // One workgroup per chain task or moment fold (a chain wavefront alone on its CU takes
+    // 28 us at 8192 positions, three together 33), more where the trial phase
+    // has over 1024 pairs of positions for each (P = 8 at 8192 positions:
+    // 39.6 us per generation with 32 workgroups, 42.2 with 16, 40.0 with 64).
+    // One CU per XCD stays free for the walk: workgroups go to the XCDs in
+    // turn, and one that found its XCD full would hold up the grid barriers
+    // until the walk ends.
+    const size_t trial_pairs = static_cast<size_t>(P) * h->stride / 2;
+    const size_t folds = static_cast<size_t>(P) * (m.use_first + m.use_third);
+    size_t nwg = std::max(static_cast<size_t>(h->MG) * h->TB + folds, trial_pairs / 1024);
+    if (m.normalize && m.renormalize) nwg = std::max<size_t>(nwg, P);  // a workgroup renormalizes a member at a time
+    if (const char *user = std::getenv("DEAC_EVOLVE_WORKGROUPS")) nwg = std::max(std::atoi(user), 1);
+    h->nwg = static_cast<int>(std::clamp<size_t>(nwg, 1, std::max(maxwg - 8, 1)));
 
     // Device buffers.
-    const size_t kmat_n = static_cast<size_t>(h->TB) * deac::kChainTau * h->stride;
     const size_t pop_n = static_cast<size_t>(h->MG) * deac::kChainRows * h->stride;
     deac_status st = DEAC_OK;
     auto A = [&](auto *&ptr, size_t n) {
         if (st == DEAC_OK) st = h->alloc(ptr, n);
     };
-    A(h->kmat, kmat_n);
+    A(h->kmat, m.T * m.Kc);
+    A(h->ktile, deac::ktile_doubles(h->TB, h->stride));
     A(h->obs, T);
     A(h->sig, T);
     A(h->pop0, pop_n);
@@ -312,22 +309,19 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     A(h->iter, 4);
     for (int k = 0; k < 2; k++) {
         A(h->ctl[k], static_cast<size_t>(h->batch) * P);
-        A(h->raw[k], static_cast<size_t>(h->batch) * P * Kc);
+        A(h->raw[k], static_cast<size_t>(h->batch) * P * h->rstride);
         A(h->gen_start[k], static_cast<size_t>(h->batch) * 4);
     }
     A(h->state, 4);
     A(h->init_start, static_cast<size_t>(P) * 4);
     A(h->skip_rows, 256 * 4);
     A(h->lane_tab, static_cast<size_t>(64) * 64 * 16 * 4);
-    if (!m.nterm.empty()) A(h->nterm, Kc);
-    if (!m.fterm.empty()) A(h->fterm, Kc);
-    if (!m.tterm.empty()) A(h->tterm, Kc);
+    if (!m.nterm.empty()) A(h->nterm, Kc + 1);
+    if (!m.fterm.empty()) A(h->fterm, Kc + 1);
+    if (!m.tterm.empty()) A(h->tterm, Kc + 1);
     if (m.use_nfm) A(h->nfm_dt, T);
     if (st != DEAC_OK) return fail(st);
 
-    // K rows [tau][stride], zero padded to whole tau blocks and chunks.
-    std::vector<double> kl(kmat_n, 0.0);
-    for (size_t t = 0; t < m.T; t++) std::memcpy(&kl[t * h->stride], &m.kernel[t * m.Kc], m.Kc * sizeof(double));
     // Jump tables: T^(nsign*G) by rows for the walk, T^(l*chunk) by nibbles
     // for the mask generator.
     std::vector<uint64_t> rows(256 * 4), tabs(static_cast<size_t>(64) * 64 * 16 * 4);
@@ -344,7 +338,9 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     auto up = [&](void *dst, const void *src, size_t bytes) {
         if (st == DEAC_OK && hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) != hipSuccess) st = DEAC_ERR_DEVICE;
     };
-    up(h->kmat, kl.data(), kl.size() * sizeof(double));
+    up(h->kmat, m.kernel.data(), m.T * m.Kc * sizeof(double));
+    if (st == DEAC_OK && deac::launch_ktile(h->kmat, h->ktile, T, Kc, h->TB, h->stride, h->stream) != hipSuccess)
+        st = DEAC_ERR_DEVICE;
     up(h->obs, m.isf.data(), m.T * sizeof(double));
     up(h->sig, m.err.data(), m.T * sizeof(double));
     up(h->skip_rows, rows.data(), rows.size() * sizeof(uint64_t));
@@ -470,7 +466,10 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ea.nfm_error = m.nfm_error;
     ea.nfm_dt = h->nfm_dt;
     ea.fold_ks = m.bdsf;
+    ea.rstride = h->rstride;
+    ea.local = deac::evolve_local(ea.P, ea.T, nsign);
     ea.kmat = h->kmat;
+    ea.ktile = h->ktile;
     ea.nterm = h->nterm;
     ea.fterm = h->fterm;
     ea.tterm = h->tterm;
@@ -500,12 +499,12 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ma.P = static_cast<int>(P);
     ma.Kc = static_cast<int>(Kc);
     ma.chunk = h->chunk;
+    ma.rstride = h->rstride;
 
     // Generation loop: ii = 0 .. N-2 (deac.cpp:1138), in batches.  Batch b
     // uses buffer set b%2.  Its walk runs on the draw stream while batch b-1
-    // evolves (on a CU of its own: the walk kernel holds enough LDS that it
-    // cannot share one with an evolution workgroup), then its mask draws and
-    // its evolution run on the evolution stream; the mask kernel spreads over
+    // evolves, then its mask draws and its evolution run on the evolution
+    // stream; the mask kernel spreads over
     // every CU and costs less alone than beside the evolution.  The evolution
     // of b is queued before the host has read batch b-1's status.  Behind a
     // stop it changes nothing: the stop test sits at the top of a generation,
@@ -513,8 +512,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     // stops at its first generation (its status and its statistics entry,
     // past the stop, are never read).  Batches start at 8
     // generations and double up to the buffer size, so that the first walk,
-    // which nothing hides, is short.  When the evolution fills every CU the
-    // walk runs in line on the evolution stream.
+    // which nothing hides, is short.
     const size_t total = N - 1;
     std::vector<std::pair<size_t, int>> plan;  // first generation, generations
     for (size_t g = 0, len = std::min(8, h->batch); g < total;) {
@@ -523,8 +521,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         g += static_cast<size_t>(nb);
         len = std::min(2 * len, static_cast<size_t>(h->batch));
     }
-    // the split loop's kernels leave room on the CUs for the walk
-    hipStream_t d = split || h->overlap ? h->draw_stream : s;
+    hipStream_t d = h->draw_stream;
     auto draws = [&](size_t b) -> deac_status {
         const int k = static_cast<int>(b & 1);
         hipEvent_t *e = h->kev[k];

@@ -23,6 +23,7 @@
 
 #include "device_common.hpp"
 #include "evolve_common.hpp"
+#include "fold_common.hpp"
 #include "kernels.hpp"
 
 namespace deac {
@@ -30,7 +31,6 @@ namespace deac {
 namespace {
 
 constexpr int kWave = 64;
-constexpr int kEvoThreads = 256;
 constexpr int kEvoWaves = kEvoThreads / kWave;
 
 // Grid-wide barrier of the persistent evolution kernel.  The wait is
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256) void mask_kernel(MaskArgs a)
         o[3] ^= e[3];
     }
     for (int w = 0; w < 4; w++) s[w] = o[w];
-    uint64_t *raw = a.raw + wave * a.Kc;
+    uint64_t *raw = a.raw + wave * a.rstride;
     const int k0 = lane * a.chunk;
     for (int c2 = 0; c2 < a.chunk; c2++) {
         const uint64_t x = xnext(s);
@@ -204,217 +204,260 @@ __global__ __launch_bounds__(256) void mask_kernel(MaskArgs a)
 
 namespace {
 
-// LDS of the chain phase: kStages buffers of the kernel-matrix chunk
-// [16 tau][kChunk] and of the genome chunk [4 members][kChunk].  Rows are
-// padded by one pair so the 16 tau rows start on different banks.
-constexpr int kRowPad = kChunk + 2;
-constexpr int kKBuf = kChainTau * kRowPad;
-constexpr int kSBuf = kChainRows * kRowPad;
-constexpr int kChainLds = kStages * (kKBuf + kSBuf);
-
-// Register-staged copies of one chunk: 20 rows of 1 KB (kChunk doubles), 16
-// kernel-matrix rows then 4 genome rows, dealt round-robin to the helper
-// waves 1-3 (7, 7 and 6 rows); lane l moves bytes [16l, 16l+16) of a row.
-// Plain 16-byte loads into a ring of registers, kAhead chunks in flight per
-// wave, then ds_write_b128 into the chunk's LDS stage: LDS-DMA copies
-// (global_load_lds) stall at issue after a few are in flight per CU.
-constexpr int kCopiesPerChunk = kChainTau + kChainRows;
-constexpr int kHelperCopies = (kCopiesPerChunk + 2) / 3;
-constexpr int kAhead = 4;
-static_assert(kChunk == 128, "one copy per row: 64 lanes x 16 bytes");
-static_assert(kStages >= 2, "the chunk written at step ch must not be the one read at step ch");
-
 // Two doubles as a native vector: plain 16-byte loads and stores that stay
 // in registers (HIP's double2 struct is copied through memory).
 typedef double dvec2 __attribute__((ext_vector_type(2)));
+typedef uint64_t uvec2 __attribute__((ext_vector_type(2)));
 
-// A helper wave's copy rows (the same for the whole task, scalar): row j of
-// the wave is copy q = wid-1 + 3j of a chunk -- kernel row q (q < 16), genome
-// row q-16 (q < 20) or, for the third wave's seventh slot, none.  base: the
-// row's start in global memory (rows past the last timeslice, and the empty
-// slot, read the first kernel row; their values are discarded); off: the
-// row's offset in stage 0 of the LDS buffers, step: the stage stride.
-typedef __attribute__((address_space(1))) const dvec2 global_dvec2;
+// Chains: units of 8 positions, chunks of 16 units; K units in flight per
+// wavefront (one 16-byte load each, 17.6 ns a unit), genome units read ahead
+// from LDS, and the LDS of a wavefront: two chunks of 4 genome rows, padded
+// so that the rows start 8 banks apart.
+constexpr int kChunkUnits = kChunk / kUnit;
+constexpr int kRing = 2 * kChunkUnits;
+constexpr int kReadAhead = 4;
+constexpr int kSRow = kChunk + 4;
+constexpr int kChainLds = 2 * kChainRows * kSRow;
+static_assert(kChainLds >= kFoldLds, "a wave's LDS serves its folds as well");
+static_assert(kKtilePad >= kRing, "the K ring reads past the last unit");
+static_assert((kEvoWaves * kChainLds + kResidLds) * sizeof(double) <= kEvoLds, "chains and members' state fit in LDS");
 
-struct HelperRows {
-    const double *b0, *b1, *b2, *b3, *b4, *b5, *b6;
-    int o0, o1, o2, o3, o4, o5, o6;
-    int k0, k1, k2, k3, k4, k5, k6;  // stage stride of the row's buffer
-};
-
-__device__ __forceinline__ void helper_row(const EvoArgs &a, const double *const *srows, int tb, int q,
-                                           const double *&b, int &o, int &k)
+// One chunk of the chains: kr[h .. h+15] hold its K units and are refilled
+// with those two chunks on; sr holds the genome units about to be used.
+template <int H>
+__device__ __forceinline__ void chain_chunk(double &acc, dvec2 (&kr)[kRing], dvec2 (&sr)[kReadAhead], const dvec2 *&ka,
+                                            const double *here, const double *next)
 {
-    if (q < kChainTau) {
-        const int t = tb * kChainTau + q;
-        b = a.kmat + (t < a.T ? static_cast<size_t>(t) * a.stride : 0);
-        o = q * kRowPad;
-        k = kKBuf;
-    } else if (q < kCopiesPerChunk) {
-        b = srows[q - kChainTau];
-        o = kStages * kKBuf + (q - kChainTau) * kRowPad;
-        k = kSBuf;
-    } else {
-        b = a.kmat;
-        o = -1;
-        k = 0;
+#pragma unroll
+    for (int i = 0; i < kChunkUnits; i++) {
+        const dvec2 k = kr[H + i], s = sr[i % kReadAhead];
+        const int j = i + kReadAhead;
+        const double *p = j < kChunkUnits ? here + j * kUnit : next + (j - kChunkUnits) * kUnit;
+        // each load issues behind an MFMA, whose result the next one waits for
+        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.x, s.x, acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        sr[i % kReadAhead] = dvec2{p[0], p[4]};
+        __builtin_amdgcn_sched_barrier(0);
+        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.y, s.y, acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        kr[H + i] = ka[i * kWave];
+        __builtin_amdgcn_sched_barrier(0);
     }
+    ka += kChunkUnits * kWave;
 }
 
-__device__ __forceinline__ HelperRows helper_rows(const EvoArgs &a, const double *const *srows, int tb, int wid)
-{
-    HelperRows h;
-    helper_row(a, srows, tb, wid - 1, h.b0, h.o0, h.k0);
-    helper_row(a, srows, tb, wid + 2, h.b1, h.o1, h.k1);
-    helper_row(a, srows, tb, wid + 5, h.b2, h.o2, h.k2);
-    helper_row(a, srows, tb, wid + 8, h.b3, h.o3, h.k3);
-    helper_row(a, srows, tb, wid + 11, h.b4, h.o4, h.k4);
-    helper_row(a, srows, tb, wid + 14, h.b5, h.o5, h.k5);
-    helper_row(a, srows, tb, wid + 17, h.b6, h.o6, h.k6);
-    return h;
-}
-
-// One ring slot: a helper wave's 7 rows of one chunk, in named registers (no
-// array, so nothing is indexed at run time).
-struct RowRing {
-    dvec2 v0, v1, v2, v3, v4, v5, v6;
-};
-static_assert(kHelperCopies == 7, "RowRing holds 7 rows");
-
-__device__ __forceinline__ dvec2 load_row(const double *base, int chunk, int lane)
-{
-    // (a global-address-space pointer: a flat load would also count against
-    // the LDS counter, which the helpers drain before every barrier)
-    return ((global_dvec2 *)(base + static_cast<size_t>(chunk) * kChunk))[lane];
-}
-
-__device__ __forceinline__ void store_row(double *lds, int stage, int off, int step, int lane, const dvec2 &v)
-{
-    if (off >= 0) reinterpret_cast<dvec2 *>(lds + off + stage * step)[lane] = v;
-}
-
-__device__ __forceinline__ void load_chunk(const HelperRows &h, int chunk, int lane, RowRing &r)
-{
-    r.v0 = load_row(h.b0, chunk, lane);
-    r.v1 = load_row(h.b1, chunk, lane);
-    r.v2 = load_row(h.b2, chunk, lane);
-    r.v3 = load_row(h.b3, chunk, lane);
-    r.v4 = load_row(h.b4, chunk, lane);
-    r.v5 = load_row(h.b5, chunk, lane);
-    r.v6 = load_row(h.b6, chunk, lane);
-}
-
-__device__ __forceinline__ void store_chunk(double *lds, int stage, const HelperRows &h, int lane, const RowRing &r)
-{
-    store_row(lds, stage, h.o0, h.k0, lane, r.v0);
-    store_row(lds, stage, h.o1, h.k1, lane, r.v1);
-    store_row(lds, stage, h.o2, h.k2, lane, r.v2);
-    store_row(lds, stage, h.o3, h.k3, lane, r.v3);
-    store_row(lds, stage, h.o4, h.k4, lane, r.v4);
-    store_row(lds, stage, h.o5, h.k5, lane, r.v5);
-    store_row(lds, stage, h.o6, h.k6, lane, r.v6);
-}
-
-// Workgroup barrier for the chunk pipeline.  Every wave retires what the
-// others depend on before arriving: the helpers their LDS writes, the
-// compute wave its LDS reads (DEAC_WAIT_LDS).
-__device__ __forceinline__ void chunk_barrier()
-{
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-// Model ISF E[i][t] of one (tau block, member group) task; the whole
-// workgroup takes part: wave 0 runs the chains, waves 1-3 stage chunks.
+// Model ISF E[i][t] of one (tau block, member group) task on one wavefront:
 // E = sum over the concatenated genome (positive sign, then negative sign)
 // as one sequential FMA chain per (member, tau) starting from zero
-// (matrix_multiply_LxM_by_MxN called twice, deac.cpp:1386-1394).
-__device__ void chain_task(const EvoArgs &a, double *lds, int tb, int mg, bool init)
+// (matrix_multiply_LxM_by_MxN called twice, deac.cpp:1386-1394), 64 chains
+// (16 tau x 4 members) advanced 4 positions per v_mfma_f64_4x4x4_4b_f64, which
+// is bit for bit four fused multiply-adds in ascending position order: block b
+// holds tau rows 4b..4b+3 of the task, every block the same 4 members.  A:
+// lane l holds tau row l&15 at position l>>4 of the MFMA's four; B: member l&3
+// at the same position (the same for the four blocks).  buf: kChainLds
+// doubles of LDS of this wavefront.
+//
+// Bound: the chain, 8.8 ns per dependent MFMA (18 us at 8192 positions).  The
+// wavefront brings its own operands: K, tiled in operand order, straight
+// into a ring of registers, the genome rows by coalesced loads through LDS,
+// which puts them in operand order.  Nothing is shared between wavefronts, so
+// no barrier sits in the chain.  Measured per 8 positions: the MFMAs alone
+// 17.2 ns, genome operands loaded lane by lane from the rows 25 (75 with four
+// wavefronts on the CU, the L1 takes 45 cycles for such a load), 16-byte genome
+// loads put in order by v_permlane swaps 45, chunks staged by helper
+// wavefronts with a barrier per 128 positions 34.
+__device__ __forceinline__ void chain_task(const EvoArgs &a, const double *r0, const double *r1, const double *r2,
+                                           const double *r3, int tb, int mg, double *buf)
 {
-    // the wave index as a scalar: every per-row choice below is then uniform
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
-    __shared__ const double *srows[kChainRows];
-    if (threadIdx.x < kChainRows) srows[threadIdx.x] = chain_row(a, mg * kChainRows + threadIdx.x, init);
-    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1);
     const int nchunk = a.stride / kChunk;
-    // Chunk c travels in ring slot c % kAhead (r0..r3); at step ch the
-    // helpers write chunk ch+1 into LDS stage (ch+1) % kStages and load chunk
-    // ch+1+kAhead into the slot it left.  Loads past the last chunk re-read
-    // it; the steps run to a multiple of kAhead (the extra ones only meet at
-    // the barrier), so every load is unconditional.
-    static_assert(kAhead == 4, "four ring slots r0..r3");
-    // The compute wave and the helpers run loops of their own, each meeting
-    // the other at one barrier per step (the same count: the steps run to a
-    // multiple of kAhead).
-    const int nsteps = (nchunk + kAhead - 1) / kAhead * kAhead;
+    const dvec2 *ka = reinterpret_cast<const dvec2 *>(a.ktile) +
+                      static_cast<size_t>(tb) * nchunk * kChunkUnits * kWave + lane;
+    struct Stage {
+        dvec2 v0, v1, v2, v3;
+    };
+    auto load = [&](int c, Stage &r) __attribute__((always_inline)) {
+        const int k = min(c, nchunk - 1) * kChunk + 2 * lane;
+        r.v0 = *reinterpret_cast<const dvec2 *>(r0 + k);
+        r.v1 = *reinterpret_cast<const dvec2 *>(r1 + k);
+        r.v2 = *reinterpret_cast<const dvec2 *>(r2 + k);
+        r.v3 = *reinterpret_cast<const dvec2 *>(r3 + k);
+    };
+    auto put = [&](int c, const Stage &r) __attribute__((always_inline)) {
+        double *p = buf + (c & 1) * (kChainRows * kSRow) + 2 * lane;
+        *reinterpret_cast<dvec2 *>(p) = r.v0;
+        *reinterpret_cast<dvec2 *>(p + kSRow) = r.v1;
+        *reinterpret_cast<dvec2 *>(p + 2 * kSRow) = r.v2;
+        *reinterpret_cast<dvec2 *>(p + 3 * kSRow) = r.v3;
+    };
+    const double *even = buf + (lane & 3) * kSRow + (lane >> 4), *odd = even + kChainRows * kSRow;
+    Stage s0, s1;
+    dvec2 kr[kRing], sr[kReadAhead];
+    load(0, s0);
+    load(1, s1);
+#pragma unroll
+    for (int i = 0; i < kRing; i++) kr[i] = ka[i * kWave];
+    ka += kRing * kWave;
+    __builtin_amdgcn_sched_barrier(0);
+    put(0, s0);
+    load(2, s0);
+#pragma unroll
+    for (int j = 0; j < kReadAhead; j++) sr[j] = dvec2{even[j * kUnit], even[j * kUnit + 4]};
     double acc = 0.0;
-    if (wid == 0) {
-        chunk_barrier();  // chunk 0 staged
-        for (int ch = 0; ch < nsteps; ch++) {
-            if (ch < nchunk) {
-                // 64 chains (16 tau x 4 members) advanced 4 positions per
-                // v_mfma_f64_4x4x4_4b_f64, which is bit for bit four fused
-                // multiply-adds in ascending position order: block b holds
-                // tau rows 4b..4b+3 of the task, every block the same 4
-                // members.  A: lane l reads tau row l&15 at position
-                // j + (l>>4); B: member l&3 at the same position (a broadcast
-                // across the blocks).
-                const int st = ch % kStages;
-                const double *kb = lds + st * kKBuf + (lane & 15) * kRowPad + (lane >> 4);
-                const double *sb = lds + kStages * kKBuf + st * kSBuf + (lane & 3) * kRowPad + (lane >> 4);
-                double ka[kChunk / 4], sa[kChunk / 4];
-#pragma unroll
-                for (int j = 0; j < kChunk / 4; j++) {
-                    ka[j] = kb[4 * j];
-                    sa[j] = sb[4 * j];
-                }
-#pragma unroll
-                for (int j = 0; j < kChunk / 4; j++) acc = __builtin_amdgcn_mfma_f64_4x4x4f64(ka[j], sa[j], acc, 0, 0, 0);
-                DEAC_WAIT_LDS();  // the stage may be refilled after the barrier
-            }
-            chunk_barrier();
+    for (int c = 0;; c += 2) {
+        put(c + 1, s1);
+        load(c + 3, s1);
+        chain_chunk<0>(acc, kr, sr, ka, even, odd);
+        if (c + 1 >= nchunk) break;
+        put(c + 2, s0);
+        load(c + 4, s0);
+        chain_chunk<kChunkUnits>(acc, kr, sr, ka, odd, even);
+        if (c + 2 >= nchunk) break;
+    }
+    // 4x4x4_4b output: lane l holds row l>>4 of block (l>>2)&3, column l&3
+    const int i = mg * kChainRows + (lane & 3), t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
+    if (i < a.P && t < a.T) a.emod[static_cast<size_t>(i) * a.T + t] = acc;
+}
+
+// The state of the members as one workgroup sees it: in its LDS, where every
+// workgroup repeats the selection (EvoArgs::local), or in global memory.
+struct Members {
+    double *fitness, *cr, *f;  // [P], [P][nsign], [P][nsign]
+    int *cur;                  // [P]
+};
+
+__device__ __forceinline__ const double *row_of(const EvoArgs &a, const int *cur, int i, bool spare)
+{
+    return ((cur[i] != 0) != spare ? a.pop1 : a.pop0) + static_cast<size_t>(i) * a.stride;
+}
+
+__device__ __forceinline__ void control(const EvoArgs &a, const Members &s, const MemberCtl &c, int i, int sg,
+                                        double &cr, double &f)
+{
+    cr = (c.flags >> (2 * sg)) & 1 ? c.cr_value[sg] : s.cr[i * a.nsign + sg];
+    f = (c.flags >> (2 * sg + 1)) & 1 ? c.f_value[sg] : s.f[i * a.nsign + sg];
+}
+
+// u < cr for the draw u = r 2^-53, as r < ceil(cr 2^53) in whole numbers
+__device__ __forceinline__ uint64_t cross_limit(double cr)
+{
+    return !(cr > 0.0) ? 0 : cr >= 1.0 ? UINT64_C(1) << 53 : static_cast<uint64_t>(ceil(cr * 0x1.0p53));
+}
+
+// Trial vectors of one member over genome blocks [b0, b1) of 128 positions,
+// two per lane, into its spare row (deac.cpp:1261-1308); the padding stays
+// zero.  The parent, donor and draw values are all loaded, whichever the
+// crossover keeps, so the loads issue together instead of behind the
+// comparison, and those of two blocks are in flight at once.
+// Bound: memory (40 bytes read and 8 written per position).
+__device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s, const MemberCtl &c,
+                                             const uint64_t *raw, int i, int b0, int b1)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    double cr, f0, f1;
+    control(a, s, c, i, 0, cr, f0);
+    const uint64_t lim0 = cross_limit(cr);
+    f1 = f0;
+    if (a.nsign == 2) control(a, s, c, i, 1, cr, f1);
+    const uint64_t lim1 = cross_limit(cr);
+    const double *r1 = row_of(a, s.cur, c.mutant[0], false), *r2 = row_of(a, s.cur, c.mutant[1], false);
+    const double *r3 = row_of(a, s.cur, c.mutant[2], false), *rp = row_of(a, s.cur, i, false);
+    double *out = const_cast<double *>(row_of(a, s.cur, i, true));
+    struct Load {
+        uvec2 u;
+        dvec2 x1, x2, x3, xp;
+    };
+    auto load = [&](int b, Load &v) __attribute__((always_inline)) {
+        const int k = b * kChunk + 2 * lane;
+        if (k < a.Kc) v.u = *reinterpret_cast<const uvec2 *>(raw + k);
+        v.x1 = *reinterpret_cast<const dvec2 *>(r1 + k);
+        v.x2 = *reinterpret_cast<const dvec2 *>(r2 + k);
+        v.x3 = *reinterpret_cast<const dvec2 *>(r3 + k);
+        v.xp = *reinterpret_cast<const dvec2 *>(rp + k);
+    };
+    auto value = [&](bool neg, uint64_t r, double d1, double d2, double d3, double p) __attribute__((always_inline)) {
+        const double w = fma(neg ? f1 : f0, d2 - d3, d1);
+        return r < (neg ? lim1 : lim0) ? (a.allow_neg ? w : fabs(w)) : p;
+    };
+    auto store = [&](int b, const Load &v) __attribute__((always_inline)) {
+        const int k = b * kChunk + 2 * lane;
+        dvec2 o = {0.0, 0.0};
+        if (k < a.Kc) o.x = value(k >= a.G, v.u.x, v.x1.x, v.x2.x, v.x3.x, v.xp.x);
+        if (k + 1 < a.Kc) o.y = value(k + 1 >= a.G, v.u.y, v.x1.y, v.x2.y, v.x3.y, v.xp.y);
+        // the negative sign's zero frequency repeats the positive one's
+        if (a.nsign == 2 && (k == a.G || k + 1 == a.G)) {
+            const double z = value(false, raw[0], r1[0], r2[0], r3[0], rp[0]);
+            if (k == a.G) o.x = z;
+            else o.y = z;
         }
-    } else {
-        RowRing r0, r1, r2, r3;
-        const HelperRows hr = helper_rows(a, srows, tb, wid);
-        const int last = nchunk - 1;
-        load_chunk(hr, 0, lane, r0);
-        load_chunk(hr, min(1, last), lane, r1);
-        load_chunk(hr, min(2, last), lane, r2);
-        load_chunk(hr, min(3, last), lane, r3);
-        store_chunk(lds, 0, hr, lane, r0);
-        load_chunk(hr, min(kAhead, last), lane, r0);
-        DEAC_WAIT_LDS();
-        chunk_barrier();
-        // step ch: chunk ch+1 into LDS stage (ch+1) % kStages, then chunk
-        // ch+1+kAhead into the ring slot it left
-        auto step = [&](int ch, RowRing &rs) __attribute__((always_inline)) {
-            if (ch + 1 < nchunk) store_chunk(lds, (ch + 1) % kStages, hr, lane, rs);
-            load_chunk(hr, min(ch + 1 + kAhead, last), lane, rs);
-            DEAC_WAIT_LDS();  // chunk ch+1 is in LDS before the barrier
-            chunk_barrier();
-        };
-        for (int ch0 = 0; ch0 < nsteps; ch0 += kAhead) {
-            step(ch0, r1);
-            step(ch0 + 1, r2);
-            step(ch0 + 2, r3);
-            step(ch0 + 3, r0);
+        *reinterpret_cast<dvec2 *>(out + k) = o;
+    };
+    int b = b0;
+    for (; b + 1 < b1; b += 2) {
+        Load v0 = {}, v1 = {};
+        load(b, v0);
+        load(b + 1, v1);
+        store(b, v0);
+        store(b + 1, v1);
+    }
+    if (b < b1) {
+        Load v0 = {};
+        load(b, v0);
+        store(b, v0);
+    }
+}
+
+// Sums d[0..n) squared in tau order from LDS, the last one fused when fused
+// is set (deac.cpp:120-126); 8 reads ahead of the adds.
+__device__ __forceinline__ double chi_sum(const double *d, int n, bool fused, double acc)
+{
+    const int m = fused ? n - 1 : n;
+    int t = 0;
+    for (; t + 8 <= m; t += 8) {
+        double v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = d[t + e];
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc = acc + v[e] * v[e];
+    }
+    for (; t < m; t++) acc = acc + d[t] * d[t];
+    if (fused) acc = fma(d[n - 1], d[n - 1], acc);
+    return acc;
+}
+
+// Member i's fitness from its chi^2 sum (deac.cpp:957-976, 1539-1555) and
+// the greedy selection (deac.cpp:1556-1571), by one lane.
+__device__ __forceinline__ void select_member(const EvoArgs &a, const Members &s, int g, int i, double chi, bool init)
+{
+    double fit = chi / static_cast<double>(a.T);
+    if (a.use_first) {
+        const double d = a.mom[i * 4 + 1] - a.first_moment;
+        fit += (d * d) / a.first_moment;
+    }
+    if (a.use_third) {
+        const double q = (a.third_moment - a.mom[i * 4 + 2]) / a.third_moment_error;
+        fit = fma(q, q, fit);
+    }
+    if (init) {
+        s.fitness[i] = fit;
+    } else if (fit <= s.fitness[i]) {
+        const MemberCtl &c = a.ctl[static_cast<size_t>(g) * a.P + i];
+        s.fitness[i] = fit;
+        s.cur[i] ^= 1;
+        for (int sg = 0; sg < a.nsign; sg++) {
+            double cr, f;
+            control(a, s, c, i, sg, cr, f);
+            s.cr[i * a.nsign + sg] = cr;
+            s.f[i * a.nsign + sg] = f;
         }
     }
-    if (wid == 0) {
-        // 4x4x4_4b output: lane l holds row l>>4 of block (l>>2)&3, column l&3
-        const int i = mg * kChainRows + (lane & 3), t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
-        if (i < a.P && t < a.T) a.emod[static_cast<size_t>(i) * a.T + t] = acc;
-    }
-    __syncthreads();
 }
 
 }  // namespace
 
 // Phase timestamps (s_memtime) of workgroup 0, compiled in only for
 // profiling builds: slot 0 top of generation, 1 after the trial barrier,
-// 2 after the chain barrier, 3 after the selection barrier.
+// 2 after the chain barrier, 3 after the selection.
 #ifdef DEAC_PHASE_TIMERS
 __device__ unsigned long long deac_phase_clock[4];
 #define DEAC_PHASE(slot)                                                                      \
@@ -431,30 +474,56 @@ __device__ unsigned long long deac_phase_clock[4];
     } while (0)
 #endif
 
-// One workgroup per CU (its LDS fills the CU), so one wave per SIMD: the
-// register file is the wave's, and the helpers' row ring fits beside the rest.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void evolve_kernel(EvoArgs a)
+// Per generation: trial vectors, barrier, chains and moment rows, barrier,
+// selection.  Where the population's residuals fit in LDS (a.local) every
+// workgroup repeats the whole selection and keeps the members' state itself,
+// which saves the third barrier: a grid barrier costs from 1 us (10
+// workgroups) to 8 us (255, the cache fences of an XCD's workgroups queue),
+// a repeated selection of 8 members 1.3 us.  One workgroup per CU is launched
+// (evolve_max_workgroups); a second handle's workgroup still fits beside it.
+__global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a)
 {
 #ifdef DEAC_PHASE_TIMERS
     unsigned long long phase_t0 = 0;
 #endif
-    extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte aligned: ds_write_b128
-    __shared__ double dsh[kEvoWaves][kWave];
+    extern __shared__ __attribute__((aligned(16))) double lds[];
     __shared__ int stop_flag;
+    __shared__ double scale;
     const int lane = threadIdx.x & (kWave - 1);
-    const int wid = threadIdx.x / kWave;
+    // the wave index as a scalar: what depends on it alone is then uniform
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int nwg = gridDim.x;
     const int total_waves = nwg * kEvoWaves;
     // Waves are numbered wave-slot-major so that consecutive tasks land on
     // different workgroups (and CUs).
     const int gwave = wid * nwg + blockIdx.x;
-    const size_t gthread = static_cast<size_t>(blockIdx.x) * kEvoThreads + threadIdx.x;
-    const size_t nthreads = static_cast<size_t>(nwg) * kEvoThreads;
     unsigned target = 0;
     const int nchain = a.MG * a.TB;
-    const int mgrp = (a.P + 7) / 8;  // moment tasks: 8 members x {first, third} per wave
-    const int nmom = (a.use_first || a.use_third) ? mgrp : 0;
-    const int half = a.stride / 2;
+    const int nmom = a.use_first + a.use_third;  // moment folds per member
+    const int ntask = nchain + nmom * a.P;
+    const int nblk = a.stride / kChunk;
+    const int run = static_cast<int>(
+        min(max(static_cast<long>(a.P) * nblk / total_waves, 1L), static_cast<long>(min(nblk, 8))));
+    const int runs = (nblk + run - 1) / run;  // per member
+    const int Tp = a.T | 1;  // odd row stride: lanes of different members read different banks
+
+    Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
+    double *resid = lds + kEvoWaves * kChainLds;  // [P][Tp] residuals (a.local), behind the chains' buffers
+    if (a.local) {
+        s.fitness = resid + static_cast<size_t>(a.P) * Tp;
+        s.cr = s.fitness + a.P;
+        s.f = s.cr + a.P * a.nsign;
+        s.cur = reinterpret_cast<int *>(s.f + a.P * a.nsign);
+        for (int i = threadIdx.x; i < a.P; i += kEvoThreads) {
+            s.cur[i] = a.cur[i];
+            s.fitness[i] = a.fitness[i];
+            for (int sg = 0; sg < a.nsign; sg++) {
+                s.cr[i * a.nsign + sg] = a.cr_old[i * a.nsign + sg];
+                s.f[i * a.nsign + sg] = a.f_old[i * a.nsign + sg];
+            }
+        }
+    }
+    __syncthreads();
 
     for (int g = 0; g <= a.ngen; g++) {
         const bool init = a.init_mode != 0;
@@ -462,27 +531,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             if (g == a.ngen) break;
             DEAC_PHASE(0);
             // Top of the generation: best fitness, statistics, stop test
-            // (deac.cpp:1145-1166).  The fitnesses are staged in LDS with one
-            // coalesced load (the chain buffers are idle here) and scanned
-            // by thread 0 in the reference's order.
-            auto top = [&](const double *fit) __attribute__((always_inline)) {
-                double mn = fit[0];
-                for (int i = 0; i < a.P; i++)
-                    if (fit[i] < mn) mn = fit[i];
-                const long ii = a.gen0 + g;
-                if (blockIdx.x == 0 && a.track_stats) {
-                    double s = 0.0;
-                    for (int i = 0; i < a.P; i++) s += fit[i];
-                    double q = 0.0;
-                    const int p4 = a.P & ~3;
-                    for (int i = 0; i < a.P; i++) {
-                        const double v = fit[i];
-                        if (i < p4) q = q + v * v;
-                        else q = fma(v, v, q);
+            // (deac.cpp:1145-1166), scanned by one thread in the reference's
+            // order, 8 values read ahead; the statistics by workgroup 0 only.
+            const double *fit = s.fitness;
+            if (!a.local && a.P <= kResidLds) {
+                for (int i = threadIdx.x; i < a.P; i += kEvoThreads) lds[i] = a.fitness[i];
+                fit = lds;
+                __syncthreads();
+            }
+            if (threadIdx.x == 0) {
+                double mn = fit[0], sum = 0.0, sq = 0.0;
+                const int p4 = a.P & ~3;
+                for (int i0 = 0; i0 < a.P; i0 += 8) {
+                    double v[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] = fit[min(i0 + e, a.P - 1)];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        if (i0 + e >= a.P) break;
+                        if (v[e] < mn) mn = v[e];
+                        sum = sum + v[e];
+                        sq = i0 + e < p4 ? sq + v[e] * v[e] : fma(v[e], v[e], sq);
                     }
-                    a.stats[ii] = s / static_cast<double>(a.P);
+                }
+                if (blockIdx.x == 0 && a.track_stats) {
+                    const long ii = a.gen0 + g;
+                    a.stats[ii] = sum / static_cast<double>(a.P);
                     a.stats[a.stats_len + ii] = mn;
-                    a.stats[2 * a.stats_len + ii] = q / static_cast<double>(a.P);
+                    a.stats[2 * a.stats_len + ii] = sq / static_cast<double>(a.P);
                 }
                 const bool stop = mn <= a.stop;
                 if (stop && blockIdx.x == 0) {
@@ -490,128 +566,123 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                     a.status[1] = g;
                 }
                 stop_flag = stop ? 1 : 0;
-            };
-            if (a.P <= kChainLds) {
-                for (int i = threadIdx.x; i < a.P; i += kEvoThreads) lds[i] = a.fitness[i];
-                __syncthreads();
-                if (threadIdx.x == 0) top(lds);
-            } else if (threadIdx.x == 0) {
-                top(a.fitness);
             }
             __syncthreads();
             if (stop_flag) break;
 
-            // Trial vectors into each member's spare buffer, two genome
-            // positions per work item; the padding stays zero.
+            // Trial vectors into each member's spare buffer: a wave takes runs
+            // of up to 8 blocks of one member, whose controls it then reads
+            // once; shorter runs where they would leave waves without work.
             const MemberCtl *ctlg = a.ctl + static_cast<size_t>(g) * a.P;
-            const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.Kc;
-            const size_t items = static_cast<size_t>(a.P) * half;
-            for (size_t it = gthread; it < items; it += nthreads) {
-                const int i = static_cast<int>(it / half);
-                const int kp = static_cast<int>(it % half);
-                const MemberCtl &c = ctlg[i];
-                const uint64_t *raw = rawg + static_cast<size_t>(i) * a.Kc;
-                double v[2];
-                for (int e = 0; e < 2; e++) {
-                    const int k = 2 * kp + e;
-                    if (k >= a.Kc) v[e] = 0.0;
-                    else if (a.nsign == 2 && k == a.G) v[e] = trial_value(a, c, raw, i, 0);  // deac.cpp:1305-1308
-                    else v[e] = trial_value(a, c, raw, i, k);
+            const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.rstride;
+            if (!a.renorm) {
+                for (int it = gwave; it < a.P * runs; it += total_waves) {
+                    const int i = it / runs, b0 = it % runs * run;
+                    trial_blocks(a, s, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, min(b0 + run, nblk));
                 }
-                double *dst = (a.cur[i] ? a.pop0 : a.pop1) + static_cast<size_t>(i) * a.stride;
-                *reinterpret_cast<double2 *>(dst + 2 * kp) = make_double2(v[0], v[1]);
+            } else {
+                // With per-generation renormalization (deac.cpp:1342-1364) a
+                // workgroup takes whole members: it forms the trial, folds
+                // its zeroth moment on one wave and scales it.
+                const int share = (nblk + kEvoWaves - 1) / kEvoWaves;
+                for (int i = blockIdx.x; i < a.P; i += nwg) {
+                    const int b0 = min(wid * share, nblk), b1 = min(b0 + share, nblk);
+                    trial_blocks(a, s, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, b1);
+                    double *x = const_cast<double *>(row_of(a, s.cur, i, true));
+                    __builtin_amdgcn_s_waitcnt(0);
+                    __syncthreads();
+                    if (wid == 0) {
+                        const double norm = wave_fold(x, a.nterm, a.Kc, a.G, lds);
+                        if (lane == 0) scale = a.zeroth / norm;
+                    }
+                    __syncthreads();
+                    for (int b = b0; b < b1; b++) {
+                        dvec2 *p2 = reinterpret_cast<dvec2 *>(x) + b * (kChunk / 2) + lane;
+                        *p2 = *p2 * scale;
+                    }
+                    __syncthreads();
+                }
             }
             if (!grid_barrier(a.bar, target, a.status)) return;
             DEAC_PHASE(1);
-
-            if (a.renorm) {
-                // Per-generation renormalization (deac.cpp:1342-1364).
-                for (int i = gwave; i < a.P; i += total_waves)
-                    if (lane == 0) {
-                        const double *src = (a.cur[i] ? a.pop0 : a.pop1) + static_cast<size_t>(i) * a.stride;
-                        a.mom[i * 4 + 0] = fold_row(src, a.nterm, a.Kc, a.G);
-                    }
-                if (!grid_barrier(a.bar, target, a.status)) return;
-                for (size_t it = gthread; it < items; it += nthreads) {
-                    const int i = static_cast<int>(it / half);
-                    const int kp = static_cast<int>(it % half);
-                    double *dst = (a.cur[i] ? a.pop0 : a.pop1) + static_cast<size_t>(i) * a.stride;
-                    double2 *p2 = reinterpret_cast<double2 *>(dst + 2 * kp);
-                    double2 v = *p2;
-                    const double scale = a.zeroth / a.mom[i * 4 + 0];
-                    v.x *= scale;
-                    v.y *= scale;
-                    *p2 = v;
-                }
-                if (!grid_barrier(a.bar, target, a.status)) return;
-            }
         }
 
-        // Model ISF chains (one workgroup per task) and moment rows.
-        for (int task = blockIdx.x; task < nchain; task += nwg) chain_task(a, lds, task % a.TB, task / a.TB, init);
-        for (int task = gwave; task < nmom; task += total_waves) {
-            const int il = lane & 7, rr = lane >> 3;
-            const int i = task * 8 + il;
-            if (i < a.P && rr < 2) {
-                const double *row = rr == 0 ? a.fterm : a.tterm;
-                const bool used = rr == 0 ? a.use_first : a.use_third;
-                if (used) a.mom[i * 4 + 1 + rr] = fold_row(chain_row(a, i, init), row, a.Kc, a.G);
+        // Model ISF chains and moment rows, one wave per task: of the trials,
+        // or of the current genomes for the initial fitness.
+        for (int task = gwave; task < ntask; task += total_waves) {
+            double *buf = lds + wid * kChainLds;
+            if (task < nchain) {
+                const int tb = task % a.TB, mg = task / a.TB;
+                auto row = [&](int m) { return row_of(a, s.cur, min(mg * kChainRows + m, a.P - 1), !init); };
+                chain_task(a, row(0), row(1), row(2), row(3), tb, mg, buf);
+            } else {
+                const int i = (task - nchain) / nmom;
+                const bool third = !a.use_first || (task - nchain) % nmom != 0;
+                const double m = wave_fold(row_of(a, s.cur, i, !init), third ? a.tterm : a.fterm, a.Kc, a.G, buf);
+                if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }
         }
         if (!grid_barrier(a.bar, target, a.status)) return;
         DEAC_PHASE(2);
 
-        // Fitness and greedy selection, one wavefront per member
-        // (deac.cpp:1539-1572; initial fitness deac.cpp:957-976).
-        for (int i = gwave; i < a.P; i += total_waves) {
-            double chi = 0.0;
-            const int tlast = (a.T & 1) ? a.T - 1 : -1;  // fused element of the reduction
-            for (int t0 = 0; t0 < a.T; t0 += kWave) {
-                const int t = t0 + lane;
-                double d = 0.0;
-                if (t < a.T) d = (a.obs[t] - a.emod[static_cast<size_t>(i) * a.T + t]) / a.sig[t];
-                dsh[wid][lane] = d;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                if (lane == 0) {
-                    const int n = min(kWave, a.T - t0);
-                    for (int u = 0; u < n; u++) {
-                        const double du = dsh[wid][u];
-                        if (t0 + u == tlast) chi = fma(du, du, chi);
-                        else chi = chi + du * du;
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
+        // Fitness and greedy selection.
+        if (a.local) {
+            const int total = a.P * a.T;
+            for (int idx = threadIdx.x; idx < total; idx += kEvoThreads) {
+                const int i = idx / a.T, t = idx % a.T;
+                resid[i * Tp + t] = (a.obs[t] - a.emod[idx]) / a.sig[t];
             }
-            if (lane == 0) {
-                double fit = chi / static_cast<double>(a.T);
-                if (a.use_first) {
-                    const double d = a.mom[i * 4 + 1] - a.first_moment;
-                    fit += (d * d) / a.first_moment;
+            __syncthreads();
+            for (int i = threadIdx.x; i < a.P; i += kEvoThreads)
+                select_member(a, s, g, i, chi_sum(resid + i * Tp, a.T, a.T & 1, 0.0), init);
+            __syncthreads();
+        } else {
+            // one wavefront per member, residuals in windows of kResidWave
+            double *d = lds + wid * kResidWave;
+            for (int i = gwave; i < a.P; i += total_waves) {
+                double chi = 0.0;
+                for (int t0 = 0; t0 < a.T; t0 += kResidWave) {
+                    const int n = min(kResidWave, a.T - t0);
+                    for (int u = lane; u < n; u += kWave)
+                        d[u] = (a.obs[t0 + u] - a.emod[static_cast<size_t>(i) * a.T + t0 + u]) / a.sig[t0 + u];
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    chi = chi_sum(d, n, (a.T & 1) && t0 + n == a.T, chi);
+                    __builtin_amdgcn_wave_barrier();
                 }
-                if (a.use_third) {
-                    const double q = (a.third_moment - a.mom[i * 4 + 2]) / a.third_moment_error;
-                    fit = fma(q, q, fit);
-                }
-                if (init) {
-                    a.fitness[i] = fit;
-                } else if (fit <= a.fitness[i]) {
-                    const MemberCtl &c = a.ctl[static_cast<size_t>(g) * a.P + i];
-                    a.fitness[i] = fit;
-                    a.cur[i] ^= 1;
-                    for (int sg = 0; sg < a.nsign; sg++) {
-                        double cr, f;
-                        control_of(a, c, i, sg, cr, f);
-                        a.cr_old[i * a.nsign + sg] = cr;
-                        a.f_old[i * a.nsign + sg] = f;
-                    }
-                }
+                if (lane == 0) select_member(a, s, g, i, chi, init);
             }
+            if (!grid_barrier(a.bar, target, a.status)) return;
         }
-        if (!grid_barrier(a.bar, target, a.status)) return;
         DEAC_PHASE(3);
         if (init) break;
+    }
+    if (a.local && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < a.P; i += kEvoThreads) {
+            a.cur[i] = s.cur[i];
+            a.fitness[i] = s.fitness[i];
+            for (int sg = 0; sg < a.nsign; sg++) {
+                a.cr_old[i * a.nsign + sg] = s.cr[i * a.nsign + sg];
+                a.f_old[i * a.nsign + sg] = s.f[i * a.nsign + sg];
+            }
+        }
+}
+
+// K rows [T][Kc] into the chains' operand order: [tau block][unit of 8
+// positions][lane][2], lane l holding tau row l&15 at positions l>>4 and
+// (l>>4)+4 of the unit.  Past T and Kc -0.0: with genomes padded with +0.0
+// the products are -0.0 and leave every chain exactly as it is.
+__global__ __launch_bounds__(256) void ktile_kernel(const double *rows, double *ktile, int T, int Kc, int TB, int nunit)
+{
+    const size_t total = (static_cast<size_t>(TB) * nunit + kKtilePad) * kWave * 2;
+    for (size_t o = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; o < total;
+         o += static_cast<size_t>(gridDim.x) * 256) {
+        const int e = static_cast<int>(o & 1), l = static_cast<int>((o >> 1) & (kWave - 1));
+        const size_t tu = o >> 7;
+        const int t = static_cast<int>(tu / nunit) * kChainTau + (l & 15);  // past T in the units of padding
+        const int k = static_cast<int>(tu % nunit) * kUnit + (l >> 4) + 4 * e;
+        ktile[o] = t < T && k < Kc ? rows[static_cast<size_t>(t) * Kc + k] : -0.0;
     }
 }
 
@@ -647,7 +718,15 @@ hipError_t launch_evolve(const EvoArgs &a, int nwg, hipStream_t s)
 {
     void *args[] = {const_cast<EvoArgs *>(&a)};
     return hipLaunchKernel(reinterpret_cast<const void *>(evolve_kernel), dim3(nwg), dim3(kEvoThreads), args,
-                           kChainLds * sizeof(double), s);
+                           kEvoLds, s);
+}
+
+hipError_t launch_ktile(const double *rows, double *ktile, int T, int Kc, int TB, int stride, hipStream_t s)
+{
+    const size_t total = ktile_doubles(TB, stride);
+    const unsigned blocks = static_cast<unsigned>(std::min<size_t>((total + 255) / 256, 8192));
+    hipLaunchKernelGGL(ktile_kernel, dim3(blocks), dim3(256), 0, s, rows, ktile, T, Kc, TB, stride / kUnit);
+    return hipGetLastError();
 }
 
 hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s)
@@ -660,10 +739,10 @@ int evolve_max_workgroups(int device)
 {
     int per_cu = 0, cus = 0;
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(evolve_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kChainLds * sizeof(double)) != hipSuccess)
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kEvoLds) != hipSuccess)
         return 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(evolve_kernel),
-                                                     kEvoThreads, kChainLds * sizeof(double)) != hipSuccess)
+                                                     kEvoThreads, kEvoLds) != hipSuccess)
         return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
     // One workgroup per CU: the grid barrier needs every workgroup resident,

@@ -9,15 +9,25 @@
 
 namespace deac {
 
-// Exact FP64 model-ISF contraction: one compute wavefront holds 4 members x
-// 16 timeslices, one sequential FMA chain per output on
-// v_mfma_f64_4x4x4_4b_f64; the kernel-matrix and genome chunks of kChunk
-// positions come from LDS, kStages buffers, filled by the helper waves from a
-// ring of registers a few chunks ahead.
+// Exact FP64 model-ISF contraction: one wavefront holds 4 members x 16
+// timeslices, one sequential FMA chain per output on v_mfma_f64_4x4x4_4b_f64,
+// its operands loaded in units of 8 positions.  Rows are padded to kChunk.
 constexpr int kChainRows = 4;
 constexpr int kChainTau = 16;
+constexpr int kUnit = 8;
 constexpr int kChunk = 128;
-constexpr int kStages = 2;
+constexpr int kKtilePad = 32;  // units past the last, which the chains load ahead and do not use
+
+// Evolution kernel: 4 wavefronts per workgroup; its registers and LDS leave
+// room for a second workgroup on the CU (another handle's).
+constexpr int kEvoThreads = 256;
+constexpr size_t kEvoLds = 78 * 1024;
+constexpr int kResidLds = 5632;   // doubles of LDS for residuals and the members' state
+constexpr int kResidWave = 1024;  // residuals per wave and window, where a wave selects a member
+static_assert(kEvoThreads / 64 * kResidWave <= kResidLds, "the waves' windows fit in LDS");
+// Every workgroup repeats the selection while that is at most this many
+// residuals, 16 per thread.
+constexpr int kLocalResid = 4096;
 
 // Random choices of one member in one generation, produced by walk_kernel.
 struct MemberCtl {
@@ -41,13 +51,15 @@ struct WalkArgs {
 struct MaskArgs {
     const MemberCtl *ctl;        // [ngen][P]
     const uint64_t *lane_tab;    // [64][64][16][4] nibble tables of T^(lane*chunk)
-    uint64_t *raw;               // [ngen][P][Kc] 53-bit draws (x >> 11)
-    int ngen, P, Kc, chunk;
+    uint64_t *raw;               // [ngen][P][rstride] 53-bit draws (x >> 11)
+    int ngen, P, Kc, chunk, rstride;
 };
 
 struct EvoArgs {
     int P, T, G, nsign, Kc;
     int stride;                  // row stride of K and of the populations: Kc padded to kChunk
+    int rstride;                 // row stride of the draws: Kc padded to whole 16-byte pairs
+    int local;                   // every workgroup repeats the selection (evolve_local)
     int MG, TB;                  // member groups of kChainRows, tau blocks of kChainTau
     int use_first, use_third, renorm, allow_neg, init_mode, track_stats;
     double stop, zeroth, first_moment, third_moment, third_moment_error;
@@ -55,7 +67,8 @@ struct EvoArgs {
     double nfm_value, nfm_error;
     const double *nfm_dt;
     int fold_ks;                 // the trials' model ISF as a rounded-product fold (bdsf; split loop only)
-    const double *kmat;          // [TB*16][stride], zero padded
+    const double *kmat;          // [T][Kc] rows (bdsf folds)
+    const double *ktile;         // K in the chains' operand order (launch_ktile)
     const double *nterm, *fterm, *tterm;   // [Kc] or null
     const double *obs, *sig;     // [T]
     double *pop0, *pop1;         // [MG*4][stride] each, member-major rows, zero padded
@@ -65,7 +78,7 @@ struct EvoArgs {
     double *emod;                // [P][T]
     double *mom;                 // [P][4]: normalization, first, third moment
     const MemberCtl *ctl;        // [ngen][P]
-    const uint64_t *raw;         // [ngen][P][Kc]
+    const uint64_t *raw;         // [ngen][P][rstride]
     double *stats;               // [3][stats_len]: mean, minimum, squared mean
     size_t stats_len;
     unsigned *bar;               // grid barrier counter, zero at launch
@@ -78,6 +91,19 @@ struct EvoArgs {
 
 hipError_t launch_walk(const WalkArgs &a, hipStream_t s);
 hipError_t launch_mask(const MaskArgs &a, hipStream_t s);
+// Whether the evolution kernel's workgroups repeat the selection: the
+// residuals are few, and they and the members' state fit in LDS.
+inline int evolve_local(int P, int T, int nsign)
+{
+    const long resid = static_cast<long>(P) * (T | 1);
+    return resid <= kLocalResid && resid + static_cast<long>(P) * (2 + 2 * nsign) <= kResidLds;
+}
+// Doubles of the K operand of TB tau blocks.
+inline size_t ktile_doubles(int TB, int stride)
+{
+    return (static_cast<size_t>(TB) * (stride / kUnit) + kKtilePad) * 64 * 2;
+}
+hipError_t launch_ktile(const double *rows, double *ktile, int T, int Kc, int TB, int stride, hipStream_t s);
 hipError_t launch_evolve(const EvoArgs &a, int nwg, hipStream_t s);
 hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s);
 // Workgroups of the evolution kernel that are co-resident on the device: one

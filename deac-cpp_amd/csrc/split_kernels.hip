@@ -102,13 +102,13 @@ __global__ __launch_bounds__(kThreads) void split_trial_kernel(EvoArgs a, int g)
     if (blockIdx.x == 0) top_of_generation(a, g);
     const int half = a.stride / 2;
     const MemberCtl *ctlg = a.ctl + static_cast<size_t>(g) * a.P;
-    const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.Kc;
+    const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.rstride;
     const size_t items = static_cast<size_t>(a.P) * half;
     for (size_t it = grid_thread(); it < items; it += grid_threads()) {
         const int i = static_cast<int>(it / half);
         const int kp = static_cast<int>(it % half);
         const MemberCtl &c = ctlg[i];
-        const uint64_t *raw = rawg + static_cast<size_t>(i) * a.Kc;
+        const uint64_t *raw = rawg + static_cast<size_t>(i) * a.rstride;
         double v[2];
         for (int e = 0; e < 2; e++) {
             const int k = 2 * kp + e;
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kThreads) void split_fold_kernel(EvoArgs a)
     const size_t total = static_cast<size_t>(a.P) * a.T;
     for (size_t idx = grid_thread(); idx < total; idx += grid_threads()) {
         const int n = static_cast<int>(idx / a.T), t = static_cast<int>(idx % a.T);
-        a.emod[idx] = fold_row(chain_row(a, n, false), a.kmat + static_cast<size_t>(t) * a.stride, a.Kc, a.G);
+        a.emod[idx] = fold_row(chain_row(a, n, false), a.kmat + static_cast<size_t>(t) * a.Kc, a.Kc, a.G);
     }
 }
 
