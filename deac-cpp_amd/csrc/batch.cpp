@@ -656,7 +656,6 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
             ia.stride = b.Lpad;
             ia.nsub = b.S;
             ia.sublen = b.Lsub;
-            ia.tab0 = 1;
             ia.allow_neg = b.m.allow_negative;
             ia.zeroth = b.m.zeroth_moment;
             BATCH_HIP(deac::launch_initial_population(ia, s));

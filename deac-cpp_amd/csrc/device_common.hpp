@@ -45,6 +45,46 @@ __device__ __forceinline__ int parity64(uint64_t x)
     return __popc(static_cast<uint32_t>(x) ^ static_cast<uint32_t>(x >> 32)) & 1;
 }
 
+// The lane's jump M^lane s of a state s that all 64 lanes share, from the
+// interleaved tables of lane_tables (host_model.hpp): 128 coalesced 1 KB loads
+// a wavefront.  (The same tables one after another, each lane gathering its
+// 32-byte entries, took four times as long.)
+__device__ __forceinline__ void lane_jump(const uint64_t *tab, const uint64_t (&s)[4], uint64_t (&out)[4])
+{
+    typedef uint32_t quad __attribute__((ext_vector_type(4)));
+    const int voff = (threadIdx.x & 63) * 16;
+    uint32_t u[8];
+    for (int w = 0; w < 4; w++) {
+        u[2 * w] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s[w]));
+        u[2 * w + 1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s[w] >> 32));
+    }
+    // the entry's address is scalar (buffer loads take it as one offset), 24 loads in flight
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t *>(tab), 0, 64 * 16 * 2048, 0x00020000);
+    constexpr int kHold = 12;
+    quad e0[kHold], e1[kHold], lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
+    auto load = [&](int n) __attribute__((always_inline)) {
+        const uint32_t v = (u[n >> 3] >> ((n & 7) * 4)) & 15;
+        const int off = static_cast<int>((n * 16 + v) * 2048);
+        e0[n % kHold] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, off, 0);
+        e1[n % kHold] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + 1024, off, 0);
+    };
+#pragma unroll
+    for (int n = 0; n < kHold; n++) load(n);
+#pragma unroll
+    for (int n = 0; n < 64; n++) {
+        lo ^= e0[n % kHold];
+        hi ^= e1[n % kHold];
+        // (the sums stay here, so that the entries' registers are free again)
+        asm volatile("" : "+v"(lo), "+v"(hi));
+        if (n + kHold < 64) load(n + kHold);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    out[0] = (static_cast<uint64_t>(lo.y) << 32) | lo.x;
+    out[1] = (static_cast<uint64_t>(lo.w) << 32) | lo.z;
+    out[2] = (static_cast<uint64_t>(hi.y) << 32) | hi.x;
+    out[3] = (static_cast<uint64_t>(hi.w) << 32) | hi.z;
+}
+
 }  // namespace deac
 
 // s_waitcnt with vmcnt <= n (n < 64) and the other counters unconstrained.

@@ -45,14 +45,18 @@ struct deac_handle {
     long *iter = nullptr;               // [2][2]: split loop generation counters, per buffer set
     int *host_status = nullptr;         // [3][4], pinned: status of the sets, then of the initial fitness
     deac::MemberCtl *ctl[2] = {};
-    uint64_t *raw[2] = {}, *gen_start[2] = {};
+    uint64_t *raw[2] = {};
+    uint64_t *gen_start[3] = {};        // by batch index modulo 3 (see the generation loop)
     uint64_t *state = nullptr, *skip_rows = nullptr, *lane_tab = nullptr;
+    uint64_t *tab1 = nullptr, *tab2 = nullptr, *skip_tab_dev = nullptr;  // wide walk
+    bool wide = false;
     uint64_t *init_start = nullptr;     // [P][4]: random state at each member's first initial draw
     std::vector<uint64_t> skip_tab;     // nibble table of T^Kc, host side
     double *stats = nullptr;            // statistics histories, kept between runs and grown on demand
     size_t stats_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // per set: walk start, walk end, mask start, mask end, evolve start,
+    // per set: walk start, walk end (fused path: of the first batch), mask
+    // start, mask end, evolve start,
     // evolve end (draws free), status copied
     hipEvent_t kev[2][7] = {};
     deac_run_profile last{};
@@ -265,6 +269,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     h->TB = (T + deac::kChainTau - 1) / deac::kChainTau;
     h->stride = round_up(Kc, deac::kChunk);
     h->rstride = round_up(Kc, 2);
+    h->wide = deac::walk_is_wide(P, m.tau_cr, m.tau_f);
     h->chunk = (Kc + 63) / 64;
     // RNG batch: generations whose mask draws are buffered at once (<= 256 MiB
     // per buffer set).
@@ -310,30 +315,38 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     for (int k = 0; k < 2; k++) {
         A(h->ctl[k], static_cast<size_t>(h->batch) * P);
         A(h->raw[k], static_cast<size_t>(h->batch) * P * h->rstride);
-        A(h->gen_start[k], static_cast<size_t>(h->batch) * 4);
     }
+    for (uint64_t *&p : h->gen_start) A(p, static_cast<size_t>(h->batch) * 4);
     A(h->state, 4);
     A(h->init_start, static_cast<size_t>(P) * 4);
     A(h->skip_rows, 256 * 4);
-    A(h->lane_tab, static_cast<size_t>(64) * 64 * 16 * 4);
+    constexpr size_t kTab = 64 * 16 * 4;  // words of a nibble table
+    A(h->lane_tab, deac::kLaneTabWords);
+    if (h->wide) {
+        A(h->tab1, deac::kLaneTabWords);
+        A(h->tab2, deac::kLaneTabWords);
+        A(h->skip_tab_dev, kTab);
+    }
     if (!m.nterm.empty()) A(h->nterm, Kc + 1);
     if (!m.fterm.empty()) A(h->fterm, Kc + 1);
     if (!m.tterm.empty()) A(h->tterm, Kc + 1);
     if (m.use_nfm) A(h->nfm_dt, T);
     if (st != DEAC_OK) return fail(st);
 
-    // Jump tables: T^(nsign*G) by rows for the walk, T^(l*chunk) by nibbles
-    // for the mask generator.
-    std::vector<uint64_t> rows(256 * 4), tabs(static_cast<size_t>(64) * 64 * 16 * 4);
+    // Jump tables: T^(nsign*G) by rows for the serial walk and by nibbles for
+    // the wide one, T^(l*chunk) by lanes for the mask generator, T^(l*c1) and
+    // T^(l*(nsign*G+3)) for the wide walk.
+    std::vector<uint64_t> rows(256 * 4), tabs(deac::kLaneTabWords), tabs1, tabs2;
     const deac::Gf2Matrix skip = deac::transition_power(static_cast<uint64_t>(Kc));
     deac::matrix_rows(skip, rows.data());
-    h->skip_tab.resize(64 * 16 * 4);
+    h->skip_tab.resize(kTab);
     deac::nibble_table(skip, h->skip_tab.data());
-    const deac::Gf2Matrix step = deac::transition_power(static_cast<uint64_t>(h->chunk));
-    deac::Gf2Matrix acc = deac::Gf2Matrix::identity();
-    for (int l = 0; l < 64; l++) {
-        deac::nibble_table(acc, tabs.data() + static_cast<size_t>(l) * 64 * 16 * 4);
-        acc = step * acc;
+    deac::lane_tables(deac::transition_power(static_cast<uint64_t>(h->chunk)), tabs.data());
+    if (h->wide) {
+        tabs1.resize(deac::kLaneTabWords);
+        tabs2.resize(deac::kLaneTabWords);
+        deac::lane_tables(deac::transition_power(static_cast<uint64_t>(deac::walk_c1(P, m.nsign))), tabs1.data());
+        deac::lane_tables(deac::transition_power(static_cast<uint64_t>(Kc) + 3), tabs2.data());
     }
     auto up = [&](void *dst, const void *src, size_t bytes) {
         if (st == DEAC_OK && hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) != hipSuccess) st = DEAC_ERR_DEVICE;
@@ -345,6 +358,11 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     up(h->sig, m.err.data(), m.T * sizeof(double));
     up(h->skip_rows, rows.data(), rows.size() * sizeof(uint64_t));
     up(h->lane_tab, tabs.data(), tabs.size() * sizeof(uint64_t));
+    if (h->wide) {
+        up(h->tab1, tabs1.data(), tabs1.size() * sizeof(uint64_t));
+        up(h->tab2, tabs2.data(), tabs2.size() * sizeof(uint64_t));
+        up(h->skip_tab_dev, h->skip_tab.data(), h->skip_tab.size() * sizeof(uint64_t));
+    }
     if (h->nterm) up(h->nterm, m.nterm.data(), m.Kc * sizeof(double));
     if (h->fterm) up(h->fterm, m.fterm.data(), m.Kc * sizeof(double));
     if (h->tterm) up(h->tterm, m.tterm.data(), m.Kc * sizeof(double));
@@ -353,6 +371,12 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     // zero past Kc and past P.
     for (double *p : {h->pop0, h->pop1})
         if (st == DEAC_OK && hipMemsetAsync(p, 0, pop_n * sizeof(double), h->stream) != hipSuccess)
+            st = DEAC_ERR_DEVICE;
+    // Records: behind a stop, mask draws run over records that no walk has
+    // written (nothing reads those draws).
+    for (deac::MemberCtl *p : h->ctl)
+        if (st == DEAC_OK &&
+            hipMemsetAsync(p, 0, static_cast<size_t>(h->batch) * P * sizeof(deac::MemberCtl), h->stream) != hipSuccess)
             st = DEAC_ERR_DEVICE;
     if (st != DEAC_OK) return fail(st);
     *out = h;
@@ -437,7 +461,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ia.stride = h->stride;
     ia.nsub = 64;
     ia.sublen = h->chunk;
-    ia.tab0 = 0;
+    ia.lane_tab = true;
     ia.allow_neg = m.allow_negative;
     ia.zeroth = m.zeroth_moment;
     DEAC_HIP(deac::launch_initial_population(ia, s));
@@ -489,6 +513,11 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     deac::WalkArgs wa{};
     wa.state = h->state;
     wa.skip_rows = h->skip_rows;
+    wa.tab1 = h->tab1;
+    wa.tab2 = h->tab2;
+    wa.skip_tab = h->skip_tab_dev;
+    wa.wide = h->wide;
+    wa.c1 = deac::walk_c1(static_cast<int>(P), nsign);
     wa.P = static_cast<int>(P);
     wa.nsign = nsign;
     wa.mod_magic = ~UINT64_C(0) / P;
@@ -502,37 +531,36 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ma.rstride = h->rstride;
 
     // Generation loop: ii = 0 .. N-2 (deac.cpp:1138), in batches.  Batch b
-    // uses buffer set b%2.  Its walk runs on the draw stream while batch b-1
-    // evolves, then its mask draws and its evolution run on the evolution
-    // stream; the mask kernel spreads over
-    // every CU and costs less alone than beside the evolution.  The evolution
-    // of b is queued before the host has read batch b-1's status.  Behind a
-    // stop it changes nothing: the stop test sits at the top of a generation,
-    // so the fitnesses it finds are those that stopped batch b-1, and it
-    // stops at its first generation (its status and its statistics entry,
-    // past the stop, are never read).  Batches start at 8
-    // generations and double up to the buffer size, so that the first walk,
-    // which nothing hides, is short.
+    // uses buffer set b%2.  Its walk runs beside the evolution of batch b-1, on
+    // a workgroup of the same launch (two streams may share a hardware queue
+    // and then run one after the other); its mask draws, which spread over
+    // every CU and cost less alone, follow before its own evolution.  The
+    // evolution of b is queued before the host has read batch b-1's status.
+    // Behind a stop it changes nothing: the stop test sits at the top of a
+    // generation, so the fitnesses it finds are those that stopped batch b-1,
+    // and it stops at its first generation (its status and its statistics
+    // entry, past the stop, are never read).  Batches start at 8 generations,
+    // so that the first walk, which nothing hides, is short, and grow by half
+    // up to the buffer size: the walk beside a batch then has one and a half
+    // times its generations to walk, which a member's walk (0.7 us) still
+    // hides behind the generations of the smallest runs (8 us, 8 members).
     const size_t total = N - 1;
     std::vector<std::pair<size_t, int>> plan;  // first generation, generations
     for (size_t g = 0, len = std::min(8, h->batch); g < total;) {
         const int nb = static_cast<int>(std::min(len, total - g));
         plan.emplace_back(g, nb);
         g += static_cast<size_t>(nb);
-        len = std::min(2 * len, static_cast<size_t>(h->batch));
+        len = std::min(len + len / 2, static_cast<size_t>(h->batch));
+        if (len < 2) len = std::min(2, h->batch);
     }
-    hipStream_t d = h->draw_stream;
-    auto draws = [&](size_t b) -> deac_status {
+    hipStream_t d = h->draw_stream;  // split loop: the draws of the next batch
+    auto walk_args = [&](size_t b) {
         const int k = static_cast<int>(b & 1);
-        hipEvent_t *e = h->kev[k];
-        if (b >= 2) DEAC_HIP(hipStreamWaitEvent(d, e[5], 0));  // batch b-2 done with the set
-        wa.gen_start = h->gen_start[k];
+        // three sets of generation starts: a stop in batch b is answered from
+        // its set while the launch of b+1, queued behind, may walk b+2
+        wa.gen_start = h->gen_start[b % 3];
         wa.ctl = h->ctl[k];
-        wa.ngen = plan[b].second;
-        DEAC_HIP(hipEventRecord(e[0], d));
-        DEAC_HIP(deac::launch_walk(wa, d));
-        DEAC_HIP(hipEventRecord(e[1], d));
-        return DEAC_OK;
+        wa.ngen = b < plan.size() ? plan[b].second : 0;
     };
     auto evolve = [&](size_t b) -> deac_status {
         const int k = static_cast<int>(b & 1);
@@ -547,13 +575,14 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         ma.ctl = h->ctl[k];
         ma.raw = h->raw[k];
         ma.ngen = plan[b].second;
-        DEAC_HIP(hipStreamWaitEvent(s, e[1], 0));  // walk done
+        walk_args(b + 1);
+        wa.halt = ea.status;
         DEAC_HIP(hipEventRecord(e[2], s));
         DEAC_HIP(deac::launch_mask(ma, s));
         DEAC_HIP(hipEventRecord(e[3], s));
         DEAC_HIP(deac::launch_zero_u32(sy, 8, s));
         DEAC_HIP(hipEventRecord(e[4], s));
-        DEAC_HIP(deac::launch_evolve(ea, h->nwg, s));
+        DEAC_HIP(deac::launch_evolve(ea, wa, s));
         DEAC_HIP(hipEventRecord(e[5], s));
         DEAC_HIP(hipMemcpyAsync(h->host_status + 4 * k, sy + 4, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
         DEAC_HIP(hipEventRecord(e[6], s));
@@ -570,14 +599,17 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         ea.ngen = 0;
         ea.bar = h->sync + 8;
         ea.status = reinterpret_cast<int *>(h->sync + 12);
+        ea.nwg = h->nwg;
         DEAC_HIP(deac::launch_zero_u32(h->sync + 8, 8, s));
-        DEAC_HIP(deac::launch_evolve(ea, h->nwg, s));
+        DEAC_HIP(deac::launch_evolve(ea, deac::WalkArgs{}, s));
         DEAC_HIP(hipMemcpyAsync(h->host_status + 8, h->sync + 12, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
         ea.init_mode = 0;
         DEAC_HIP(hipEventRecord(h->ev0, s));
-        DEAC_HIP(hipStreamWaitEvent(d, h->ev0, 0));  // RNG state uploaded
-        DEAC_TRY(draws(0));
-        if (plan.size() > 1) DEAC_TRY(draws(1));
+        walk_args(0);
+        wa.halt = nullptr;
+        DEAC_HIP(hipEventRecord(h->kev[0][0], s));
+        DEAC_HIP(deac::launch_walk(wa, s));
+        DEAC_HIP(hipEventRecord(h->kev[0][1], s));
         DEAC_TRY(evolve(0));
         for (size_t b = 0; b < plan.size(); b++) {
             if (b + 1 < plan.size()) DEAC_TRY(evolve(b + 1));
@@ -586,7 +618,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             DEAC_HIP(hipEventSynchronize(e[6]));
             if (b == 0 && h->host_status[8 + 2]) return DEAC_ERR_DEVICE;  // initial fitness: barrier timeout
             float t_walk = 0, t_mask = 0, t_evo = 0;
-            DEAC_HIP(hipEventElapsedTime(&t_walk, e[0], e[1]));
+            if (b == 0) DEAC_HIP(hipEventElapsedTime(&t_walk, e[0], e[1]));
             DEAC_HIP(hipEventElapsedTime(&t_mask, e[2], e[3]));
             DEAC_HIP(hipEventElapsedTime(&t_evo, e[4], e[5]));
             prof.walk_ms += t_walk;
@@ -596,18 +628,16 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             const int *status = h->host_status + 4 * k;
             if (status[2]) return DEAC_ERR_DEVICE;  // a grid barrier timed out
             if (status[0]) {
-                // RNG state at the top of the stopping generation; the set is
-                // not rewritten before this copy (draws of b+2 not queued)
+                // RNG state at the top of the stopping generation
                 stopped_at = static_cast<long>(plan[b].first) + status[1];
                 uint64_t st4[4];
-                DEAC_HIP(hipMemcpy(st4, h->gen_start[k] + static_cast<size_t>(status[1]) * 4, sizeof st4,
+                DEAC_HIP(hipMemcpy(st4, h->gen_start[b % 3] + static_cast<size_t>(status[1]) * 4, sizeof st4,
                                    hipMemcpyDeviceToHost));
                 std::memcpy(rng.s, st4, sizeof st4);
                 done += static_cast<size_t>(status[1]);
                 return DEAC_OK;
             }
             done += static_cast<size_t>(plan[b].second);
-            if (b + 2 < plan.size()) DEAC_TRY(draws(b + 2));
         }
         return DEAC_OK;
     };

@@ -30,8 +30,10 @@ __global__ __launch_bounds__(kThreads) void init_draw_kernel(InitArgs a)
     if (row >= a.rows) return;
     const uint64_t *st = a.start + row * 4;
     uint64_t s[4] = {st[0], st[1], st[2], st[3]};
-    if (sub >= a.tab0) {
-        const uint64_t *tab = a.tab + static_cast<size_t>(sub - a.tab0) * (64 * 16 * 4);
+    if (a.lane_tab) {
+        lane_jump(a.tab, s, s);
+    } else if (sub > 0) {
+        const uint64_t *tab = a.tab + static_cast<size_t>(sub - 1) * (64 * 16 * 4);
         uint64_t o[4] = {0, 0, 0, 0};
 #pragma unroll 4
         for (int n = 0; n < 64; n++) {

@@ -13,11 +13,13 @@ struct InitArgs {
     const uint64_t *start;   // [rows][4]: random state at each member's first draw
     const long *offset;      // [rows / P] offset of each instance's population from pop, or null (0)
     double *pop;             // member rows of `stride` doubles
-    const uint64_t *tab;     // nibble tables of T^(k*sublen) for sub-streams k = tab0 .. nsub-1
+    const uint64_t *tab;     // lane_tab: lane_tables of T^sublen (64 sub-streams, one wavefront per member);
+                             // else nibble tables of T^(k*sublen) for sub-streams k = 1 .. nsub-1
     const double *nterm;     // [Kc] normalization weights, or null: populations are not normalized
     long rows;               // members of all instances
     int P, G, nsign, stride;
-    int nsub, sublen, tab0;  // sub-streams per member and draws of each; first sub-stream with a table
+    int nsub, sublen;        // sub-streams per member and draws of each
+    bool lane_tab;
     int allow_neg;
     double zeroth;
 };

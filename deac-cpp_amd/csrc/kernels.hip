@@ -3,10 +3,10 @@
 // One generation of the reference loop (deac.cpp:1138-1573) is split in
 // two independent parts:
 //   * the random choices, which depend only on the xoshiro256+ stream:
-//       walk_kernel  - one wavefront walks the sequential, data-dependent
+//       walk         - one wavefront walks the sequential, data-dependent
 //                      part of the stream (jDE F/CR redraws, rejection-
 //                      sampled donor indices) and skips each member's 2G
-//                      crossover-mask draws with one GF(2) jump;
+//                      crossover-mask draws with GF(2) jumps;
 //       mask_kernel  - one wavefront per member regenerates the mask draws:
 //                      lane l jumps to draw l*chunk with a nibble table and
 //                      steps chunk draws;
@@ -38,7 +38,7 @@ constexpr int kEvoWaves = kEvoThreads / kWave;
 // caller leaves the kernel, so a broken launch cannot hang the device.
 constexpr unsigned kBarrierSpins = 1u << 24;
 
-__device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, int *status)
+__device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, int nwg, int *status)
 {
     // Each wave drains its own memory operations; then one thread per
     // workgroup publishes the workgroup's stores at agent scope (L2 write-back,
@@ -47,7 +47,7 @@ __device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, in
     __shared__ int timed_out;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    target += gridDim.x;
+    target += nwg;
     if (threadIdx.x == 0) {
         timed_out = 0;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -93,21 +93,254 @@ __device__ __forceinline__ uint32_t mod_p_uniform(uint64_t x, uint64_t magic, ui
     return r;
 }
 
+// s <- M s from M's nibble table: 64 lookups of 32 bytes.
+__device__ __forceinline__ void nibble_jump(const uint64_t *tab, uint64_t (&s)[4])
+{
+    uint64_t o[4] = {0, 0, 0, 0};
+#pragma unroll 16
+    for (int n = 0; n < 64; n++) {
+        const int v = static_cast<int>((s[n >> 4] >> ((n & 15) * 4)) & 15);
+        const uint64_t *e = tab + (n * 16 + v) * 4;
+        o[0] ^= e[0];
+        o[1] ^= e[1];
+        o[2] ^= e[2];
+        o[3] ^= e[3];
+    }
+    for (int w = 0; w < 4; w++) s[w] = o[w];
+}
+
+// Lane q's copy of a state, in every lane (q uniform).
+__device__ __forceinline__ void lane_state(const uint64_t (&s)[4], int q, uint64_t (&out)[4])
+{
+    for (int w = 0; w < 4; w++) {
+        const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(s[w]), q);
+        const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(s[w] >> 32), q);
+        out[w] = (static_cast<uint64_t>(hi) << 32) | lo;
+    }
+}
+
+// u < p for the draw x, u = (x >> 11) 2^-53, in whole numbers: x < below, or
+// all draws.
+struct DrawLimit {
+    uint64_t below;
+    bool all;
+};
+
+__device__ __forceinline__ DrawLimit draw_limit(double p)
+{
+    if (!(p > 0.0)) return {0, false};
+    if (p >= 1.0) return {0, true};
+    return {static_cast<uint64_t>(ceil(p * 0x1.0p53)) << 11, false};
+}
+
+__device__ __forceinline__ bool passes(const DrawLimit &l, uint64_t x) { return l.all || x < l.below; }
+
 }  // namespace
 
 // ---------------------------------------------------------------- walk
 
-__global__ __launch_bounds__(64) void walk_kernel(WalkArgs a)
-{
-    __shared__ uint64_t rows[256 * 4];
-    const int lane = threadIdx.x;
-    for (int k = lane; k < 256 * 4; k += kWave) rows[k] = a.skip_rows[k];
-    __syncthreads();
+namespace {
 
+// Whether the batch that runs beside this walk has met its stop test, looked
+// up every few generations: what the walk draws is then not used.
+constexpr int kWalkPoll = 16;
+
+__device__ __forceinline__ bool stopped(const WalkArgs &a)
+{
+    return a.halt && __hip_atomic_load(a.halt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
+// Which draws of a sequence are values: bit i+1 where bit i is a test (not a
+// value) whose limit the draw passed.  carry: whether draw 0 is a value; set
+// to whether draw 64 is.  Runs of passed draws alternate test, value, test,
+// ..., which an addition resolves for all runs at once: a run's values are
+// its positions of the parity opposite to its first.
+__device__ __forceinline__ uint64_t value_bits(uint64_t passed, bool &carry)
+{
+    const uint64_t kEven = UINT64_C(0x5555555555555555);
+    passed &= ~static_cast<uint64_t>(carry ? 1 : 0);
+    const uint64_t follows = (passed << 1) | (carry ? 1 : 0);
+    const uint64_t odd_starts = passed & ~kEven & ~follows;
+    const uint64_t sum = odd_starts + passed;
+    carry = sum < passed;
+    return (kEven ^ (sum << 1)) & follows;
+}
+
+// Walk of a.ngen generations by one wavefront (deac.cpp:1180-1240): the
+// sequential, data-dependent part of the stream -- which draws are F/CR
+// redraws, how many draws each member's rejection-sampled donors take -- with
+// the draws themselves made in parallel.
+//
+// jDE controls (CR+, F+, CR-, F- per member, a test draw each and a value
+// draw where the test passes): lane l jumps to draw l*c1 of the generation
+// and makes c1 draws into LDS; windows of 64 draws are then told apart into
+// tests and values at once.  Donors: lane l jumps to where member m0+l starts
+// if every member before it takes exactly 3 donor draws (its crossover draws
+// are skipped in the same jump); e, the draws really taken beyond that, is
+// uniform, so all lanes try their member at offset e, the lanes up to the
+// first one that rejects a draw are right, and the rest try again from there.
+// The lane behind the last member is where the next block, or the next
+// generation, starts.
+//
+// Bound: latency of one wavefront, mostly the jumps' table loads (128 of 1 KB
+// each, from L2).  Walking member by member took 0.7 us per member: per
+// generation 356 us at 512 members, 45 at 64.
+__device__ void walk_wide(const WalkArgs &a, uint64_t *lds)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    uint64_t *draws = lds;                                                   // [kWave][c1 | 1]
+    uint32_t *res = reinterpret_cast<uint32_t *>(lds + kWave * (a.c1 | 1));  // [kWalkDraws][kWave]
+    uint32_t *flags = res + kWalkDraws * kWave;                              // [P]
+    const int c1 = a.c1, pitch = a.c1 | 1;
+    const uint32_t P = static_cast<uint32_t>(a.P);
+    const int tests = 2 * a.nsign * a.P;
+    const DrawLimit lim = draw_limit(a.tau_cr);  // tau_f is the same (walk_is_wide)
+    // lanes that usually cover a generation's controls
+    const int n1 = min(kWave, (tests + tests / 4 + 8 + c1 - 1) / c1);
+    uint64_t s[4] = {a.state[0], a.state[1], a.state[2], a.state[3]};  // uniform: where the next draw is
+    for (int g = 0; g < a.ngen; g++) {
+        if (g % kWalkPoll == 0 && stopped(a)) return;
+        if (lane < 4) a.gen_start[static_cast<size_t>(g) * 4 + lane] = s[lane & 3];
+        MemberCtl *ctl = a.ctl + static_cast<size_t>(g) * a.P;
+        for (int i = lane; i < a.P; i += kWave) flags[i] = 0;
+
+        int k0 = 0;          // tests before the current window
+        bool carry = false;  // the window's first draw is a value
+        int end = -1;        // draw behind the last control, of the current round
+        while (end < 0) {
+            uint64_t start[4] = {s[0], s[1], s[2], s[3]};
+            if (lane < n1) {
+                lane_jump(a.tab1, s, start);
+                uint64_t t[4] = {start[0], start[1], start[2], start[3]};
+                for (int j = 0; j < c1; j++) draws[lane * pitch + j] = xnext(t);
+            }
+            asm volatile("" ::: "memory");
+            const int avail = n1 * c1;
+            for (int w = 0; w < avail && end < 0; w += kWave) {
+                const int o = w + lane;
+                const uint64_t x = o < avail ? draws[o / c1 * pitch + o % c1] : 0;
+                const bool in = o < avail;
+                const uint64_t valid = __ballot(in);
+                const uint64_t passed = __ballot(in && passes(lim, x));
+                const uint64_t values = value_bits(passed, carry) & valid;
+                const uint64_t below = (UINT64_C(1) << lane) - 1;
+                const uint64_t test_bits = valid & ~values;
+                // the test of this draw, or the one its value belongs to
+                const int k = k0 + __popcll(test_bits & below) - ((values >> lane) & 1 ? 1 : 0);
+                if (((values >> lane) & 1) && k < tests) {
+                    const int i = k / (2 * a.nsign), sg = (k / 2) % a.nsign;
+                    if (k & 1) ctl[i].f_value[sg] = 2.0 * to_unit(x);
+                    else ctl[i].cr_value[sg] = to_unit(x);
+                    __hip_atomic_fetch_or(&flags[i], (k & 1 ? 2u : 1u) << (2 * sg), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+                // the first draw that is a test past the last one ends the controls
+                const uint64_t past = __ballot(in && !((values >> lane) & 1) && k >= tests);
+                if (past) end = w + __builtin_ctzll(past);
+                k0 += __popcll(test_bits);
+                if (w + kWave > avail) carry = (passed & test_bits) >> (avail - w - 1) & 1;
+            }
+            if (end < 0 && k0 == tests && !carry) end = avail;
+            // on to the next round, or to the draw behind the controls
+            const int to = end < 0 ? avail : end;
+            const int q = min(to / c1, n1 - 1);
+            lane_state(start, q, s);
+            for (int j = q * c1; j < to; j++) (void)xnext_uniform(s);
+        }
+
+        for (int m0 = 0; m0 < a.P;) {
+            const int cnt = min(kWave - 1, a.P - m0);  // members tried in this block
+            uint64_t start[4] = {s[0], s[1], s[2], s[3]};
+            if (lane <= cnt) lane_jump(a.tab2, s, start);
+            uint64_t t[4] = {start[0], start[1], start[2], start[3]};
+            int made = 0;
+            auto more = [&]() {
+#pragma unroll 2
+                for (int j = 0; j < 4; j++) res[(made + j) * kWave + lane] = mod_p(xnext(t), a.mod_magic, P);
+                made += 4;
+                asm volatile("" ::: "memory");
+            };
+            const uint32_t i = static_cast<uint32_t>(m0 + lane);
+            int cur = 0, e = 0;
+            bool room = true;
+            while (cur < cnt && room) {
+                while (made < e + 4 && made + 4 <= kWalkDraws) more();
+                // donor indices (deac.cpp:200-216) from draw e on
+                uint32_t m[3] = {i, i, i};
+                int got = 0, d = e;
+                while (got < 3 && d < made) {
+                    const uint32_t r = res[d++ * kWave + lane];
+                    if (r == i || (got > 0 && r == m[0]) || (got > 1 && r == m[1])) continue;
+                    if (got == 0) m[0] = r;
+                    else if (got == 1) m[1] = r;
+                    else m[2] = r;
+                    got++;
+                }
+                const bool mine = lane >= cur && lane < cnt;
+                const uint64_t bad = __ballot(mine && (got < 3 || d - e > 3));
+                const int f = bad ? __builtin_ctzll(bad) : cnt;
+                const bool whole = f < cnt && __builtin_amdgcn_readlane(static_cast<uint32_t>(got), f) == 3;
+                if (mine && (lane < f || (lane == f && whole))) {
+                    MemberCtl &c = ctl[i];
+                    c.flags = flags[i];
+                    c.mutant[0] = m[0];
+                    c.mutant[1] = m[1];
+                    c.mutant[2] = m[2];
+                    c.mask_steps = static_cast<uint32_t>(d);
+                    for (int w = 0; w < 4; w++) c.mask_state[w] = start[w];
+                }
+                cur = f;
+                if (whole) {
+                    e = static_cast<int>(__builtin_amdgcn_readlane(static_cast<uint32_t>(d), f)) - 3;
+                    cur = f + 1;
+                } else if (f < cnt) {  // this member needs more draws than were made
+                    if (made + 4 <= kWalkDraws) more();
+                    else room = false;  // a new block starts at it
+                }
+            }
+            // a member that one block cannot settle at its start would need
+            // more than kWalkDraws draws for three donors: walked one by one
+            if (cur == 0) {
+                uint32_t m[3] = {static_cast<uint32_t>(m0), static_cast<uint32_t>(m0), static_cast<uint32_t>(m0)};
+                const uint32_t i0 = static_cast<uint32_t>(m0);
+                uint64_t first[4] = {s[0], s[1], s[2], s[3]};
+                uint32_t steps = 0;
+                for (int got = 0; got < 3; steps++) {
+                    const uint32_t r = mod_p_uniform(xnext_uniform(s), a.mod_magic, P);
+                    if (r == i0 || (got > 0 && r == m[0]) || (got > 1 && r == m[1])) continue;
+                    m[got++] = r;
+                }
+                if (lane == 0) {
+                    MemberCtl &c = ctl[m0];
+                    c.flags = flags[m0];
+                    for (int w = 0; w < 3; w++) c.mutant[w] = m[w];
+                    c.mask_steps = steps;
+                    for (int w = 0; w < 4; w++) c.mask_state[w] = first[w];
+                }
+                nibble_jump(a.skip_tab, s);
+                m0 += 1;
+                continue;
+            }
+            lane_state(start, cur, s);
+            for (int j = 0; j < e; j++) (void)xnext_uniform(s);
+            m0 += cur;
+        }
+    }
+    if (lane < 4) a.state[lane] = s[lane & 3];
+}
+
+// The same member by member.
+__device__ void walk_serial(const WalkArgs &a, uint64_t *rows)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int k = lane; k < 256 * 4; k += kWave) rows[k] = a.skip_rows[k];
+    asm volatile("" ::: "memory");
     // Every lane carries the same state; lane 0 writes the records.
     uint64_t s[4] = {a.state[0], a.state[1], a.state[2], a.state[3]};
     const uint32_t P = static_cast<uint32_t>(a.P);
+    const DrawLimit lim_cr = draw_limit(a.tau_cr), lim_f = draw_limit(a.tau_f);
     for (int g = 0; g < a.ngen; g++) {
+        if (g % kWalkPoll == 0 && stopped(a)) return;
         if (lane == 0)
             for (int w = 0; w < 4; w++) a.gen_start[static_cast<size_t>(g) * 4 + w] = s[w];
         MemberCtl *ctl = a.ctl + static_cast<size_t>(g) * a.P;
@@ -116,11 +349,11 @@ __global__ __launch_bounds__(64) void walk_kernel(WalkArgs a)
             uint32_t flags = 0;
             double crv[2] = {0.0, 0.0}, fv[2] = {0.0, 0.0};
             for (int sg = 0; sg < a.nsign; sg++) {
-                if (to_unit(xnext_uniform(s)) < a.tau_cr) {
+                if (passes(lim_cr, xnext_uniform(s))) {
                     flags |= 1u << (2 * sg);
                     crv[sg] = to_unit(xnext_uniform(s));
                 }
-                if (to_unit(xnext_uniform(s)) < a.tau_f) {
+                if (passes(lim_f, xnext_uniform(s))) {
                     flags |= 2u << (2 * sg);
                     fv[sg] = 2.0 * to_unit(xnext_uniform(s));
                 }
@@ -144,6 +377,7 @@ __global__ __launch_bounds__(64) void walk_kernel(WalkArgs a)
                 ctl[i].mutant[0] = m0;
                 ctl[i].mutant[1] = m1;
                 ctl[i].mutant[2] = m2;
+                ctl[i].mask_steps = 0;
                 for (int w = 0; w < 4; w++) ctl[i].mask_state[w] = s[w];
             }
             // s <- T^(nsign*G) s: lane l forms output bits l, 64+l, 128+l,
@@ -169,6 +403,21 @@ __global__ __launch_bounds__(64) void walk_kernel(WalkArgs a)
         for (int w = 0; w < 4; w++) a.state[w] = s[w];
 }
 
+// One wavefront.
+__device__ __forceinline__ void walk(const WalkArgs &a, uint64_t *lds)
+{
+    if (a.wide) walk_wide(a, lds);
+    else walk_serial(a, lds);
+}
+
+}  // namespace
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void walk_kernel(WalkArgs a)
+{
+    extern __shared__ uint64_t walk_lds[];
+    walk(a, walk_lds);
+}
+
 // ---------------------------------------------------------------- masks
 
 __global__ __launch_bounds__(256) void mask_kernel(MaskArgs a)
@@ -178,19 +427,8 @@ __global__ __launch_bounds__(256) void mask_kernel(MaskArgs a)
     if (wave >= static_cast<size_t>(a.ngen) * a.P) return;
     const MemberCtl &c = a.ctl[wave];
     uint64_t s[4] = {c.mask_state[0], c.mask_state[1], c.mask_state[2], c.mask_state[3]};
-    // s <- T^(lane*chunk) s from the lane's nibble table.
-    const uint64_t *tab = a.lane_tab + static_cast<size_t>(lane) * (64 * 16 * 4);
-    uint64_t o[4] = {0, 0, 0, 0};
-#pragma unroll 4
-    for (int n = 0; n < 64; n++) {
-        const int v = static_cast<int>((s[n >> 4] >> ((n & 15) * 4)) & 15);
-        const uint64_t *e = tab + (n * 16 + v) * 4;
-        o[0] ^= e[0];
-        o[1] ^= e[1];
-        o[2] ^= e[2];
-        o[3] ^= e[3];
-    }
-    for (int w = 0; w < 4; w++) s[w] = o[w];
+    for (uint32_t k = 0; k < c.mask_steps; k++) (void)xnext(s);
+    lane_jump(a.lane_tab, s, s);  // T^(lane*chunk)
     uint64_t *raw = a.raw + wave * a.rstride;
     const int k0 = lane * a.chunk;
     for (int c2 = 0; c2 < a.chunk; c2++) {
@@ -481,7 +719,7 @@ __device__ unsigned long long deac_phase_clock[4];
 // workgroups) to 8 us (255, the cache fences of an XCD's workgroups queue),
 // a repeated selection of 8 members 1.3 us.  One workgroup per CU is launched
 // (evolve_max_workgroups); a second handle's workgroup still fits beside it.
-__global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a)
+__global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a, WalkArgs next)
 {
 #ifdef DEAC_PHASE_TIMERS
     unsigned long long phase_t0 = 0;
@@ -492,7 +730,13 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const int lane = threadIdx.x & (kWave - 1);
     // the wave index as a scalar: what depends on it alone is then uniform
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int nwg = gridDim.x;
+    const int nwg = a.nwg;
+    if (blockIdx.x == nwg) {
+        // the workgroup behind the evolution's: it walks the next batch and
+        // takes no part in the barriers
+        if (wid == 0) walk(next, reinterpret_cast<uint64_t *>(lds));
+        return;
+    }
     const int total_waves = nwg * kEvoWaves;
     // Waves are numbered wave-slot-major so that consecutive tasks land on
     // different workgroups (and CUs).
@@ -562,8 +806,8 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 }
                 const bool stop = mn <= a.stop;
                 if (stop && blockIdx.x == 0) {
-                    a.status[0] = 1;
                     a.status[1] = g;
+                    __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 stop_flag = stop ? 1 : 0;
             }
@@ -603,7 +847,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                     __syncthreads();
                 }
             }
-            if (!grid_barrier(a.bar, target, a.status)) return;
+            if (!grid_barrier(a.bar, target, nwg, a.status)) return;
             DEAC_PHASE(1);
         }
 
@@ -622,7 +866,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }
         }
-        if (!grid_barrier(a.bar, target, a.status)) return;
+        if (!grid_barrier(a.bar, target, nwg, a.status)) return;
         DEAC_PHASE(2);
 
         // Fitness and greedy selection.
@@ -653,7 +897,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 }
                 if (lane == 0) select_member(a, s, g, i, chi, init);
             }
-            if (!grid_barrier(a.bar, target, a.status)) return;
+            if (!grid_barrier(a.bar, target, nwg, a.status)) return;
         }
         DEAC_PHASE(3);
         if (init) break;
@@ -696,7 +940,7 @@ __global__ void zero_u32_kernel(unsigned *p, size_t n)
 
 hipError_t launch_walk(const WalkArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(walk_kernel, dim3(1), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(walk_kernel, dim3(1), dim3(64), walk_lds_bytes(a), s, a);
     return hipGetLastError();
 }
 
@@ -708,17 +952,18 @@ hipError_t launch_mask(const MaskArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-// A regular launch: the device holds one cooperative queue, which one
+// The batch's evolution and, where next.ngen > 0, the walk of the next batch
+// on one more workgroup.  A regular launch: the device holds one cooperative queue, which one
 // process keeps once it has used it, so cooperative launches from a second
 // process fail.  The grid never exceeds the co-resident limit that
 // evolve_max_workgroups reports (one workgroup per CU, bounded by LDS), so on
 // an otherwise idle device every workgroup is resident; if one is not, the
 // bounded grid barrier reports a timeout instead of hanging.
-hipError_t launch_evolve(const EvoArgs &a, int nwg, hipStream_t s)
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, hipStream_t s)
 {
-    void *args[] = {const_cast<EvoArgs *>(&a)};
-    return hipLaunchKernel(reinterpret_cast<const void *>(evolve_kernel), dim3(nwg), dim3(kEvoThreads), args,
-                           kEvoLds, s);
+    if (next.ngen > 0 && walk_lds_bytes(next) > kEvoLds) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(evolve_kernel, dim3(a.nwg + (next.ngen > 0 ? 1 : 0)), dim3(kEvoThreads), kEvoLds, s, a, next);
+    return hipGetLastError();
 }
 
 hipError_t launch_ktile(const double *rows, double *ktile, int T, int Kc, int TB, int stride, hipStream_t s)

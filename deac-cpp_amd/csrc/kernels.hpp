@@ -31,18 +31,24 @@ constexpr int kLocalResid = 4096;
 
 // Random choices of one member in one generation, produced by walk_kernel.
 struct MemberCtl {
-    uint64_t mask_state[4];  // xoshiro256+ state at the member's first crossover-mask draw
+    uint64_t mask_state[4];  // xoshiro256+ state mask_steps draws before the member's first crossover-mask draw
     uint32_t mutant[3];      // donor indices r1, r2, r3 (deac.cpp:200-216)
     uint32_t flags;          // bit 2s: CR of sign s redrawn; bit 2s+1: F of sign s redrawn
     double cr_value[2];      // redrawn CR per sign
     double f_value[2];       // redrawn F per sign
+    uint32_t mask_steps;
 };
 
 struct WalkArgs {
     uint64_t *state;             // in/out, 4 words
     uint64_t *gen_start;         // [ngen][4] state at the top of each generation
     MemberCtl *ctl;              // [ngen][P]
-    const uint64_t *skip_rows;   // rows of T^(nsign*G), 256 x 4 words
+    const uint64_t *skip_rows;   // rows of T^(nsign*G), 256 x 4 words (serial walk)
+    const uint64_t *tab1;        // lane_tables of T^c1 (wide walk)
+    const uint64_t *tab2;        // lane_tables of T^(nsign*G+3) (wide walk)
+    const uint64_t *skip_tab;    // nibble table of T^(nsign*G) (wide walk)
+    int wide, c1;
+    const int *halt;             // status of the batch that evolves beside the walk, or null
     int ngen, P, nsign;
     uint64_t mod_magic;          // floor((2^64-1)/P)
     double tau_cr, tau_f;
@@ -50,7 +56,7 @@ struct WalkArgs {
 
 struct MaskArgs {
     const MemberCtl *ctl;        // [ngen][P]
-    const uint64_t *lane_tab;    // [64][64][16][4] nibble tables of T^(lane*chunk)
+    const uint64_t *lane_tab;    // lane_tables of T^chunk
     uint64_t *raw;               // [ngen][P][rstride] 53-bit draws (x >> 11)
     int ngen, P, Kc, chunk, rstride;
 };
@@ -85,10 +91,36 @@ struct EvoArgs {
     int *status;                 // [0] stopped, [1] generation index within the batch, [2] barrier timeout
     long gen0;                   // generation index of the batch's first generation
     int ngen;
+    int nwg;                     // workgroups that evolve
     long *iter;                  // split loop under graph capture: [0] gen0, [1] generation within the batch
                                  // (read in place of gen0 and the kernels' g), or null
 };
 
+// Wide walk: draws per lane and round for the jDE controls, donor draws per
+// member that one block looks ahead, members it holds flags of.
+constexpr int kWalkControls = 33;
+constexpr int kWalkDraws = 48;
+constexpr int kWalkMaxP = 4096;
+// The wide walk from here on (us per generation, serial and wide: 16 members
+// 11.4 and 14.3, 24 members 16.7 and 14.4, 64 members 43 and 19, 512 members
+// 340 and 65); its one test per control needs equal redraw probabilities.
+constexpr int kWalkWideP = 20;
+inline bool walk_is_wide(int P, double tau_cr, double tau_f)
+{
+    return P >= kWalkWideP && P <= kWalkMaxP && tau_cr == tau_f;
+}
+inline int walk_c1(int P, int nsign)
+{
+    const int tests = 2 * nsign * P;
+    const int c = (tests + tests / 4 + 8 + 63) / 64;
+    return c < 4 ? 4 : c > kWalkControls ? kWalkControls : c;
+}
+inline size_t walk_lds_bytes(const WalkArgs &a)
+{
+    if (!a.wide) return 256 * 4 * sizeof(uint64_t);
+    return (64 * static_cast<size_t>(a.c1 | 1)) * sizeof(uint64_t) +
+           (static_cast<size_t>(kWalkDraws) * 64 + a.P) * sizeof(uint32_t);
+}
 hipError_t launch_walk(const WalkArgs &a, hipStream_t s);
 hipError_t launch_mask(const MaskArgs &a, hipStream_t s);
 // Whether the evolution kernel's workgroups repeat the selection: the
@@ -104,7 +136,7 @@ inline size_t ktile_doubles(int TB, int stride)
     return (static_cast<size_t>(TB) * (stride / kUnit) + kKtilePad) * 64 * 2;
 }
 hipError_t launch_ktile(const double *rows, double *ktile, int T, int Kc, int TB, int stride, hipStream_t s);
-hipError_t launch_evolve(const EvoArgs &a, int nwg, hipStream_t s);
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, hipStream_t s);
 hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s);
 // Workgroups of the evolution kernel that are co-resident on the device: one
 // per CU.
