@@ -46,7 +46,7 @@ __device__ __forceinline__ int parity64(uint64_t x)
 }
 
 // The lane's jump M^lane s of a state s that all 64 lanes share, from the
-// interleaved tables of lane_tables (host_model.hpp): 128 coalesced 1 KB loads
+// interleaved tables of launch_lane_tables (init_kernels.hpp): 128 coalesced 1 KB loads
 // a wavefront.  (The same tables one after another, each lane gathering its
 // 32-byte entries, took four times as long.)
 __device__ __forceinline__ void lane_jump(const uint64_t *tab, const uint64_t (&s)[4], uint64_t (&out)[4])

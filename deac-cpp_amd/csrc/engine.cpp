@@ -49,6 +49,7 @@ struct deac_handle {
     uint64_t *gen_start[3] = {};        // by batch index modulo 3 (see the generation loop)
     uint64_t *state = nullptr, *skip_rows = nullptr, *lane_tab = nullptr;
     uint64_t *tab1 = nullptr, *tab2 = nullptr, *skip_tab_dev = nullptr;  // wide walk
+    uint64_t *columns = nullptr;        // matrices the lane tables are made of
     bool wide = false;
     uint64_t *init_start = nullptr;     // [P][4]: random state at each member's first initial draw
     std::vector<uint64_t> skip_tab;     // nibble table of T^Kc, host side
@@ -322,6 +323,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     A(h->skip_rows, 256 * 4);
     constexpr size_t kTab = 64 * 16 * 4;  // words of a nibble table
     A(h->lane_tab, deac::kLaneTabWords);
+    A(h->columns, deac::kLaneTabSets * 256 * 4);
     if (h->wide) {
         A(h->tab1, deac::kLaneTabWords);
         A(h->tab2, deac::kLaneTabWords);
@@ -336,17 +338,21 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     // Jump tables: T^(nsign*G) by rows for the serial walk and by nibbles for
     // the wide one, T^(l*chunk) by lanes for the mask generator, T^(l*c1) and
     // T^(l*(nsign*G+3)) for the wide walk.
-    std::vector<uint64_t> rows(256 * 4), tabs(deac::kLaneTabWords), tabs1, tabs2;
+    std::vector<uint64_t> rows(256 * 4);
     const deac::Gf2Matrix skip = deac::transition_power(static_cast<uint64_t>(Kc));
     deac::matrix_rows(skip, rows.data());
     h->skip_tab.resize(kTab);
     deac::nibble_table(skip, h->skip_tab.data());
-    deac::lane_tables(deac::transition_power(static_cast<uint64_t>(h->chunk)), tabs.data());
+    const int sets = h->wide ? 3 : 1;
+    deac::LaneTabArgs la{};
+    la.columns = h->columns;
+    la.tab[0] = h->lane_tab;
+    la.tab[1] = h->tab1;
+    la.tab[2] = h->tab2;
+    std::vector<deac::Gf2Matrix> steps{deac::transition_power(static_cast<uint64_t>(h->chunk))};
     if (h->wide) {
-        tabs1.resize(deac::kLaneTabWords);
-        tabs2.resize(deac::kLaneTabWords);
-        deac::lane_tables(deac::transition_power(static_cast<uint64_t>(deac::walk_c1(P, m.nsign))), tabs1.data());
-        deac::lane_tables(deac::transition_power(static_cast<uint64_t>(Kc) + 3), tabs2.data());
+        steps.push_back(deac::transition_power(static_cast<uint64_t>(deac::walk_c1(P, m.nsign))));
+        steps.push_back(deac::transition_power(static_cast<uint64_t>(Kc) + 3));
     }
     auto up = [&](void *dst, const void *src, size_t bytes) {
         if (st == DEAC_OK && hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) != hipSuccess) st = DEAC_ERR_DEVICE;
@@ -357,12 +363,9 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     up(h->obs, m.isf.data(), m.T * sizeof(double));
     up(h->sig, m.err.data(), m.T * sizeof(double));
     up(h->skip_rows, rows.data(), rows.size() * sizeof(uint64_t));
-    up(h->lane_tab, tabs.data(), tabs.size() * sizeof(uint64_t));
-    if (h->wide) {
-        up(h->tab1, tabs1.data(), tabs1.size() * sizeof(uint64_t));
-        up(h->tab2, tabs2.data(), tabs2.size() * sizeof(uint64_t));
-        up(h->skip_tab_dev, h->skip_tab.data(), h->skip_tab.size() * sizeof(uint64_t));
-    }
+    if (h->wide) up(h->skip_tab_dev, h->skip_tab.data(), h->skip_tab.size() * sizeof(uint64_t));
+    up(h->columns, steps.data(), steps.size() * sizeof(deac::Gf2Matrix));
+    if (st == DEAC_OK && deac::launch_lane_tables(la, sets, h->stream) != hipSuccess) st = DEAC_ERR_DEVICE;
     if (h->nterm) up(h->nterm, m.nterm.data(), m.Kc * sizeof(double));
     if (h->fterm) up(h->fterm, m.fterm.data(), m.Kc * sizeof(double));
     if (h->tterm) up(h->tterm, m.tterm.data(), m.Kc * sizeof(double));

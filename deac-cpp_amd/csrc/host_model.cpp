@@ -126,20 +126,6 @@ void nibble_table(const Gf2Matrix &m, uint64_t *tab)
         }
 }
 
-void lane_tables(const Gf2Matrix &m, uint64_t *tabs)
-{
-    std::vector<uint64_t> step(64 * 16 * 4), tab(64 * 16 * 4);
-    nibble_table(m, step.data());
-    Gf2Matrix acc = Gf2Matrix::identity();
-    for (int l = 0; l < 64; l++) {
-        nibble_table(acc, tab.data());
-        for (size_t e = 0; e < 64 * 16; e++)
-            for (int h = 0; h < 2; h++)
-                std::memcpy(tabs + ((e * 2 + h) * 64 + l) * 2, &tab[e * 4 + 2 * h], 2 * sizeof(uint64_t));
-        for (auto &col : acc.col) nibble_apply(step.data(), col);
-    }
-}
-
 void nibble_apply(const uint64_t *tab, uint64_t s[4])
 {
     uint64_t o[4] = {0, 0, 0, 0};

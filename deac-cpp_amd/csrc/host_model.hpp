@@ -43,11 +43,6 @@ Gf2Matrix transition_power(uint64_t n);
 void matrix_rows(const Gf2Matrix &m, uint64_t *rows);
 // 4-bit lookup table: tab[n][v] = M * (v << 4n), 64 x 16 x 4 words.
 void nibble_table(const Gf2Matrix &m, uint64_t *tab);
-// Nibble tables of M^0 .. M^63, interleaved: tabs[n][v][half][l][2] is half
-// (words 0-1, 2-3) of M^l * (v << 4n), so that 64 lanes that jump one common
-// state by different powers load side by side.  64 x 16 x 2 x 64 x 2 words.
-constexpr size_t kLaneTabWords = 64 * 16 * 4 * 64;
-void lane_tables(const Gf2Matrix &m, uint64_t *tabs);
 // M s by a nibble table.
 void nibble_apply(const uint64_t *tab, uint64_t s[4]);
 

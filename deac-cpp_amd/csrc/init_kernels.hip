@@ -1,5 +1,6 @@
-// gfx950 kernels of the initial populations (deac.cpp:430-458, 584-602): the
-// draws of every member in parallel, then the normalization.  The host only
+// gfx950 kernels of the engines' set-up: jump tables, and the initial
+// populations (deac.cpp:430-458, 584-602): the draws of every member in
+// parallel, then the normalization.  The host only
 // computes the random state at each member's first draw (one GF(2) jump per
 // member).  Compiled with -ffp-contract=off.
 #include <hip/hip_runtime.h>
@@ -80,7 +81,70 @@ __global__ __launch_bounds__(kThreads) void init_normalize_kernel(InitArgs a)
     for (int k = lane; k < Kc; k += kWave) x[k] *= scale;
 }
 
+// One workgroup per matrix: thread b carries column b of M^l from power to
+// power by nibble lookups in LDS, and every power's 16 sums of four columns go
+// out to the lane's place.  (On the host a set of tables took 2 ms.)
+__global__ __launch_bounds__(kThreads) void lane_tables_kernel(LaneTabArgs a)
+{
+    typedef uint64_t pair __attribute__((ext_vector_type(2)));
+    struct State {
+        pair h[2];
+    };
+    __shared__ State step[64][16];  // nibble table of M
+    __shared__ State col[256];
+    const int b = threadIdx.x, n = b >> 2, v0 = (b & 3) * 4;
+    uint64_t *out = a.tab[blockIdx.x];
+    // the 4 of a nibble's 16 sums of columns that this thread forms
+    auto sums = [&](State (&s)[4]) {
+        const State c0 = col[4 * n], c1 = col[4 * n + 1], c2 = col[4 * n + 2], c3 = col[4 * n + 3];
+        for (int h = 0; h < 2; h++) {
+            pair base = {0, 0};
+            if (v0 & 4) base ^= c2.h[h];
+            if (v0 & 8) base ^= c3.h[h];
+            s[0].h[h] = base;
+            s[1].h[h] = base ^ c0.h[h];
+            s[2].h[h] = base ^ c1.h[h];
+            s[3].h[h] = s[1].h[h] ^ c1.h[h];
+        }
+    };
+    const pair *m = reinterpret_cast<const pair *>(a.columns) + (static_cast<size_t>(blockIdx.x) * 256 + b) * 2;
+    col[b].h[0] = m[0];
+    col[b].h[1] = m[1];
+    __syncthreads();
+    State s[4];
+    sums(s);
+    for (int j = 0; j < 4; j++) step[n][v0 + j] = s[j];
+    State c;  // column b of M^l, from the identity on
+    for (int h = 0; h < 2; h++)
+        c.h[h] = pair{b >> 6 == 2 * h ? UINT64_C(1) << (b & 63) : 0, b >> 6 == 2 * h + 1 ? UINT64_C(1) << (b & 63) : 0};
+    for (int l = 0; l < 64; l++) {
+        __syncthreads();
+        col[b] = c;
+        __syncthreads();
+        sums(s);
+        for (int j = 0; j < 4; j++)
+            for (int h = 0; h < 2; h++)
+                reinterpret_cast<pair *>(out)[((n * 16 + v0 + j) * 2 + h) * 64 + l] = s[j].h[h];
+        const uint64_t w[4] = {c.h[0].x, c.h[0].y, c.h[1].x, c.h[1].y};
+        pair o0 = {0, 0}, o1 = {0, 0};
+#pragma unroll
+        for (int q = 0; q < 64; q++) {
+            const State &e = step[q][(w[q >> 4] >> ((q & 15) * 4)) & 15];
+            o0 ^= e.h[0];
+            o1 ^= e.h[1];
+        }
+        c.h[0] = o0;
+        c.h[1] = o1;
+    }
+}
+
 }  // namespace
+
+hipError_t launch_lane_tables(const LaneTabArgs &a, int sets, hipStream_t s)
+{
+    hipLaunchKernelGGL(lane_tables_kernel, dim3(sets), dim3(kThreads), 0, s, a);
+    return hipGetLastError();
+}
 
 hipError_t launch_initial_population(const InitArgs &a, hipStream_t s)
 {

@@ -1,5 +1,5 @@
-// Initial populations on the device (deac.cpp:430-458, 584-602), for the
-// single-instance engine and the batch.
+// Device set-up of the engines: initial populations (deac.cpp:430-458,
+// 584-602), for the single-instance engine and the batch, and jump tables.
 #pragma once
 
 #include <hip/hip_runtime_api.h>
@@ -23,6 +23,17 @@ struct InitArgs {
     int allow_neg;
     double zeroth;
 };
+
+// Nibble tables of M^0 .. M^63, interleaved by lane: tab[n][v][half][l][2] is
+// half (words 0-1, 2-3) of M^l * (v << 4n), so that 64 lanes that jump one
+// common state by different powers load side by side (lane_jump).
+constexpr size_t kLaneTabWords = 64 * 16 * 4 * 64;
+constexpr int kLaneTabSets = 3;
+struct LaneTabArgs {
+    const uint64_t *columns;         // [sets][256][4]: the columns of each M
+    uint64_t *tab[kLaneTabSets];
+};
+hipError_t launch_lane_tables(const LaneTabArgs &a, int sets, hipStream_t s);
 
 // Draws every member's genome, then normalizes it when nterm is given.
 hipError_t launch_initial_population(const InitArgs &a, hipStream_t s);
