@@ -288,7 +288,15 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     // until the walk ends.
     const size_t trial_pairs = static_cast<size_t>(P) * h->stride / 2;
     const size_t folds = static_cast<size_t>(P) * (m.use_first + m.use_third);
-    size_t nwg = std::max(static_cast<size_t>(h->MG) * h->TB + folds, trial_pairs / 1024);
+    size_t tasks = static_cast<size_t>(h->MG) * h->TB + folds;
+    if (m.bdsf) {
+        // folds draw less memory than chains: four to a CU, once 64 have a CU
+        // of their own (32 members, 65 timeslices, 4096 positions: 42.7 us per
+        // generation with 64 workgroups, 49.8 with 160)
+        tasks = static_cast<size_t>(P) * h->TB + folds;
+        tasks = std::max(std::min<size_t>(tasks, 64), tasks / 4);
+    }
+    size_t nwg = std::max(tasks, trial_pairs / 1024);
     if (m.normalize && m.renormalize) nwg = std::max<size_t>(nwg, P);  // a workgroup renormalizes a member at a time
     if (const char *user = std::getenv("DEAC_EVOLVE_WORKGROUPS")) nwg = std::max(std::atoi(user), 1);
     h->nwg = static_cast<int>(std::clamp<size_t>(nwg, 1, std::max(maxwg - 8, 1)));
@@ -414,10 +422,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         return DEAC_ERR_INVALID_ARGUMENT;
     }
     const deac::Model &m = h->m;
-    // bdsf always runs the split loop: its trial contraction is the
-    // reference build's rounded-product fold (split_fold_kernel), not the
-    // fused kernel's exact FMA chains
-    const bool split = o->ks_precision != DEAC_PRECISION_FP64 || o->split_loop != 0 || m.bdsf;
+    const bool split = o->ks_precision != DEAC_PRECISION_FP64 || o->split_loop != 0;
     const size_t N = o->number_of_generations, P = m.P, Kc = m.Kc;
     const int nsign = m.nsign;
     hipStream_t s = h->stream;
@@ -494,8 +499,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ea.nfm_dt = h->nfm_dt;
     ea.fold_ks = m.bdsf;
     ea.rstride = h->rstride;
-    ea.local = deac::evolve_local(ea.P, ea.T, nsign);
-    ea.kmat = h->kmat;
+    ea.local = deac::evolve_local(ea.P, ea.T, nsign, m.use_nfm);
     ea.ktile = h->ktile;
     ea.nterm = h->nterm;
     ea.fterm = h->fterm;

@@ -456,8 +456,8 @@ constexpr int kRing = 2 * kChunkUnits;
 constexpr int kReadAhead = 4;
 constexpr int kSRow = kChunk + 4;
 constexpr int kChainLds = 2 * kChainRows * kSRow;
-static_assert(kChainLds >= kFoldLds, "a wave's LDS serves its folds as well");
-static_assert(kKtilePad >= kRing, "the K ring reads past the last unit");
+static_assert(kChainLds >= kFoldLds && kChainLds >= kFoldTaskLds, "a wave's LDS serves its folds as well");
+static_assert(kKtilePad >= kRing && kKtilePad >= kFoldRing, "the K rings read past the last unit");
 static_assert((kEvoWaves * kChainLds + kResidLds) * sizeof(double) <= kEvoLds, "chains and members' state fit in LDS");
 
 // One chunk of the chains: kr[h .. h+15] hold its K units and are refilled
@@ -663,11 +663,35 @@ __device__ __forceinline__ double chi_sum(const double *d, int n, bool fused, do
     return acc;
 }
 
-// Member i's fitness from its chi^2 sum (deac.cpp:957-976, 1539-1555) and
-// the greedy selection (deac.cpp:1556-1571), by one lane.
-__device__ __forceinline__ void select_member(const EvoArgs &a, const Members &s, int g, int i, double chi, bool init)
+// acc + the products w[0..n) added in tau order from LDS: the -1st moment
+// (deac.cpp:1398-1416), whose last product is fused where T is odd.
+__device__ __forceinline__ double product_sum(const EvoArgs &a, const double *w, int i, int t0, int n, double acc)
+{
+    const bool fused = (a.T & 1) && t0 + n == a.T;
+    const int m = fused ? n - 1 : n;
+    int t = 0;
+    for (; t + 8 <= m; t += 8) {
+        double v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = w[t + e];
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc = acc + v[e];
+    }
+    for (; t < m; t++) acc = acc + w[t];
+    if (fused) acc = fma(a.emod[static_cast<size_t>(i) * a.T + a.T - 1], a.nfm_dt[a.T - 1], acc);
+    return acc;
+}
+
+// Member i's fitness from its chi^2 sum and -1st moment (deac.cpp:957-976,
+// 1539-1555) and the greedy selection (deac.cpp:1556-1571), by one lane.
+__device__ __forceinline__ void select_member(const EvoArgs &a, const Members &s, int g, int i, double chi, double nfm,
+                                              bool init)
 {
     double fit = chi / static_cast<double>(a.T);
+    if (a.use_nfm) {
+        const double q = (a.nfm_value - nfm) / a.nfm_error;
+        fit = fma(q, q, fit);
+    }
     if (a.use_first) {
         const double d = a.mom[i * 4 + 1] - a.first_moment;
         fit += (d * d) / a.first_moment;
@@ -719,6 +743,9 @@ __device__ unsigned long long deac_phase_clock[4];
 // workgroups) to 8 us (255, the cache fences of an XCD's workgroups queue),
 // a repeated selection of 8 members 1.3 us.  One workgroup per CU is launched
 // (evolve_max_workgroups); a second handle's workgroup still fits beside it.
+// FOLD: the trials' model ISF as rounded-product folds (bdsf; its initial
+// population goes through the chains of the other form, deac.cpp:860).
+template <bool FOLD>
 __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a, WalkArgs next)
 {
 #ifdef DEAC_PHASE_TIMERS
@@ -742,9 +769,9 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     // different workgroups (and CUs).
     const int gwave = wid * nwg + blockIdx.x;
     unsigned target = 0;
-    const int nchain = a.MG * a.TB;
+    const int ks = (FOLD ? a.P : a.MG) * a.TB;  // contraction tasks
     const int nmom = a.use_first + a.use_third;  // moment folds per member
-    const int ntask = nchain + nmom * a.P;
+    const int ntask = ks + nmom * a.P;
     const int nblk = a.stride / kChunk;
     const int run = static_cast<int>(
         min(max(static_cast<long>(a.P) * nblk / total_waves, 1L), static_cast<long>(min(nblk, 8))));
@@ -752,9 +779,11 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const int Tp = a.T | 1;  // odd row stride: lanes of different members read different banks
 
     Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
-    double *resid = lds + kEvoWaves * kChainLds;  // [P][Tp] residuals (a.local), behind the chains' buffers
+    // [P][Tp] residuals and -1st-moment products (a.local), behind the chains' buffers
+    double *resid = lds + kEvoWaves * kChainLds;
+    double *moment = resid + static_cast<size_t>(a.P) * Tp;
     if (a.local) {
-        s.fitness = resid + static_cast<size_t>(a.P) * Tp;
+        s.fitness = moment + (a.use_nfm ? static_cast<size_t>(a.P) * Tp : 0);
         s.cr = s.fitness + a.P;
         s.f = s.cr + a.P * a.nsign;
         s.cur = reinterpret_cast<int *>(s.f + a.P * a.nsign);
@@ -770,7 +799,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     __syncthreads();
 
     for (int g = 0; g <= a.ngen; g++) {
-        const bool init = a.init_mode != 0;
+        const bool init = !FOLD && a.init_mode != 0;
         if (!init) {
             if (g == a.ngen) break;
             DEAC_PHASE(0);
@@ -855,13 +884,20 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         // or of the current genomes for the initial fitness.
         for (int task = gwave; task < ntask; task += total_waves) {
             double *buf = lds + wid * kChainLds;
-            if (task < nchain) {
+            if (task < ks) {
                 const int tb = task % a.TB, mg = task / a.TB;
-                auto row = [&](int m) { return row_of(a, s.cur, min(mg * kChainRows + m, a.P - 1), !init); };
-                chain_task(a, row(0), row(1), row(2), row(3), tb, mg, buf);
+                if constexpr (FOLD) {
+                    const double e = fold_task(a.ktile + static_cast<size_t>(tb) * a.stride * kChainTau,
+                                               row_of(a, s.cur, mg, true), nblk, a.Kc, (a.G & 1) != 0, buf);
+                    const int t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
+                    if ((lane & 3) == 0 && t < a.T) a.emod[static_cast<size_t>(mg) * a.T + t] = e;
+                } else {
+                    auto row = [&](int m) { return row_of(a, s.cur, min(mg * kChainRows + m, a.P - 1), !init); };
+                    chain_task(a, row(0), row(1), row(2), row(3), tb, mg, buf);
+                }
             } else {
-                const int i = (task - nchain) / nmom;
-                const bool third = !a.use_first || (task - nchain) % nmom != 0;
+                const int i = (task - ks) / nmom;
+                const bool third = !a.use_first || (task - ks) % nmom != 0;
                 const double m = wave_fold(row_of(a, s.cur, i, !init), third ? a.tterm : a.fterm, a.Kc, a.G, buf);
                 if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }
@@ -874,28 +910,37 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             const int total = a.P * a.T;
             for (int idx = threadIdx.x; idx < total; idx += kEvoThreads) {
                 const int i = idx / a.T, t = idx % a.T;
-                resid[i * Tp + t] = (a.obs[t] - a.emod[idx]) / a.sig[t];
+                const double e = a.emod[idx];
+                resid[i * Tp + t] = (a.obs[t] - e) / a.sig[t];
+                if (a.use_nfm) moment[i * Tp + t] = e * a.nfm_dt[t];
             }
             __syncthreads();
-            for (int i = threadIdx.x; i < a.P; i += kEvoThreads)
-                select_member(a, s, g, i, chi_sum(resid + i * Tp, a.T, a.T & 1, 0.0), init);
+            for (int i = threadIdx.x; i < a.P; i += kEvoThreads) {
+                const double chi = chi_sum(resid + i * Tp, a.T, a.T & 1, 0.0);
+                select_member(a, s, g, i, chi, a.use_nfm ? product_sum(a, moment + i * Tp, i, 0, a.T, 0.0) : 0.0, init);
+            }
             __syncthreads();
         } else {
-            // one wavefront per member, residuals in windows of kResidWave
-            double *d = lds + wid * kResidWave;
+            // one wavefront per member, residuals in windows
+            const int window = a.use_nfm ? kResidWave / 2 : kResidWave;
+            double *d = lds + wid * kResidWave, *p = d + window;
             for (int i = gwave; i < a.P; i += total_waves) {
-                double chi = 0.0;
-                for (int t0 = 0; t0 < a.T; t0 += kResidWave) {
-                    const int n = min(kResidWave, a.T - t0);
-                    for (int u = lane; u < n; u += kWave)
-                        d[u] = (a.obs[t0 + u] - a.emod[static_cast<size_t>(i) * a.T + t0 + u]) / a.sig[t0 + u];
+                double chi = 0.0, nfm = 0.0;
+                for (int t0 = 0; t0 < a.T; t0 += window) {
+                    const int n = min(window, a.T - t0);
+                    for (int u = lane; u < n; u += kWave) {
+                        const double e = a.emod[static_cast<size_t>(i) * a.T + t0 + u];
+                        d[u] = (a.obs[t0 + u] - e) / a.sig[t0 + u];
+                        if (a.use_nfm) p[u] = e * a.nfm_dt[t0 + u];
+                    }
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                     chi = chi_sum(d, n, (a.T & 1) && t0 + n == a.T, chi);
+                    if (a.use_nfm) nfm = product_sum(a, p, i, t0, n, nfm);
                     __builtin_amdgcn_wave_barrier();
                 }
-                if (lane == 0) select_member(a, s, g, i, chi, init);
+                if (lane == 0) select_member(a, s, g, i, chi, nfm, init);
             }
             if (!grid_barrier(a.bar, target, nwg, a.status)) return;
         }
@@ -913,10 +958,10 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         }
 }
 
-// K rows [T][Kc] into the chains' operand order: [tau block][unit of 8
-// positions][lane][2], lane l holding tau row l&15 at positions l>>4 and
-// (l>>4)+4 of the unit.  Past T and Kc -0.0: with genomes padded with +0.0
-// the products are -0.0 and leave every chain exactly as it is.
+// K rows [T][Kc] into operand order: [tau block][unit of 8 positions][lane][2],
+// lane l holding tau row l&15 at positions l>>4 and (l>>4)+4 of the unit.  Past
+// T and Kc -0.0: with genomes padded with +0.0 the products are -0.0 and leave
+// every sum exactly as it is.
 __global__ __launch_bounds__(256) void ktile_kernel(const double *rows, double *ktile, int T, int Kc, int TB, int nunit)
 {
     const size_t total = (static_cast<size_t>(TB) * nunit + kKtilePad) * kWave * 2;
@@ -962,7 +1007,8 @@ hipError_t launch_mask(const MaskArgs &a, hipStream_t s)
 hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, hipStream_t s)
 {
     if (next.ngen > 0 && walk_lds_bytes(next) > kEvoLds) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(evolve_kernel, dim3(a.nwg + (next.ngen > 0 ? 1 : 0)), dim3(kEvoThreads), kEvoLds, s, a, next);
+    hipLaunchKernelGGL(a.fold_ks && !a.init_mode ? evolve_kernel<true> : evolve_kernel<false>,
+                       dim3(a.nwg + (next.ngen > 0 ? 1 : 0)), dim3(kEvoThreads), kEvoLds, s, a, next);
     return hipGetLastError();
 }
 
@@ -982,18 +1028,19 @@ hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s)
 
 int evolve_max_workgroups(int device)
 {
-    int per_cu = 0, cus = 0;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(evolve_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kEvoLds) != hipSuccess)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(evolve_kernel),
-                                                     kEvoThreads, kEvoLds) != hipSuccess)
-        return 0;
+    int per_cu = 1, cus = 0;
+    for (const void *k : {reinterpret_cast<const void *>(evolve_kernel<false>),
+                          reinterpret_cast<const void *>(evolve_kernel<true>)}) {
+        int n = 0;
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kEvoLds) != hipSuccess) return 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kEvoThreads, kEvoLds) != hipSuccess) return 0;
+        per_cu = std::min(per_cu, n);
+    }
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
     // One workgroup per CU: the grid barrier needs every workgroup resident,
     // and a second one per CU is not guaranteed to be even where the
     // occupancy estimate allows it.
-    return std::min(per_cu, 1) * cus;
+    return per_cu * cus;
 }
 
 }  // namespace deac

@@ -72,9 +72,8 @@ struct EvoArgs {
     int use_nfm;                 // -1st-moment term of the fitness (bdsf): weights nfm_dt [T]
     double nfm_value, nfm_error;
     const double *nfm_dt;
-    int fold_ks;                 // the trials' model ISF as a rounded-product fold (bdsf; split loop only)
-    const double *kmat;          // [T][Kc] rows (bdsf folds)
-    const double *ktile;         // K in the chains' operand order (launch_ktile)
+    int fold_ks;                 // the trials' model ISF as a rounded-product fold (bdsf)
+    const double *ktile;         // K in the chains' and folds' operand order (launch_ktile)
     const double *nterm, *fterm, *tterm;   // [Kc] or null
     const double *obs, *sig;     // [T]
     double *pop0, *pop1;         // [MG*4][stride] each, member-major rows, zero padded
@@ -125,10 +124,10 @@ hipError_t launch_walk(const WalkArgs &a, hipStream_t s);
 hipError_t launch_mask(const MaskArgs &a, hipStream_t s);
 // Whether the evolution kernel's workgroups repeat the selection: the
 // residuals are few, and they and the members' state fit in LDS.
-inline int evolve_local(int P, int T, int nsign)
+inline int evolve_local(int P, int T, int nsign, int use_nfm)
 {
     const long resid = static_cast<long>(P) * (T | 1);
-    return resid <= kLocalResid && resid + static_cast<long>(P) * (2 + 2 * nsign) <= kResidLds;
+    return resid <= kLocalResid && resid * (1 + use_nfm) + static_cast<long>(P) * (2 + 2 * nsign) <= kResidLds;
 }
 // Doubles of the K operand of TB tau blocks.
 inline size_t ktile_doubles(int TB, int stride)

@@ -29,6 +29,7 @@
 
 #include "device_common.hpp"
 #include "evolve_common.hpp"
+#include "fold_common.hpp"
 #include "split_kernels.hpp"
 
 namespace deac {
@@ -226,17 +227,16 @@ __global__ __launch_bounds__(kThreads) void split_model_kernel(EvoArgs a, const 
 }
 
 // The trials' model ISF as the detailed-balance (bdsf) reference build sums
-// it (its loop inlines matrix_multiply_LxM_by_MxN, deac.cpp:110-118,
-// 1389-1390, as a fold of rounded products, the last of an odd count fused):
-// one thread per (member, tau), straight into emod.
-__global__ __launch_bounds__(kThreads) void split_fold_kernel(EvoArgs a)
+// it, straight into emod: one wavefront per member and 16 timeslices.
+__global__ __launch_bounds__(kWave) void split_fold_kernel(EvoArgs a)
 {
     if (stopped(a)) return;
-    const size_t total = static_cast<size_t>(a.P) * a.T;
-    for (size_t idx = grid_thread(); idx < total; idx += grid_threads()) {
-        const int n = static_cast<int>(idx / a.T), t = static_cast<int>(idx % a.T);
-        a.emod[idx] = fold_row(chain_row(a, n, false), a.kmat + static_cast<size_t>(t) * a.Kc, a.Kc, a.G);
-    }
+    __shared__ __attribute__((aligned(16))) double buf[kFoldTaskLds];
+    const int lane = threadIdx.x, tb = blockIdx.x % a.TB, i = blockIdx.x / a.TB;
+    const double e = fold_task(a.ktile + static_cast<size_t>(tb) * a.stride * kChainTau, chain_row(a, i, false),
+                               a.stride / kFoldBlock, a.Kc, (a.G & 1) != 0, buf);
+    const int t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
+    if ((lane & 3) == 0 && t < a.T) a.emod[static_cast<size_t>(i) * a.T + t] = e;
 }
 
 // First and third moment rows of the contraction's genomes, one thread per
@@ -383,9 +383,7 @@ hipError_t launch_split_model(const EvoArgs &a, const float *part, int slices, i
 
 hipError_t launch_split_fold(const EvoArgs &a, hipStream_t s)
 {
-    const size_t total = static_cast<size_t>(a.P) * a.T;
-    const int blocks = static_cast<int>(std::min<size_t>((total + kThreads - 1) / kThreads, 4096));
-    hipLaunchKernelGGL(split_fold_kernel, dim3(blocks), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL(split_fold_kernel, dim3(a.P * a.TB), dim3(kWave), 0, s, a);
     return hipGetLastError();
 }
 

@@ -19,6 +19,15 @@ pytestmark = pytest.mark.gpu
     (6, 5, 191, {}), (12, 48, 192, {}), (8, 65, 193, {}), (4, 3, 256, {}), (13, 64, 321, {}),
     (8, 20, 127, dict(zero_temperature=True)), (8, 20, 385, dict(zero_temperature=True)),
     (63, 65, 70, {}), (64, 64, 70, {}), (64, 65, 70, {}), (65, 63, 40, dict(normalize=True)), (130, 31, 33, {}),
+    # bdsf folds: chunks of 32 positions, odd lengths fuse the last, both forms of the -1st moment's sum
+    (4, 2, 2, dict(spectra_type="bdsf")), (6, 17, 31, dict(spectra_type="bdsf")),
+    (5, 16, 32, dict(spectra_type="bdsf", use_negative_first_moment=True)),
+    (9, 33, 33, dict(spectra_type="bdsf", use_negative_first_moment=True)),
+    (8, 65, 127, dict(spectra_type="bdsf", use_negative_first_moment=True, normalize=True)),
+    (13, 18, 257, dict(spectra_type="bdsf", model="hyperbolic")),
+    (70, 66, 129, dict(spectra_type="bdsf", use_negative_first_moment=True)),
+    (66, 600, 40, dict(spectra_type="bdsf", use_negative_first_moment=True)),
+    (5, 1101, 21, dict(spectra_type="bdsf", use_negative_first_moment=True)),
     (130, 33, 33, {}), (10, 20, 255, dict(first_moment=1.5)),
     (6, 20, 64, dict(normalize=True, third_moment=900.0, third_moment_error=9.0)),
     (5, 9, 193, dict(normalize=True, renormalize=True, first_moment=1.5, third_moment=900.0, third_moment_error=9.0)),
@@ -35,6 +44,9 @@ def test_plain_path_shapes_match_oracle(P, T, G, kw):
                                stop_minimum_fitness=0.0, **kw), seed)
     with da.Engine(da.make_problem(tau, isf, 1e-2 * isf, freq, 1.35, population_size=P, **kw)) as e:
         g = e.run(seed, N, 0.0)
+        if "bdsf" in kw.values():
+            split = e.run(seed, N, 0.0, split_loop=True)
+            assert gc.bit_diff(g["minimum"], split["minimum"]) is None and g["rng"] == split["rng"]
     for k in ("minimum", "mean", "squared_mean", "dsf", "fitness"):
         assert gc.bit_diff(g[k], o[k]) is None, (k, gc.bit_diff(g[k], o[k]))
     assert g["rng"] == o["rng"]
