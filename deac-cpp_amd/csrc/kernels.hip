@@ -460,10 +460,35 @@ static_assert(kChainLds >= kFoldLds && kChainLds >= kFoldTaskLds, "a wave's LDS 
 static_assert(kKtilePad >= kRing && kKtilePad >= kFoldRing, "the K rings read past the last unit");
 static_assert((kEvoWaves * kChainLds + kResidLds) * sizeof(double) <= kEvoLds, "chains and members' state fit in LDS");
 
+// A tau block's K units from a moving chunk on, as buffer loads: the base is
+// scalar and the unit an immediate offset from one of four lane offsets, so a
+// load is one instruction with one address register (with 64-bit lane
+// addresses a unit took 28 ns, 24.5 this way).
+struct KUnits {
+    static_assert(kChunkUnits == 16, "four lane offsets, four units each");
+    const char *base;
+    int vo[4];
+    __device__ __forceinline__ KUnits(const double *p)
+        : base(reinterpret_cast<const char *>(p))
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            vo[k] = (threadIdx.x & (kWave - 1)) * 16 + k * 4096;
+            asm("" : "+v"(vo[k]));  // a register each
+        }
+    }
+    __device__ __forceinline__ dvec2 load(int i) const
+    {
+        const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(base), 0, kChunkUnits * 1024, 0x00020000);
+        return __builtin_bit_cast(dvec2, __builtin_amdgcn_raw_buffer_load_b128(r, vo[i >> 2] + (i & 3) * 1024, 0, 0));
+    }
+    __device__ __forceinline__ void advance() { base += kChunkUnits * 1024; }
+};
+
 // One chunk of the chains: kr[h .. h+15] hold its K units and are refilled
 // with those two chunks on; sr holds the genome units about to be used.
 template <int H>
-__device__ __forceinline__ void chain_chunk(double &acc, dvec2 (&kr)[kRing], dvec2 (&sr)[kReadAhead], const dvec2 *&ka,
+__device__ __forceinline__ void chain_chunk(double &acc, dvec2 (&kr)[kRing], dvec2 (&sr)[kReadAhead], KUnits &ku,
                                             const double *here, const double *next)
 {
 #pragma unroll
@@ -478,10 +503,10 @@ __device__ __forceinline__ void chain_chunk(double &acc, dvec2 (&kr)[kRing], dve
         __builtin_amdgcn_sched_barrier(0);
         acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.y, s.y, acc, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        kr[H + i] = ka[i * kWave];
+        kr[H + i] = ku.load(i);
         __builtin_amdgcn_sched_barrier(0);
     }
-    ka += kChunkUnits * kWave;
+    ku.advance();
 }
 
 // Model ISF E[i][t] of one (tau block, member group) task on one wavefront:
@@ -509,8 +534,7 @@ __device__ __forceinline__ void chain_task(const EvoArgs &a, const double *r0, c
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int nchunk = a.stride / kChunk;
-    const dvec2 *ka = reinterpret_cast<const dvec2 *>(a.ktile) +
-                      static_cast<size_t>(tb) * nchunk * kChunkUnits * kWave + lane;
+    KUnits ku(a.ktile + static_cast<size_t>(tb) * nchunk * kChunkUnits * (2 * kWave));
     struct Stage {
         dvec2 v0, v1, v2, v3;
     };
@@ -534,8 +558,10 @@ __device__ __forceinline__ void chain_task(const EvoArgs &a, const double *r0, c
     load(0, s0);
     load(1, s1);
 #pragma unroll
-    for (int i = 0; i < kRing; i++) kr[i] = ka[i * kWave];
-    ka += kRing * kWave;
+    for (int i = 0; i < kRing; i++) {
+        kr[i] = ku.load(i % kChunkUnits);
+        if (i % kChunkUnits == kChunkUnits - 1) ku.advance();
+    }
     __builtin_amdgcn_sched_barrier(0);
     put(0, s0);
     load(2, s0);
@@ -545,11 +571,11 @@ __device__ __forceinline__ void chain_task(const EvoArgs &a, const double *r0, c
     for (int c = 0;; c += 2) {
         put(c + 1, s1);
         load(c + 3, s1);
-        chain_chunk<0>(acc, kr, sr, ka, even, odd);
+        chain_chunk<0>(acc, kr, sr, ku, even, odd);
         if (c + 1 >= nchunk) break;
         put(c + 2, s0);
         load(c + 4, s0);
-        chain_chunk<kChunkUnits>(acc, kr, sr, ka, odd, even);
+        chain_chunk<kChunkUnits>(acc, kr, sr, ku, odd, even);
         if (c + 2 >= nchunk) break;
     }
     // 4x4x4_4b output: lane l holds row l>>4 of block (l>>2)&3, column l&3
