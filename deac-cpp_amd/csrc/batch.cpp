@@ -11,6 +11,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -25,7 +26,8 @@
 #include "deac_engine.h"
 #include "host_model.hpp"
 #include "init_kernels.hpp"
-#include "ks_layout.hpp"
+#include "kernels.hpp"
+#include "pack_kernels.hpp"
 
 namespace {
 
@@ -254,6 +256,25 @@ deac_status plan_model(BatchModel &b, std::string &why)
     return DEAC_OK;
 }
 
+// Device memory for the rows of one kernel matrix while they are packed.
+struct TempRows {
+    double *rows = nullptr;
+    int *ex = nullptr;
+    ~TempRows()
+    {
+        if (rows) (void)hipFree(rows);
+        if (ex) (void)hipFree(ex);
+    }
+    bool alloc(size_t values, size_t exponents)
+    {
+        if (hipMalloc(reinterpret_cast<void **>(&rows), values * sizeof(double)) == hipSuccess &&
+            (exponents == 0 || hipMalloc(reinterpret_cast<void **>(&ex), exponents * sizeof(int)) == hipSuccess))
+            return true;
+        (void)hipGetLastError();
+        return false;
+    }
+};
+
 // K in the mixed kernel's operand order (batch_kernels.hpp, BatchDesc::kmix),
 // each row scaled by 2^-ex[t] with ex[t] the exponent of its largest
 // magnitude (the split loop's scaling, ks_layout.hpp), and 2^ex[t] itself.
@@ -268,39 +289,24 @@ deac_status upload_mixed(deac_batch *h, BatchModel &b, int precision)
         for (size_t k = 0; k < L; k++) mx = std::fmax(mx, std::fabs(m.kernel[t * L + k]));
         ex[t] = mx > 0.0 ? std::ilogb(mx) : 0;
     }
-    auto scaled = [&](size_t row, size_t pos) {
-        return row < T && pos < L ? std::ldexp(m.kernel[row * L + pos], -ex[row]) : 0.0;
-    };
-    const size_t tile = static_cast<size_t>(b.Lpad) * 16;  // values per 16-row tile
-    std::vector<uint32_t> img(static_cast<size_t>(b.ntm) * tile, 0);  // 4 bytes per value either way
-    if (precision == DEAC_PRECISION_FP32) {
-        // [tile][unit of 16 positions][lane][4]: row 16 tile + l % 16, position 16 u + 4 e + l / 16
-        float *f = reinterpret_cast<float *>(img.data());
-        for (int tt = 0; tt < b.ntm; tt++)
-            for (int u = 0; u < b.Lpad / 16; u++)
-                for (int l = 0; l < 64; l++)
-                    for (int e = 0; e < 4; e++)
-                        f[((static_cast<size_t>(tt) * (b.Lpad / 16) + u) * 64 + l) * 4 + e] = static_cast<float>(
-                            scaled(16 * tt + (l & 15), 16 * static_cast<size_t>(u) + 4 * e + (l >> 4)));
-    } else {
-        // [tile][32-position block][lane][8 hi, 8 lo]: row 16 tile + l % 16, position 32 u + 8 (l / 16) + e
-        uint16_t *q = reinterpret_cast<uint16_t *>(img.data());
-        for (int tt = 0; tt < b.ntm; tt++)
-            for (int u = 0; u < b.Lpad / 32; u++)
-                for (int l = 0; l < 64; l++)
-                    for (int e = 0; e < 8; e++) {
-                        uint16_t hi, lo;
-                        deac::bf16_split(scaled(16 * tt + (l & 15), 32 * static_cast<size_t>(u) + 8 * (l >> 4) + e),
-                                         hi, lo);
-                        const size_t o = ((static_cast<size_t>(tt) * (b.Lpad / 32) + u) * 64 + l) * 16 + e;
-                        q[o] = hi;
-                        q[o + 8] = lo;
-                    }
-    }
+    // rows up as they are, packed on the device: FP32 [tile][unit of 16
+    // positions][lane][4], BF16X3 [tile][32-position block][lane][8 hi, 8 lo]
+    const bool f32 = precision == DEAC_PRECISION_FP32;
     uint32_t *dk = nullptr;
-    deac_status st = h->alloc(dk, img.size());
+    deac_status st = h->alloc(dk, static_cast<size_t>(b.ntm) * b.Lpad * 16);  // 4 bytes per value either way
     if (st != DEAC_OK) return st;
-    if (hipMemcpy(dk, img.data(), img.size() * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess)
+    TempRows rows;
+    int *dex = nullptr;
+    if (!rows.alloc(T * L, T)) return DEAC_ERR_OUT_OF_MEMORY;
+    dex = rows.ex;
+    if (hipMemcpyAsync(rows.rows, m.kernel.data(), T * L * sizeof(double), hipMemcpyHostToDevice, h->stream) !=
+            hipSuccess ||
+        hipMemcpyAsync(dex, ex.data(), T * sizeof(int), hipMemcpyHostToDevice, h->stream) != hipSuccess)
+        return DEAC_ERR_DEVICE;
+    const deac::PackArgs pk{rows.rows, dex, static_cast<int>(T), static_cast<int>(L), b.ntm, b.Lpad / (f32 ? 16 : 32)};
+    if ((f32 ? deac::launch_pack_fp32_units(pk, reinterpret_cast<float *>(dk), h->stream)
+             : deac::launch_pack_bf16x3(pk, dk, nullptr, h->stream)) != hipSuccess ||
+        hipStreamSynchronize(h->stream) != hipSuccess)
         return DEAC_ERR_DEVICE;
     if (!b.kscale) {
         std::vector<double> sc(T);
@@ -318,16 +324,6 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     const deac::Model &m = b.m;
     const int T = static_cast<int>(m.T), L = static_cast<int>(m.Kc);
     const int nkb2 = b.Lpad / 8;
-    std::vector<double> kt(static_cast<size_t>(std::max(b.ntt, 1)) * nkb2 * 64 * 2, -0.0);
-    for (int t = 0; t < b.ntt; t++)
-        for (int kb2 = 0; kb2 < nkb2; kb2++)
-            for (int l = 0; l < 64; l++)
-                for (int e = 0; e < 2; e++) {
-                    const int tau = t * 16 + (l & 15), slot = (2 * kb2 + e) * 4 + (l >> 4);
-                    double v = -0.0;
-                    if (tau < T && slot < L) v = m.kernel[static_cast<size_t>(tau) * L + slot];
-                    kt[((static_cast<size_t>(t) * nkb2 + kb2) * 64 + l) * 2 + e] = v;
-                }
     // Rows ntt*16 .. T-1 for v_mfma_f64_4x4x4_4b: per 8 positions, 4 nrem
     // pairs (row r + nrem * position k of a 4-position block; the pair holds
     // the two blocks).  Lane l with l & 3 < nrem reads entry
@@ -360,7 +356,10 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     auto A = [&](auto *&p, size_t n) {
         if (st == DEAC_OK) st = h->alloc(p, n);
     };
-    A(b.ktile, kt.size());
+    const size_t ktile_n = static_cast<size_t>(std::max(b.ntt, 1)) * b.Lpad * 16;
+    A(b.ktile, ktile_n + deac::kKtilePad * 128);  // (launch_ktile writes a margin)
+    TempRows tmp;
+    if (st == DEAC_OK && !tmp.alloc(m.T * m.Kc, 0)) st = DEAC_ERR_OUT_OF_MEMORY;
     A(b.krem, kr.size());
     A(b.obs, m.T);
     A(b.sig, m.T);
@@ -385,7 +384,12 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     auto up = [&](void *dst, const void *src, size_t bytes) {
         if (st == DEAC_OK && hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) != hipSuccess) st = DEAC_ERR_DEVICE;
     };
-    up(b.ktile, kt.data(), kt.size() * sizeof(double));
+    up(tmp.rows, m.kernel.data(), m.T * m.Kc * sizeof(double));
+    // [tile][8 positions][lane][2] (the plain engine's order), -0.0 past T and L
+    if (st == DEAC_OK &&
+        deac::launch_ktile(tmp.rows, b.ktile, std::min(T, b.ntt * 16), L, std::max(b.ntt, 1), b.Lpad, h->stream) !=
+            hipSuccess)
+        st = DEAC_ERR_DEVICE;
     up(b.krem, kr.data(), kr.size() * sizeof(double));
     up(b.obs, m.isf.data(), m.T * sizeof(double));
     up(b.sig, m.err.data(), m.T * sizeof(double));
@@ -395,16 +399,16 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
     if (b.mterm) up(b.mterm, mt.data(), mt.size() * sizeof(double));
     if (m.bdsf && st == DEAC_OK) {
         // [Lpad][fold_rows]: the timeslices of a position contiguous
-        const int rw = b.fold_rows;
-        std::vector<double> kf(static_cast<size_t>(b.Lpad) * rw, 0.0);
-        for (int t = 0; t < T; t++)
-            for (int k = 0; k < L; k++)
-                kf[static_cast<size_t>(k) * rw + t] = m.kernel[static_cast<size_t>(t) * L + k];
-        A(b.kfold, kf.size());
+        A(b.kfold, static_cast<size_t>(b.Lpad) * b.fold_rows);
         if (m.use_nfm) A(b.nfm_dt, m.T);
-        up(b.kfold, kf.data(), kf.size() * sizeof(double));
+        const deac::PackArgs pk{tmp.rows, nullptr, T, L, 0, 0};
+        if (st == DEAC_OK &&
+            deac::launch_pack_transposed(pk, b.fold_rows, b.Lpad, b.kfold, h->stream) != hipSuccess)
+            st = DEAC_ERR_DEVICE;
         if (b.nfm_dt) up(b.nfm_dt, m.nfm_dt.data(), m.T * sizeof(double));
     }
+    // the packing reads the temporary rows
+    if (hipStreamSynchronize(h->stream) != hipSuccess && st == DEAC_OK) st = DEAC_ERR_DEVICE;
     return st;
 }
 

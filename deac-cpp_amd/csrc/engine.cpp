@@ -14,6 +14,7 @@
 #include "init_kernels.hpp"
 #include "kernels.hpp"
 #include "ks_layout.hpp"
+#include "pack_kernels.hpp"
 #include "precision_kernels.hpp"
 #include "split_kernels.hpp"
 
@@ -136,46 +137,39 @@ deac_status prepare_split(deac_handle *h, int precision)
     const deac::Model &m = h->m;
     sp.y = deac::ks_layout(m, precision, m.P);
     const deac::KsLayout &y = sp.y;
-    auto up = [](void *dst, const void *src, size_t bytes) {
-        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess ? DEAC_OK : DEAC_ERR_DEVICE;
-    };
+    if (precision != DEAC_PRECISION_FP64) {
+        DEAC_TRY(h->alloc(sp.part, static_cast<size_t>(y.slices) * y.mpad() * y.npad()));
+        DEAC_TRY(h->alloc(sp.ex, y.T));
+        DEAC_HIP(hipMemcpy(sp.ex, y.ex.data(), y.T * sizeof(int), hipMemcpyHostToDevice));
+    }
+    // K padded with -0.0 at FP64 (with genomes padded with +0.0 the padded
+    // products are -0.0 and leave every chain exactly as it is), 0 otherwise
+    const deac::PackArgs pk{h->kmat, sp.ex, static_cast<int>(y.T), static_cast<int>(y.L), y.Mt, static_cast<int>(y.Kb)};
     if (precision == DEAC_PRECISION_FP64) {
-        std::vector<double> A;
-        deac::ks_kernel_fp64(m, y, A);
         double *a = nullptr, *b = nullptr;
-        DEAC_TRY(h->alloc(a, A.size()));
+        DEAC_TRY(h->alloc(a, y.a_count()));
         sp.A = a;
         DEAC_TRY(h->alloc(b, y.b_count()));
         sp.B = b;
-        DEAC_TRY(up(a, A.data(), A.size() * sizeof(double)));
+        DEAC_HIP(deac::launch_pack_fp64(pk, -0.0, a, h->stream));
     } else if (precision == DEAC_PRECISION_FP32) {
-        std::vector<float> A;
-        deac::ks_kernel_fp32(m, y, A);
         float *a = nullptr, *b = nullptr;
-        DEAC_TRY(h->alloc(a, A.size()));
+        DEAC_TRY(h->alloc(a, y.a_count()));
         sp.A = a;
         DEAC_TRY(h->alloc(b, y.b_count()));
         sp.B = b;
-        DEAC_TRY(up(a, A.data(), A.size() * sizeof(float)));
+        DEAC_HIP(deac::launch_pack_fp32(pk, a, h->stream));
     } else {
-        std::vector<uint16_t> Ah, Al;
-        deac::ks_kernel_bf16x3(m, y, Ah, Al);
         uint16_t *ah = nullptr, *al = nullptr, *bh = nullptr, *bl = nullptr;
-        DEAC_TRY(h->alloc(ah, Ah.size()));
+        DEAC_TRY(h->alloc(ah, y.a_count()));
         sp.A = ah;
-        DEAC_TRY(h->alloc(al, Al.size()));
+        DEAC_TRY(h->alloc(al, y.a_count()));
         sp.Al = al;
         DEAC_TRY(h->alloc(bh, y.b_count()));
         sp.B = bh;
         DEAC_TRY(h->alloc(bl, y.b_count()));
         sp.Bl = bl;
-        DEAC_TRY(up(ah, Ah.data(), Ah.size() * sizeof(uint16_t)));
-        DEAC_TRY(up(al, Al.data(), Al.size() * sizeof(uint16_t)));
-    }
-    if (precision != DEAC_PRECISION_FP64) {
-        DEAC_TRY(h->alloc(sp.part, static_cast<size_t>(y.slices) * y.mpad() * y.npad()));
-        DEAC_TRY(h->alloc(sp.ex, y.T));
-        DEAC_TRY(up(sp.ex, y.ex.data(), y.T * sizeof(int)));
+        DEAC_HIP(deac::launch_pack_bf16x3(pk, ah, al, h->stream));
     }
     sp.precision = precision;
     return DEAC_OK;

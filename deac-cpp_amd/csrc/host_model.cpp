@@ -4,9 +4,13 @@
 // evaluates the expressions below.
 #include "host_model.hpp"
 
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <system_error>
+#include <thread>
 
 namespace deac {
 
@@ -240,6 +244,29 @@ static double trapezoid_weight(const std::vector<double> &f, size_t j)  // deac.
     return 0.5 * (f[j + 1] - f[j - 1]);
 }
 
+// fn(i) for i < rows, on several host threads where the rows hold enough
+// values (an exponential each) to pay for starting them.
+template <class F>
+static void parallel_rows(size_t rows, size_t values, F fn)
+{
+    const size_t most = std::clamp<size_t>(std::thread::hardware_concurrency(), 1, 16);
+    const size_t nt = std::min({rows, most, values >> 15});
+    std::vector<std::thread> th;
+    std::atomic<size_t> next{0};
+    auto work = [&] {
+        for (size_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < rows;) fn(i);
+    };
+    for (size_t t = 1; t < nt; t++) {
+        try {
+            th.emplace_back(work);
+        } catch (const std::system_error &) {  // no more threads: the ones there are do it
+            break;
+        }
+    }
+    work();
+    for (auto &x : th) x.join();
+}
+
 Model build_model(const deac_problem &p)
 {
     Model m;
@@ -278,7 +305,7 @@ Model build_model(const deac_problem &p)
 
     // Kernel matrix, deac.cpp:318-401.
     m.kernel.assign(m.T * Kc, 0.0);
-    for (size_t i = 0; i < m.T; i++) {
+    parallel_rows(m.T, m.T * Kc, [&](size_t i) {
         const double t = m.tau[i];
         double *kp = &m.kernel[i * Kc];
         double *km = m.nsign == 2 ? kp + G : nullptr;
@@ -321,7 +348,7 @@ Model build_model(const deac_problem &p)
                 km[j] = per * df * std::exp(tmb * w);
             }
         }
-    }
+    });
 
     // Normalization / first-moment / third-moment vectors (deac.cpp:495-538,
     // 628-668, 728-768).  which: 0 = normalization, 1 = first, 3 = third.

@@ -17,6 +17,7 @@
 #include "deac_engine.h"
 #include "host_model.hpp"
 #include "ks_layout.hpp"
+#include "pack_kernels.hpp"
 #include "precision_kernels.hpp"
 
 namespace {
@@ -128,14 +129,39 @@ extern "C" deac_status deac_model_isf(const deac_problem *p, const double *genom
     Buffers buf;
     const size_t asz = y.a_count(), bsz = y.b_count();
 
+    // K and the genomes go up as they are and are packed on the device, the
+    // genomes in blocks of whole tiles of at most about 256 MiB
+    double *krows, *grows;
+    const size_t L = y.L;
+    const size_t block = std::min<size_t>(static_cast<size_t>(y.Nt) * 16,
+                                          std::max<size_t>(1, (size_t(1) << 21) / L) * 16);
+    if (!buf.alloc(krows, m.T * L) || !buf.alloc(grows, block * L)) return DEAC_ERR_OUT_OF_MEMORY;
+    PREC_HIP(hipMemcpyAsync(krows, m.kernel.data(), m.T * L * sizeof(double), hipMemcpyHostToDevice, s));
+    auto pack_genomes = [&](auto pack) -> deac_status {
+        for (size_t n0 = 0; n0 < count; n0 += block) {
+            const size_t n = std::min(block, count - n0);
+            PREC_HIP(hipMemcpyAsync(grows, genomes + n0 * L, n * L * sizeof(double), hipMemcpyHostToDevice, s));
+            const int tiles = static_cast<int>((n + 15) / 16);
+            PREC_HIP(pack(deac::PackArgs{grows, nullptr, static_cast<int>(n), static_cast<int>(L), tiles, Kb},
+                          n0 / 16 * y.Kb * 64 * y.per));
+        }
+        return DEAC_OK;
+    };
+    int *ex = nullptr;
+    if (!y.ex.empty()) {
+        if (!buf.alloc(ex, m.T)) return DEAC_ERR_OUT_OF_MEMORY;
+        PREC_HIP(hipMemcpyAsync(ex, y.ex.data(), m.T * sizeof(int), hipMemcpyHostToDevice, s));
+    }
+    const deac::PackArgs pk{krows, ex, T, static_cast<int>(L), y.Mt, Kb};
     if (precision == DEAC_PRECISION_FP64) {
-        std::vector<double> A, B;
-        deac::ks_kernel_fp64(m, y, A);
-        deac::ks_genomes_fp64(y, genomes, B);
         double *dA, *dB, *dE;
         if (!buf.alloc(dA, asz) || !buf.alloc(dB, bsz) || !buf.alloc(dE, E.size())) return DEAC_ERR_OUT_OF_MEMORY;
-        PREC_HIP(hipMemcpyAsync(dA, A.data(), asz * sizeof(double), hipMemcpyHostToDevice, s));
-        PREC_HIP(hipMemcpyAsync(dB, B.data(), bsz * sizeof(double), hipMemcpyHostToDevice, s));
+        // -0.0 past K's rows and positions: with genomes padded with +0.0 the
+        // padded products are -0.0 and leave every chain exactly as it is
+        PREC_HIP(deac::launch_pack_fp64(pk, -0.0, dA, s));
+        const deac_status st = pack_genomes(
+            [&](const deac::PackArgs &a, size_t at) { return deac::launch_pack_fp64(a, 0.0, dB + at, s); });
+        if (st != DEAC_OK) return st;
         PREC_HIP(deac::launch_ks_fp64(dA, dB, dE, T, N, y.Mt, y.Nt, Kb, s, e0, e1, nullptr));
         PREC_HIP(hipMemcpyAsync(E.data(), dE, E.size() * sizeof(double), hipMemcpyDeviceToHost, s));
         PREC_HIP(hipStreamSynchronize(s));
@@ -143,35 +169,28 @@ extern "C" deac_status deac_model_isf(const deac_problem *p, const double *genom
         const size_t mn = y.mpad() * y.npad();
         float *part, *out;
         if (!buf.alloc(part, static_cast<size_t>(y.slices) * mn) || !buf.alloc(out, mn)) return DEAC_ERR_OUT_OF_MEMORY;
-        // Each branch queues the slice sum before its host operands are
-        // freed (a few ms for large stacks), so the end event follows the
-        // contraction directly.
         if (precision == DEAC_PRECISION_FP32) {
-            std::vector<float> A, B;
-            deac::ks_kernel_fp32(m, y, A);
-            deac::ks_genomes_fp32(y, genomes, B);
             float *dA, *dB;
             if (!buf.alloc(dA, asz) || !buf.alloc(dB, bsz)) return DEAC_ERR_OUT_OF_MEMORY;
-            PREC_HIP(hipMemcpyAsync(dA, A.data(), asz * sizeof(float), hipMemcpyHostToDevice, s));
-            PREC_HIP(hipMemcpyAsync(dB, B.data(), bsz * sizeof(float), hipMemcpyHostToDevice, s));
+            PREC_HIP(deac::launch_pack_fp32(pk, dA, s));
+            const deac_status st = pack_genomes(
+                [&](const deac::PackArgs &a, size_t at) { return deac::launch_pack_fp32(a, dB + at, s); });
+            if (st != DEAC_OK) return st;
             PREC_HIP(deac::launch_ks_fp32(dA, dB, part, y.Mt, y.Nt, Kb, y.kb_per_slice, y.slices, s, e0, nullptr,
                                           nullptr));
-            PREC_HIP(deac::launch_reduce_slices(part, out, y.slices, mn, s, nullptr, e1));
         } else {
-            std::vector<uint16_t> Ah, Al, Bh, Bl;
-            deac::ks_kernel_bf16x3(m, y, Ah, Al);
-            deac::ks_genomes_bf16x3(y, genomes, Bh, Bl);
             uint16_t *dAh, *dAl, *dBh, *dBl;
             if (!buf.alloc(dAh, asz) || !buf.alloc(dAl, asz) || !buf.alloc(dBh, bsz) || !buf.alloc(dBl, bsz))
                 return DEAC_ERR_OUT_OF_MEMORY;
-            PREC_HIP(hipMemcpyAsync(dAh, Ah.data(), asz * 2, hipMemcpyHostToDevice, s));
-            PREC_HIP(hipMemcpyAsync(dAl, Al.data(), asz * 2, hipMemcpyHostToDevice, s));
-            PREC_HIP(hipMemcpyAsync(dBh, Bh.data(), bsz * 2, hipMemcpyHostToDevice, s));
-            PREC_HIP(hipMemcpyAsync(dBl, Bl.data(), bsz * 2, hipMemcpyHostToDevice, s));
+            PREC_HIP(deac::launch_pack_bf16x3(pk, dAh, dAl, s));
+            const deac_status st = pack_genomes([&](const deac::PackArgs &a, size_t at) {
+                return deac::launch_pack_bf16x3(a, dBh + at, dBl + at, s);
+            });
+            if (st != DEAC_OK) return st;
             PREC_HIP(deac::launch_ks_bf16x3(dAh, dAl, dBh, dBl, part, y.Mt, y.Nt, Kb, y.kb_per_slice, y.slices, s,
                                             e0, nullptr, nullptr));
-            PREC_HIP(deac::launch_reduce_slices(part, out, y.slices, mn, s, nullptr, e1));
         }
+        PREC_HIP(deac::launch_reduce_slices(part, out, y.slices, mn, s, nullptr, e1));
         std::vector<float> E32(mn);
         PREC_HIP(hipMemcpyAsync(E32.data(), out, E32.size() * sizeof(float), hipMemcpyDeviceToHost, s));
         PREC_HIP(hipStreamSynchronize(s));
