@@ -122,6 +122,11 @@ struct deac_batch {
                                                // each member's first initial draw
     long *init_off = nullptr;                  // instances, model by model: offset of the population in pop
     size_t init_rows = 0;
+    double *best_rows = nullptr;               // [genomes of all instances]: best members, gathered for the readback
+    long *best_off = nullptr;                  // per instance: offset in best_rows, of its population, P, Kc, Lpad
+    std::vector<size_t> best_at;               // offset in best_rows, host side
+    double *stats_ws = nullptr;                // statistics histories, kept between runs and grown on demand
+    size_t stats_cap = 0;
     double *scratch = nullptr;                 // this device's statistics scratch (deac_batch_run_noalloc)
     std::vector<long> reached;                 // per instance: generation reached by the last run (absolute)
     std::vector<char> epar_valid;              // per instance: epar holds the current population's model ISF
@@ -531,11 +536,24 @@ deac_status deac_batch_create(const deac_problem *problems, size_t count, deac_b
         for (size_t i : b->insts) init_off.push_back(static_cast<long>(h->pop_off[i]));
         h->init_rows += b->insts.size() * b->m.P;
     }
+    h->best_at.resize(count);
+    size_t nbest = 0;
+    std::vector<long> best_off;
+    for (size_t i = 0; i < count; i++) {
+        const BatchModel &b = *h->models[h->model_of[i]];
+        h->best_at[i] = nbest;
+        for (size_t v : {nbest, h->pop_off[i], b.m.P, b.m.Kc, static_cast<size_t>(b.Lpad)})
+            best_off.push_back(static_cast<long>(v));
+        nbest += b.m.Kc;
+    }
+    A(h->best_rows, nbest);
+    A(h->best_off, best_off.size());
     A(h->init_start, h->init_rows * 4);
     A(h->init_off, count);
     A(h->descs, 3 * count);  // evolution launches, and the evaluation launches of mixed K.S before and after
     if (st != DEAC_OK) return st;
     BATCH_HIP(hipMemcpy(h->init_off, init_off.data(), count * sizeof(long), hipMemcpyHostToDevice));
+    BATCH_HIP(hipMemcpy(h->best_off, best_off.data(), best_off.size() * sizeof(long), hipMemcpyHostToDevice));
     // pinned host sides of the per-round descriptor upload and status read
     if (hipHostMalloc(reinterpret_cast<void **>(&h->hdescs), 3 * count * sizeof(deac::BatchDesc)) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void **>(&h->hstatus), 2 * count * sizeof(long)) != hipSuccess) {
@@ -671,31 +689,24 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
         BATCH_HIP(hipStreamSynchronize(s));
     }
 
-    // Statistics buffers for the instances that track them.
+    // Statistics buffers for the instances that track them, packed.
     std::vector<double *> stats(n, nullptr);
-    struct Freer {
-        deac_batch *h;
-        std::vector<double *> &v;
-        bool own;
-        ~Freer()
-        {
-            if (own)
-                for (double *p : v)
-                    if (p) h->release(p);
-        }
-    } freer{h, stats, stats_pool == nullptr};
-    if (stats_pool) {
-        size_t off = 0;
-        for (size_t i = 0; i < n; i++)
-            if (options[i].track_stats) {
-                stats[i] = stats_pool + off;
-                off += 3 * options[i].number_of_generations;
-            }
-    } else {
-        for (size_t i = 0; i < n; i++)
-            if (options[i].track_stats && h->alloc(stats[i], 3 * options[i].number_of_generations) != DEAC_OK)
-                return DEAC_ERR_OUT_OF_MEMORY;
+    size_t stats_n = 0;
+    for (size_t i = 0; i < n; i++)
+        if (options[i].track_stats) stats_n += 3 * options[i].number_of_generations;
+    if (!stats_pool && stats_n > h->stats_cap) {
+        h->release(h->stats_ws);
+        h->stats_ws = nullptr;
+        h->stats_cap = 0;
+        if (h->alloc(h->stats_ws, stats_n) != DEAC_OK) return DEAC_ERR_OUT_OF_MEMORY;
+        h->stats_cap = stats_n;
     }
+    double *const stats_base_ptr = stats_pool ? stats_pool : h->stats_ws;
+    for (size_t i = 0, off = 0; i < n; i++)
+        if (options[i].track_stats) {
+            stats[i] = stats_base_ptr + off;
+            off += 3 * options[i].number_of_generations;
+        }
 
     // Launch slices: every active instance evolves up to `slice` generations
     // per launch; stopped or finished instances leave the next launch.
@@ -1023,10 +1034,18 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
     h->last = prof;
 
     // Epilogue per instance (deac.cpp:1576-1685), as deac_run.
+    // The best members' rows are gathered on the device: one copy each for the
+    // fitnesses, the random states, the rows and the statistics.
+    const size_t last = n - 1;
+    std::vector<double> rows(h->best_at[last] + h->models[h->model_of[last]]->m.Kc), stats_host(stats_n);
+    BATCH_HIP(deac::launch_gather_best(h->best_off, n, h->fitness, deac::kBatchMaxP, h->pop, h->best_rows, s));
+    BATCH_HIP(hipStreamSynchronize(s));
+    BATCH_HIP(hipMemcpy(rows.data(), h->best_rows, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
+    if (stats_n)
+        BATCH_HIP(hipMemcpy(stats_host.data(), stats_base_ptr, stats_n * sizeof(double), hipMemcpyDeviceToHost));
     std::vector<double> fit_all(n * deac::kBatchMaxP);
     BATCH_HIP(hipMemcpy(fit_all.data(), h->fitness, fit_all.size() * sizeof(double), hipMemcpyDeviceToHost));
     BATCH_HIP(hipMemcpy(rng_host.data(), h->rng, rng_host.size() * sizeof(uint64_t), hipMemcpyDeviceToHost));
-    std::vector<double> row;
     for (size_t i = 0; i < n; i++) {
         const BatchModel &b = *h->models[h->model_of[i]];
         const deac::Model &m = b.m;
@@ -1040,18 +1059,14 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
                 minimum = fit[k];
                 best = k;
             }
-        row.resize(m.Kc);
-        BATCH_HIP(hipMemcpy(row.data(), h->pop + h->pop_off[i] + best * b.Lpad, m.Kc * sizeof(double),
-                            hipMemcpyDeviceToHost));
-        deac::output_transform(m, row.data(), r->dsf, r->frequency);
+        deac::output_transform(m, &rows[h->best_at[i]], r->dsf, r->frequency);
         size_t generation = stopped_at[i] >= 0 ? static_cast<size_t>(stopped_at[i] - base[i]) : N - 2;
         if (stats[i]) {
-            std::vector<double> hs(3 * N, 0.0);
+            const double *hs = &stats_host[static_cast<size_t>(stats[i] - stats_base_ptr)];
             const size_t k = generation + 1;
-            BATCH_HIP(hipMemcpy(hs.data(), stats[i], 3 * N * sizeof(double), hipMemcpyDeviceToHost));
-            if (r->stats_mean) std::memcpy(r->stats_mean, hs.data(), k * sizeof(double));
-            if (r->stats_minimum) std::memcpy(r->stats_minimum, hs.data() + N, k * sizeof(double));
-            if (r->stats_squared_mean) std::memcpy(r->stats_squared_mean, hs.data() + 2 * N, k * sizeof(double));
+            if (r->stats_mean) std::memcpy(r->stats_mean, hs, k * sizeof(double));
+            if (r->stats_minimum) std::memcpy(r->stats_minimum, hs + N, k * sizeof(double));
+            if (r->stats_squared_mean) std::memcpy(r->stats_squared_mean, hs + 2 * N, k * sizeof(double));
         }
         if (generation + 2 == N) {  // deac.cpp:1677-1685
             generation += 1;

@@ -138,7 +138,32 @@ __global__ __launch_bounds__(kThreads) void lane_tables_kernel(LaneTabArgs a)
     }
 }
 
+// One workgroup per instance.  (A copy per instance from the host took 25 us.)
+__global__ __launch_bounds__(kThreads) void gather_best_kernel(const long *table, const double *fitness, int pitch,
+                                                               const double *pop, double *out)
+{
+    const long *t = table + static_cast<size_t>(blockIdx.x) * 5;
+    const double *fit = fitness + static_cast<size_t>(blockIdx.x) * pitch;
+    int best = 0;
+    double minimum = fit[0];
+    for (int k = 0; k < t[2]; k++)
+        if (fit[k] < minimum) {
+            minimum = fit[k];
+            best = k;
+        }
+    const double *row = pop + t[1] + best * t[4];
+    for (long k = threadIdx.x; k < t[3]; k += kThreads) out[t[0] + k] = row[k];
+}
+
 }  // namespace
+
+hipError_t launch_gather_best(const long *table, size_t n, const double *fitness, int pitch, const double *pop,
+                              double *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(gather_best_kernel, dim3(static_cast<unsigned>(n)), dim3(kThreads), 0, s, table, fitness, pitch,
+                       pop, out);
+    return hipGetLastError();
+}
 
 hipError_t launch_lane_tables(const LaneTabArgs &a, int sets, hipStream_t s)
 {

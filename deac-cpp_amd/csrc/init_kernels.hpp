@@ -1,4 +1,4 @@
-// Device set-up of the engines: initial populations (deac.cpp:430-458,
+// Device set-up and readback of the engines: initial populations (deac.cpp:430-458,
 // 584-602), for the single-instance engine and the batch, and jump tables.
 #pragma once
 
@@ -37,5 +37,11 @@ hipError_t launch_lane_tables(const LaneTabArgs &a, int sets, hipStream_t s);
 
 // Draws every member's genome, then normalizes it when nterm is given.
 hipError_t launch_initial_population(const InitArgs &a, hipStream_t s);
+
+// Best member of each of n instances (the first of the lowest fitnesses,
+// deac.cpp:128-138) into out; table: per instance 5 values, its offset in out
+// and in pop, members, genome length, row stride; fitness rows of `pitch`.
+hipError_t launch_gather_best(const long *table, size_t n, const double *fitness, int pitch, const double *pop,
+                              double *out, hipStream_t s);
 
 }  // namespace deac
