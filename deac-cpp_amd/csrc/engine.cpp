@@ -33,7 +33,7 @@ struct deac_handle {
     int device = 0;
     hipStream_t stream = nullptr;       // evolution
     hipStream_t draw_stream = nullptr;  // RNG walk, batches ahead of the evolution
-    int MG = 0, TB = 0, stride = 0, rstride = 0, nwg = 0, chunk = 0, batch = 0;
+    int MG = 0, TB = 0, stride = 0, rstride = 0, nwg = 0, maxwg = 0, chunk = 0, batch = 0;
     std::vector<void *> allocations;
     double *kmat = nullptr, *ktile = nullptr, *nterm = nullptr, *fterm = nullptr, *tterm = nullptr, *obs = nullptr, *sig = nullptr;
     double *nfm_dt = nullptr;           // -1st-moment weights over tau (bdsf), or null
@@ -41,13 +41,15 @@ struct deac_handle {
     double *emod = nullptr, *mom = nullptr;
     int *cur = nullptr;
     // Two buffer sets, used by batches of even and odd index: grid barrier
-    // counter ([0]) and status ([4..6]) per set, and the batch's draws.
+    // counter ([0]) and status ([4..6]) per set, and the batch's mask draws.
+    // Three sets of the walk's records, four of its generation starts (see
+    // the generation loop).
     unsigned *sync = nullptr;           // [2][8]
     long *iter = nullptr;               // [2][2]: split loop generation counters, per buffer set
     int *host_status = nullptr;         // [3][4], pinned: status of the sets, then of the initial fitness
-    deac::MemberCtl *ctl[2] = {};
+    deac::MemberCtl *ctl[3] = {};
     uint64_t *raw[2] = {};
-    uint64_t *gen_start[3] = {};        // by batch index modulo 3 (see the generation loop)
+    uint64_t *gen_start[4] = {};
     uint64_t *state = nullptr, *skip_rows = nullptr, *lane_tab = nullptr;
     uint64_t *tab1 = nullptr, *tab2 = nullptr, *skip_tab_dev = nullptr;  // wide walk
     uint64_t *columns = nullptr;        // matrices the lane tables are made of
@@ -57,9 +59,9 @@ struct deac_handle {
     double *stats = nullptr;            // statistics histories, kept between runs and grown on demand
     size_t stats_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // per set: walk start, walk end (fused path: of the first batch), mask
-    // start, mask end, evolve start,
-    // evolve end (draws free), status copied
+    // per set: walk start, walk end, mask end (fused path: the first batch's
+    // masks between the first two), evolve start, evolve end (draws free),
+    // status copied (split loop)
     hipEvent_t kev[2][7] = {};
     deac_run_profile last{};
     // Split loop: contraction operands of the precision it last ran at.
@@ -265,7 +267,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     h->stride = round_up(Kc, deac::kChunk);
     h->rstride = round_up(Kc, 2);
     h->wide = deac::walk_is_wide(P, m.tau_cr, m.tau_f);
-    h->chunk = (Kc + 63) / 64;
+    h->chunk = round_up((Kc + 63) / 64, 2);
     // RNG batch: generations whose mask draws are buffered at once (<= 256 MiB
     // per buffer set).
     const size_t per_gen = static_cast<size_t>(P) * h->rstride * sizeof(uint64_t);
@@ -273,6 +275,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
 
     const int maxwg = deac::evolve_max_workgroups(device);
     if (maxwg <= 0) return fail(DEAC_ERR_DEVICE);
+    h->maxwg = maxwg;
     // One workgroup per chain task or moment fold (a chain wavefront alone on its CU takes
     // 28 us at 8192 positions, three together 33), more where the trial phase
     // has over 1024 pairs of positions for each (P = 8 at 8192 positions:
@@ -315,10 +318,8 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     A(h->mom, static_cast<size_t>(P) * 4);
     A(h->sync, 16);
     A(h->iter, 4);
-    for (int k = 0; k < 2; k++) {
-        A(h->ctl[k], static_cast<size_t>(h->batch) * P);
-        A(h->raw[k], static_cast<size_t>(h->batch) * P * h->rstride);
-    }
+    for (deac::MemberCtl *&p : h->ctl) A(p, static_cast<size_t>(h->batch) * P);
+    for (uint64_t *&p : h->raw) A(p, static_cast<size_t>(h->batch) * P * h->rstride);
     for (uint64_t *&p : h->gen_start) A(p, static_cast<size_t>(h->batch) * 4);
     A(h->state, 4);
     A(h->init_start, static_cast<size_t>(P) * 4);
@@ -377,8 +378,8 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     for (double *p : {h->pop0, h->pop1})
         if (st == DEAC_OK && hipMemsetAsync(p, 0, pop_n * sizeof(double), h->stream) != hipSuccess)
             st = DEAC_ERR_DEVICE;
-    // Records: behind a stop, mask draws run over records that no walk has
-    // written (nothing reads those draws).
+    // Records: behind a stop, mask draws may run over records that no walk
+    // has written (nothing reads those draws).
     for (deac::MemberCtl *p : h->ctl)
         if (st == DEAC_OK &&
             hipMemsetAsync(p, 0, static_cast<size_t>(h->batch) * P * sizeof(deac::MemberCtl), h->stream) != hipSuccess)
@@ -531,98 +532,99 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ma.chunk = h->chunk;
     ma.rstride = h->rstride;
 
-    // Generation loop: ii = 0 .. N-2 (deac.cpp:1138), in batches.  Batch b
-    // uses buffer set b%2.  Its walk runs beside the evolution of batch b-1, on
-    // a workgroup of the same launch (two streams may share a hardware queue
-    // and then run one after the other); its mask draws, which spread over
-    // every CU and cost less alone, follow before its own evolution.  The
-    // evolution of b is queued before the host has read batch b-1's status.
-    // Behind a stop it changes nothing: the stop test sits at the top of a
-    // generation, so the fitnesses it finds are those that stopped batch b-1,
-    // and it stops at its first generation (its status and its statistics
-    // entry, past the stop, are never read).  Batches start at 8 generations,
-    // so that the first walk, which nothing hides, is short, and grow by half
-    // up to the buffer size: the walk beside a batch then has one and a half
-    // times its generations to walk, which a member's walk (0.7 us) still
-    // hides behind the generations of the smallest runs (8 us, 8 members).
+    // Generation loop: ii = 0 .. N-2 (deac.cpp:1138), in batches.  The launch
+    // that evolves batch b also makes, on workgroups of its own, the mask draws
+    // of batch b+1 and the walk of batch b+2 (two streams may share a hardware
+    // queue and then run one after the other).  The evolution of b+1 is queued
+    // before the host has read batch b's status.  Behind a stop it changes
+    // nothing: the stop test sits at the top of a generation, so the fitnesses
+    // it finds are those that stopped batch b, and it stops at its first
+    // generation (its status and its statistics entry, past the stop, are
+    // never read).  Batches start at 8 generations, so that the first masks,
+    // which nothing hides, are few, and grow by a quarter up to the buffer
+    // size: the walk beside a batch then has one and a half times its
+    // generations to walk, which a member's walk (0.7 us) still hides behind
+    // the generations of the smallest runs (8 us, 8 members).
     const size_t total = N - 1;
     std::vector<std::pair<size_t, int>> plan;  // first generation, generations
     for (size_t g = 0, len = std::min(8, h->batch); g < total;) {
         const int nb = static_cast<int>(std::min(len, total - g));
         plan.emplace_back(g, nb);
         g += static_cast<size_t>(nb);
-        len = std::min(len + len / 2, static_cast<size_t>(h->batch));
+        len = std::min(len + len / 4, static_cast<size_t>(h->batch));
         if (len < 2) len = std::min(2, h->batch);
     }
     hipStream_t d = h->draw_stream;  // split loop: the draws of the next batch
-    auto walk_args = [&](size_t b) {
-        const int k = static_cast<int>(b & 1);
-        // three sets of generation starts: a stop in batch b is answered from
-        // its set while the launch of b+1, queued behind, may walk b+2
-        wa.gen_start = h->gen_start[b % 3];
-        wa.ctl = h->ctl[k];
+    auto walk_args = [&](size_t b, const int *halt) {
+        // four sets of generation starts: a stop in batch b is answered from
+        // its set while the launch of b+1, queued behind, may walk b+3
+        wa.gen_start = h->gen_start[b % 4];
+        wa.ctl = h->ctl[b % 3];
+        wa.halt = halt;
         wa.ngen = b < plan.size() ? plan[b].second : 0;
+    };
+    auto mask_args = [&](size_t b, const int *halt) {
+        ma.ctl = h->ctl[b % 3];
+        ma.raw = h->raw[b & 1];
+        ma.halt = halt;
+        ma.ngen = b < plan.size() ? plan[b].second : 0;
+        // up to a workgroup per CU: a wavefront per SIMD, beside the evolution's
+        ma.nwg = static_cast<int>(std::min<size_t>((static_cast<size_t>(ma.ngen) * P + 3) / 4, h->maxwg));
     };
     auto evolve = [&](size_t b) -> deac_status {
         const int k = static_cast<int>(b & 1);
         hipEvent_t *e = h->kev[k];
         unsigned *sy = h->sync + 8 * k;
-        ea.ctl = h->ctl[k];
+        ea.ctl = h->ctl[b % 3];
         ea.raw = h->raw[k];
         ea.bar = sy;
         ea.status = reinterpret_cast<int *>(sy + 4);
+        ea.host_status = h->host_status + 4 * k;
+        ea.clear = h->sync + 8 * (k ^ 1);
         ea.gen0 = static_cast<long>(plan[b].first);
         ea.ngen = plan[b].second;
-        ma.ctl = h->ctl[k];
-        ma.raw = h->raw[k];
-        ma.ngen = plan[b].second;
-        walk_args(b + 1);
-        wa.halt = ea.status;
-        DEAC_HIP(hipEventRecord(e[2], s));
-        DEAC_HIP(deac::launch_mask(ma, s));
-        DEAC_HIP(hipEventRecord(e[3], s));
-        DEAC_HIP(deac::launch_zero_u32(sy, 8, s));
+        mask_args(b + 1, ea.status);
+        walk_args(b + 2, ea.status);
+        std::fill_n(ea.host_status, 4, 0);  // read for batch b-2 by now
         DEAC_HIP(hipEventRecord(e[4], s));
-        DEAC_HIP(deac::launch_evolve(ea, wa, s));
+        DEAC_HIP(deac::launch_evolve(ea, wa, ma, s));
         DEAC_HIP(hipEventRecord(e[5], s));
-        DEAC_HIP(hipMemcpyAsync(h->host_status + 4 * k, sy + 4, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
-        DEAC_HIP(hipEventRecord(e[6], s));
         return DEAC_OK;
     };
     deac_run_profile prof{};
     size_t done = 0;          // generations evolved
     long stopped_at = -1;     // generation index of the stop, if any
     auto pipeline = [&]() -> deac_status {
-        // Initial fitness (deac.cpp:857-976), on buffer set 1; its status
-        // goes to host slot 2.
+        // Initial fitness (deac.cpp:857-976), on buffer set 1, with the first
+        // walk beside it; then the first masks with the second walk.
+        DEAC_HIP(deac::launch_zero_u32(h->sync, 16, s));
         ea.init_mode = 1;
         ea.gen0 = 0;
         ea.ngen = 0;
         ea.bar = h->sync + 8;
         ea.status = reinterpret_cast<int *>(h->sync + 12);
+        ea.host_status = h->host_status + 8;
         ea.nwg = h->nwg;
-        DEAC_HIP(deac::launch_zero_u32(h->sync + 8, 8, s));
-        DEAC_HIP(deac::launch_evolve(ea, deac::WalkArgs{}, s));
-        DEAC_HIP(hipMemcpyAsync(h->host_status + 8, h->sync + 12, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
+        std::fill_n(ea.host_status, 4, 0);
+        walk_args(0, nullptr);
+        DEAC_HIP(deac::launch_evolve(ea, wa, deac::MaskArgs{}, s));
         ea.init_mode = 0;
         DEAC_HIP(hipEventRecord(h->ev0, s));
-        walk_args(0);
-        wa.halt = nullptr;
+        mask_args(0, nullptr);
+        walk_args(1, nullptr);
         DEAC_HIP(hipEventRecord(h->kev[0][0], s));
-        DEAC_HIP(deac::launch_walk(wa, s));
+        DEAC_HIP(deac::launch_mask(ma, wa, s));
         DEAC_HIP(hipEventRecord(h->kev[0][1], s));
         DEAC_TRY(evolve(0));
         for (size_t b = 0; b < plan.size(); b++) {
             if (b + 1 < plan.size()) DEAC_TRY(evolve(b + 1));
             const int k = static_cast<int>(b & 1);
             hipEvent_t *e = h->kev[k];
-            DEAC_HIP(hipEventSynchronize(e[6]));
+            DEAC_HIP(hipEventSynchronize(e[5]));
             if (b == 0 && h->host_status[8 + 2]) return DEAC_ERR_DEVICE;  // initial fitness: barrier timeout
-            float t_walk = 0, t_mask = 0, t_evo = 0;
-            if (b == 0) DEAC_HIP(hipEventElapsedTime(&t_walk, e[0], e[1]));
-            DEAC_HIP(hipEventElapsedTime(&t_mask, e[2], e[3]));
+            float t_mask = 0, t_evo = 0;
+            if (b == 0) DEAC_HIP(hipEventElapsedTime(&t_mask, e[0], e[1]));
             DEAC_HIP(hipEventElapsedTime(&t_evo, e[4], e[5]));
-            prof.walk_ms += t_walk;
             prof.mask_ms += t_mask;
             prof.evolve_ms += t_evo;
             prof.evolve_launches += 1;
@@ -632,7 +634,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
                 // RNG state at the top of the stopping generation
                 stopped_at = static_cast<long>(plan[b].first) + status[1];
                 uint64_t st4[4];
-                DEAC_HIP(hipMemcpy(st4, h->gen_start[b % 3] + static_cast<size_t>(status[1]) * 4, sizeof st4,
+                DEAC_HIP(hipMemcpy(st4, h->gen_start[b % 4] + static_cast<size_t>(status[1]) * 4, sizeof st4,
                                    hipMemcpyDeviceToHost));
                 std::memcpy(rng.s, st4, sizeof st4);
                 done += static_cast<size_t>(status[1]);
@@ -750,7 +752,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             DEAC_HIP(hipEventRecord(e[0], d));
             DEAC_HIP(deac::launch_walk(wa, d));
             DEAC_HIP(hipEventRecord(e[1], d));
-            DEAC_HIP(deac::launch_mask(ma, d));
+            DEAC_HIP(deac::launch_mask(ma, deac::WalkArgs{}, d));
             DEAC_HIP(hipEventRecord(e[2], d));
             return DEAC_OK;
         };

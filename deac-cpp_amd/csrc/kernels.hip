@@ -7,9 +7,9 @@
 //                      part of the stream (jDE F/CR redraws, rejection-
 //                      sampled donor indices) and skips each member's 2G
 //                      crossover-mask draws with GF(2) jumps;
-//       mask_kernel  - one wavefront per member regenerates the mask draws:
-//                      lane l jumps to draw l*chunk with a nibble table and
-//                      steps chunk draws;
+//       mask draws   - one wavefront per member regenerates them: lane l
+//                      jumps to draw l*chunk with a nibble table and steps
+//                      chunk draws;
 //   * evolve_kernel - a persistent kernel (all workgroups co-resident) that runs a batch of
 //     generations: best-fitness/stats/stop test, trial vectors (DE/rand/1,
 //     binomial crossover, |.|, zero-frequency match), the model ISF
@@ -38,7 +38,7 @@ constexpr int kEvoWaves = kEvoThreads / kWave;
 // caller leaves the kernel, so a broken launch cannot hang the device.
 constexpr unsigned kBarrierSpins = 1u << 24;
 
-__device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, int nwg, int *status)
+__device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, int nwg, const EvoArgs &a)
 {
     // Each wave drains its own memory operations; then one thread per
     // workgroup publishes the workgroup's stores at agent scope (L2 write-back,
@@ -57,7 +57,8 @@ __device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, in
             __builtin_amdgcn_s_sleep(1);
             if (++spins == kBarrierSpins) {
                 timed_out = 1;
-                __hip_atomic_store(status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(a.status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(a.host_status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 break;
             }
         }
@@ -141,13 +142,13 @@ __device__ __forceinline__ bool passes(const DrawLimit &l, uint64_t x) { return 
 
 namespace {
 
-// Whether the batch that runs beside this walk has met its stop test, looked
-// up every few generations: what the walk draws is then not used.
+// Whether the batch that runs beside these draws has met its stop test (the
+// walk looks every few generations): what they make is then not used.
 constexpr int kWalkPoll = 16;
 
-__device__ __forceinline__ bool stopped(const WalkArgs &a)
+__device__ __forceinline__ bool stopped(const int *halt)
 {
-    return a.halt && __hip_atomic_load(a.halt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    return halt && __hip_atomic_load(halt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
 // Which draws of a sequence are values: bit i+1 where bit i is a test (not a
@@ -199,7 +200,7 @@ __device__ void walk_wide(const WalkArgs &a, uint64_t *lds)
     const int n1 = min(kWave, (tests + tests / 4 + 8 + c1 - 1) / c1);
     uint64_t s[4] = {a.state[0], a.state[1], a.state[2], a.state[3]};  // uniform: where the next draw is
     for (int g = 0; g < a.ngen; g++) {
-        if (g % kWalkPoll == 0 && stopped(a)) return;
+        if (g % kWalkPoll == 0 && stopped(a.halt)) return;
         if (lane < 4) a.gen_start[static_cast<size_t>(g) * 4 + lane] = s[lane & 3];
         MemberCtl *ctl = a.ctl + static_cast<size_t>(g) * a.P;
         for (int i = lane; i < a.P; i += kWave) flags[i] = 0;
@@ -340,7 +341,7 @@ __device__ void walk_serial(const WalkArgs &a, uint64_t *rows)
     const uint32_t P = static_cast<uint32_t>(a.P);
     const DrawLimit lim_cr = draw_limit(a.tau_cr), lim_f = draw_limit(a.tau_f);
     for (int g = 0; g < a.ngen; g++) {
-        if (g % kWalkPoll == 0 && stopped(a)) return;
+        if (g % kWalkPoll == 0 && stopped(a.halt)) return;
         if (lane == 0)
             for (int w = 0; w < 4; w++) a.gen_start[static_cast<size_t>(g) * 4 + w] = s[w];
         MemberCtl *ctl = a.ctl + static_cast<size_t>(g) * a.P;
@@ -420,22 +421,63 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 
 // ---------------------------------------------------------------- masks
 
-__global__ __launch_bounds__(256) void mask_kernel(MaskArgs a)
+namespace {
+
+// Crossover-mask draws: one wavefront per member of a generation, lane l makes
+// draws l*chunk on.  first, step: the wavefront's members; buf: kMaskLds
+// doubles of LDS of this wavefront.
+//
+// Bound: alone on the chip the stores (8 bytes per draw); beside an evolution
+// one wavefront's instruction issue.  Rounds of 16 draws per lane go
+// through LDS, so that 8 lanes together store one line of 128 bytes.  Lane by
+// lane, 64 lines per store, 512 members of 8192 draws took 22 us, 64 members
+// of 32768 draws 37.
+__device__ void mask_draws(const MaskArgs &a, size_t first, size_t step, double *buf)
 {
+    typedef uint64_t pair __attribute__((ext_vector_type(2)));
     const int lane = threadIdx.x & (kWave - 1);
-    const size_t wave = (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-    if (wave >= static_cast<size_t>(a.ngen) * a.P) return;
-    const MemberCtl &c = a.ctl[wave];
-    uint64_t s[4] = {c.mask_state[0], c.mask_state[1], c.mask_state[2], c.mask_state[3]};
-    for (uint32_t k = 0; k < c.mask_steps; k++) (void)xnext(s);
-    lane_jump(a.lane_tab, s, s);  // T^(lane*chunk)
-    uint64_t *raw = a.raw + wave * a.rstride;
-    const int k0 = lane * a.chunk;
-    for (int c2 = 0; c2 < a.chunk; c2++) {
-        const uint64_t x = xnext(s);
-        const int k = k0 + c2;
-        if (k < a.Kc) raw[k] = x >> 11;
+    uint64_t *mine = reinterpret_cast<uint64_t *>(buf) + lane * kMaskRow;
+    const pair *from = reinterpret_cast<const pair *>(buf) + (lane >> 3) * (kMaskRow / 2) + (lane & 7);
+    for (size_t wave = first; wave < static_cast<size_t>(a.ngen) * a.P; wave += step) {
+        if (stopped(a.halt)) return;
+        const MemberCtl &c = a.ctl[wave];
+        uint64_t s[4] = {c.mask_state[0], c.mask_state[1], c.mask_state[2], c.mask_state[3]};
+        for (uint32_t k = 0; k < c.mask_steps; k++) (void)xnext(s);
+        lane_jump(a.lane_tab, s, s);  // T^(lane*chunk)
+        uint64_t *raw = a.raw + wave * a.rstride;
+        for (int c0 = 0; c0 < a.chunk; c0 += kMaskRound) {
+            const int n = min(kMaskRound, a.chunk - c0);
+            for (int j = 0; j < n; j++) mine[j] = xnext(s) >> 11;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // 8 lanes' draws at a time, a pair per lane
+            int k = (lane >> 3) * a.chunk + c0 + 2 * (lane & 7);
+            const bool in = 2 * (lane & 7) < n;
+            for (int r = 0; r < 8; r++, k += 8 * a.chunk)
+                if (in && k < a.Kc) *reinterpret_cast<pair *>(raw + k) = from[r * 8 * (kMaskRow / 2)];
+            __builtin_amdgcn_wave_barrier();
+        }
     }
+}
+
+}  // namespace
+
+template <bool WALK>
+__global__ __launch_bounds__(256) void mask_kernel(MaskArgs a, WalkArgs next)
+{
+    extern __shared__ __attribute__((aligned(16))) double mask_lds[];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    int block = blockIdx.x;
+    if constexpr (WALK) {
+        if (block == 0) {
+            if (wid == 0) walk(next, reinterpret_cast<uint64_t *>(mask_lds));
+            return;
+        }
+        block--;
+    }
+    const size_t waves = static_cast<size_t>(a.ngen) * a.P;
+    mask_draws(a, static_cast<size_t>(block) * kEvoWaves + wid, waves, mask_lds + wid * kMaskLds);
 }
 
 // ---------------------------------------------------------------- evolution
@@ -772,7 +814,8 @@ __device__ unsigned long long deac_phase_clock[4];
 // FOLD: the trials' model ISF as rounded-product folds (bdsf; its initial
 // population goes through the chains of the other form, deac.cpp:860).
 template <bool FOLD>
-__global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a, WalkArgs next)
+__global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a, WalkArgs next,
+                                                                                              MaskArgs masks)
 {
 #ifdef DEAC_PHASE_TIMERS
     unsigned long long phase_t0 = 0;
@@ -784,12 +827,18 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     // the wave index as a scalar: what depends on it alone is then uniform
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int nwg = a.nwg;
-    if (blockIdx.x == nwg) {
-        // the workgroup behind the evolution's: it walks the next batch and
-        // takes no part in the barriers
-        if (wid == 0) walk(next, reinterpret_cast<uint64_t *>(lds));
+    if (blockIdx.x >= nwg) {
+        // the workgroups behind the evolution's draw for the batches to come
+        // and take no part in the barriers: the walk, then the masks
+        const int behind = blockIdx.x - nwg - (next.ngen > 0 ? 1 : 0);
+        if (behind >= 0)
+            mask_draws(masks, static_cast<size_t>(wid) * masks.nwg + behind,
+                       static_cast<size_t>(masks.nwg) * kEvoWaves, lds + wid * kMaskLds);
+        else if (wid == 0)
+            walk(next, reinterpret_cast<uint64_t *>(lds));
         return;
     }
+    if (blockIdx.x == 0 && a.clear && threadIdx.x < 8) a.clear[threadIdx.x] = 0;
     const int total_waves = nwg * kEvoWaves;
     // Waves are numbered wave-slot-major so that consecutive tasks land on
     // different workgroups (and CUs).
@@ -863,6 +912,8 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 if (stop && blockIdx.x == 0) {
                     a.status[1] = g;
                     __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(a.host_status + 1, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    __hip_atomic_store(a.host_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 }
                 stop_flag = stop ? 1 : 0;
             }
@@ -902,7 +953,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                     __syncthreads();
                 }
             }
-            if (!grid_barrier(a.bar, target, nwg, a.status)) return;
+            if (!grid_barrier(a.bar, target, nwg, a)) return;
             DEAC_PHASE(1);
         }
 
@@ -928,7 +979,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }
         }
-        if (!grid_barrier(a.bar, target, nwg, a.status)) return;
+        if (!grid_barrier(a.bar, target, nwg, a)) return;
         DEAC_PHASE(2);
 
         // Fitness and greedy selection.
@@ -968,7 +1019,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 }
                 if (lane == 0) select_member(a, s, g, i, chi, nfm, init);
             }
-            if (!grid_barrier(a.bar, target, nwg, a.status)) return;
+            if (!grid_barrier(a.bar, target, nwg, a)) return;
         }
         DEAC_PHASE(3);
         if (init) break;
@@ -1015,26 +1066,32 @@ hipError_t launch_walk(const WalkArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_mask(const MaskArgs &a, hipStream_t s)
+hipError_t launch_mask(const MaskArgs &a, const WalkArgs &next, hipStream_t s)
 {
     const size_t waves = static_cast<size_t>(a.ngen) * a.P;
-    const size_t blocks = (waves * kWave + 255) / 256;
-    hipLaunchKernelGGL(mask_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a);
+    const unsigned blocks = static_cast<unsigned>((waves + kEvoWaves - 1) / kEvoWaves);
+    const size_t lds = kEvoWaves * kMaskLds * sizeof(double);
+    if (next.ngen > 0)
+        hipLaunchKernelGGL(mask_kernel<true>, dim3(blocks + 1), dim3(kEvoThreads), std::max(lds, walk_lds_bytes(next)), s,
+                           a, next);
+    else
+        hipLaunchKernelGGL(mask_kernel<false>, dim3(blocks), dim3(kEvoThreads), lds, s, a, next);
     return hipGetLastError();
 }
 
-// The batch's evolution and, where next.ngen > 0, the walk of the next batch
-// on one more workgroup.  A regular launch: the device holds one cooperative queue, which one
+// A regular launch: the device holds one cooperative queue, which one
 // process keeps once it has used it, so cooperative launches from a second
-// process fail.  The grid never exceeds the co-resident limit that
-// evolve_max_workgroups reports (one workgroup per CU, bounded by LDS), so on
-// an otherwise idle device every workgroup is resident; if one is not, the
-// bounded grid barrier reports a timeout instead of hanging.
-hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, hipStream_t s)
+// process fail.  The evolution's workgroups never exceed the co-resident limit
+// that evolve_max_workgroups reports (one workgroup per CU, bounded by LDS) and
+// are dispatched first, so on an otherwise idle device every one of them is
+// resident; if one is not, the bounded grid barrier reports a timeout instead
+// of hanging.
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s)
 {
     if (next.ngen > 0 && walk_lds_bytes(next) > kEvoLds) return hipErrorInvalidValue;
     hipLaunchKernelGGL(a.fold_ks && !a.init_mode ? evolve_kernel<true> : evolve_kernel<false>,
-                       dim3(a.nwg + (next.ngen > 0 ? 1 : 0)), dim3(kEvoThreads), kEvoLds, s, a, next);
+                       dim3(a.nwg + (next.ngen > 0 ? 1 : 0) + (masks.ngen > 0 ? masks.nwg : 0)), dim3(kEvoThreads), kEvoLds, s,
+                       a, next, masks);
     return hipGetLastError();
 }
 

@@ -58,8 +58,16 @@ struct MaskArgs {
     const MemberCtl *ctl;        // [ngen][P]
     const uint64_t *lane_tab;    // lane_tables of T^chunk
     uint64_t *raw;               // [ngen][P][rstride] 53-bit draws (x >> 11)
-    int ngen, P, Kc, chunk, rstride;
+    const int *halt;             // status of the batch that evolves beside the draws, or null
+    int ngen, P, Kc, rstride;
+    int chunk;                   // draws per lane, even
+    int nwg;                     // workgroups (beside the evolution)
 };
+// LDS of a wavefront that makes mask draws: rounds of 16 per lane.
+constexpr int kMaskRound = 16;
+constexpr int kMaskRow = kMaskRound + 2;
+constexpr int kMaskLds = 64 * kMaskRow;  // doubles
+static_assert(kEvoThreads / 64 * kMaskLds * sizeof(double) <= kEvoLds, "mask draws fit beside the evolution");
 
 struct EvoArgs {
     int P, T, G, nsign, Kc;
@@ -88,6 +96,8 @@ struct EvoArgs {
     size_t stats_len;
     unsigned *bar;               // grid barrier counter, zero at launch
     int *status;                 // [0] stopped, [1] generation index within the batch, [2] barrier timeout
+    int *host_status;            // the same in pinned host memory, or null (split loop)
+    unsigned *clear;             // barrier counter and status (8 words) of the next launch, or null
     long gen0;                   // generation index of the batch's first generation
     int ngen;
     int nwg;                     // workgroups that evolve
@@ -121,7 +131,8 @@ inline size_t walk_lds_bytes(const WalkArgs &a)
            (static_cast<size_t>(kWalkDraws) * 64 + a.P) * sizeof(uint32_t);
 }
 hipError_t launch_walk(const WalkArgs &a, hipStream_t s);
-hipError_t launch_mask(const MaskArgs &a, hipStream_t s);
+// Mask draws, and where next.ngen > 0 a walk on one more workgroup.
+hipError_t launch_mask(const MaskArgs &a, const WalkArgs &next, hipStream_t s);
 // Whether the evolution kernel's workgroups repeat the selection: the
 // residuals are few, and they and the members' state fit in LDS.
 inline int evolve_local(int P, int T, int nsign, int use_nfm)
@@ -135,7 +146,9 @@ inline size_t ktile_doubles(int TB, int stride)
     return (static_cast<size_t>(TB) * (stride / kUnit) + kKtilePad) * 64 * 2;
 }
 hipError_t launch_ktile(const double *rows, double *ktile, int T, int Kc, int TB, int stride, hipStream_t s);
-hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, hipStream_t s);
+// The evolution of a batch and beside it the mask draws of the next one and
+// the walk of the one after, where they have generations.
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s);
 hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s);
 // Workgroups of the evolution kernel that are co-resident on the device: one
 // per CU.

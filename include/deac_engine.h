@@ -188,8 +188,8 @@ const char *deac_last_error_message(void);
  * handle's stream (no counterpart in the reference, which has no timers). */
 typedef struct deac_run_profile {
     double loop_ms;              /* whole generation loop */
-    double walk_ms;              /* RNG walk kernels (fused path: the first batch; the others walk inside evolve_ms) */
-    double mask_ms;              /* crossover-mask kernels */
+    double walk_ms;              /* RNG walk kernels (split loop; the fused path walks beside its other kernels) */
+    double mask_ms;              /* crossover-mask kernels (fused path: the first batch; the others inside evolve_ms) */
     double evolve_ms;            /* fused generation kernels */
     size_t generations;          /* generations evolved */
     size_t evolve_launches;      /* launches of the fused generation kernel */
