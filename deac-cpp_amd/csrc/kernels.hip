@@ -654,9 +654,11 @@ __device__ __forceinline__ uint64_t cross_limit(double cr)
 // two per lane, into its spare row (deac.cpp:1261-1308); the padding stays
 // zero.  The parent, donor and draw values are all loaded, whichever the
 // crossover keeps, so the loads issue together instead of behind the
-// comparison, and those of two blocks are in flight at once.
-// Bound: memory (40 bytes read and 8 written per position).
-__device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s, const MemberCtl &c,
+// comparison, two blocks' ahead of the two being formed.
+// Bound: memory (40 bytes read and 8 written per position): 512 members of
+// 8192 positions take 67 us with the top of the generation and the barrier
+// (3.5 TB/s without them); 96 with runs of 8 blocks and nothing read ahead.
+__device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s, const int *cur, const MemberCtl &c,
                                              const uint64_t *raw, int i, int b0, int b1)
 {
     const int lane = threadIdx.x & (kWave - 1);
@@ -666,9 +668,9 @@ __device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s,
     f1 = f0;
     if (a.nsign == 2) control(a, s, c, i, 1, cr, f1);
     const uint64_t lim1 = cross_limit(cr);
-    const double *r1 = row_of(a, s.cur, c.mutant[0], false), *r2 = row_of(a, s.cur, c.mutant[1], false);
-    const double *r3 = row_of(a, s.cur, c.mutant[2], false), *rp = row_of(a, s.cur, i, false);
-    double *out = const_cast<double *>(row_of(a, s.cur, i, true));
+    const double *r1 = row_of(a, cur, c.mutant[0], false), *r2 = row_of(a, cur, c.mutant[1], false);
+    const double *r3 = row_of(a, cur, c.mutant[2], false), *rp = row_of(a, cur, i, false);
+    double *out = const_cast<double *>(row_of(a, cur, i, true));
     struct Load {
         uvec2 u;
         dvec2 x1, x2, x3, xp;
@@ -698,18 +700,87 @@ __device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s,
         }
         *reinterpret_cast<dvec2 *>(out + k) = o;
     };
-    int b = b0;
-    for (; b + 1 < b1; b += 2) {
-        Load v0 = {}, v1 = {};
-        load(b, v0);
-        load(b + 1, v1);
-        store(b, v0);
-        store(b + 1, v1);
+    Load v0 = {}, v1 = {}, w0 = {}, w1 = {};
+    auto two = [&](int b, Load &x, Load &y) __attribute__((always_inline)) {
+        if (b < b1) load(b, x);
+        if (b + 1 < b1) load(b + 1, y);
+    };
+    auto put = [&](int b, const Load &x, const Load &y) __attribute__((always_inline)) {
+        store(b, x);
+        if (b + 1 < b1) store(b + 1, y);
+    };
+    two(b0, v0, v1);
+    for (int b = b0;; b += 4) {
+        two(b + 2, w0, w1);
+        put(b, v0, v1);
+        if (b + 2 >= b1) break;
+        two(b + 4, v0, v1);
+        put(b + 2, w0, w1);
+        if (b + 4 >= b1) break;
     }
-    if (b < b1) {
-        Load v0 = {};
-        load(b, v0);
-        store(b, v0);
+}
+
+// Lowest fitness as the reference's scan finds it (deac.cpp:128-138: the first
+// of equal ones, no value but the first may be NaN), by one whole wavefront.
+__device__ __forceinline__ double lowest(const double *fit, int P)
+{
+    double mn = fit[0];
+    if (P <= 32) {  // (64 values take 0.4 us in a row, 0.6 in parallel)
+        for (int i = 1; i < P; i++) mn = fit[i] < mn ? fit[i] : mn;
+        return mn;
+    }
+    const double first = mn;
+    int at = 0;
+    for (int i = threadIdx.x & (kWave - 1); i < P; i += kWave) {
+        const double v = fit[i];
+        if (v < mn) {
+            mn = v;
+            at = i;
+        }
+    }
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) {
+        const double v = __shfl_xor(mn, m);
+        const int i = __shfl_xor(at, m);
+        if (v < mn || (v == mn && i < at)) {
+            mn = v;
+            at = i;
+        }
+    }
+    return first != first ? first : mn;
+}
+
+// Mean and squared mean of the fitnesses of generation g in the reference's
+// order (deac.cpp:1145-1160), by one wavefront: staged in its LDS (kChainLds
+// doubles), 8 values read ahead.
+__device__ __forceinline__ void statistics(const EvoArgs &a, const double *fit, int g, double mn, double *buf)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    constexpr int kWindow = kChainLds & ~7;
+    double sum = 0.0, sq = 0.0;
+    const int p4 = a.P & ~3;
+    for (int w0 = 0; w0 < a.P; w0 += kWindow) {
+        const int n = min(kWindow, a.P - w0);
+        for (int i = lane; i < n; i += kWave) buf[i] = fit[w0 + i];
+        asm volatile("" ::: "memory");  // (one wavefront: LDS keeps its order)
+        for (int i0 = 0; i0 < n; i0 += 8) {
+            double v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = buf[min(i0 + e, n - 1)];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if (i0 + e >= n) break;
+                sum = sum + v[e];
+                sq = w0 + i0 + e < p4 ? sq + v[e] * v[e] : fma(v[e], v[e], sq);
+            }
+        }
+        asm volatile("" ::: "memory");
+    }
+    const long ii = a.gen0 + g;
+    if (lane == 0) {
+        a.stats[ii] = sum / static_cast<double>(a.P);
+        a.stats[a.stats_len + ii] = mn;
+        a.stats[2 * a.stats_len + ii] = sq / static_cast<double>(a.P);
     }
 }
 
@@ -821,8 +892,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     unsigned long long phase_t0 = 0;
 #endif
     extern __shared__ __attribute__((aligned(16))) double lds[];
-    __shared__ int stop_flag;
-    __shared__ double scale;
+    __shared__ double minimum, scale;
     const int lane = threadIdx.x & (kWave - 1);
     // the wave index as a scalar: what depends on it alone is then uniform
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -848,12 +918,19 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const int nmom = a.use_first + a.use_third;  // moment folds per member
     const int ntask = ks + nmom * a.P;
     const int nblk = a.stride / kChunk;
-    const int run = static_cast<int>(
-        min(max(static_cast<long>(a.P) * nblk / total_waves, 1L), static_cast<long>(min(nblk, 8))));
-    const int runs = (nblk + run - 1) / run;  // per member
+    // This wave's share of the trials' blocks: equal shares, across members.
+    // (In runs of 8 blocks of one member, 4096 of them for 992 waves, the fifth
+    // round was nearly empty.)
+    const size_t blocks = static_cast<size_t>(a.P) * nblk;
+    const int share0 = static_cast<int>(gwave * blocks / total_waves);
+    const int nshare = static_cast<int>((gwave + 1) * blocks / total_waves) - share0;
+    const int share_i = share0 / nblk, share_b = share0 % nblk;
     const int Tp = a.T | 1;  // odd row stride: lanes of different members read different banks
 
     Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
+    // Where each member's current genome is: a copy in LDS of the members' state
+    // in global memory where it fits.
+    const bool copy = !a.local && a.P <= 2 * kResidLds;
     // [P][Tp] residuals and -1st-moment products (a.local), behind the chains' buffers
     double *resid = lds + kEvoWaves * kChainLds;
     double *moment = resid + static_cast<size_t>(a.P) * Tp;
@@ -871,6 +948,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             }
         }
     }
+    const int *cur = s.cur;
     __syncthreads();
 
     for (int g = 0; g <= a.ngen; g++) {
@@ -878,57 +956,40 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         if (!init) {
             if (g == a.ngen) break;
             DEAC_PHASE(0);
-            // Top of the generation: best fitness, statistics, stop test
-            // (deac.cpp:1145-1166), scanned by one thread in the reference's
-            // order, 8 values read ahead; the statistics by workgroup 0 only.
-            const double *fit = s.fitness;
-            if (!a.local && a.P <= kResidLds) {
-                for (int i = threadIdx.x; i < a.P; i += kEvoThreads) lds[i] = a.fitness[i];
-                fit = lds;
-                __syncthreads();
+            // Top of the generation: best fitness and stop test
+            // (deac.cpp:1145-1166); the statistics are left to the chains'
+            // phase, which one wave's scan does not lengthen.
+            if (copy) {
+                int *to = reinterpret_cast<int *>(resid);
+                for (int i = threadIdx.x; i < a.P; i += kEvoThreads) to[i] = a.cur[i];
+                cur = to;
             }
-            if (threadIdx.x == 0) {
-                double mn = fit[0], sum = 0.0, sq = 0.0;
-                const int p4 = a.P & ~3;
-                for (int i0 = 0; i0 < a.P; i0 += 8) {
-                    double v[8];
-#pragma unroll
-                    for (int e = 0; e < 8; e++) v[e] = fit[min(i0 + e, a.P - 1)];
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        if (i0 + e >= a.P) break;
-                        if (v[e] < mn) mn = v[e];
-                        sum = sum + v[e];
-                        sq = i0 + e < p4 ? sq + v[e] * v[e] : fma(v[e], v[e], sq);
-                    }
-                }
-                if (blockIdx.x == 0 && a.track_stats) {
-                    const long ii = a.gen0 + g;
-                    a.stats[ii] = sum / static_cast<double>(a.P);
-                    a.stats[a.stats_len + ii] = mn;
-                    a.stats[2 * a.stats_len + ii] = sq / static_cast<double>(a.P);
-                }
-                const bool stop = mn <= a.stop;
-                if (stop && blockIdx.x == 0) {
-                    a.status[1] = g;
-                    __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(a.host_status + 1, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    __hip_atomic_store(a.host_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                }
-                stop_flag = stop ? 1 : 0;
+            if (wid == 0) {
+                const double mn = lowest(s.fitness, a.P);
+                if (lane == 0) minimum = mn;
             }
             __syncthreads();
-            if (stop_flag) break;
+            if (minimum <= a.stop) {
+                if (blockIdx.x == 0 && wid == 0) {
+                    if (a.track_stats) statistics(a, s.fitness, g, minimum, lds);
+                    if (lane == 0) {
+                        a.status[1] = g;
+                        __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(a.host_status + 1, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        __hip_atomic_store(a.host_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                }
+                break;
+            }
 
-            // Trial vectors into each member's spare buffer: a wave takes runs
-            // of up to 8 blocks of one member, whose controls it then reads
-            // once; shorter runs where they would leave waves without work.
+            // Trial vectors into each member's spare buffer.
             const MemberCtl *ctlg = a.ctl + static_cast<size_t>(g) * a.P;
             const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.rstride;
             if (!a.renorm) {
-                for (int it = gwave; it < a.P * runs; it += total_waves) {
-                    const int i = it / runs, b0 = it % runs * run;
-                    trial_blocks(a, s, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, min(b0 + run, nblk));
+                for (int i = share_i, b0 = share_b, left = nshare; left > 0; i++, b0 = 0) {
+                    const int n = min(nblk - b0, left);
+                    trial_blocks(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, b0 + n);
+                    left -= n;
                 }
             } else {
                 // With per-generation renormalization (deac.cpp:1342-1364) a
@@ -937,8 +998,9 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 const int share = (nblk + kEvoWaves - 1) / kEvoWaves;
                 for (int i = blockIdx.x; i < a.P; i += nwg) {
                     const int b0 = min(wid * share, nblk), b1 = min(b0 + share, nblk);
-                    trial_blocks(a, s, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, b1);
-                    double *x = const_cast<double *>(row_of(a, s.cur, i, true));
+                    if (b0 < b1)
+                        trial_blocks(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, b1);
+                    double *x = const_cast<double *>(row_of(a, cur, i, true));
                     __builtin_amdgcn_s_waitcnt(0);
                     __syncthreads();
                     if (wid == 0) {
@@ -965,20 +1027,22 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 const int tb = task % a.TB, mg = task / a.TB;
                 if constexpr (FOLD) {
                     const double e = fold_task(a.ktile + static_cast<size_t>(tb) * a.stride * kChainTau,
-                                               row_of(a, s.cur, mg, true), nblk, a.Kc, (a.G & 1) != 0, buf);
+                                               row_of(a, cur, mg, true), nblk, a.Kc, (a.G & 1) != 0, buf);
                     const int t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
                     if ((lane & 3) == 0 && t < a.T) a.emod[static_cast<size_t>(mg) * a.T + t] = e;
                 } else {
-                    auto row = [&](int m) { return row_of(a, s.cur, min(mg * kChainRows + m, a.P - 1), !init); };
+                    auto row = [&](int m) { return row_of(a, cur, min(mg * kChainRows + m, a.P - 1), !init); };
                     chain_task(a, row(0), row(1), row(2), row(3), tb, mg, buf);
                 }
             } else {
                 const int i = (task - ks) / nmom;
                 const bool third = !a.use_first || (task - ks) % nmom != 0;
-                const double m = wave_fold(row_of(a, s.cur, i, !init), third ? a.tterm : a.fterm, a.Kc, a.G, buf);
+                const double m = wave_fold(row_of(a, cur, i, !init), third ? a.tterm : a.fterm, a.Kc, a.G, buf);
                 if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }
         }
+        if (gwave == total_waves - 1 && a.track_stats && !init)
+            statistics(a, s.fitness, g, minimum, lds + wid * kChainLds);
         if (!grid_barrier(a.bar, target, nwg, a)) return;
         DEAC_PHASE(2);
 
