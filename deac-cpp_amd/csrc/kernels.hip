@@ -637,12 +637,25 @@ __device__ __forceinline__ const double *row_of(const EvoArgs &a, const int *cur
     return ((cur[i] != 0) != spare ? a.pop1 : a.pop0) + static_cast<size_t>(i) * a.stride;
 }
 
-__device__ __forceinline__ void control(const EvoArgs &a, const Members &s, const MemberCtl &c, int i, int sg,
-                                        double &cr, double &f)
-{
-    cr = (c.flags >> (2 * sg)) & 1 ? c.cr_value[sg] : s.cr[i * a.nsign + sg];
-    f = (c.flags >> (2 * sg + 1)) & 1 ? c.f_value[sg] : s.f[i * a.nsign + sg];
-}
+// CR and F of member i in a generation, per sign (the second repeats the first
+// where there is one sign): redrawn or the member's own.  Both are loaded
+// whichever holds, so that a member costs one memory latency and not one per
+// value.
+struct Controls {
+    double cr[2] = {0.0, 0.0}, f[2] = {0.0, 0.0};
+    __device__ __forceinline__ Controls() {}
+    __device__ __forceinline__ Controls(const EvoArgs &a, const Members &s, const MemberCtl &c, int i)
+    {
+        const int j = i * a.nsign, j1 = j + a.nsign - 1, two = a.nsign - 1;
+        const double c0 = s.cr[j], c1 = s.cr[j1], f0 = s.f[j], f1 = s.f[j1];
+        const double n0 = c.cr_value[0], n1 = c.cr_value[1], m0 = c.f_value[0], m1 = c.f_value[1];
+        const uint32_t flags = c.flags;
+        cr[0] = flags & 1 ? n0 : c0;
+        f[0] = flags & 2 ? m0 : f0;
+        cr[1] = !two ? cr[0] : flags & 4 ? n1 : c1;
+        f[1] = !two ? f[0] : flags & 8 ? m1 : f1;
+    }
+};
 
 // u < cr for the draw u = r 2^-53, as r < ceil(cr 2^53) in whole numbers
 __device__ __forceinline__ uint64_t cross_limit(double cr)
@@ -650,45 +663,55 @@ __device__ __forceinline__ uint64_t cross_limit(double cr)
     return !(cr > 0.0) ? 0 : cr >= 1.0 ? UINT64_C(1) << 53 : static_cast<uint64_t>(ceil(cr * 0x1.0p53));
 }
 
-// Trial vectors of one member over genome blocks [b0, b1) of 128 positions,
-// two per lane, into its spare row (deac.cpp:1261-1308); the padding stays
-// zero.  The parent, donor and draw values are all loaded, whichever the
-// crossover keeps, so the loads issue together instead of behind the
-// comparison, two blocks' ahead of the two being formed.
-// Bound: memory (40 bytes read and 8 written per position): 512 members of
-// 8192 positions take 67 us with the top of the generation and the barrier
-// (3.5 TB/s without them); 96 with runs of 8 blocks and nothing read ahead.
-__device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s, const int *cur, const MemberCtl &c,
-                                             const uint64_t *raw, int i, int b0, int b1)
-{
-    const int lane = threadIdx.x & (kWave - 1);
-    double cr, f0, f1;
-    control(a, s, c, i, 0, cr, f0);
-    const uint64_t lim0 = cross_limit(cr);
-    f1 = f0;
-    if (a.nsign == 2) control(a, s, c, i, 1, cr, f1);
-    const uint64_t lim1 = cross_limit(cr);
-    const double *r1 = row_of(a, cur, c.mutant[0], false), *r2 = row_of(a, cur, c.mutant[1], false);
-    const double *r3 = row_of(a, cur, c.mutant[2], false), *rp = row_of(a, cur, i, false);
-    double *out = const_cast<double *>(row_of(a, cur, i, true));
+// A member's trial vector (deac.cpp:1261-1308), in blocks of 128 genome
+// positions, two per lane: load() fetches a block's parent, donor and draw
+// values, form() the trial values, zero past the genome.  The values are all
+// loaded, whichever the crossover keeps, so the loads issue together instead
+// of behind the comparison.
+struct Trial {
+    const EvoArgs &a;
+    const uint64_t *raw;
+    const double *r1, *r2, *r3, *rp;
+    double *out;  // the member's spare row
+    double f0, f1;
+    uint64_t lim0, lim1;
     struct Load {
         uvec2 u;
         dvec2 x1, x2, x3, xp;
     };
-    auto load = [&](int b, Load &v) __attribute__((always_inline)) {
-        const int k = b * kChunk + 2 * lane;
+    __device__ __forceinline__ Trial(const EvoArgs &ea, const Members &s, const int *cur, const MemberCtl &c,
+                                     const uint64_t *draws, int i)
+        : a(ea), raw(draws)
+    {
+        r1 = row_of(a, cur, c.mutant[0], false);
+        r2 = row_of(a, cur, c.mutant[1], false);
+        r3 = row_of(a, cur, c.mutant[2], false);
+        rp = row_of(a, cur, i, false);
+        out = const_cast<double *>(row_of(a, cur, i, true));
+        const Controls k(a, s, c, i);
+        f0 = k.f[0];
+        f1 = k.f[1];
+        lim0 = cross_limit(k.cr[0]);
+        lim1 = cross_limit(k.cr[1]);
+    }
+    static __device__ __forceinline__ int position(int b) { return b * kChunk + 2 * (threadIdx.x & (kWave - 1)); }
+    __device__ __forceinline__ void load(int b, Load &v) const
+    {
+        const int k = position(b);
         if (k < a.Kc) v.u = *reinterpret_cast<const uvec2 *>(raw + k);
         v.x1 = *reinterpret_cast<const dvec2 *>(r1 + k);
         v.x2 = *reinterpret_cast<const dvec2 *>(r2 + k);
         v.x3 = *reinterpret_cast<const dvec2 *>(r3 + k);
         v.xp = *reinterpret_cast<const dvec2 *>(rp + k);
-    };
-    auto value = [&](bool neg, uint64_t r, double d1, double d2, double d3, double p) __attribute__((always_inline)) {
+    }
+    __device__ __forceinline__ double value(bool neg, uint64_t r, double d1, double d2, double d3, double p) const
+    {
         const double w = fma(neg ? f1 : f0, d2 - d3, d1);
         return r < (neg ? lim1 : lim0) ? (a.allow_neg ? w : fabs(w)) : p;
-    };
-    auto store = [&](int b, const Load &v) __attribute__((always_inline)) {
-        const int k = b * kChunk + 2 * lane;
+    }
+    __device__ __forceinline__ dvec2 form(int b, const Load &v) const
+    {
+        const int k = position(b);
         dvec2 o = {0.0, 0.0};
         if (k < a.Kc) o.x = value(k >= a.G, v.u.x, v.x1.x, v.x2.x, v.x3.x, v.xp.x);
         if (k + 1 < a.Kc) o.y = value(k + 1 >= a.G, v.u.y, v.x1.y, v.x2.y, v.x3.y, v.xp.y);
@@ -698,16 +721,30 @@ __device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s,
             if (k == a.G) o.x = z;
             else o.y = z;
         }
-        *reinterpret_cast<dvec2 *>(out + k) = o;
-    };
+        return o;
+    }
+    __device__ __forceinline__ void store(int b, const dvec2 &o) const
+    {
+        *reinterpret_cast<dvec2 *>(out + position(b)) = o;
+    }
+};
+
+// Blocks [b0, b1) of a trial vector into the spare row, two blocks' loads
+// ahead of the two being formed.
+// Bound: memory (40 bytes read and 8 written per position): 512 members of
+// 8192 positions take 67 us with the top of the generation and the barrier
+// (3.5 TB/s without them); 96 with runs of 8 blocks and nothing read ahead.
+__device__ __forceinline__ void trial_blocks(const Trial &t, int b0, int b1)
+{
+    typedef Trial::Load Load;
     Load v0 = {}, v1 = {}, w0 = {}, w1 = {};
     auto two = [&](int b, Load &x, Load &y) __attribute__((always_inline)) {
-        if (b < b1) load(b, x);
-        if (b + 1 < b1) load(b + 1, y);
+        if (b < b1) t.load(b, x);
+        if (b + 1 < b1) t.load(b + 1, y);
     };
     auto put = [&](int b, const Load &x, const Load &y) __attribute__((always_inline)) {
-        store(b, x);
-        if (b + 1 < b1) store(b + 1, y);
+        t.store(b, t.form(b, x));
+        if (b + 1 < b1) t.store(b + 1, t.form(b + 1, y));
     };
     two(b0, v0, v1);
     for (int b = b0;; b += 4) {
@@ -718,6 +755,87 @@ __device__ __forceinline__ void trial_blocks(const EvoArgs &a, const Members &s,
         put(b + 2, w0, w1);
         if (b + 4 >= b1) break;
     }
+}
+
+// A trial vector and its zeroth moment (deac.cpp:1342-1352) by one workgroup:
+// waves 1 to 3 form the blocks of one stage, store them and leave their products
+// in LDS while wave 0 folds the stage before.  Returns the moment in wave 0.
+// buf: 2 stages in LDS.
+// Bound: the fold's chain of MFMAs, 9 us at 4096 positions.  The trial phase
+// took 25 us there with trial, fold and scaling one after the other, 29 with
+// the fold's wave forming the trial as it went; 20.5 this way.
+constexpr int kStageBlocks = 9;
+constexpr int kStage = kStageBlocks * kChunk;
+static_assert(kStageBlocks % (kEvoWaves - 1) == 0 && kFoldBlock == kChunk);
+static_assert(2 * kStage <= kEvoWaves * kChainLds, "the stages fit in front of the members' state");
+
+__device__ __forceinline__ double trial_fold(const Trial &t, const double *w, int nblk, double *buf)
+{
+    constexpr int kEach = kStageBlocks / (kEvoWaves - 1);
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const int Kc = t.a.Kc, G = t.a.G, nstage = (nblk + kStageBlocks - 1) / kStageBlocks;
+    const bool godd = (G & 1) != 0;
+    double acc = 0.0;
+    for (int c = -1; c < nstage; c++) {
+        if (wid == 0 && c >= 0) {
+            FoldFused f = {{-1, -1}, {1.0, 1.0}};
+            if (godd) {
+                f.w[0] = w[G - 1];
+                f.w[1] = w[Kc - 1];
+            }
+            const double *here = buf + (c & 1) * kStage + (lane >> 4);
+            fold_pair v[kFoldAhead];
+#pragma unroll
+            for (int u = 0; u < kFoldAhead; u++) v[u] = fold_pair{here[8 * u], here[8 * u + 4]};
+            const int b0 = c * kStageBlocks, b1 = min(b0 + kStageBlocks, nblk);
+            for (int b = b0; b < b1; b++, here += kChunk) {
+                // (a stage's last block reads ahead into its own start)
+                const double *next = b + 1 < b1 ? here + kChunk : here;
+                f.k[0] = godd ? G - 1 - b * kChunk : -1;
+                f.k[1] = godd ? Kc - 1 - b * kChunk : -1;
+                const bool fused = (f.k[0] >= 0 && f.k[0] < kChunk) || (f.k[1] >= 0 && f.k[1] < kChunk);
+                if (fused) fold_block<true>(acc, v, here, next, f);
+                else fold_block<false>(acc, v, here, next, f);
+            }
+        }
+        if (wid != 0 && c + 1 < nstage) {
+            Trial::Load v[kEach] = {};
+            dvec2 wk[kEach];
+            const int j0 = (wid - 1) * kEach, b0 = (c + 1) * kStageBlocks + j0;
+#pragma unroll
+            for (int j = 0; j < kEach; j++)
+                if (b0 + j < nblk) {
+                    t.load(b0 + j, v[j]);
+                    wk[j] = *reinterpret_cast<const dvec2 *>(w + min(Trial::position(b0 + j), (Kc - 1) & ~1));
+                }
+#pragma unroll
+            for (int j = 0; j < kEach; j++)
+                if (b0 + j < nblk) {
+                    const int k = Trial::position(b0 + j);
+                    const dvec2 x = t.form(b0 + j, v[j]);
+                    t.store(b0 + j, x);
+                    dvec2 p = x * wk[j];
+                    if (godd) {  // a fused element's first factor in place of its product
+                        if (k == G - 1 || k == Kc - 1) p.x = x.x;
+                        if (k + 1 == G - 1 || k + 1 == Kc - 1) p.y = x.y;
+                    }
+                    if (k >= Kc) p.x = 0.0;
+                    if (k + 1 >= Kc) p.y = 0.0;
+                    reinterpret_cast<dvec2 *>(buf + ((c + 1) & 1) * kStage + (j0 + j) * kChunk)[lane] = p;
+                }
+        }
+        if (c == nstage - 1) __builtin_amdgcn_s_waitcnt(0);  // the trial, before it is scaled
+        __syncthreads();
+    }
+    return acc;
+}
+
+// Blocks [b0, b1) of a row times a factor.
+__device__ __forceinline__ void scale_blocks(double *x, double scale, int b0, int b1)
+{
+    dvec2 *p = reinterpret_cast<dvec2 *>(x) + (threadIdx.x & (kWave - 1));
+#pragma unroll 8
+    for (int b = b0; b < b1; b++) p[b * (kChunk / 2)] = p[b * (kChunk / 2)] * scale;
 }
 
 // Lowest fitness as the reference's scan finds it (deac.cpp:128-138: the first
@@ -821,38 +939,50 @@ __device__ __forceinline__ double product_sum(const EvoArgs &a, const double *w,
     return acc;
 }
 
-// Member i's fitness from its chi^2 sum and -1st moment (deac.cpp:957-976,
-// 1539-1555) and the greedy selection (deac.cpp:1556-1571), by one lane.
-__device__ __forceinline__ void select_member(const EvoArgs &a, const Members &s, int g, int i, double chi, double nfm,
-                                              bool init)
-{
-    double fit = chi / static_cast<double>(a.T);
-    if (a.use_nfm) {
-        const double q = (a.nfm_value - nfm) / a.nfm_error;
-        fit = fma(q, q, fit);
+// The greedy selection of a member (deac.cpp:1556-1571), by one lane: what it
+// needs beside the new fitness is loaded ahead of the sums.
+struct Selection {
+    const EvoArgs &a;
+    const Members &s;
+    int i;
+    bool init;
+    double old, first, third;
+    Controls next;
+    __device__ __forceinline__ Selection(const EvoArgs &ea, const Members &members, int g, int member, bool initial)
+        : a(ea), s(members), i(member), init(initial), old(s.fitness[i]), first(a.use_first ? a.mom[i * 4 + 1] : 0.0),
+          third(a.use_third ? a.mom[i * 4 + 2] : 0.0)
+    {
+        // (the initial fitness has no control records)
+        if (!init) next = Controls(a, s, a.ctl[static_cast<size_t>(g) * a.P + i], i);
     }
-    if (a.use_first) {
-        const double d = a.mom[i * 4 + 1] - a.first_moment;
-        fit += (d * d) / a.first_moment;
-    }
-    if (a.use_third) {
-        const double q = (a.third_moment - a.mom[i * 4 + 2]) / a.third_moment_error;
-        fit = fma(q, q, fit);
-    }
-    if (init) {
-        s.fitness[i] = fit;
-    } else if (fit <= s.fitness[i]) {
-        const MemberCtl &c = a.ctl[static_cast<size_t>(g) * a.P + i];
-        s.fitness[i] = fit;
-        s.cur[i] ^= 1;
-        for (int sg = 0; sg < a.nsign; sg++) {
-            double cr, f;
-            control(a, s, c, i, sg, cr, f);
-            s.cr[i * a.nsign + sg] = cr;
-            s.f[i * a.nsign + sg] = f;
+    // from the chi^2 sum and the -1st moment (deac.cpp:957-976, 1539-1555)
+    __device__ __forceinline__ void take(double chi, double nfm) const
+    {
+        double fit = chi / static_cast<double>(a.T);
+        if (a.use_nfm) {
+            const double q = (a.nfm_value - nfm) / a.nfm_error;
+            fit = fma(q, q, fit);
+        }
+        if (a.use_first) {
+            const double d = first - a.first_moment;
+            fit += (d * d) / a.first_moment;
+        }
+        if (a.use_third) {
+            const double q = (a.third_moment - third) / a.third_moment_error;
+            fit = fma(q, q, fit);
+        }
+        if (init) {
+            s.fitness[i] = fit;
+        } else if (fit <= old) {
+            s.fitness[i] = fit;
+            s.cur[i] ^= 1;
+            for (int sg = 0; sg < a.nsign; sg++) {
+                s.cr[i * a.nsign + sg] = sg ? next.cr[1] : next.cr[0];
+                s.f[i * a.nsign + sg] = sg ? next.f[1] : next.f[0];
+            }
         }
     }
-}
+};
 
 }  // namespace
 
@@ -988,30 +1118,28 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             if (!a.renorm) {
                 for (int i = share_i, b0 = share_b, left = nshare; left > 0; i++, b0 = 0) {
                     const int n = min(nblk - b0, left);
-                    trial_blocks(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, b0 + n);
+                    trial_blocks(Trial(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i), b0, b0 + n);
                     left -= n;
                 }
             } else {
                 // With per-generation renormalization (deac.cpp:1342-1364) a
-                // workgroup takes whole members: it forms the trial, folds
-                // its zeroth moment on one wave and scales it.
-                const int share = (nblk + kEvoWaves - 1) / kEvoWaves;
-                for (int i = blockIdx.x; i < a.P; i += nwg) {
-                    const int b0 = min(wid * share, nblk), b1 = min(b0 + share, nblk);
-                    if (b0 < b1)
-                        trial_blocks(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i, b0, b1);
-                    double *x = const_cast<double *>(row_of(a, cur, i, true));
-                    __builtin_amdgcn_s_waitcnt(0);
-                    __syncthreads();
-                    if (wid == 0) {
-                        const double norm = wave_fold(x, a.nterm, a.Kc, a.G, lds);
-                        if (lane == 0) scale = a.zeroth / norm;
+                // workgroup takes whole members, or where there are more
+                // members than workgroups every wave has one of its own.
+                const bool alone = a.P > nwg;
+                for (int i = alone ? gwave : static_cast<int>(blockIdx.x); i < a.P; i += alone ? total_waves : nwg) {
+                    const Trial t(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i);
+                    if (alone) {
+                        trial_blocks(t, 0, nblk);
+                        __builtin_amdgcn_s_waitcnt(0);
+                        scale_blocks(t.out, a.zeroth / wave_fold(t.out, a.nterm, a.Kc, a.G, lds + wid * kChainLds), 0,
+                                     nblk);
+                        continue;
                     }
+                    const double norm = trial_fold(t, a.nterm, nblk, lds);
+                    if (threadIdx.x == 0) scale = a.zeroth / norm;
                     __syncthreads();
-                    for (int b = b0; b < b1; b++) {
-                        dvec2 *p2 = reinterpret_cast<dvec2 *>(x) + b * (kChunk / 2) + lane;
-                        *p2 = *p2 * scale;
-                    }
+                    const int share = (nblk + kEvoWaves - 1) / kEvoWaves;
+                    scale_blocks(t.out, scale, min(wid * share, nblk), min((wid + 1) * share, nblk));
                     __syncthreads();
                 }
             }
@@ -1057,8 +1185,9 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             }
             __syncthreads();
             for (int i = threadIdx.x; i < a.P; i += kEvoThreads) {
+                const Selection sel(a, s, g, i, init);
                 const double chi = chi_sum(resid + i * Tp, a.T, a.T & 1, 0.0);
-                select_member(a, s, g, i, chi, a.use_nfm ? product_sum(a, moment + i * Tp, i, 0, a.T, 0.0) : 0.0, init);
+                sel.take(chi, a.use_nfm ? product_sum(a, moment + i * Tp, i, 0, a.T, 0.0) : 0.0);
             }
             __syncthreads();
         } else {
@@ -1066,6 +1195,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             const int window = a.use_nfm ? kResidWave / 2 : kResidWave;
             double *d = lds + wid * kResidWave, *p = d + window;
             for (int i = gwave; i < a.P; i += total_waves) {
+                const Selection sel(a, s, g, i, init);
                 double chi = 0.0, nfm = 0.0;
                 for (int t0 = 0; t0 < a.T; t0 += window) {
                     const int n = min(window, a.T - t0);
@@ -1081,7 +1211,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                     if (a.use_nfm) nfm = product_sum(a, p, i, t0, n, nfm);
                     __builtin_amdgcn_wave_barrier();
                 }
-                if (lane == 0) select_member(a, s, g, i, chi, nfm, init);
+                if (lane == 0) sel.take(chi, nfm);
             }
             if (!grid_barrier(a.bar, target, nwg, a)) return;
         }
