@@ -478,6 +478,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ea.stride = h->stride;
     ea.MG = h->MG;
     ea.TB = h->TB;
+    ea.by_tau = m.bdsf ? deac::evolve_by_tau(ea.P, 1, ea.TB) : deac::evolve_by_tau(ea.MG, deac::kChainRows, ea.TB);
     ea.use_first = m.use_first;
     ea.use_third = m.use_third;
     ea.renorm = m.normalize && m.renormalize;

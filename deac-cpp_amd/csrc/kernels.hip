@@ -527,25 +527,42 @@ struct KUnits {
     __device__ __forceinline__ void advance() { base += kChunkUnits * 1024; }
 };
 
+// A member group's four genome rows, read the same way, 128 positions a load.
+struct GenomeRows {
+    const double *row[kChainRows];
+    int vo;  // this lane's two positions, bytes
+    __device__ __forceinline__ dvec2 load(int m, int chunk) const
+    {
+        const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(row[m]), 0, -1, 0x00020000);
+        return __builtin_bit_cast(dvec2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, static_cast<unsigned>(chunk) * (kChunk * 8), 0));
+    }
+};
+
 // One chunk of the chains: kr[h .. h+15] hold its K units and are refilled
-// with those two chunks on; sr holds the genome units about to be used.
+// with those two chunks on; sr holds the genome units about to be used.  st,
+// the genome rows of the next chunk, goes to its place in LDS (to) and is
+// refilled from chunk `ahead`.  Every instruction beside the MFMAs has its
+// place behind one, whose result the next one waits for.
 template <int H>
 __device__ __forceinline__ void chain_chunk(double &acc, dvec2 (&kr)[kRing], dvec2 (&sr)[kReadAhead], KUnits &ku,
-                                            const double *here, const double *next)
+                                            const double *here, const double *next, dvec2 (&st)[kChainRows],
+                                            const GenomeRows &rows, double *to, int ahead)
 {
 #pragma unroll
     for (int i = 0; i < kChunkUnits; i++) {
         const dvec2 k = kr[H + i], s = sr[i % kReadAhead];
         const int j = i + kReadAhead;
         const double *p = j < kChunkUnits ? here + j * kUnit : next + (j - kChunkUnits) * kUnit;
-        // each load issues behind an MFMA, whose result the next one waits for
         acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.x, s.x, acc, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         sr[i % kReadAhead] = dvec2{p[0], p[4]};
         __builtin_amdgcn_sched_barrier(0);
+        if (i < kChainRows) *reinterpret_cast<dvec2 *>(to + i * kSRow) = st[i % kChainRows];
+        __builtin_amdgcn_sched_barrier(0);
         acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.y, s.y, acc, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         kr[H + i] = ku.load(i);
+        if (i >= kChainRows && i < 2 * kChainRows) st[i % kChainRows] = rows.load(i % kChainRows, ahead);
         __builtin_amdgcn_sched_barrier(0);
     }
     ku.advance();
@@ -571,55 +588,47 @@ __device__ __forceinline__ void chain_chunk(double &acc, dvec2 (&kr)[kRing], dve
 // wavefronts on the CU, the L1 takes 45 cycles for such a load), 16-byte genome
 // loads put in order by v_permlane swaps 45, chunks staged by helper
 // wavefronts with a barrier per 128 positions 34.
-__device__ __forceinline__ void chain_task(const EvoArgs &a, const double *r0, const double *r1, const double *r2,
-                                           const double *r3, int tb, int mg, double *buf)
+__device__ __forceinline__ void chain_task(const EvoArgs &a, const GenomeRows &rows, int tb, int mg, double *buf)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int nchunk = a.stride / kChunk;
     KUnits ku(a.ktile + static_cast<size_t>(tb) * nchunk * kChunkUnits * (2 * kWave));
-    struct Stage {
-        dvec2 v0, v1, v2, v3;
-    };
-    auto load = [&](int c, Stage &r) __attribute__((always_inline)) {
-        const int k = min(c, nchunk - 1) * kChunk + 2 * lane;
-        r.v0 = *reinterpret_cast<const dvec2 *>(r0 + k);
-        r.v1 = *reinterpret_cast<const dvec2 *>(r1 + k);
-        r.v2 = *reinterpret_cast<const dvec2 *>(r2 + k);
-        r.v3 = *reinterpret_cast<const dvec2 *>(r3 + k);
-    };
-    auto put = [&](int c, const Stage &r) __attribute__((always_inline)) {
-        double *p = buf + (c & 1) * (kChainRows * kSRow) + 2 * lane;
-        *reinterpret_cast<dvec2 *>(p) = r.v0;
-        *reinterpret_cast<dvec2 *>(p + kSRow) = r.v1;
-        *reinterpret_cast<dvec2 *>(p + 2 * kSRow) = r.v2;
-        *reinterpret_cast<dvec2 *>(p + 3 * kSRow) = r.v3;
-    };
+    double *to_even = buf + 2 * lane, *to_odd = to_even + kChainRows * kSRow;
     const double *even = buf + (lane & 3) * kSRow + (lane >> 4), *odd = even + kChainRows * kSRow;
-    Stage s0, s1;
+    dvec2 s0[kChainRows], s1[kChainRows];
     dvec2 kr[kRing], sr[kReadAhead];
+    auto load = [&](int c, dvec2 (&st)[kChainRows]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++) st[m] = rows.load(m, min(c, nchunk - 1));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // the loads in about the order of the loop, whose waits hold for its first
+    // turn as well
+    auto fill = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kChunkUnits; i++) {
+            kr[h + i] = ku.load(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ku.advance();
+    };
     load(0, s0);
     load(1, s1);
+    fill(0);
 #pragma unroll
-    for (int i = 0; i < kRing; i++) {
-        kr[i] = ku.load(i % kChunkUnits);
-        if (i % kChunkUnits == kChunkUnits - 1) ku.advance();
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    put(0, s0);
+    for (int m = 0; m < kChainRows; m++) *reinterpret_cast<dvec2 *>(to_even + m * kSRow) = s0[m];
     load(2, s0);
+    fill(kChunkUnits);
 #pragma unroll
     for (int j = 0; j < kReadAhead; j++) sr[j] = dvec2{even[j * kUnit], even[j * kUnit + 4]};
     double acc = 0.0;
-    for (int c = 0;; c += 2) {
-        put(c + 1, s1);
-        load(c + 3, s1);
-        chain_chunk<0>(acc, kr, sr, ku, even, odd);
-        if (c + 1 >= nchunk) break;
-        put(c + 2, s0);
-        load(c + 4, s0);
-        chain_chunk<kChunkUnits>(acc, kr, sr, ku, odd, even);
-        if (c + 2 >= nchunk) break;
+    // two chunks a turn and an odd one behind the loop: with an exit between
+    // the two the waits let 19 loads stay in flight, not 39
+    for (int c = 0; c + 1 < nchunk; c += 2) {
+        chain_chunk<0>(acc, kr, sr, ku, even, odd, s1, rows, to_odd, min(c + 3, nchunk - 1));
+        chain_chunk<kChunkUnits>(acc, kr, sr, ku, odd, even, s0, rows, to_even, min(c + 4, nchunk - 1));
     }
+    if (nchunk & 1) chain_chunk<0>(acc, kr, sr, ku, even, odd, s1, rows, to_odd, nchunk - 1);
     // 4x4x4_4b output: lane l holds row l>>4 of block (l>>2)&3, column l&3
     const int i = mg * kChainRows + (lane & 3), t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
     if (i < a.P && t < a.T) a.emod[static_cast<size_t>(i) * a.T + t] = acc;
@@ -1044,9 +1053,17 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     // different workgroups (and CUs).
     const int gwave = wid * nwg + blockIdx.x;
     unsigned target = 0;
-    const int ks = (FOLD ? a.P : a.MG) * a.TB;  // contraction tasks
+    // The contraction's tasks and the moment folds of this workgroup's XCD
+    // (workgroups go to the XCDs in turn), in equal ranges: neighbouring tasks
+    // share a tau block's K or a member group's rows in its L2.
+    const int nx = min(kXcds, nwg), xcd = blockIdx.x % nx;
+    const int xwg = (nwg - xcd + nx - 1) / nx, xwave = wid * xwg + blockIdx.x / nx;  // workgroups here, this wave
+    const int before = xcd * (nwg / nx) + min(xcd, nwg % nx);                        // workgroups of lower XCDs
+    const int groups = FOLD ? a.P : a.MG;
     const int nmom = a.use_first + a.use_third;  // moment folds per member
-    const int ntask = ks + nmom * a.P;
+    auto share = [&](int all, int wgs) { return static_cast<int>(static_cast<long>(all) * wgs / nwg); };
+    const int ks0 = share(groups * a.TB, before), nks = share(groups * a.TB, before + xwg) - ks0;
+    const int mom0 = share(nmom * a.P, before), nmoms = share(nmom * a.P, before + xwg) - mom0;
     const int nblk = a.stride / kChunk;
     // This wave's share of the trials' blocks: equal shares, across members.
     // (In runs of 8 blocks of one member, 4096 of them for 992 waves, the fifth
@@ -1149,22 +1166,31 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
 
         // Model ISF chains and moment rows, one wave per task: of the trials,
         // or of the current genomes for the initial fitness.
-        for (int task = gwave; task < ntask; task += total_waves) {
+        for (int n = xwave; n < nks + nmoms; n += xwg * kEvoWaves) {
             double *buf = lds + wid * kChainLds;
-            if (task < ks) {
-                const int tb = task % a.TB, mg = task / a.TB;
+            if (n < nks) {
+                const int task = ks0 + n;
+                const int tb = a.by_tau ? task / groups : task % a.TB, mg = a.by_tau ? task % groups : task / a.TB;
                 if constexpr (FOLD) {
                     const double e = fold_task(a.ktile + static_cast<size_t>(tb) * a.stride * kChainTau,
                                                row_of(a, cur, mg, true), nblk, a.Kc, (a.G & 1) != 0, buf);
                     const int t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
                     if ((lane & 3) == 0 && t < a.T) a.emod[static_cast<size_t>(mg) * a.T + t] = e;
                 } else {
-                    auto row = [&](int m) { return row_of(a, cur, min(mg * kChainRows + m, a.P - 1), !init); };
-                    chain_task(a, row(0), row(1), row(2), row(3), tb, mg, buf);
+                    GenomeRows rows;
+                    const int first = mg * kChainRows;
+                    const int c = cur[min(first + (lane & (kChainRows - 1)), a.P - 1)];
+#pragma unroll
+                    for (int m = 0; m < kChainRows; m++) {
+                        const bool second = (__builtin_amdgcn_readlane(c, m) != 0) == init;
+                        rows.row[m] = (second ? a.pop1 : a.pop0) + static_cast<size_t>(min(first + m, a.P - 1)) * a.stride;
+                    }
+                    rows.vo = lane * 16;
+                    chain_task(a, rows, tb, mg, buf);
                 }
             } else {
-                const int i = (task - ks) / nmom;
-                const bool third = !a.use_first || (task - ks) % nmom != 0;
+                const int task = mom0 + n - nks, i = task / nmom;
+                const bool third = !a.use_first || task % nmom != 0;
                 const double m = wave_fold(row_of(a, cur, i, !init), third ? a.tterm : a.fterm, a.Kc, a.G, buf);
                 if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }

@@ -75,6 +75,7 @@ struct EvoArgs {
     int rstride;                 // row stride of the draws: Kc padded to whole 16-byte pairs
     int local;                   // every workgroup repeats the selection (evolve_local)
     int MG, TB;                  // member groups of kChainRows, tau blocks of kChainTau
+    int by_tau;                  // contraction tasks in order of tau blocks, else of member groups (evolve_by_tau)
     int use_first, use_third, renorm, allow_neg, init_mode, track_stats;
     double stop, zeroth, first_moment, third_moment, third_moment_error;
     int use_nfm;                 // -1st-moment term of the fitness (bdsf): weights nfm_dt [T]
@@ -139,6 +140,16 @@ inline int evolve_local(int P, int T, int nsign, int use_nfm)
 {
     const long resid = static_cast<long>(P) * (T | 1);
     return resid <= kLocalResid && resid * (1 + use_nfm) + static_cast<long>(P) * (2 + 2 * nsign) <= kResidLds;
+}
+// Whether an XCD's range of contraction tasks reads fewer rows in order of tau
+// blocks (16 K rows each) than in order of member groups (`rows` genome rows).
+constexpr int kXcds = 8;
+inline int evolve_by_tau(int groups, int rows, int TB)
+{
+    const long n = (static_cast<long>(groups) * TB + kXcds - 1) / kXcds;
+    const long tau = kChainTau * ((n - 1) / groups + 2) + rows * (n < groups ? n : groups);
+    const long member = kChainTau * (n < TB ? n : TB) + rows * ((n - 1) / TB + 2);
+    return tau < member;
 }
 // Doubles of the K operand of TB tau blocks.
 inline size_t ktile_doubles(int TB, int stride)
