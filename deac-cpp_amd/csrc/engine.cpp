@@ -45,7 +45,7 @@ struct deac_handle {
     // Three sets of the walk's records, four of its generation starts (see
     // the generation loop).
     unsigned *sync = nullptr;           // [2][8]
-    long *iter = nullptr;               // [2][2]: split loop generation counters, per buffer set
+    long *iter = nullptr;               // [2][4]: split loop generation counters, per buffer set
     int *host_status = nullptr;         // [3][4], pinned: status of the sets, then of the initial fitness
     deac::MemberCtl *ctl[3] = {};
     uint64_t *raw[2] = {};
@@ -62,7 +62,7 @@ struct deac_handle {
     // per set: walk start, walk end, mask end (fused path: the first batch's
     // masks between the first two), evolve start, evolve end (draws free),
     // status copied (split loop)
-    hipEvent_t kev[2][7] = {};
+    hipEvent_t kev[3][7] = {};
     deac_run_profile last{};
     // Split loop: contraction operands of the precision it last ran at.
     struct Split {
@@ -317,7 +317,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     A(h->emod, static_cast<size_t>(P) * T);
     A(h->mom, static_cast<size_t>(P) * 4);
     A(h->sync, 16);
-    A(h->iter, 4);
+    A(h->iter, 8);
     for (deac::MemberCtl *&p : h->ctl) A(p, static_cast<size_t>(h->batch) * P);
     for (uint64_t *&p : h->raw) A(p, static_cast<size_t>(h->batch) * P * h->rstride);
     for (uint64_t *&p : h->gen_start) A(p, static_cast<size_t>(h->batch) * 4);
@@ -674,8 +674,9 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         ea.status = reinterpret_cast<int *>(h->sync + 4);
         const int *halt = ea.status;
         // model ISF (and moment rows) of the contraction's genomes: the
-        // current ones for the initial fitness, the trials otherwise
-        auto evaluate = [&](const deac::EvoArgs &a, int init) -> deac_status {
+        // current ones for the initial fitness, the trials otherwise; packed:
+        // the genome operand is there already
+        auto evaluate = [&](const deac::EvoArgs &a, int init, bool packed) -> deac_status {
             if (y.precision == DEAC_PRECISION_FP64 && a.fold_ks && !init) {
                 DEAC_HIP(deac::launch_split_fold(a, s));
             } else if (y.precision == DEAC_PRECISION_FP64) {
@@ -686,29 +687,36 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             } else {
                 if (y.precision == DEAC_PRECISION_FP32) {
                     float *B = static_cast<float *>(sp.B);
-                    DEAC_HIP(deac::launch_split_pack_fp32(a, init, B, y.Nt, Kb, s));
+                    if (!packed) DEAC_HIP(deac::launch_split_pack_fp32(a, init, B, y.Nt, Kb, s));
                     DEAC_HIP(deac::launch_ks_fp32(static_cast<const float *>(sp.A), B, sp.part, y.Mt, y.Nt, Kb,
                                                   y.kb_per_slice, y.slices, s, nullptr, nullptr, halt));
                 } else {
-                    DEAC_HIP(deac::launch_split_pack_bf16x3(a, init, sp.B, sp.Bl, y.Nt, Kb, s));
+                    if (!packed) DEAC_HIP(deac::launch_split_pack_bf16x3(a, init, sp.B, sp.Bl, y.Nt, Kb, s));
                     DEAC_HIP(deac::launch_ks_bf16x3(sp.A, sp.Al, sp.B, sp.Bl, sp.part, y.Mt, y.Nt, Kb, y.kb_per_slice,
                                                     y.slices, s, nullptr, nullptr, halt));
                 }
-                DEAC_HIP(deac::launch_split_model(a, sp.part, y.slices, static_cast<int>(y.npad()),
-                                                  y.mpad() * y.npad(), sp.ex, s));
             }
             if (a.use_first || a.use_third) DEAC_HIP(deac::launch_split_moments(a, init, s));
             return DEAC_OK;
         };
+        auto select = [&](const deac::EvoArgs &a, int g, int init) -> deac_status {
+            if (y.precision == DEAC_PRECISION_FP64)
+                DEAC_HIP(deac::launch_split_select(a, g, init, s));
+            else
+                DEAC_HIP(deac::launch_split_model_select(a, g, init, sp.part, y.slices, static_cast<int>(y.npad()),
+                                                         static_cast<int>(y.mpad()), sp.ex, s));
+            return DEAC_OK;
+        };
         // One generation g of a batch: top and trials, renormalization,
         // contraction, moments, selection; with a.iter, the generation comes
-        // from the device counter, which the last kernel advances.
+        // from the device counter, which they advance.
         auto one_generation = [&](const deac::EvoArgs &a, int g) -> deac_status {
-            DEAC_HIP(deac::launch_split_trial(a, g, s));  // with the top of generation g
+            const bool fp64 = y.precision == DEAC_PRECISION_FP64, pack = !fp64 && !a.renorm;
+            // with the top of generation g
+            DEAC_HIP(deac::launch_split_trial(a, g, pack ? y.precision : DEAC_PRECISION_FP64, sp.B, sp.Bl, Kb, s));
             if (a.renorm) DEAC_HIP(deac::launch_split_renorm(a, s));
-            DEAC_TRY(evaluate(a, 0));
-            DEAC_HIP(deac::launch_split_select(a, g, 0, s));
-            if (a.iter) DEAC_HIP(deac::launch_split_iter(a.iter, 0, 0, s));
+            DEAC_TRY(evaluate(a, 0, pack));
+            DEAC_TRY(select(a, g, 0));
             return DEAC_OK;
         };
         // Graphs: the kernels of graph_len generations captured once per
@@ -736,30 +744,28 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         };
         // Initial fitness (deac.cpp:857-976).
         DEAC_HIP(deac::launch_zero_u32(h->sync, 8, s));
-        DEAC_TRY(evaluate(ea, 1));
-        DEAC_HIP(deac::launch_split_select(ea, 0, 1, s));
+        DEAC_TRY(evaluate(ea, 1, false));
+        DEAC_TRY(select(ea, 0, 1));
         DEAC_HIP(hipEventRecord(h->ev0, s));
         DEAC_HIP(hipStreamWaitEvent(d, h->ev0, 0));  // RNG state uploaded
-        auto walk = [&](size_t b) -> deac_status {
-            const int k = static_cast<int>(b & 1);
-            hipEvent_t *e = h->kev[k];
-            if (b >= 2) DEAC_HIP(hipStreamWaitEvent(d, e[5], 0));  // batch b-2 done with the set
-            wa.gen_start = h->gen_start[k];
-            wa.ctl = h->ctl[k];
-            wa.ngen = plan[b].second;
-            ma.ctl = h->ctl[k];
-            ma.raw = h->raw[k];
-            ma.ngen = plan[b].second;
-            DEAC_HIP(hipEventRecord(e[0], d));
+        // Draws of batch b, into the buffers of batch b-2 once that is done.
+        auto draw = [&](size_t b) -> deac_status {
+            hipEvent_t *ev = h->kev[b % 3];
+            walk_args(b, halt);
+            mask_args(b, halt);
+            wa.ctl = h->ctl[b & 1];  // (two sets, which the graphs hold)
+            ma.ctl = h->ctl[b & 1];
+            if (b >= 2) DEAC_HIP(hipStreamWaitEvent(d, h->kev[(b - 2) % 3][5], 0));
+            DEAC_HIP(hipEventRecord(ev[0], d));
             DEAC_HIP(deac::launch_walk(wa, d));
-            DEAC_HIP(hipEventRecord(e[1], d));
+            DEAC_HIP(hipEventRecord(ev[1], d));
             DEAC_HIP(deac::launch_mask(ma, deac::WalkArgs{}, d));
-            DEAC_HIP(hipEventRecord(e[2], d));
+            DEAC_HIP(hipEventRecord(ev[2], d));
             return DEAC_OK;
         };
         auto generations = [&](size_t b) -> deac_status {
             const int k = static_cast<int>(b & 1);
-            hipEvent_t *e = h->kev[k];
+            hipEvent_t *e = h->kev[b % 3];
             const int nb = plan[b].second;
             DEAC_HIP(hipStreamWaitEvent(s, e[2], 0));  // draws ready
             DEAC_HIP(hipEventRecord(e[3], s));
@@ -770,8 +776,8 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             int g = 0;
             if (graph_len > 0 && nb >= graph_len) {
                 deac::EvoArgs eg = ea;
-                eg.iter = h->iter + 2 * k;
-                DEAC_HIP(deac::launch_split_iter(eg.iter, eg.gen0, 1, s));
+                eg.iter = h->iter + 4 * k;
+                DEAC_HIP(deac::launch_split_iter(eg.iter, eg.gen0, s));
                 if (!gexec[k] && !capture(k, eg)) graph_len = 0;
                 if (gexec[k]) {
                     for (; g + graph_len <= nb; g += graph_len) {
@@ -787,13 +793,17 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             DEAC_HIP(hipEventRecord(e[6], s));
             return DEAC_OK;
         };
-        DEAC_TRY(walk(0));
-        if (plan.size() > 1) DEAC_TRY(walk(1));
+        DEAC_TRY(draw(0));
+        if (plan.size() > 1) DEAC_TRY(draw(1));
         DEAC_TRY(generations(0));
         for (size_t b = 0; b < plan.size(); b++) {
+            // The draws are queued while batch b runs, ahead of batch b+1, whose
+            // launches keep the host for most of a batch (behind them, or after
+            // batch b, they left 0.2 ms between batches of 0.8 ms).
+            if (b + 2 < plan.size()) DEAC_TRY(draw(b + 2));
             if (b + 1 < plan.size()) DEAC_TRY(generations(b + 1));
             const int k = static_cast<int>(b & 1);
-            hipEvent_t *e = h->kev[k];
+            hipEvent_t *e = h->kev[b % 3];
             DEAC_HIP(hipEventSynchronize(e[6]));
             float t_walk = 0, t_mask = 0, t_evo = 0;
             DEAC_HIP(hipEventElapsedTime(&t_walk, e[0], e[1]));
@@ -809,14 +819,13 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
             if (status[0]) {
                 stopped_at = static_cast<long>(plan[b].first) + status[1];
                 uint64_t st4[4];
-                DEAC_HIP(hipMemcpy(st4, h->gen_start[k] + static_cast<size_t>(status[1]) * 4, sizeof st4,
+                DEAC_HIP(hipMemcpy(st4, h->gen_start[b % 4] + static_cast<size_t>(status[1]) * 4, sizeof st4,
                                    hipMemcpyDeviceToHost));
                 std::memcpy(rng.s, st4, sizeof st4);
                 done += static_cast<size_t>(status[1]);
                 return DEAC_OK;
             }
             done += static_cast<size_t>(plan[b].second);
-            if (b + 2 < plan.size()) DEAC_TRY(walk(b + 2));
         }
         return DEAC_OK;
     };

@@ -103,7 +103,7 @@ struct EvoArgs {
     int ngen;
     int nwg;                     // workgroups that evolve
     long *iter;                  // split loop under graph capture: [0] gen0, [1] generation within the batch
-                                 // (read in place of gen0 and the kernels' g), or null
+                                 // (read in place of gen0 and the kernels' g; the selection reads [2]), or null
 };
 
 // Wide walk: draws per lane and round for the jDE controls, donor draws per

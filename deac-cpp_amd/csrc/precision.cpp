@@ -194,11 +194,11 @@ extern "C" deac_status deac_model_isf(const deac_problem *p, const double *genom
         std::vector<float> E32(mn);
         PREC_HIP(hipMemcpyAsync(E32.data(), out, E32.size() * sizeof(float), hipMemcpyDeviceToHost, s));
         PREC_HIP(hipStreamSynchronize(s));
-        const size_t Npad = y.npad();
+        const size_t Mpad = y.mpad();
         for (int n = 0; n < N; n++)
             for (int t = 0; t < T; t++)
                 E[static_cast<size_t>(n) * T + t] =
-                    std::ldexp(static_cast<double>(E32[static_cast<size_t>(t) * Npad + n]), y.ex[t]);
+                    std::ldexp(static_cast<double>(E32[static_cast<size_t>(n) * Mpad + t]), y.ex[t]);
     }
     if (kernel_ms) {
         float ms = 0.0f;

@@ -18,11 +18,12 @@
 //                          B[nt][kb][lane] = S[16 nt + lane%16][4 kb + lane/16];
 //   16x16x32 (BF16):       A[mt][kb][lane][e] = K[16 mt + lane%16][32 kb + 8 (lane/16) + e],
 //                          B likewise with S.
-// Outputs: FP64 E[n][t] directly; FP32/BF16 partial tiles [slice][Mpad][Npad]
+// Outputs: FP64 E[n][t] directly; FP32/BF16 partial tiles [slice][Npad][Mpad]
 // reduced in slice order by reduce_slices.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "precision_kernels.hpp"
@@ -80,79 +81,162 @@ __device__ __forceinline__ void store_partial(float *part, int slice, int Mpad, 
                                               f4 acc)
 {
     // lane l holds rows 4 (l/16) + v of the tile, column l%16
-    float *p = part + (static_cast<size_t>(slice) * Mpad + mt * 16 + 4 * (lane >> 4)) * Npad + nt * 16 + (lane & 15);
-    for (int v = 0; v < 4; v++) p[static_cast<size_t>(v) * Npad] = acc[v];
+    float *p = part + (static_cast<size_t>(slice) * Npad + nt * 16 + (lane & 15)) * Mpad + mt * 16 + 4 * (lane >> 4);
+    *reinterpret_cast<f4 *>(p) = acc;
 }
 
-// grid (Mt, ceil(Nt/4), slices): one output tile per wave over one slice
-__global__ __launch_bounds__(256) void ks_fp32_kernel(const float *__restrict__ A, const float *__restrict__ B,
-                                                      float *__restrict__ part, int Mt, int Nt, int Kb, int kb_per_slice,
-                                                      const int *halt)
+// What one wavefront contracts: MB tau tiles x NB genome tiles over one slice.  The workgroups (one wavefront each) of an XCD, which they go to in
+// turn, take a range of (slice, genome tiles, tau tiles), tau tiles fastest,
+// so that a slice's genomes come through one L2.
+constexpr int kXcds = 8;
+template <int MB, int NB>
+struct SliceTask {
+    int slice, mt[MB], nt[NB];
+    bool mine;
+    __device__ __forceinline__ SliceTask(int Mt, int Nt, int slices)
+    {
+        const int mp = (Mt + MB - 1) / MB, ng = (Nt + NB - 1) / NB;
+        const int task = blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+        slice = task / (mp * ng);
+        mine = slice < slices;
+        // past the last tile: the last one again
+        for (int m = 0; m < MB; m++) mt[m] = min(task % mp * MB + m, Mt - 1);
+        for (int n = 0; n < NB; n++) nt[n] = min(task / mp % ng * NB + n, Nt - 1);
+    }
+    __device__ __forceinline__ void store(float *part, int Mt, int Nt, const f4 (&acc)[MB][NB]) const
+    {
+        for (int m = 0; m < MB; m++)
+            for (int n = 0; n < NB; n++)
+                if ((m == 0 || mt[m] != mt[m - 1]) && (n == 0 || nt[n] != nt[n - 1]))
+                    store_partial(part, slice, Mt * 16, Nt * 16, mt[m], nt[n], threadIdx.x, acc[m][n]);
+    }
+};
+
+// FP32: two tau tiles per wavefront or one, whichever gives the fullest SIMD
+// fewer tiles (one reads more, 320 bytes per MFMA instead of 192 at NB = 4): T =
+// 257, 64 genomes, 114 slices make 1026 wavefronts of two, 22.8 us, or 1938 of
+// one, 16.0.
+constexpr int kSimds = 1024;
+inline int slice_tasks(int MB, int NB, int Mt, int Nt, int slices)
+{
+    return slices * ((Mt + MB - 1) / MB) * ((Nt + NB - 1) / NB);
+}
+inline bool two_tau_tiles(int NB, int Mt, int Nt, int slices)
+{
+    auto fullest = [&](int MB) { return (slice_tasks(MB, NB, Mt, Nt, slices) + kSimds - 1) / kSimds * MB; };
+    return fullest(2) <= fullest(1);
+}
+
+// Bound: the matrix cores (32 cycles per MFMA) and the operands from L2.  T =
+// 257, 64 genomes of 32768 positions: 16.0 us (71 TFLOP/s); one output tile per
+// wavefront (512 bytes per MFMA) 24.8.
+template <int MB, int NB>
+__global__ __launch_bounds__(64) void ks_fp32_kernel(const float *__restrict__ A, const float *__restrict__ B,
+                                                     float *__restrict__ part, int Mt, int Nt, int Kb, int kb_per_slice,
+                                                     int slices, const int *halt)
 {
     if (halt && *halt) return;
-    const int lane = threadIdx.x & 63;
-    const int mt = blockIdx.x, nt = blockIdx.y * 4 + static_cast<int>(threadIdx.x >> 6), slice = blockIdx.z;
-    if (nt >= Nt) return;
-    const int kb0 = slice * kb_per_slice, kb1 = min(kb0 + kb_per_slice, Kb);
-    const float *a = A + static_cast<size_t>(mt) * Kb * 64 + lane;
-    const float *b = B + static_cast<size_t>(nt) * Kb * 64 + lane;
-    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    float ra[kDepth], rb[kDepth];
+    const SliceTask<MB, NB> t(Mt, Nt, slices);
+    if (!t.mine) return;
+    // a slice's length is a multiple of kDepth
+    const int kb0 = t.slice * kb_per_slice, turns = (min(kb0 + kb_per_slice, Kb) - kb0) / kDepth;
+    const float *a[MB], *b[NB];
+    for (int m = 0; m < MB; m++) a[m] = A + (static_cast<size_t>(t.mt[m]) * Kb + kb0) * 64 + threadIdx.x;
+    for (int n = 0; n < NB; n++) b[n] = B + (static_cast<size_t>(t.nt[n]) * Kb + kb0) * 64 + threadIdx.x;
+    f4 acc[MB][NB] = {};
+    float ra[kDepth][MB], rb[kDepth][NB];
+    // (the scheduler would gather the loads in front of their use)
+    auto load = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kDepth; i++) {
-        ra[i] = a[static_cast<size_t>(kb0 + i) * 64];
-        rb[i] = b[static_cast<size_t>(kb0 + i) * 64];
-    }
-    for (int kb = kb0; kb < kb1; kb += kDepth) {
+        for (int m = 0; m < MB; m++) ra[i][m] = a[m][i * 64];
+#pragma unroll
+        for (int n = 0; n < NB; n++) rb[i][n] = b[n][i * 64];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto advance = [&]() __attribute__((always_inline)) {
+        for (int m = 0; m < MB; m++) a[m] += kDepth * 64;
+        for (int n = 0; n < NB; n++) b[n] += kDepth * 64;
+    };
+    auto contract = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+#pragma unroll
+            for (int m = 0; m < MB; m++)
+                acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[i][m], rb[i][n], acc[m][n], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int i = 0; i < kDepth; i++) load(i);
+    for (int turn = 1; turn < turns; turn++) {
+        advance();
 #pragma unroll
         for (int i = 0; i < kDepth; i++) {
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[i], rb[i], acc, 0, 0, 0);
-            const size_t nk = static_cast<size_t>(min(kb + i + kDepth, kb1 - 1)) * 64;
-            ra[i] = a[nk];
-            rb[i] = b[nk];
+            contract(i);
+            load(i);
         }
     }
-    store_partial(part, slice, Mt * 16, Nt * 16, mt, nt, lane, acc);
+#pragma unroll
+    for (int i = 0; i < kDepth; i++) contract(i);
+    t.store(part, Mt, Nt, acc);
 }
 
-__global__ __launch_bounds__(256) void ks_bf16x3_kernel(const bf8 *__restrict__ Ah, const bf8 *__restrict__ Al,
-                                                        const bf8 *__restrict__ Bh, const bf8 *__restrict__ Bl,
-                                                        float *__restrict__ part, int Mt, int Nt, int Kb,
-                                                        int kb_per_slice, const int *halt)
+template <int MB, int NB>
+__global__ __launch_bounds__(64) void ks_bf16x3_kernel(const bf8 *__restrict__ Ah, const bf8 *__restrict__ Al,
+                                                       const bf8 *__restrict__ Bh, const bf8 *__restrict__ Bl,
+                                                       float *__restrict__ part, int Mt, int Nt, int Kb,
+                                                       int kb_per_slice, int slices, const int *halt)
 {
     if (halt && *halt) return;
-    const int lane = threadIdx.x & 63;
-    const int mt = blockIdx.x, nt = blockIdx.y * 4 + static_cast<int>(threadIdx.x >> 6), slice = blockIdx.z;
-    if (nt >= Nt) return;
-    const int kb0 = slice * kb_per_slice, kb1 = min(kb0 + kb_per_slice, Kb);
-    const size_t aoff = static_cast<size_t>(mt) * Kb * 64 + lane, boff = static_cast<size_t>(nt) * Kb * 64 + lane;
-    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    bf8 rah[kDepth16], ral[kDepth16], rbh[kDepth16], rbl[kDepth16];
+    const SliceTask<MB, NB> t(Mt, Nt, slices);
+    if (!t.mine) return;
+    // a slice's length is a multiple of kDepth16
+    const int kb0 = t.slice * kb_per_slice, turns = (min(kb0 + kb_per_slice, Kb) - kb0) / kDepth16;
+    size_t a[MB], b[NB];
+    for (int m = 0; m < MB; m++) a[m] = (static_cast<size_t>(t.mt[m]) * Kb + kb0) * 64 + threadIdx.x;
+    for (int n = 0; n < NB; n++) b[n] = (static_cast<size_t>(t.nt[n]) * Kb + kb0) * 64 + threadIdx.x;
+    f4 acc[MB][NB] = {};
+    bf8 ah[kDepth16][MB], al[kDepth16][MB], bh[kDepth16][NB], bl[kDepth16][NB];
+    auto load = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kDepth16; i++) {
-        const size_t k = static_cast<size_t>(kb0 + i) * 64;
-        rah[i] = Ah[aoff + k];
-        ral[i] = Al[aoff + k];
-        rbh[i] = Bh[boff + k];
-        rbl[i] = Bl[boff + k];
-    }
-    for (int kb = kb0; kb < kb1; kb += kDepth16) {
+        for (int m = 0; m < MB; m++) ah[i][m] = Ah[a[m] + i * 64], al[i][m] = Al[a[m] + i * 64];
+#pragma unroll
+        for (int n = 0; n < NB; n++) bh[i][n] = Bh[b[n] + i * 64], bl[i][n] = Bl[b[n] + i * 64];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto advance = [&]() __attribute__((always_inline)) {
+        for (int m = 0; m < MB; m++) a[m] += kDepth16 * 64;
+        for (int n = 0; n < NB; n++) b[n] += kDepth16 * 64;
+    };
+    // one product of the three for every tile, small terms first
+    auto product = [&](const bf8 (&x)[MB], const bf8 (&y)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+#pragma unroll
+            for (int m = 0; m < MB; m++)
+                acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[m], y[n], acc[m][n], 0, 0, 0);
+    };
+    auto contract = [&](int i) __attribute__((always_inline)) {
+        product(al[i], bh[i]);
+        product(ah[i], bl[i]);
+        product(ah[i], bh[i]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int i = 0; i < kDepth16; i++) load(i);
+    for (int turn = 1; turn < turns; turn++) {
+        advance();
 #pragma unroll
         for (int i = 0; i < kDepth16; i++) {
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ral[i], rbh[i], acc, 0, 0, 0);  // small terms first
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rah[i], rbl[i], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rah[i], rbh[i], acc, 0, 0, 0);
-            const size_t nk = static_cast<size_t>(min(kb + i + kDepth16, kb1 - 1)) * 64;
-            rah[i] = Ah[aoff + nk];
-            ral[i] = Al[aoff + nk];
-            rbh[i] = Bh[boff + nk];
-            rbl[i] = Bl[boff + nk];
+            contract(i);
+            load(i);
         }
     }
-    store_partial(part, slice, Mt * 16, Nt * 16, mt, nt, lane, acc);
+#pragma unroll
+    for (int i = 0; i < kDepth16; i++) contract(i);
+    t.store(part, Mt, Nt, acc);
 }
 
-// E32[m][n] = sum over slices (in order, FP32) of part[slice][m][n]
+// E32[n][m] = sum over slices (in order, FP32) of part[slice][n][m]
 __global__ __launch_bounds__(256) void reduce_slices_kernel(const float *__restrict__ part, float *__restrict__ out,
                                                             int slices, size_t mn)
 {
@@ -177,19 +261,35 @@ hipError_t launch_ks_fp64(const double *A, const double *B, double *E, int T, in
 hipError_t launch_ks_fp32(const float *A, const float *B, float *part, int Mt, int Nt, int Kb, int kb_per_slice,
                           int slices, hipStream_t s, hipEvent_t start, hipEvent_t stop, const int *halt)
 {
-    hipExtLaunchKernelGGL(ks_fp32_kernel, dim3(Mt, (Nt + 3) / 4, slices), dim3(256), 0, s, start, stop, 0, A, B, part,
-                          Mt, Nt, Kb, kb_per_slice, halt);
-    return hipGetLastError();
+    auto go = [&](auto kernel, int MB, int NB) {
+        const unsigned grid = (slice_tasks(MB, NB, Mt, Nt, slices) + kXcds - 1) / kXcds * kXcds;
+        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, s, start, stop, 0, A, B, part, Mt, Nt, Kb, kb_per_slice,
+                              slices, halt);
+        return hipGetLastError();
+    };
+    const bool two = two_tau_tiles(std::min(Nt, 4), Mt, Nt, slices);
+    if (Nt == 1) return two ? go(ks_fp32_kernel<2, 1>, 2, 1) : go(ks_fp32_kernel<1, 1>, 1, 1);
+    if (Nt == 2) return two ? go(ks_fp32_kernel<2, 2>, 2, 2) : go(ks_fp32_kernel<1, 2>, 1, 2);
+    if (Nt == 3) return two ? go(ks_fp32_kernel<2, 3>, 2, 3) : go(ks_fp32_kernel<1, 3>, 1, 3);
+    return two ? go(ks_fp32_kernel<2, 4>, 2, 4) : go(ks_fp32_kernel<1, 4>, 1, 4);
 }
 
 hipError_t launch_ks_bf16x3(const void *Ah, const void *Al, const void *Bh, const void *Bl, float *part, int Mt,
                             int Nt, int Kb, int kb_per_slice, int slices, hipStream_t s, hipEvent_t start,
                             hipEvent_t stop, const int *halt)
 {
-    hipExtLaunchKernelGGL(ks_bf16x3_kernel, dim3(Mt, (Nt + 3) / 4, slices), dim3(256), 0, s, start, stop, 0,
-                          static_cast<const bf8 *>(Ah), static_cast<const bf8 *>(Al), static_cast<const bf8 *>(Bh),
-                          static_cast<const bf8 *>(Bl), part, Mt, Nt, Kb, kb_per_slice, halt);
-    return hipGetLastError();
+    auto go = [&](auto kernel, int MB, int NB) {
+        const unsigned grid = (slice_tasks(MB, NB, Mt, Nt, slices) + kXcds - 1) / kXcds * kXcds;
+        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, s, start, stop, 0, static_cast<const bf8 *>(Ah),
+                              static_cast<const bf8 *>(Al), static_cast<const bf8 *>(Bh), static_cast<const bf8 *>(Bl),
+                              part, Mt, Nt, Kb, kb_per_slice, slices, halt);
+        return hipGetLastError();
+    };
+    // (two genome tiles at most: their operands of four k-blocks take 128
+    // registers.  Two tau tiles always: one, where it fills the SIMDs better,
+    // reads 6 KB per three MFMAs instead of 4, 30.4 and 32.0 ms for 600
+    // generations at T = 257 and 64 genomes of 32768 positions.)
+    return Nt == 1 ? go(ks_bf16x3_kernel<2, 1>, 2, 1) : go(ks_bf16x3_kernel<2, 2>, 2, 2);
 }
 
 hipError_t launch_reduce_slices(const float *part, float *out, int slices, size_t mn, hipStream_t s, hipEvent_t start,

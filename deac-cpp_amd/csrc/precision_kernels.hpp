@@ -20,10 +20,10 @@ constexpr int kSweepDepth16 = 4;
 // E[n][t] (FP64, exact chains); operands in 16x16x4 lane order, Kb = genome / 4.
 hipError_t launch_ks_fp64(const double *A, const double *B, double *E, int T, int N, int Mt, int Nt, int Kb,
                           hipStream_t s, hipEvent_t start, hipEvent_t stop, const int *halt);
-// Partial FP32 tiles [slices][16 Mt][16 Nt]; Kb = genome / 4.
+// Partial FP32 tiles [slices][16 Nt][16 Mt]; Kb = genome / 4.
 hipError_t launch_ks_fp32(const float *A, const float *B, float *part, int Mt, int Nt, int Kb, int kb_per_slice,
                           int slices, hipStream_t s, hipEvent_t start, hipEvent_t stop, const int *halt);
-// Partial FP32 tiles from bfloat16 hi/lo operands in 16x16x32 lane order; Kb = genome / 32.
+// The same from bfloat16 hi/lo operands in 16x16x32 lane order; Kb = genome / 32.
 hipError_t launch_ks_bf16x3(const void *Ah, const void *Al, const void *Bh, const void *Bl, float *part, int Mt,
                             int Nt, int Kb, int kb_per_slice, int slices, hipStream_t s, hipEvent_t start,
                             hipEvent_t stop, const int *halt);

@@ -8,15 +8,17 @@
 //   split_trial_kernel    best fitness, statistics, stop test (workgroup 0),
 //                         trial vectors into each member's spare buffer
 //   split_renorm_*        per-generation renormalization, when enabled
-//   split_pack_*          trial rows into the contraction's operand layout
+//   split_pack_*          rows into the contraction's operand layout: at FP64,
+//                         where the trials are renormalized, and for the
+//                         initial fitness (the trial kernel packs the rest)
 //   ks_*_kernel           the contraction: FP64 exact chains straight into
 //                         the model ISF, or FP32 / BF16x3 genome slices
 //   split_fold_kernel     (bdsf at FP64, in place of the two above) the
 //                         reference build's rounded-product fold
-//   split_model_kernel    FP32 slices summed in slice order and scaled back
-//                         per tau row into the FP64 model ISF
 //   split_moment_kernel   first / third moment rows, when used
-//   split_select_kernel   chi^2 and greedy selection
+//   split_select_kernel   the FP32 slices summed in slice order and scaled back
+//                         per tau row into the FP64 model ISF; chi^2 and greedy
+//                         selection
 //
 // A stop found at the top of generation g sets status[0]; every later kernel
 // (of this batch and of any batch queued behind it) reads it first and
@@ -77,7 +79,7 @@ __device__ void top_scan(const EvoArgs &a, int g, Fit fit)
 // one coalesced load (up to kTopLds of them), so the sequential scans do not
 // wait on a load each.
 constexpr int kTopLds = 512;
-constexpr int kSelectLds = 4096;  // residuals staged per member (32 KB)
+constexpr int kSelectLds = 4096;  // residuals staged per member at a time (32 KB)
 
 __device__ void top_of_generation(const EvoArgs &a, int g)
 {
@@ -91,34 +93,95 @@ __device__ void top_of_generation(const EvoArgs &a, int g)
     }
 }
 
-// Trial vectors of generation g into each member's spare buffer, two genome
-// positions per work item (deac.cpp:1261-1308); the padding stays zero.
-// Workgroup 0 first runs the top of generation g: it reads only the
-// fitnesses, which no trial writes, and if its stop test fires the trials
-// are never selected (every later kernel of the generation returns).
-__global__ __launch_bounds__(kThreads) void split_trial_kernel(EvoArgs a, int g)
+// Round-to-nearest-even FP32 -> bfloat16 bits (finite inputs).
+__device__ __forceinline__ uint32_t bf16_rne(float x)
 {
+    uint32_t u = __float_as_uint(x);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return u >> 16;
+}
+
+// x = hi + lo with hi = bf16(x) and lo = bf16(x - hi), the remainder taken in
+// FP32, into half e of word e/2.
+__device__ __forceinline__ void bf16_split(float x, int e, uint32_t (&hi)[4], uint32_t (&lo)[4])
+{
+    const uint32_t h = bf16_rne(x);
+    const uint32_t r = bf16_rne(x - __uint_as_float(h << 16));
+    hi[e >> 1] |= h << (16 * (e & 1));
+    lo[e >> 1] |= r << (16 * (e & 1));
+}
+
+// Trial vectors of generation g into each member's spare buffer
+// (deac.cpp:1261-1308; the padding stays zero), and into the contraction's
+// operand B (Bl: the BF16x3 remainders) where its precision is PACK, in the
+// layout that the pack kernels below write (they fill what the genomes do not
+// reach, once, for the initial fitness).  Workgroup 0 runs the top of the
+// generation: it reads only the fitnesses, which no trial writes, and if its
+// stop test fires the trials are never selected (every later kernel of the
+// generation returns).  The others take 16 members x 128 positions each, a
+// member's 128 per wavefront, so that rows and operand are both whole lines.
+//
+// Bound: memory (40 bytes read, 12 written per position).  64 members of 32768
+// positions: 19.3 us; with a kernel of its own for the operand 17.4 and 9.7.
+constexpr int kTileMembers = 16;
+constexpr int kTileRow = kChunk + 4;  // floats: the operand's readers meet no bank twice
+template <int PACK>
+__global__ __launch_bounds__(kThreads) void split_trial_kernel(EvoArgs a, int g, void *B, void *Bl, int Kb)
+{
+    constexpr int kWaves = kThreads / kWave, kEach = kTileMembers / kWaves;
+    __shared__ __attribute__((aligned(16))) float tile[PACK == DEAC_PRECISION_FP64 ? 1 : kTileMembers][kTileRow];
     if (stopped(a)) return;
     if (a.iter) g = static_cast<int>(a.iter[1]);
-    if (blockIdx.x == 0) top_of_generation(a, g);
-    const int half = a.stride / 2;
+    if (blockIdx.x == 0) {
+        // (the selection reads the generation here and moves the counter on)
+        if (a.iter && threadIdx.x == 0) a.iter[2] = g;
+        top_of_generation(a, g);
+        return;
+    }
+    const int nblk = a.stride / kChunk;
+    const int nt = (blockIdx.x - 1) / nblk, b = (blockIdx.x - 1) % nblk;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
     const MemberCtl *ctlg = a.ctl + static_cast<size_t>(g) * a.P;
     const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.rstride;
-    const size_t items = static_cast<size_t>(a.P) * half;
-    for (size_t it = grid_thread(); it < items; it += grid_threads()) {
-        const int i = static_cast<int>(it / half);
-        const int kp = static_cast<int>(it % half);
-        const MemberCtl &c = ctlg[i];
-        const uint64_t *raw = rawg + static_cast<size_t>(i) * a.rstride;
-        double v[2];
-        for (int e = 0; e < 2; e++) {
-            const int k = 2 * kp + e;
-            if (k >= a.Kc) v[e] = 0.0;
-            else if (a.nsign == 2 && k == a.G) v[e] = trial_value(a, c, raw, i, 0);  // deac.cpp:1305-1308
-            else v[e] = trial_value(a, c, raw, i, k);
+    auto member = [&](int j) { return nt * kTileMembers + wid + j * kWaves; };
+    auto trial = [&](int j) {
+        const int i = min(member(j), a.P - 1);
+        return Trial(a, s, a.cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i);
+    };
+    const Trial t[kEach] = {trial(0), trial(1), trial(2), trial(3)};
+    Trial::Load v[kEach] = {};
+#pragma unroll
+    for (int j = 0; j < kEach; j++) t[j].load(b, v[j]);
+#pragma unroll
+    for (int j = 0; j < kEach; j++) {
+        const bool in = member(j) < a.P;
+        const dvec2 o = in ? t[j].form(b, v[j]) : dvec2{0.0, 0.0};
+        if (in) t[j].store(b, o);
+        if constexpr (PACK != DEAC_PRECISION_FP64)
+            *reinterpret_cast<float2 *>(&tile[wid + j * kWaves][2 * lane]) =
+                make_float2(static_cast<float>(o.x), static_cast<float>(o.y));
+    }
+    if constexpr (PACK == DEAC_PRECISION_FP32) {
+        __syncthreads();
+        const int per = kChunk / 4;  // k-blocks of a tile, 64 values each
+        float4 *to = reinterpret_cast<float4 *>(static_cast<float *>(B) + (static_cast<size_t>(nt) * Kb + b * per) * 64);
+        for (int u = threadIdx.x; u < per * 16; u += kThreads) {
+            const int kb = u >> 4, k = 4 * kb + ((u >> 2) & 3), m = 4 * (u & 3);
+            if (b * per + kb < Kb) to[u] = make_float4(tile[m][k], tile[m + 1][k], tile[m + 2][k], tile[m + 3][k]);
         }
-        double *dst = (a.cur[i] ? a.pop0 : a.pop1) + static_cast<size_t>(i) * a.stride;
-        *reinterpret_cast<double2 *>(dst + 2 * kp) = make_double2(v[0], v[1]);
+    } else if constexpr (PACK == DEAC_PRECISION_BF16X3) {
+        __syncthreads();
+        const int per = kChunk / 32, kb = threadIdx.x / kWave;
+        static_assert(kThreads / kWave == kChunk / 32, "a k-block per wavefront");
+        uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
+        const float *x = &tile[lane & 15][32 * kb + 8 * (lane >> 4)];
+        for (int e = 0; e < 8; e++) bf16_split(x[e], e, hi, lo);
+        if (b * per + kb < Kb) {
+            const size_t slot = (static_cast<size_t>(nt) * Kb + b * per + kb) * 64 + lane;
+            static_cast<uint4 *>(B)[slot] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+            static_cast<uint4 *>(Bl)[slot] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        }
     }
 }
 
@@ -170,17 +233,8 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(EvoArgs a, int ini
     }
 }
 
-// Round-to-nearest-even FP32 -> bfloat16 bits (finite inputs).
-__device__ __forceinline__ uint32_t bf16_rne(float x)
-{
-    uint32_t u = __float_as_uint(x);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return u >> 16;
-}
-
-// Genome operand, 16x16x32 lane order, each value split x = hi + lo with
-// hi = bf16(x) and lo = bf16(x - hi), the remainder taken in FP32:
-// slot (nt, kb, lane) holds positions 32 kb + 8 (lane/16) + e, e = 0..7.
+// Genome operand, 16x16x32 lane order, each value split into hi and lo: slot
+// (nt, kb, lane) holds positions 32 kb + 8 (lane/16) + e, e = 0..7.
 __global__ __launch_bounds__(kThreads) void split_pack_bf16x3_kernel(EvoArgs a, int init, uint4 *Bh, uint4 *Bl,
                                                                       int Nt, int Kb)
 {
@@ -195,34 +249,10 @@ __global__ __launch_bounds__(kThreads) void split_pack_bf16x3_kernel(EvoArgs a, 
         uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
         for (int e = 0; e < 8; e++) {
             const size_t k = k0 + e;
-            if (row && k < static_cast<size_t>(a.Kc)) {
-                const float f = static_cast<float>(row[k]);
-                const uint32_t h = bf16_rne(f);
-                const uint32_t r = bf16_rne(f - __uint_as_float(h << 16));
-                hi[e >> 1] |= h << (16 * (e & 1));
-                lo[e >> 1] |= r << (16 * (e & 1));
-            }
+            if (row && k < static_cast<size_t>(a.Kc)) bf16_split(static_cast<float>(row[k]), e, hi, lo);
         }
         Bh[s] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
         Bl[s] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    }
-}
-
-// Model ISF from the FP32 genome slices: emod[n][t] = 2^ex[t] * (sum over
-// slices, in slice order, in FP32, of part[slice][t][n]).
-__global__ __launch_bounds__(kThreads) void split_model_kernel(EvoArgs a, const float *part, int slices, int Npad,
-                                                               size_t mn, const int *ex)
-{
-    if (stopped(a)) return;
-    // consecutive threads take consecutive genomes: coalesced slice reads
-    const size_t total = static_cast<size_t>(a.P) * a.T;
-    for (size_t idx = grid_thread(); idx < total; idx += grid_threads()) {
-        const int t = static_cast<int>(idx / a.P), n = static_cast<int>(idx % a.P);
-        const size_t i = static_cast<size_t>(t) * Npad + n;
-        float s = 0.0f;
-#pragma unroll 8
-        for (int k = 0; k < slices; k++) s += part[static_cast<size_t>(k) * mn + i];
-        a.emod[static_cast<size_t>(n) * a.T + t] = ldexp(static_cast<double>(s), ex[t]);
     }
 }
 
@@ -253,37 +283,92 @@ __global__ __launch_bounds__(kWave) void split_moment_kernel(EvoArgs a, int init
     a.mom[i * 4 + 1 + rr] = fold_row(chain_row(a, i, init != 0), row, a.Kc, a.G);
 }
 
-// Fitness and greedy selection, one wavefront per member (deac.cpp:1539-1572;
-// the initial fitness, deac.cpp:957-976).  The wavefront forms the weighted
-// residuals; lane 0 adds their squares in tau order, the last one fused when
+// Fitness and greedy selection, one workgroup per member (deac.cpp:1539-1572;
+// the initial fitness, deac.cpp:957-976).  The workgroup forms the weighted
+// residuals; thread 0 adds their squares in tau order, the last one fused when
 // T is odd.
-__global__ __launch_bounds__(kWave) void split_select_kernel(EvoArgs a, int g, int init)
+//
+// MODEL: the model ISF from the contraction's slices part [slices][Npad][Mpad]
+// first, emod[i][t] = 2^ex[t] * (sum over slices, in slice order, in FP32).  A
+// thread takes four timeslices of a run of slices, which it loads at once; the
+// runs then take over each other's sums in order.
+//
+// Bound: latency: loads, one barrier per run, thread 0's sum.  257 timeslices,
+// 114 slices, 64 members: 13.3 us; as two kernels, with a part of each
+// sum's loads in flight, 9.2 and 7.5.
+constexpr int kSliceRun = 8;  // slices a thread loads at once
+template <bool MODEL>
+__global__ __launch_bounds__(MODEL ? 1024 : kWave) void split_select_kernel(EvoArgs a, int g, int init, const float *part,
+                                                                            int slices, int Npad, int Mpad, const int *ex)
 {
+    constexpr int kTauEach = 4;
     if (stopped(a)) return;
-    if (a.iter && !init) g = static_cast<int>(a.iter[1]);
-    extern __shared__ double dsh[];  // T residuals (T <= kSelectLds), else one window of kWave
-    const int i = blockIdx.x, lane = threadIdx.x;
-    double chi = 0.0;
-    const int tlast = (a.T & 1) ? a.T - 1 : -1;
-    auto residual = [&](int t) { return (a.obs[t] - a.emod[static_cast<size_t>(i) * a.T + t]) / a.sig[t]; };
-    auto add = [&](int t, double du) { chi = t == tlast ? fma(du, du, chi) : chi + du * du; };
-    if (a.T <= kSelectLds) {
-        // every residual at once (their loads all in flight), then the sum
-        for (int t = lane; t < a.T; t += kWave) dsh[t] = residual(t);
-        __syncthreads();
-        if (lane == 0)
-            for (int t = 0; t < a.T; t++) add(t, dsh[t]);
-    } else {
-        for (int t0 = 0; t0 < a.T; t0 += kWave) {
-            const int t = t0 + lane;
-            dsh[lane] = t < a.T ? residual(t) : 0.0;
-            __syncthreads();
-            if (lane == 0)
-                for (int u = 0; u < min(kWave, a.T - t0); u++) add(t0 + u, dsh[u]);
-            __syncthreads();
-        }
+    if (a.iter && !init) {
+        g = static_cast<int>(a.iter[2]);
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.iter[1] = g + 1;
     }
-    if (lane != 0) return;
+    extern __shared__ __attribute__((aligned(16))) double dsh[];  // a window of residuals, and MODEL their sums
+    const int i = blockIdx.x;
+    const Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
+    Controls next;  // loaded ahead of their use
+    double old = 0.0;
+    if (threadIdx.x == 0 && !init) {
+        old = a.fitness[i];
+        next = Controls(a, s, a.ctl[static_cast<size_t>(g) * a.P + i], i);
+    }
+    double chi = 0.0;
+    for (int t0 = 0; t0 < a.T; t0 += kSelectLds) {
+        const int n = min(kSelectLds, a.T - t0);
+        if constexpr (MODEL) {
+            const int cols = (n + kTauEach - 1) / kTauEach, runs = static_cast<int>(blockDim.x) / cols;
+            const int col = threadIdx.x % cols, run = threadIdx.x / cols;
+            const int each = (slices + runs - 1) / runs, k0 = run * each, k1 = min(k0 + each, slices);
+            const float4 *from = reinterpret_cast<const float4 *>(part + static_cast<size_t>(i) * Mpad + t0) + col;
+            const size_t step = static_cast<size_t>(Npad) * Mpad / 4;
+            float4 *sums = reinterpret_cast<float4 *>(dsh + (min(kSelectLds, a.T) + 1) / 2 * 2);
+            float4 v[kSliceRun];
+            auto load = [&](int k) {
+#pragma unroll
+                for (int u = 0; u < kSliceRun; u++)
+                    if (k + u < k1) v[u] = from[(k + u) * step];
+            };
+            load(k0);
+            for (int r = 0; r < runs; r++) {
+                if (run == r) {
+                    float4 x = r ? sums[col] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    for (int k = k0; k < k1; k += kSliceRun) {
+                        if (k > k0) load(k);
+#pragma unroll
+                        for (int u = 0; u < kSliceRun; u++)
+                            if (k + u < k1) {
+                                x.x += v[u].x;
+                                x.y += v[u].y;
+                                x.z += v[u].z;
+                                x.w += v[u].w;
+                            }
+                    }
+                    sums[col] = x;
+                }
+                __syncthreads();
+            }
+        }
+        for (int u = threadIdx.x; u < n; u += blockDim.x) {
+            const int t = t0 + u;
+            double e;
+            if constexpr (MODEL) {
+                const float *sums = reinterpret_cast<const float *>(dsh + (min(kSelectLds, a.T) + 1) / 2 * 2);
+                e = ldexp(static_cast<double>(sums[u]), ex[t]);
+                a.emod[static_cast<size_t>(i) * a.T + t] = e;
+            } else {
+                e = a.emod[static_cast<size_t>(i) * a.T + t];
+            }
+            dsh[u] = (a.obs[t] - e) / a.sig[t];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) chi = chi_sum(dsh, n, (a.T & 1) && t0 + n == a.T, chi);
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
     double fit = chi / static_cast<double>(a.T);
     if (a.use_nfm) {  // deac.cpp:961-965, 1398-1416, 1543-1547
         const double mi = fold_row(a.emod + static_cast<size_t>(i) * a.T, a.nfm_dt, a.T, a.T);
@@ -300,29 +385,22 @@ __global__ __launch_bounds__(kWave) void split_select_kernel(EvoArgs a, int g, i
     }
     if (init) {
         a.fitness[i] = fit;
-    } else if (fit <= a.fitness[i]) {
-        const MemberCtl &c = a.ctl[static_cast<size_t>(g) * a.P + i];
+    } else if (fit <= old) {
         a.fitness[i] = fit;
         a.cur[i] ^= 1;
         for (int sg = 0; sg < a.nsign; sg++) {
-            double cr, f;
-            control_of(a, c, i, sg, cr, f);
-            a.cr_old[i * a.nsign + sg] = cr;
-            a.f_old[i * a.nsign + sg] = f;
+            a.cr_old[i * a.nsign + sg] = sg ? next.cr[1] : next.cr[0];
+            a.f_old[i * a.nsign + sg] = sg ? next.f[1] : next.f[0];
         }
     }
 }
 
-// The generation counter of a captured batch: set = 1 starts a batch at
-// gen0 (generation 0 of the batch), set = 0 moves to the next generation.
-__global__ void split_iter_kernel(long *iter, long gen0, int set)
+// The generation counter of a captured batch, from the batch's first
+// generation on.
+__global__ void split_iter_kernel(long *iter, long gen0)
 {
-    if (set) {
-        iter[0] = gen0;
-        iter[1] = 0;
-    } else {
-        iter[1] += 1;
-    }
+    iter[0] = gen0;
+    iter[1] = 0;
 }
 
 unsigned grid_for(size_t work, unsigned threads)
@@ -333,10 +411,16 @@ unsigned grid_for(size_t work, unsigned threads)
 
 }  // namespace
 
-hipError_t launch_split_trial(const EvoArgs &a, int g, hipStream_t s)
+hipError_t launch_split_trial(const EvoArgs &a, int g, int pack, void *B, void *Bl, int Kb, hipStream_t s)
 {
-    const size_t items = static_cast<size_t>(a.P) * (a.stride / 2);
-    hipLaunchKernelGGL(split_trial_kernel, dim3(grid_for(items, kThreads)), dim3(kThreads), 0, s, a, g);
+    const size_t tiles = static_cast<size_t>((a.P + kTileMembers - 1) / kTileMembers) * (a.stride / kChunk);
+    const dim3 grid(static_cast<unsigned>(tiles) + 1), threads(kThreads);
+    if (pack == DEAC_PRECISION_FP32)
+        hipLaunchKernelGGL(split_trial_kernel<DEAC_PRECISION_FP32>, grid, threads, 0, s, a, g, B, Bl, Kb);
+    else if (pack == DEAC_PRECISION_BF16X3)
+        hipLaunchKernelGGL(split_trial_kernel<DEAC_PRECISION_BF16X3>, grid, threads, 0, s, a, g, B, Bl, Kb);
+    else
+        hipLaunchKernelGGL(split_trial_kernel<DEAC_PRECISION_FP64>, grid, threads, 0, s, a, g, B, Bl, Kb);
     return hipGetLastError();
 }
 
@@ -372,15 +456,6 @@ hipError_t launch_split_pack_bf16x3(const EvoArgs &a, int init, void *Bh, void *
     return hipGetLastError();
 }
 
-hipError_t launch_split_model(const EvoArgs &a, const float *part, int slices, int Npad, size_t mn, const int *ex,
-                              hipStream_t s)
-{
-    const size_t total = static_cast<size_t>(a.P) * a.T;
-    hipLaunchKernelGGL(split_model_kernel, dim3(grid_for(total, kThreads)), dim3(kThreads), 0, s, a, part, slices,
-                       Npad, mn, ex);
-    return hipGetLastError();
-}
-
 hipError_t launch_split_fold(const EvoArgs &a, hipStream_t s)
 {
     hipLaunchKernelGGL(split_fold_kernel, dim3(a.P * a.TB), dim3(kWave), 0, s, a);
@@ -396,14 +471,24 @@ hipError_t launch_split_moments(const EvoArgs &a, int init, hipStream_t s)
 
 hipError_t launch_split_select(const EvoArgs &a, int g, int init, hipStream_t s)
 {
-    const size_t lds = static_cast<size_t>(a.T <= kSelectLds ? a.T : kWave) * sizeof(double);
-    hipLaunchKernelGGL(split_select_kernel, dim3(a.P), dim3(kWave), lds, s, a, g, init);
+    const size_t lds = static_cast<size_t>(std::min(a.T, kSelectLds)) * sizeof(double);
+    hipLaunchKernelGGL(split_select_kernel<false>, dim3(a.P), dim3(kWave), lds, s, a, g, init, nullptr, 0, 0, 0, nullptr);
     return hipGetLastError();
 }
 
-hipError_t launch_split_iter(long *iter, long gen0, int set, hipStream_t s)
+hipError_t launch_split_model_select(const EvoArgs &a, int g, int init, const float *part, int slices, int Npad, int Mpad,
+                                     const int *ex, hipStream_t s)
 {
-    hipLaunchKernelGGL(split_iter_kernel, dim3(1), dim3(1), 0, s, iter, gen0, set);
+    const size_t window = static_cast<size_t>(std::min(a.T, kSelectLds));
+    const size_t lds = (window + 1) / 2 * 2 * sizeof(double) + (window + 3) / 4 * sizeof(float4);
+    hipLaunchKernelGGL(split_select_kernel<true>, dim3(a.P), dim3(1024), lds, s, a, g, init, part, slices, Npad, Mpad,
+                       ex);
+    return hipGetLastError();
+}
+
+hipError_t launch_split_iter(long *iter, long gen0, hipStream_t s)
+{
+    hipLaunchKernelGGL(split_iter_kernel, dim3(1), dim3(1), 0, s, iter, gen0);
     return hipGetLastError();
 }
 
