@@ -34,6 +34,7 @@ struct deac_handle {
     hipStream_t stream = nullptr;       // evolution
     hipStream_t draw_stream = nullptr;  // RNG walk, batches ahead of the evolution
     int MG = 0, TB = 0, stride = 0, rstride = 0, nwg = 0, maxwg = 0, chunk = 0, batch = 0;
+    bool fixed_nwg = false;             // the number of workgroups is the user's
     std::vector<void *> allocations;
     double *kmat = nullptr, *ktile = nullptr, *nterm = nullptr, *fterm = nullptr, *tterm = nullptr, *obs = nullptr, *sig = nullptr;
     double *nfm_dt = nullptr;           // -1st-moment weights over tau (bdsf), or null
@@ -295,6 +296,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     }
     size_t nwg = std::max(tasks, trial_pairs / 1024);
     if (m.normalize && m.renormalize) nwg = std::max<size_t>(nwg, P);  // a workgroup renormalizes a member at a time
+    h->fixed_nwg = std::getenv("DEAC_EVOLVE_WORKGROUPS") != nullptr;
     if (const char *user = std::getenv("DEAC_EVOLVE_WORKGROUPS")) nwg = std::max(std::atoi(user), 1);
     h->nwg = static_cast<int>(std::clamp<size_t>(nwg, 1, std::max(maxwg - 8, 1)));
 
@@ -308,13 +310,13 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     A(h->ktile, deac::ktile_doubles(h->TB, h->stride));
     A(h->obs, T);
     A(h->sig, T);
-    A(h->pop0, pop_n);
-    A(h->pop1, pop_n);
+    A(h->pop0, 2 * pop_n);
+    if (st == DEAC_OK) h->pop1 = h->pop0 + pop_n;
     A(h->cur, P);
     A(h->fitness, P);
     A(h->cr_old, static_cast<size_t>(P) * m.nsign);
     A(h->f_old, static_cast<size_t>(P) * m.nsign);
-    A(h->emod, static_cast<size_t>(P) * T);
+    A(h->emod, 2 * static_cast<size_t>(P) * T);
     A(h->mom, static_cast<size_t>(P) * 4);
     A(h->sync, 16);
     A(h->iter, 8);
@@ -496,6 +498,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     ea.fold_ks = m.bdsf;
     ea.rstride = h->rstride;
     ea.local = deac::evolve_local(ea.P, ea.T, nsign, m.use_nfm);
+    ea.fed = !h->fixed_nwg && deac::evolve_fed(ea, std::max(h->maxwg - 8, 1));
     ea.ktile = h->ktile;
     ea.nterm = h->nterm;
     ea.fterm = h->fterm;
@@ -610,6 +613,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         walk_args(0, nullptr);
         DEAC_HIP(deac::launch_evolve(ea, wa, deac::MaskArgs{}, s));
         ea.init_mode = 0;
+        if (ea.fed) ea.nwg = ea.MG * ea.TB + 1;  // the last one keeps the statistics
         DEAC_HIP(hipEventRecord(h->ev0, s));
         mask_args(0, nullptr);
         walk_args(1, nullptr);

@@ -629,6 +629,263 @@ __device__ __forceinline__ void chain_task(const EvoArgs &a, const GenomeRows &r
     if (i < a.P && t < a.T) a.emod[static_cast<size_t>(i) * a.T + t] = acc;
 }
 
+// ---- chains whose genome rows the workgroup forms as they run
+
+__device__ __forceinline__ unsigned uniform(unsigned x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// Three wavefronts form the trial vectors of the group's members, every third
+// chunk each, into a ring of chunks in LDS; the chain's wavefront follows.
+// ready[slot] is the chunk in a slot of the ring, counted since the launch
+// began, plus one; used the chunks that the chain is done with.
+constexpr int kFedSlots = 8;
+constexpr int kFeeders = kEvoWaves - 1;
+constexpr int kFedAhead = 2;  // chunks whose loads a feeder has in flight
+constexpr int kFedChunk = kChainRows * kSRow;
+static_assert(kFedSlots * kFedChunk <= kEvoWaves * kChainLds, "the ring fits in front of the members' state");
+struct Feed {
+    double *ring;
+    unsigned *ready, *used;
+    __device__ __forceinline__ double *slot(unsigned n) const { return ring + n % kFedSlots * kFedChunk; }
+    static __device__ __forceinline__ unsigned read(const unsigned *p)
+    {
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    static __device__ __forceinline__ void write(unsigned *p, unsigned v)
+    {
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+};
+
+// Until *p is at least need; there: what it held a while ago.  One piece of
+// assembly, so that the chain around it stays one block of code (as a loop in
+// the source it cost register copies and a wait for all loads in flight).  The
+// feeders never wait for anything but chunks used, so that the wait ends.
+__device__ __forceinline__ void await(const unsigned *p, unsigned there, unsigned need)
+{
+    typedef const __attribute__((address_space(3))) unsigned *Lds;
+    const unsigned at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((Lds)p));
+    unsigned v, u;
+    asm volatile("s_cmp_ge_u32 %2, %3\n\t"
+                 "s_cbranch_scc1 2f\n"
+                 "1:\n\t"
+                 "ds_read_b32 %0, %4\n\t"
+                 "s_waitcnt lgkmcnt(0)\n\t"
+                 "v_readfirstlane_b32 %1, %0\n\t"
+                 "s_cmp_ge_u32 %1, %3\n\t"
+                 "s_cbranch_scc0 1b\n"
+                 "2:"
+                 : "=&v"(v), "=&s"(u)
+                 : "s"(there), "s"(need), "v"(at)
+                 : "scc", "memory");
+}
+
+// chain_chunk on the ring: chunk n of the launch; more: another one follows.
+template <int H>
+__device__ __forceinline__ void fed_chunk(double &acc, dvec2 (&kr)[kRing], dvec2 (&sr)[kReadAhead], KUnits &ku,
+                                          const Feed &f, unsigned n, int offset, bool more)
+{
+    const double *here = f.slot(n) + offset, *next = f.slot(n + 1) + offset;
+    const unsigned need = more ? n + 2 : 0;
+    unsigned there = 0;
+#pragma unroll
+    for (int i = 0; i < kChunkUnits; i++) {
+        const dvec2 k = kr[H + i], s = sr[i % kReadAhead];
+        const int j = i + kReadAhead;
+        const double *p = j < kChunkUnits ? here + j * kUnit : next + (j - kChunkUnits) * kUnit;
+        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.x, s.x, acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i == kChunkUnits - 2 * kReadAhead) there = Feed::read(f.ready + (n + 1) % kFedSlots);
+        if (j == kChunkUnits) {  // from here on the reads are of the next chunk
+            await(f.ready + (n + 1) % kFedSlots, uniform(there), need);
+            Feed::write(f.used, n + 1);
+        }
+        sr[i % kReadAhead] = dvec2{p[0], p[4]};
+        __builtin_amdgcn_sched_barrier(0);
+        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(k.y, s.y, acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        kr[H + i] = ku.load(i);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    ku.advance();
+}
+
+// chain_task on the ring, from chunk n0 of the launch on.
+__device__ __forceinline__ void fed_chain(const EvoArgs &a, double *emod, int tb, int mg, const Feed &f, unsigned n0)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int nchunk = a.stride / kChunk, offset = (lane & 3) * kSRow + (lane >> 4);
+    KUnits ku(a.ktile + static_cast<size_t>(tb) * nchunk * kChunkUnits * (2 * kWave));
+    dvec2 kr[kRing], sr[kReadAhead];
+#pragma unroll
+    for (int h = 0; h < kRing; h += kChunkUnits) {
+#pragma unroll
+        for (int i = 0; i < kChunkUnits; i++) {
+            kr[h + i] = ku.load(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ku.advance();
+    }
+    await(f.ready + n0 % kFedSlots, n0, n0 + 1);
+    const double *first = f.slot(n0) + offset;
+#pragma unroll
+    for (int j = 0; j < kReadAhead; j++) sr[j] = dvec2{first[j * kUnit], first[j * kUnit + 4]};
+    double acc = 0.0;
+    for (int c = 0; c + 1 < nchunk; c += 2) {
+        fed_chunk<0>(acc, kr, sr, ku, f, n0 + c, offset, true);
+        fed_chunk<kChunkUnits>(acc, kr, sr, ku, f, n0 + c + 1, offset, c + 2 < nchunk);
+    }
+    if (nchunk & 1) fed_chunk<0>(acc, kr, sr, ku, f, n0 + nchunk - 1, offset, false);
+    const int i = mg * kChainRows + (lane & 3), t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
+    if (i < a.P && t < a.T) emod[static_cast<size_t>(i) * a.T + t] = acc;
+}
+
+typedef unsigned raw_quad __attribute__((ext_vector_type(4)));
+
+// Chunks feeder, feeder + 3, ... of the group's trial vectors (deac.cpp:
+// 1261-1308) into the ring, from chunk n0 of the launch on, and into the spare
+// rows where this workgroup writes them.  ctl: the members' records; raw: the
+// generation's draws.
+//
+// Bound: the operands (36 KB a chunk with the chain's: 407 ns, the chain alone
+// needs 281), and a feeder's instruction issue, so what a sign's or the genome's
+// end needs stands aside (8 members, G = 4096, T = 65: 34.1 us a generation;
+// 35.3 with a step of 390 instructions in place of 190; 39.5 with the barrier's
+// fences replaced by loads and stores past the caches; 38.6 with flat
+// addresses).  Rows are byte offsets from pop0 (both populations are one allocation) in buffer operations:
+// flat ones would have to be waited for at every LDS operation.
+__device__ __forceinline__ void feed_chain(const EvoArgs &a, const Members &s, const MemberCtl (&ctl)[kChainRows],
+                                           const uint64_t *raw, int mg, bool write, int feeder, const Feed &f, unsigned n0)
+{
+    const int lane = threadIdx.x & (kWave - 1), nchunk = a.stride / kChunk;
+    if (feeder >= nchunk) return;
+    const auto pop = __builtin_amdgcn_make_buffer_rsrc(a.pop0, 0, -1, 0x00020000);
+    const auto draws = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t *>(raw), 0, -1, 0x00020000);
+    const unsigned span = static_cast<unsigned>(reinterpret_cast<uintptr_t>(a.pop1) - reinterpret_cast<uintptr_t>(a.pop0));
+    struct Row {
+        unsigned r1, r2, r3, rp, out, u;  // byte offsets
+        double f0, f1;
+        uint64_t lim0, lim1;
+    } row[kChainRows];
+    auto offset_of = [&](unsigned i, bool spare) __attribute__((always_inline)) {
+        const unsigned j = uniform(i);
+        return ((uniform(static_cast<unsigned>(s.cur[j])) != 0) != spare ? span : 0) + j * static_cast<unsigned>(a.stride) * 8;
+    };
+#pragma unroll
+    for (int m = 0; m < kChainRows; m++) {
+        const int i = min(mg * kChainRows + m, a.P - 1);
+        Row &r = row[m];
+        r.r1 = offset_of(ctl[m].mutant[0], false);
+        r.r2 = offset_of(ctl[m].mutant[1], false);
+        r.r3 = offset_of(ctl[m].mutant[2], false);
+        r.rp = offset_of(i, false);
+        r.out = offset_of(i, true);
+        r.u = static_cast<unsigned>(i) * static_cast<unsigned>(a.rstride) * 8;
+        const Controls c(a, s, ctl[m], i);
+        r.f0 = c.f[0];
+        r.f1 = c.f[1];
+        r.lim0 = cross_limit(c.cr[0]);
+        r.lim1 = cross_limit(c.cr[1]);
+    }
+    const unsigned sign_mask = a.allow_neg ? ~0u : 0x7fffffffu;
+    auto value = [&](double fm, uint64_t lim, uint64_t u, double d1, double d2, double d3, double p)
+                     __attribute__((always_inline)) {
+        const uint64_t w = __builtin_bit_cast(uint64_t, fma(fm, d2 - d3, d1));
+        const uint64_t x = static_cast<uint64_t>(static_cast<unsigned>(w >> 32) & sign_mask) << 32 | static_cast<unsigned>(w);
+        return u < lim ? __builtin_bit_cast(double, x) : p;
+    };
+    const int vo = lane * 16, last = ((a.Kc - 1) & ~1) * 8;
+    auto load = [&](int m, int c, Trial::Load &v) __attribute__((always_inline)) {
+        const int so = min(c, nchunk - 1) * (kChunk * 8);
+        auto pair = [&](unsigned r) __attribute__((always_inline)) {
+            return __builtin_bit_cast(dvec2, __builtin_amdgcn_raw_buffer_load_b128(pop, vo, r + so, 0));
+        };
+        v.u = __builtin_bit_cast(uvec2, __builtin_amdgcn_raw_buffer_load_b128(draws, min(so + vo, last), row[m].u, 0));
+        v.x1 = pair(row[m].r1);
+        v.x2 = pair(row[m].r2);
+        v.x3 = pair(row[m].r3);
+        v.xp = pair(row[m].rp);
+    };
+    // the trial's value at the zero frequency, which the negative sign repeats
+    double zero[kChainRows];
+    {
+        double x[kChainRows][4];
+        uint64_t u[kChainRows];
+        auto one = [&](unsigned r) __attribute__((always_inline)) {
+            return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(pop, 0, r, 0));
+        };
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++) {
+            u[m] = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(draws, 0, row[m].u, 0));
+            x[m][0] = one(row[m].r1);
+            x[m][1] = one(row[m].r2);
+            x[m][2] = one(row[m].r3);
+            x[m][3] = one(row[m].rp);
+        }
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++)
+            zero[m] = value(row[m].f0, row[m].lim0, u[m], x[m][0], x[m][1], x[m][2], x[m][3]);
+    }
+    Trial::Load v[kFedAhead][kChainRows];
+#pragma unroll
+    for (int u = 0; u < kFedAhead; u++)
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++) load(m, feeder + u * kFeeders, v[u][m]);
+    auto step = [&](Trial::Load (&x)[kChainRows], int c) __attribute__((always_inline)) {
+        const unsigned n = n0 + c;
+        while (static_cast<int>(n - uniform(Feed::read(f.used))) >= kFedSlots) __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+        const bool neg = c * kChunk >= a.G;
+        dvec2 o[kChainRows];
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++) {
+            const double fm = neg ? row[m].f1 : row[m].f0;
+            const uint64_t lim = neg ? row[m].lim1 : row[m].lim0;
+            o[m].x = value(fm, lim, x[m].u.x, x[m].x1.x, x[m].x2.x, x[m].x3.x, x[m].xp.x);
+            o[m].y = value(fm, lim, x[m].u.y, x[m].x1.y, x[m].x2.y, x[m].x3.y, x[m].xp.y);
+        }
+        if ((c * kChunk <= a.G && (c + 1) * kChunk > a.G) || (c + 1) * kChunk > a.Kc) {
+            // where a sign begins inside the chunk, or the genome ends
+            const int k = Trial::position(c);
+#pragma unroll
+            for (int m = 0; m < kChainRows; m++) {
+                const Row &r = row[m];
+                if (k >= a.G) o[m].x = value(r.f1, r.lim1, x[m].u.x, x[m].x1.x, x[m].x2.x, x[m].x3.x, x[m].xp.x);
+                if (k + 1 >= a.G) o[m].y = value(r.f1, r.lim1, x[m].u.y, x[m].x1.y, x[m].x2.y, x[m].x3.y, x[m].xp.y);
+                if (k == a.G) o[m].x = zero[m];
+                if (k + 1 == a.G) o[m].y = zero[m];
+                if (k >= a.Kc) o[m].x = 0.0;
+                if (k + 1 >= a.Kc) o[m].y = 0.0;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++) load(m, c + kFedAhead * kFeeders, x[m]);
+        __builtin_amdgcn_sched_barrier(0);
+        dvec2 *to = reinterpret_cast<dvec2 *>(f.slot(n)) + lane;
+#pragma unroll
+        for (int m = 0; m < kChainRows; m++) to[m * (kSRow / 2)] = o[m];
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // the rows are in LDS (lgkmcnt 0, the other counters as they are)
+        Feed::write(f.ready + n % kFedSlots, n + 1);
+        if (write) {
+#pragma unroll
+            for (int m = 0; m < kChainRows; m++)
+                if (mg * kChainRows + m < a.P)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(raw_quad, o[m]), pop, vo,
+                                                           row[m].out + c * (kChunk * 8), 0);
+        }
+    };
+    // (two chunks a turn and an odd one behind: an exit between them costs
+    // copies of the loads in flight)
+    static_assert(kFedAhead == 2);
+    int c = feeder;
+    for (; c + kFeeders < nchunk; c += 2 * kFeeders) {
+        step(v[0], c);
+        step(v[1], c + kFeeders);
+    }
+    if (c < nchunk) step(v[0], c);
+}
+
 // Blocks [b0, b1) of a trial vector into the spare row, two blocks' loads
 // ahead of the two being formed.
 // Bound: memory (40 bytes read and 8 written per position): 512 members of
@@ -896,13 +1153,18 @@ __device__ unsigned long long deac_phase_clock[4];
 // (evolve_max_workgroups); a second handle's workgroup still fits beside it.
 // FOLD: the trials' model ISF as rounded-product folds (bdsf; its initial
 // population goes through the chains of the other form, deac.cpp:860).
-template <bool FOLD>
+// FED (EvoArgs::fed): a workgroup per contraction task, and one for the
+// statistics, which forms the trial vectors of its members beside their chains:
+// no trial phase, one barrier per generation.
+enum Form { kChains, kFold, kFed };
+template <Form FORM>
 __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void evolve_kernel(EvoArgs a, WalkArgs next,
                                                                                               MaskArgs masks)
 {
 #ifdef DEAC_PHASE_TIMERS
     unsigned long long phase_t0 = 0;
 #endif
+    constexpr bool FOLD = FORM == kFold, FED = FORM == kFed;
     extern __shared__ __attribute__((aligned(16))) double lds[];
     __shared__ double minimum, scale;
     const int lane = threadIdx.x & (kWave - 1);
@@ -969,6 +1231,28 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         }
     }
     const int *cur = s.cur;
+    __shared__ unsigned fed_ready[kFedSlots], fed_used;
+    const Feed feed = {lds, fed_ready, &fed_used};
+    // FED: this workgroup's task; one workgroup has none.  The members' records
+    // are put into LDS a generation ahead.
+    const int fed_task = ks0 + static_cast<int>(blockIdx.x) / nx;
+    const int fed_tb = a.by_tau ? fed_task / groups : fed_task % a.TB, fed_mg = a.by_tau ? fed_task % groups : fed_task / a.TB;
+    const bool fed_mine = static_cast<int>(blockIdx.x) / nx < nks;
+    __shared__ MemberCtl fed_ctl[2][kChainRows];
+    auto records = [&](int g) {
+        constexpr int kWords = sizeof(MemberCtl) / sizeof(uint64_t);
+        static_assert(kChainRows * kWords <= kWave);
+        const int m = lane / kWords;
+        const MemberCtl *from = a.ctl + static_cast<size_t>(min(g, a.ngen - 1)) * a.P;
+        if (m < kChainRows)
+            reinterpret_cast<uint64_t *>(fed_ctl[g & 1])[lane] =
+                reinterpret_cast<const uint64_t *>(from + min(fed_mg * kChainRows + m, a.P - 1))[lane % kWords];
+    };
+    if constexpr (FED) {
+        if (threadIdx.x < kFedSlots) fed_ready[threadIdx.x] = 0;
+        if (threadIdx.x == 0) fed_used = 0;
+        if (wid == 1) records(0);
+    }
     __syncthreads();
 
     for (int g = 0; g <= a.ngen; g++) {
@@ -1005,7 +1289,9 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             // Trial vectors into each member's spare buffer.
             const MemberCtl *ctlg = a.ctl + static_cast<size_t>(g) * a.P;
             const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.rstride;
-            if (!a.renorm) {
+            if constexpr (FED) {
+                // beside the chains, below
+            } else if (!a.renorm) {
                 for (int i = share_i, b0 = share_b, left = nshare; left > 0; i++, b0 = 0) {
                     const int n = min(nblk - b0, left);
                     trial_blocks(Trial(a, s, cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i), b0, b0 + n);
@@ -1033,13 +1319,32 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                     __syncthreads();
                 }
             }
-            if (!grid_barrier(a.bar, target, nwg, a)) return;
-            DEAC_PHASE(1);
+            if constexpr (!FED) {
+                if (!grid_barrier(a.bar, target, nwg, a)) return;
+                DEAC_PHASE(1);
+            }
         }
 
+        // FED: a workgroup may still select from a generation's model ISF while
+        // the next one's chains end.
+        double *const emod = FED && (g & 1) ? a.emod + static_cast<size_t>(a.P) * a.T : a.emod;
+        if constexpr (FED) {
+            const unsigned n0 = static_cast<unsigned>(g) * nblk;
+            if (fed_mine) {
+                if (wid == 0) {
+                    fed_chain(a, emod, fed_tb, fed_mg, feed, n0);
+                } else {
+                    feed_chain(a, s, fed_ctl[g & 1], a.raw + static_cast<size_t>(g) * a.P * a.rstride, fed_mg, fed_tb == 0, wid - 1,
+                               feed, n0);
+                    if (wid == 1) records(g + 1);
+                }
+            } else if (wid == 0 && a.track_stats) {
+                statistics(a, s.fitness, g, minimum, lds);
+            }
+        }
         // Model ISF chains and moment rows, one wave per task: of the trials,
         // or of the current genomes for the initial fitness.
-        for (int n = xwave; n < nks + nmoms; n += xwg * kEvoWaves) {
+        for (int n = FED ? nks + nmoms : xwave; n < nks + nmoms; n += xwg * kEvoWaves) {
             double *buf = lds + wid * kChainLds;
             if (n < nks) {
                 const int task = ks0 + n;
@@ -1068,7 +1373,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 if (lane == 0) a.mom[i * 4 + (third ? 2 : 1)] = m;
             }
         }
-        if (gwave == total_waves - 1 && a.track_stats && !init)
+        if (!FED && gwave == total_waves - 1 && a.track_stats && !init)
             statistics(a, s.fitness, g, minimum, lds + wid * kChainLds);
         if (!grid_barrier(a.bar, target, nwg, a)) return;
         DEAC_PHASE(2);
@@ -1078,7 +1383,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             const int total = a.P * a.T;
             for (int idx = threadIdx.x; idx < total; idx += kEvoThreads) {
                 const int i = idx / a.T, t = idx % a.T;
-                const double e = a.emod[idx];
+                const double e = emod[idx];
                 resid[i * Tp + t] = (a.obs[t] - e) / a.sig[t];
                 if (a.use_nfm) moment[i * Tp + t] = e * a.nfm_dt[t];
             }
@@ -1086,10 +1391,11 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             for (int i = threadIdx.x; i < a.P; i += kEvoThreads) {
                 const Selection sel(a, s, g, i, init);
                 const double chi = chi_sum(resid + i * Tp, a.T, a.T & 1, 0.0);
-                sel.take(chi, a.use_nfm ? product_sum(a, moment + i * Tp, i, 0, a.T, 0.0) : 0.0);
+                const double nfm = a.use_nfm ? product_sum(a, moment + i * Tp, i, 0, a.T, 0.0) : 0.0;
+                sel.take(chi, nfm);
             }
             __syncthreads();
-        } else {
+        } else if constexpr (!FED) {
             // one wavefront per member, residuals in windows
             const int window = a.use_nfm ? kResidWave / 2 : kResidWave;
             double *d = lds + wid * kResidWave, *p = d + window;
@@ -1182,9 +1488,10 @@ hipError_t launch_mask(const MaskArgs &a, const WalkArgs &next, hipStream_t s)
 hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s)
 {
     if (next.ngen > 0 && walk_lds_bytes(next) > kEvoLds) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(a.fold_ks && !a.init_mode ? evolve_kernel<true> : evolve_kernel<false>,
-                       dim3(a.nwg + (next.ngen > 0 ? 1 : 0) + (masks.ngen > 0 ? masks.nwg : 0)), dim3(kEvoThreads), kEvoLds, s,
-                       a, next, masks);
+    const bool fed = a.fed && !a.init_mode;
+    hipLaunchKernelGGL(fed ? evolve_kernel<kFed> : a.fold_ks && !a.init_mode ? evolve_kernel<kFold> : evolve_kernel<kChains>,
+                       dim3(a.nwg + (next.ngen > 0 ? 1 : 0) + (masks.ngen > 0 ? masks.nwg : 0)),
+                       dim3(kEvoThreads), kEvoLds, s, a, next, masks);
     return hipGetLastError();
 }
 
@@ -1205,8 +1512,9 @@ hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s)
 int evolve_max_workgroups(int device)
 {
     int per_cu = 1, cus = 0;
-    for (const void *k : {reinterpret_cast<const void *>(evolve_kernel<false>),
-                          reinterpret_cast<const void *>(evolve_kernel<true>)}) {
+    for (const void *k : {reinterpret_cast<const void *>(evolve_kernel<kChains>),
+                          reinterpret_cast<const void *>(evolve_kernel<kFold>),
+                          reinterpret_cast<const void *>(evolve_kernel<kFed>)}) {
         int n = 0;
         if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kEvoLds) != hipSuccess) return 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kEvoThreads, kEvoLds) != hipSuccess) return 0;

@@ -74,6 +74,7 @@ struct EvoArgs {
     int stride;                  // row stride of K and of the populations: Kc padded to kChunk
     int rstride;                 // row stride of the draws: Kc padded to whole 16-byte pairs
     int local;                   // every workgroup repeats the selection (evolve_local)
+    int fed;                     // trial vectors formed beside the chains (evolve_fed)
     int MG, TB;                  // member groups of kChainRows, tau blocks of kChainTau
     int by_tau;                  // contraction tasks in order of tau blocks, else of member groups (evolve_by_tau)
     int use_first, use_third, renorm, allow_neg, init_mode, track_stats;
@@ -85,11 +86,11 @@ struct EvoArgs {
     const double *ktile;         // K in the chains' and folds' operand order (launch_ktile)
     const double *nterm, *fterm, *tterm;   // [Kc] or null
     const double *obs, *sig;     // [T]
-    double *pop0, *pop1;         // [MG*4][stride] each, member-major rows, zero padded
+    double *pop0, *pop1;         // [MG*4][stride] each, one allocation, member-major rows, zero padded
     int *cur;                    // [P] buffer holding each member's current genome
     double *fitness;             // [P]
     double *cr_old, *f_old;      // [P][nsign]
-    double *emod;                // [P][T]
+    double *emod;                // [2][P][T] (the second where fed)
     double *mom;                 // [P][4]: normalization, first, third moment
     const MemberCtl *ctl;        // [ngen][P]
     const uint64_t *raw;         // [ngen][P][rstride]
@@ -140,6 +141,18 @@ inline int evolve_local(int P, int T, int nsign, int use_nfm)
 {
     const long resid = static_cast<long>(P) * (T | 1);
     return resid <= kLocalResid && resid * (1 + use_nfm) + static_cast<long>(P) * (2 + 2 * nsign) <= kResidLds;
+}
+// Whether a workgroup per contraction task forms the trial vectors of its
+// members itself, beside their chains: where the tasks have a CU each, the
+// selection is every workgroup's own, nothing but the chains reads whole trials,
+// and 32-bit offsets reach the populations.  (us a generation without and with:
+// 8 members G = 512, T = 33 13.6 and 12.7; G = 4096, T = 65 and 8 members 35.2
+// and 34.1, 16 39.8 and 36.7, 32 48.8 and 42.0, 62 66.1 and 49.8; 31 members G =
+// 2048, T = 129 38.2 and 33.4; 200 members G = 6000, T = 17 102 and 80.)
+inline int evolve_fed(const EvoArgs &a, int maxwg)
+{
+    return a.local && !a.renorm && !a.use_first && !a.use_third && !a.use_nfm && !a.fold_ks && a.MG * a.TB + 1 <= maxwg &&
+           static_cast<size_t>(a.MG) * kChainRows * a.stride * 16 < (size_t(1) << 31);
 }
 // Whether an XCD's range of contraction tasks reads fewer rows in order of tau
 // blocks (16 K rows each) than in order of member groups (`rows` genome rows).
