@@ -125,7 +125,6 @@ struct deac_batch {
     double *best_rows = nullptr;               // [genomes of all instances]: best members, gathered for the readback
     long *best_off = nullptr;                  // per instance: offset in best_rows, of its population, P, Kc, Lpad
     std::vector<size_t> best_at;               // offset in best_rows, host side
-    std::vector<double> best_host;             // the readback, kept (a new 16.8 MB vector's page faults took 3.6 ms)
     double *stats_ws = nullptr;                // statistics histories, kept between runs and grown on demand
     size_t stats_cap = 0;
     double *scratch = nullptr;                 // this device's statistics scratch (deac_batch_run_noalloc)
@@ -1060,9 +1059,7 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
     // The best members' rows are gathered on the device: one copy each for the
     // fitnesses, the random states, the rows and the statistics.
     const size_t last = n - 1;
-    std::vector<double> &rows = h->best_host;
-    rows.resize(h->best_at[last] + h->models[h->model_of[last]]->m.Kc);
-    std::vector<double> stats_host(stats_n);
+    std::vector<double> rows(h->best_at[last] + h->models[h->model_of[last]]->m.Kc), stats_host(stats_n);
     BATCH_HIP(deac::launch_gather_best(h->best_off, n, h->fitness, deac::kBatchMaxP, h->pop, h->best_rows, s));
     BATCH_HIP(hipStreamSynchronize(s));
     BATCH_HIP(hipMemcpy(rows.data(), h->best_rows, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
