@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <cmath>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -269,10 +270,15 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     h->rstride = round_up(Kc, 2);
     h->wide = deac::walk_is_wide(P, m.tau_cr, m.tau_f);
     h->chunk = round_up((Kc + 63) / 64, 2);
-    // RNG batch: generations whose mask draws are buffered at once (<= 256 MiB
-    // per buffer set).
+    // RNG batch: generations whose mask draws are buffered at once: 64 MiB per
+    // buffer set, so that the evolution finds both sets in the 256 MB cache in
+    // front of HBM (G = 4096, T = 65: 8 members 67.8 -> 65.7 ms for 2000
+    // generations, 32 members 25.4 -> 24.0 for 600, against 256 MiB), but at
+    // least 16 generations where 256 MiB hold them (a batch's launches and first
+    // draws; long genomes of large populations would have 2 to 4).
     const size_t per_gen = static_cast<size_t>(P) * h->rstride * sizeof(uint64_t);
-    h->batch = static_cast<int>(std::clamp<size_t>((size_t(256) << 20) / per_gen, 1, 1024));
+    const size_t most = (size_t(256) << 20) / per_gen;
+    h->batch = static_cast<int>(std::clamp<size_t>(std::max((size_t(64) << 20) / per_gen, std::min<size_t>(16, most)), 1, 1024));
 
     const int maxwg = deac::evolve_max_workgroups(device);
     if (maxwg <= 0) return fail(DEAC_ERR_DEVICE);
@@ -545,18 +551,21 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     // it finds are those that stopped batch b, and it stops at its first
     // generation (its status and its statistics entry, past the stop, are
     // never read).  Batches start at 8 generations, so that the first masks,
-    // which nothing hides, are few, and grow by a quarter up to the buffer
-    // size: the walk beside a batch then has one and a half times its
-    // generations to walk, which a member's walk (0.7 us) still hides behind
-    // the generations of the smallest runs (8 us, 8 members).
+    // which nothing hides, are few, and grow up to the buffer size by what
+    // keeps the walk beside a batch, of the batch after the next, no longer
+    // than the batch: by 1.1 for 8 members at G = 16 (walk 5.6 us a generation,
+    // evolution 7; 200 generations 1.79 ms, 2.06 by 1.25), by at most a quarter.
+    const double walk_us = h->wide ? 12.0 + 0.1 * static_cast<double>(P) : 0.7 * static_cast<double>(P);
+    const double generation_us = 6.0 + 0.35 * (h->stride / deac::kChunk);  // at least
+    const double grow = split ? 1.25 : std::clamp(std::sqrt(generation_us / walk_us), 1.1, 1.25);
     const size_t total = N - 1;
     std::vector<std::pair<size_t, int>> plan;  // first generation, generations
     for (size_t g = 0, len = std::min(8, h->batch); g < total;) {
         const int nb = static_cast<int>(std::min(len, total - g));
         plan.emplace_back(g, nb);
         g += static_cast<size_t>(nb);
-        len = std::min(len + len / 4, static_cast<size_t>(h->batch));
-        if (len < 2) len = std::min(2, h->batch);
+        len = std::min(std::max(static_cast<size_t>(static_cast<double>(len) * grow), len + 1),
+                       static_cast<size_t>(h->batch));
     }
     hipStream_t d = h->draw_stream;  // split loop: the draws of the next batch
     auto walk_args = [&](size_t b, const int *halt) {
@@ -590,9 +599,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         mask_args(b + 1, ea.status);
         walk_args(b + 2, ea.status);
         std::fill_n(ea.host_status, 4, 0);  // read for batch b-2 by now
-        DEAC_HIP(hipEventRecord(e[4], s));
-        DEAC_HIP(deac::launch_evolve(ea, wa, ma, s));
-        DEAC_HIP(hipEventRecord(e[5], s));
+        DEAC_HIP(deac::launch_evolve(ea, wa, ma, s, e[4], e[5]));
         return DEAC_OK;
     };
     deac_run_profile prof{};
@@ -611,7 +618,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
         ea.nwg = h->nwg;
         std::fill_n(ea.host_status, 4, 0);
         walk_args(0, nullptr);
-        DEAC_HIP(deac::launch_evolve(ea, wa, deac::MaskArgs{}, s));
+        DEAC_HIP(deac::launch_evolve(ea, wa, deac::MaskArgs{}, s, nullptr, nullptr));
         ea.init_mode = 0;
         if (ea.fed) ea.nwg = ea.MG * ea.TB + 1;  // the last one keeps the statistics
         DEAC_HIP(hipEventRecord(h->ev0, s));

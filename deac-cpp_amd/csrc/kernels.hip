@@ -17,6 +17,7 @@
 //     order, greedy selection.  Grid barriers separate the phases.
 // The file is compiled with -ffp-contract=off: every fused multiply-add is
 // written as fma().
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1485,13 +1486,14 @@ hipError_t launch_mask(const MaskArgs &a, const WalkArgs &next, hipStream_t s)
 // are dispatched first, so on an otherwise idle device every one of them is
 // resident; if one is not, the bounded grid barrier reports a timeout instead
 // of hanging.
-hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s)
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s, hipEvent_t start,
+                         hipEvent_t stop)
 {
     if (next.ngen > 0 && walk_lds_bytes(next) > kEvoLds) return hipErrorInvalidValue;
     const bool fed = a.fed && !a.init_mode;
-    hipLaunchKernelGGL(fed ? evolve_kernel<kFed> : a.fold_ks && !a.init_mode ? evolve_kernel<kFold> : evolve_kernel<kChains>,
-                       dim3(a.nwg + (next.ngen > 0 ? 1 : 0) + (masks.ngen > 0 ? masks.nwg : 0)),
-                       dim3(kEvoThreads), kEvoLds, s, a, next, masks);
+    hipExtLaunchKernelGGL(fed ? evolve_kernel<kFed> : a.fold_ks && !a.init_mode ? evolve_kernel<kFold> : evolve_kernel<kChains>,
+                          dim3(a.nwg + (next.ngen > 0 ? 1 : 0) + (masks.ngen > 0 ? masks.nwg : 0)), dim3(kEvoThreads),
+                          kEvoLds, s, start, stop, 0, a, next, masks);
     return hipGetLastError();
 }
 

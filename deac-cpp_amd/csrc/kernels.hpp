@@ -171,8 +171,11 @@ inline size_t ktile_doubles(int TB, int stride)
 }
 hipError_t launch_ktile(const double *rows, double *ktile, int T, int Kc, int TB, int stride, hipStream_t s);
 // The evolution of a batch and beside it the mask draws of the next one and
-// the walk of the one after, where they have generations.
-hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s);
+// the walk of the one after, where they have generations.  start, stop: events
+// that the dispatch itself records, or null (recorded in the stream on its two
+// sides they cost the gap between two launches 6 us).
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &next, const MaskArgs &masks, hipStream_t s, hipEvent_t start,
+                         hipEvent_t stop);
 hipError_t launch_zero_u32(unsigned *p, size_t n, hipStream_t s);
 // Workgroups of the evolution kernel that are co-resident on the device: one
 // per CU.
