@@ -46,7 +46,7 @@ struct deac_handle {
     // counter ([0]) and status ([4..6]) per set, and the batch's mask draws.
     // Three sets of the walk's records, four of its generation starts (see
     // the generation loop).
-    unsigned *sync = nullptr;           // [2][8]
+    unsigned *sync = nullptr;           // [2][kSyncWords]
     long *iter = nullptr;               // [2][4]: split loop generation counters, per buffer set
     int *host_status = nullptr;         // [3][4], pinned: status of the sets, then of the initial fitness
     deac::MemberCtl *ctl[3] = {};
@@ -324,7 +324,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     A(h->f_old, static_cast<size_t>(P) * m.nsign);
     A(h->emod, 2 * static_cast<size_t>(P) * T);
     A(h->mom, static_cast<size_t>(P) * 4);
-    A(h->sync, 16);
+    A(h->sync, 2 * deac::kSyncWords);
     A(h->iter, 8);
     for (deac::MemberCtl *&p : h->ctl) A(p, static_cast<size_t>(h->batch) * P);
     for (uint64_t *&p : h->raw) A(p, static_cast<size_t>(h->batch) * P * h->rstride);
@@ -587,13 +587,14 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     auto evolve = [&](size_t b) -> deac_status {
         const int k = static_cast<int>(b & 1);
         hipEvent_t *e = h->kev[k];
-        unsigned *sy = h->sync + 8 * k;
+        unsigned *sy = h->sync + deac::kSyncWords * k;
         ea.ctl = h->ctl[b % 3];
         ea.raw = h->raw[k];
         ea.bar = sy;
         ea.status = reinterpret_cast<int *>(sy + 4);
         ea.host_status = h->host_status + 4 * k;
-        ea.clear = h->sync + 8 * (k ^ 1);
+        ea.clear = h->sync + deac::kSyncWords * (k ^ 1);
+        ea.xbar = sy + deac::kXcdSync;
         ea.gen0 = static_cast<long>(plan[b].first);
         ea.ngen = plan[b].second;
         mask_args(b + 1, ea.status);
@@ -608,12 +609,13 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     auto pipeline = [&]() -> deac_status {
         // Initial fitness (deac.cpp:857-976), on buffer set 1, with the first
         // walk beside it; then the first masks with the second walk.
-        DEAC_HIP(deac::launch_zero_u32(h->sync, 16, s));
+        DEAC_HIP(deac::launch_zero_u32(h->sync, 2 * deac::kSyncWords, s));
         ea.init_mode = 1;
         ea.gen0 = 0;
         ea.ngen = 0;
-        ea.bar = h->sync + 8;
-        ea.status = reinterpret_cast<int *>(h->sync + 12);
+        ea.bar = h->sync + deac::kSyncWords;
+        ea.xbar = ea.bar + deac::kXcdSync;
+        ea.status = reinterpret_cast<int *>(ea.bar + 4);
         ea.host_status = h->host_status + 8;
         ea.nwg = h->nwg;
         std::fill_n(ea.host_status, 4, 0);

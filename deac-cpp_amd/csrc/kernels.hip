@@ -39,35 +39,86 @@ constexpr int kEvoWaves = kEvoThreads / kWave;
 // caller leaves the kernel, so a broken launch cannot hang the device.
 constexpr unsigned kBarrierSpins = 1u << 24;
 
-__device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned &target, int nwg, const EvoArgs &a)
-{
+// Where many workgroups take part (kXcdBarrierWgs), those of an XCD, which share
+// its L2, arrive together: the last of them writes the L2 back for all.  The
+// write-backs of an XCD's workgroups queue: with three barriers a generation,
+// 248 workgroups, T = 257, G = 16384, 64 members took 168 us a generation with
+// one each and 141 this way, 512 members G = 4096 147 and 112; with 52 workgroups
+// (two barriers) 43.3 and 43.1; below 32 it makes no difference.
+constexpr int kXcdBarrierWgs = 32;
+struct GridBarrier {
+    unsigned *bar;          // arrivals
+    unsigned *xcd = nullptr;  // arrivals of this XCD's workgroups, or null: one by one
+    unsigned mine = 0;      // of them, per barrier
+    unsigned arrivals;      // at bar, per barrier
+    unsigned epoch = 0, target = 0;
+    const EvoArgs &a;
+
+    __device__ __forceinline__ GridBarrier(const EvoArgs &ea)
+        : bar(ea.bar), arrivals(ea.nwg), a(ea)
+    {
+    }
+
     // Each wave drains its own memory operations; then one thread per
     // workgroup publishes the workgroup's stores at agent scope (L2 write-back,
     // visible to the other XCDs), arrives, waits, and invalidates this CU's
     // caches for what the other workgroups wrote.
-    __shared__ int timed_out;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    target += nwg;
-    if (threadIdx.x == 0) {
-        timed_out = 0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned spins = 0;
-        while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            __builtin_amdgcn_s_sleep(1);
-            if (++spins == kBarrierSpins) {
-                timed_out = 1;
-                __hip_atomic_store(a.status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(a.host_status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                break;
+    __device__ __forceinline__ bool wait()
+    {
+        __shared__ int timed_out;
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        target += arrivals;
+        epoch++;
+        if (threadIdx.x == 0) {
+            timed_out = 0;
+            bool last = true;
+            if (xcd)
+                last = __hip_atomic_fetch_add(xcd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == mine * epoch;
+            if (last) {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+            unsigned spins = 0;
+            while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+                __builtin_amdgcn_s_sleep(1);
+                if (++spins == kBarrierSpins) {
+                    timed_out = 1;
+                    __hip_atomic_store(a.status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(a.host_status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    break;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        __syncthreads();
+        return timed_out == 0;
     }
-    __syncthreads();
-    return timed_out == 0;
-}
+
+    // Counts the workgroups per XCD: by the number the hardware gives, which
+    // says whose L2 a workgroup's stores are in.
+    __device__ __forceinline__ bool by_xcd()
+    {
+        __shared__ unsigned counted[2];
+        constexpr int kXccId = 20 | 3 << 11;  // HW_REG_XCC_ID, 4 bits
+        unsigned *here = a.xbar + (__builtin_amdgcn_s_getreg(kXccId) % kXcds) * kXcdWords;
+        if (threadIdx.x == 0) __hip_atomic_fetch_add(here + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!wait()) return false;
+        if (threadIdx.x == 0) {
+            unsigned n = 0;
+            for (int x = 0; x < kXcds; x++)
+                n += __hip_atomic_load(a.xbar + x * kXcdWords + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+            counted[0] = __hip_atomic_load(here + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            counted[1] = n;
+        }
+        __syncthreads();
+        xcd = here;
+        mine = counted[0];
+        arrivals = counted[1];
+        epoch = 0;
+        return true;
+    }
+};
 
 // The walk's stream is wave-uniform: its step as scalar (SALU) operations,
 // the rotate as two 64-bit shifts (the funnel-shift form of xnext would put
@@ -1148,9 +1199,8 @@ __device__ unsigned long long deac_phase_clock[4];
 // Per generation: trial vectors, barrier, chains and moment rows, barrier,
 // selection.  Where the population's residuals fit in LDS (a.local) every
 // workgroup repeats the whole selection and keeps the members' state itself,
-// which saves the third barrier: a grid barrier costs from 1 us (10
-// workgroups) to 8 us (255, the cache fences of an XCD's workgroups queue),
-// a repeated selection of 8 members 1.3 us.  One workgroup per CU is launched
+// which saves the third barrier: a grid barrier costs 1 us, a repeated selection
+// of 8 members 1.3 us.  One workgroup per CU is launched
 // (evolve_max_workgroups); a second handle's workgroup still fits beside it.
 // FOLD: the trials' model ISF as rounded-product folds (bdsf; its initial
 // population goes through the chains of the other form, deac.cpp:860).
@@ -1183,12 +1233,14 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             walk(next, reinterpret_cast<uint64_t *>(lds));
         return;
     }
-    if (blockIdx.x == 0 && a.clear && threadIdx.x < 8) a.clear[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && a.clear)
+        for (int i = threadIdx.x; i < kSyncWords; i += kEvoThreads) a.clear[i] = 0;
     const int total_waves = nwg * kEvoWaves;
     // Waves are numbered wave-slot-major so that consecutive tasks land on
     // different workgroups (and CUs).
     const int gwave = wid * nwg + blockIdx.x;
-    unsigned target = 0;
+    GridBarrier barrier(a);
+    if (a.xbar && nwg >= kXcdBarrierWgs && !barrier.by_xcd()) return;
     // The contraction's tasks and the moment folds of this workgroup's XCD
     // (workgroups go to the XCDs in turn), in equal ranges: neighbouring tasks
     // share a tau block's K or a member group's rows in its L2.
@@ -1321,7 +1373,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 }
             }
             if constexpr (!FED) {
-                if (!grid_barrier(a.bar, target, nwg, a)) return;
+                if (!barrier.wait()) return;
                 DEAC_PHASE(1);
             }
         }
@@ -1376,7 +1428,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         }
         if (!FED && gwave == total_waves - 1 && a.track_stats && !init)
             statistics(a, s.fitness, g, minimum, lds + wid * kChainLds);
-        if (!grid_barrier(a.bar, target, nwg, a)) return;
+        if (!barrier.wait()) return;
         DEAC_PHASE(2);
 
         // Fitness and greedy selection.
@@ -1419,7 +1471,7 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                 }
                 if (lane == 0) sel.take(chi, nfm);
             }
-            if (!grid_barrier(a.bar, target, nwg, a)) return;
+            if (!barrier.wait()) return;
         }
         DEAC_PHASE(3);
         if (init) break;

@@ -29,6 +29,13 @@ static_assert(kEvoThreads / 64 * kResidWave <= kResidLds, "the waves' windows fi
 // residuals, 16 per thread.
 constexpr int kLocalResid = 4096;
 
+constexpr int kXcds = 8;
+// Words of a launch's synchronization: barrier counter [0], status [4..6], and
+// from kXcdSync on a line of kXcdWords per XCD.
+constexpr int kXcdSync = 32;
+constexpr int kXcdWords = 32;
+constexpr int kSyncWords = kXcdSync + kXcds * kXcdWords;
+
 // Random choices of one member in one generation, produced by walk_kernel.
 struct MemberCtl {
     uint64_t mask_state[4];  // xoshiro256+ state mask_steps draws before the member's first crossover-mask draw
@@ -97,9 +104,10 @@ struct EvoArgs {
     double *stats;               // [3][stats_len]: mean, minimum, squared mean
     size_t stats_len;
     unsigned *bar;               // grid barrier counter, zero at launch
+    unsigned *xbar;              // [kXcds][kXcdWords] the same per XCD, or null (split loop)
     int *status;                 // [0] stopped, [1] generation index within the batch, [2] barrier timeout
     int *host_status;            // the same in pinned host memory, or null (split loop)
-    unsigned *clear;             // barrier counter and status (8 words) of the next launch, or null
+    unsigned *clear;             // the next launch's words (kSyncWords), or null
     long gen0;                   // generation index of the batch's first generation
     int ngen;
     int nwg;                     // workgroups that evolve
@@ -156,7 +164,6 @@ inline int evolve_fed(const EvoArgs &a, int maxwg)
 }
 // Whether an XCD's range of contraction tasks reads fewer rows in order of tau
 // blocks (16 K rows each) than in order of member groups (`rows` genome rows).
-constexpr int kXcds = 8;
 inline int evolve_by_tau(int groups, int rows, int TB)
 {
     const long n = (static_cast<long>(groups) * TB + kXcds - 1) / kXcds;
