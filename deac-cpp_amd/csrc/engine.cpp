@@ -284,9 +284,10 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     if (maxwg <= 0) return fail(DEAC_ERR_DEVICE);
     h->maxwg = maxwg;
     // One workgroup per chain task or moment fold (a chain wavefront alone on its CU takes
-    // 28 us at 8192 positions, three together 33), more where the trial phase
-    // has over 1024 pairs of positions for each (P = 8 at 8192 positions:
-    // 39.6 us per generation with 32 workgroups, 42.2 with 16, 40.0 with 64).
+    // 28 us at 8192 positions, three together 33), more where there is a trial
+    // phase (not EvoArgs::fed) with over 1024 pairs of positions for each (P = 8
+    // at 8192 positions: 39.6 us per generation with 32 workgroups, 42.2 with 16,
+    // 40.0 with 64).
     // One CU per XCD stays free for the walk: workgroups go to the XCDs in
     // turn, and one that found its XCD full would hold up the grid barriers
     // until the walk ends.
@@ -302,6 +303,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     }
     size_t nwg = std::max(tasks, trial_pairs / 1024);
     if (m.normalize && m.renormalize) nwg = std::max<size_t>(nwg, P);  // a workgroup renormalizes a member at a time
+    // (the number of workgroups given from outside: always with a trial phase)
     h->fixed_nwg = std::getenv("DEAC_EVOLVE_WORKGROUPS") != nullptr;
     if (const char *user = std::getenv("DEAC_EVOLVE_WORKGROUPS")) nwg = std::max(std::atoi(user), 1);
     h->nwg = static_cast<int>(std::clamp<size_t>(nwg, 1, std::max(maxwg - 8, 1)));

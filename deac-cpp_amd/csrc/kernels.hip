@@ -941,8 +941,9 @@ __device__ __forceinline__ void feed_chain(const EvoArgs &a, const Members &s, c
 // Blocks [b0, b1) of a trial vector into the spare row, two blocks' loads
 // ahead of the two being formed.
 // Bound: memory (40 bytes read and 8 written per position): 512 members of
-// 8192 positions take 67 us with the top of the generation and the barrier
-// (3.5 TB/s without them); 96 with runs of 8 blocks and nothing read ahead.
+// 8192 positions take 46 us with the top of the generation and the barrier
+// (4.4 TB/s; a large copy reaches 4.7).  With a cache write-back per workgroup at
+// the barrier it was 67, with runs of 8 blocks and nothing read ahead 96.
 __device__ __forceinline__ void trial_blocks(const Trial &t, int b0, int b1)
 {
     typedef Trial::Load Load;
