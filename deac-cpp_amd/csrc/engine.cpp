@@ -258,7 +258,9 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     for (auto &set : h->kev)
         for (hipEvent_t &e : set)
             if (hipEventCreate(&e) != hipSuccess) return fail(DEAC_ERR_DEVICE);
-    if (hipHostMalloc(reinterpret_cast<void **>(&h->host_status), 12 * sizeof(int)) != hipSuccess) {
+    // coherent: kernels write it (EvoArgs::host_status), the host reads it after a dispatch's own event
+    if (hipHostMalloc(reinterpret_cast<void **>(&h->host_status), 12 * sizeof(int), hipHostMallocCoherent) !=
+        hipSuccess) {
         h->host_status = nullptr;
         return fail(DEAC_ERR_OUT_OF_MEMORY);
     }

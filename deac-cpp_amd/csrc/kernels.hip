@@ -34,6 +34,15 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kEvoWaves = kEvoThreads / kWave;
 
+// Status words for the host, by one thread: it reads them after the dispatch's
+// own stop event, which does not release at system scope, so this does, and the
+// stores have arrived in host memory before the wave ends.
+__device__ __forceinline__ void tell_host(int *status, int word, int value)
+{
+    __hip_atomic_store(status + word, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+}
+
 // Grid-wide barrier of the persistent evolution kernel.  The wait is
 // bounded: after kBarrierSpins polls the workgroup records a failure and every
 // caller leaves the kernel, so a broken launch cannot hang the device.
@@ -85,7 +94,7 @@ struct GridBarrier {
                 if (++spins == kBarrierSpins) {
                     timed_out = 1;
                     __hip_atomic_store(a.status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(a.host_status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    tell_host(a.host_status, 2, 1);
                     break;
                 }
             }
@@ -1333,8 +1342,8 @@ __global__ __launch_bounds__(kEvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
                     if (lane == 0) {
                         a.status[1] = g;
                         __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        __hip_atomic_store(a.host_status + 1, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                        __hip_atomic_store(a.host_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        tell_host(a.host_status, 1, g);
+                        tell_host(a.host_status, 0, 1);
                     }
                 }
                 break;

@@ -1,0 +1,316 @@
+// The engine's and the batch's host code (engine.cpp, batch.cpp,
+// host_model.cpp) on a stand-in for the HIP runtime: device memory is host
+// memory, streams and events only keep track of what has been waited for, and
+// no kernel runs (an evolution launch reports a stop at its first generation).
+// Allocations and launches are counted and can be made to fail, so that what
+// the host does when they do can be checked without a device.
+//
+// Usage: host_runtime SCENARIO; prints what was wrong and exits with 1.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "batch_kernels.hpp"
+#include "deac_engine.h"
+#include "init_kernels.hpp"
+#include "kernels.hpp"
+#include "pack_kernels.hpp"
+#include "precision_kernels.hpp"
+#include "split_kernels.hpp"
+
+// ---------------------------------------------------------------- runtime
+
+namespace {
+
+struct Stream {
+    bool pending = false;        // work that nothing has waited for
+    std::set<Stream *> behind;   // streams whose work this one waits for
+};
+struct Event {
+    std::set<Stream *> covers;
+};
+
+std::map<void *, size_t> live;   // device allocations
+size_t live_bytes = 0;
+long fail_malloc = 0;            // the n-th allocation from now on fails (1: the next), 0: none
+long fail_launch = 0;            // likewise the launches
+std::map<void *, unsigned> pinned;
+std::set<Stream *> streams;
+
+Stream *stream_of(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
+Event *event_of(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
+
+hipError_t launch(hipStream_t s)
+{
+    if (fail_launch > 0 && --fail_launch == 0) return hipErrorLaunchFailure;
+    if (s) stream_of(s)->pending = true;
+    return hipSuccess;
+}
+
+bool anything_in_flight()
+{
+    for (Stream *s : streams)
+        if (s->pending) return true;
+    return false;
+}
+
+}  // namespace
+
+extern "C" {
+hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int)
+{
+    *p = hipDeviceProp_t{};
+    std::strcpy(p->gcnArchName, "gfx950:sramecc+:xnack-");
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipMalloc(void **p, size_t n)
+{
+    if (fail_malloc > 0 && --fail_malloc == 0) return hipErrorOutOfMemory;
+    if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
+    live[*p] = n;
+    live_bytes += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    if (!p) return hipSuccess;
+    auto it = live.find(p);
+    if (it == live.end()) return hipErrorInvalidValue;
+    live_bytes -= it->second;
+    live.erase(it);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned flags)
+{
+    *p = std::calloc(n, 1);
+    pinned[*p] = flags;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p)
+{
+    pinned.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    return std::memcpy(d, s, n), hipSuccess;
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
+{
+    Stream *n = new Stream;
+    streams.insert(n);
+    *s = reinterpret_cast<hipStream_t>(n);
+    return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s)
+{
+    streams.erase(stream_of(s));
+    delete stream_of(s);
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s)
+{
+    for (Stream *b : stream_of(s)->behind) b->pending = false;
+    stream_of(s)->pending = false;
+    return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
+{
+    for (Stream *b : event_of(e)->covers) stream_of(s)->behind.insert(b);
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = reinterpret_cast<hipEvent_t>(new Event);
+    return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t e) { return delete event_of(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
+{
+    event_of(e)->covers = stream_of(s)->behind;
+    event_of(e)->covers.insert(stream_of(s));
+    return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e)
+{
+    for (Stream *b : event_of(e)->covers) b->pending = false;
+    return hipSuccess;
+}
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 0.0f, hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *) { return hipErrorNotSupported; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *, hipGraph_t, hipGraphNode_t *, char *, size_t)
+{
+    return hipErrorNotSupported;
+}
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+}
+
+// ---------------------------------------------------------------- kernels
+
+namespace deac {
+
+hipError_t launch_walk(const WalkArgs &, hipStream_t s) { return launch(s); }
+hipError_t launch_mask(const MaskArgs &, const WalkArgs &, hipStream_t s) { return launch(s); }
+hipError_t launch_ktile(const double *, double *, int, int, int, int, hipStream_t s) { return launch(s); }
+hipError_t launch_evolve(const EvoArgs &a, const WalkArgs &, const MaskArgs &, hipStream_t s, hipEvent_t, hipEvent_t stop)
+{
+    if (a.ngen > 0) a.host_status[0] = 1;
+    const hipError_t e = launch(s);
+    if (stop) (void)hipEventRecord(stop, s);
+    return e;
+}
+hipError_t launch_zero_u32(unsigned *, size_t, hipStream_t s) { return launch(s); }
+int evolve_max_workgroups(int) { return 256; }
+
+hipError_t launch_lane_tables(const LaneTabArgs &, int, hipStream_t s) { return launch(s); }
+hipError_t launch_initial_population(const InitArgs &, hipStream_t s) { return launch(s); }
+hipError_t launch_gather_best(const long *, size_t, const double *, int, const double *, double *, hipStream_t s)
+{
+    return launch(s);
+}
+
+hipError_t launch_pack_fp64(const PackArgs &, double, double *, hipStream_t s) { return launch(s); }
+hipError_t launch_pack_fp32(const PackArgs &, float *, hipStream_t s) { return launch(s); }
+hipError_t launch_pack_bf16x3(const PackArgs &, void *, void *, hipStream_t s) { return launch(s); }
+hipError_t launch_pack_fp32_units(const PackArgs &, float *, hipStream_t s) { return launch(s); }
+hipError_t launch_pack_transposed(const PackArgs &, int, int, double *, hipStream_t s) { return launch(s); }
+
+hipError_t launch_split_trial(const EvoArgs &, int, int, void *, void *, int, hipStream_t s) { return launch(s); }
+hipError_t launch_split_renorm(const EvoArgs &, hipStream_t s) { return launch(s); }
+hipError_t launch_split_pack_fp64(const EvoArgs &, int, double *, int, int, hipStream_t s) { return launch(s); }
+hipError_t launch_split_pack_fp32(const EvoArgs &, int, float *, int, int, hipStream_t s) { return launch(s); }
+hipError_t launch_split_pack_bf16x3(const EvoArgs &, int, void *, void *, int, int, hipStream_t s) { return launch(s); }
+hipError_t launch_split_fold(const EvoArgs &, hipStream_t s) { return launch(s); }
+hipError_t launch_split_moments(const EvoArgs &, int, hipStream_t s) { return launch(s); }
+hipError_t launch_split_select(const EvoArgs &, int, int, hipStream_t s) { return launch(s); }
+hipError_t launch_split_model_select(const EvoArgs &, int, int, const float *, int, int, int, const int *, hipStream_t s)
+{
+    return launch(s);
+}
+hipError_t launch_split_iter(long *, long, hipStream_t s) { return launch(s); }
+hipError_t launch_ks_fp64(const double *, const double *, double *, int, int, int, int, int, hipStream_t s, hipEvent_t,
+                          hipEvent_t, const int *)
+{
+    return launch(s);
+}
+hipError_t launch_ks_fp32(const float *, const float *, float *, int, int, int, int, int, hipStream_t s, hipEvent_t,
+                          hipEvent_t, const int *)
+{
+    return launch(s);
+}
+hipError_t launch_ks_bf16x3(const void *, const void *, const void *, const void *, float *, int, int, int, int, int,
+                            hipStream_t s, hipEvent_t, hipEvent_t, const int *)
+{
+    return launch(s);
+}
+
+static hipError_t batch_launch(const BatchDesc *d, int count, hipStream_t s)
+{
+    for (int i = 0; i < count; i++)
+        for (int q = 0; q < d[i].Q && d[i].mode == 0; q++) {
+            d[i].status[q][0] = 1;
+            d[i].status[q][1] = d[i].gen0;
+        }
+    return launch(s);
+}
+hipError_t launch_batch(const BatchDesc *d, int n, int, int, int, hipStream_t s) { return batch_launch(d, n, s); }
+hipError_t launch_batch_fold(const BatchDesc *d, int n, int, int, hipStream_t s) { return batch_launch(d, n, s); }
+hipError_t launch_batch_mixed(const BatchDesc *d, int n, int, int, int, int, hipStream_t s)
+{
+    return batch_launch(d, n, s);
+}
+int batch_mixed_nq(int ntm, int) { return ntm <= 9 ? 9 : 0; }
+hipError_t batch_scratch(int, double **p)
+{
+    static std::vector<double> scratch(kBatchScratchDoubles);
+    return *p = scratch.data(), hipSuccess;
+}
+hipError_t batch_role_cycles_fp64(unsigned long long *, int) { return hipErrorNotSupported; }
+hipError_t batch_role_cycles_mixed(unsigned long long *, int) { return hipErrorNotSupported; }
+
+}  // namespace deac
+
+// ---------------------------------------------------------------- scenarios
+
+namespace {
+
+int wrong = 0;
+void expect(bool ok, const std::string &what)
+{
+    if (ok) return;
+    std::printf("%s\n", what.c_str());
+    wrong = 1;
+}
+
+struct Problem {
+    std::vector<double> tau, isf, err, freq;
+    deac_problem p{};
+    Problem(size_t T, size_t G) : tau(T), isf(T), err(T), freq(G)
+    {
+        for (size_t t = 0; t < T; t++) {
+            tau[t] = 0.37 * static_cast<double>(t) / static_cast<double>(T - 1);
+            isf[t] = 1.0 - 0.5 * tau[t];
+            err[t] = 0.01 * isf[t];
+        }
+        (void)deac_frequency_grid(G, 48.0, freq.data());
+        p.number_of_timeslices = T;
+        p.imaginary_time = tau.data();
+        p.isf = isf.data();
+        p.isf_error = err.data();
+        p.genome_size = G;
+        p.frequency = freq.data();
+        p.temperature = 1.35;
+        p.spectra_type = DEAC_BFULL;
+        p.population_size = 8;
+        p.first_moment = p.third_moment = -1.0;
+        p.crossover_probability = p.differential_weight = 0.9;
+        p.self_adapting_crossover_probability = p.self_adapting_differential_weight_probability = 0.1;
+    }
+};
+
+// The kernel writes the status into pinned memory that the host reads after
+// the dispatch's own event: memory that neither side may hold in a cache.
+void status_memory()
+{
+    Problem q(9, 32);
+    deac_handle *h = nullptr;
+    expect(deac_create(&q.p, &h, nullptr) == DEAC_OK, "deac_create failed");
+    expect(pinned.size() == 1, "one pinned allocation expected");
+    for (auto &[ptr, flags] : pinned)
+        expect((flags & hipHostMallocCoherent) != 0, "the status memory is not asked for as coherent");
+    deac_destroy(h);
+    expect(live.empty(), "device memory left after deac_destroy");
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const std::map<std::string, void (*)()> scenarios = {
+        {"status_memory", status_memory},
+    };
+    auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
+    if (it == scenarios.end()) return std::printf("no such scenario\n"), 2;
+    it->second();
+    return wrong;
+}
