@@ -297,9 +297,23 @@ __global__ __launch_bounds__(kWave) void split_moment_kernel(EvoArgs a, int init
 // 114 slices, 64 members: 13.3 us; as two kernels, with a part of each
 // sum's loads in flight, 9.2 and 7.5.
 constexpr int kSliceRun = 8;  // slices a thread loads at once
+constexpr int kSelectThreads = 1024;
+
+// Runs of slices: as many as the threads hold, but none of fewer slices than a
+// thread loads at once (a turn with its barrier costs 0.15 us among 1024 threads:
+// with all the runs that fit, FP32, 8 members, G = 4096, a generation took 181 us
+// at 2 timeslices, 134 at 8, 70 at 17 and 38 at 65; 22.6, 22.5, 23.0 and 25.3 with
+// this).
+__host__ __device__ __forceinline__ int slice_runs(int cols, int slices, int threads)
+{
+    const int held = threads / cols, full = (slices + kSliceRun - 1) / kSliceRun;
+    return held < full ? held : full;
+}
+
 template <bool MODEL>
-__global__ __launch_bounds__(MODEL ? 1024 : kWave) void split_select_kernel(EvoArgs a, int g, int init, const float *part,
-                                                                            int slices, int Npad, int Mpad, const int *ex)
+__global__ __launch_bounds__(MODEL ? kSelectThreads : kWave) void split_select_kernel(EvoArgs a, int g, int init,
+                                                                                      const float *part, int slices,
+                                                                                      int Npad, int Mpad, const int *ex)
 {
     constexpr int kTauEach = 4;
     if (stopped(a)) return;
@@ -320,17 +334,21 @@ __global__ __launch_bounds__(MODEL ? 1024 : kWave) void split_select_kernel(EvoA
     for (int t0 = 0; t0 < a.T; t0 += kSelectLds) {
         const int n = min(kSelectLds, a.T - t0);
         if constexpr (MODEL) {
-            const int cols = (n + kTauEach - 1) / kTauEach, runs = static_cast<int>(blockDim.x) / cols;
+            const int cols = (n + kTauEach - 1) / kTauEach, runs = slice_runs(cols, slices, blockDim.x);
             const int col = threadIdx.x % cols, run = threadIdx.x / cols;
             const int each = (slices + runs - 1) / runs, k0 = run * each, k1 = min(k0 + each, slices);
             const float4 *from = reinterpret_cast<const float4 *>(part + static_cast<size_t>(i) * Mpad + t0) + col;
             const size_t step = static_cast<size_t>(Npad) * Mpad / 4;
             float4 *sums = reinterpret_cast<float4 *>(dsh + (min(kSelectLds, a.T) + 1) / 2 * 2);
             float4 v[kSliceRun];
+            // past the run the last slice again, as zeros: a sum that starts
+            // from +0 is never -0, so that they leave it as it is
             auto load = [&](int k) {
 #pragma unroll
+                for (int u = 0; u < kSliceRun; u++) v[u] = from[min(k + u, slices - 1) * step];
+#pragma unroll
                 for (int u = 0; u < kSliceRun; u++)
-                    if (k + u < k1) v[u] = from[(k + u) * step];
+                    if (k + u >= k1) v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             };
             load(k0);
             for (int r = 0; r < runs; r++) {
@@ -339,13 +357,12 @@ __global__ __launch_bounds__(MODEL ? 1024 : kWave) void split_select_kernel(EvoA
                     for (int k = k0; k < k1; k += kSliceRun) {
                         if (k > k0) load(k);
 #pragma unroll
-                        for (int u = 0; u < kSliceRun; u++)
-                            if (k + u < k1) {
-                                x.x += v[u].x;
-                                x.y += v[u].y;
-                                x.z += v[u].z;
-                                x.w += v[u].w;
-                            }
+                        for (int u = 0; u < kSliceRun; u++) {
+                            x.x += v[u].x;
+                            x.y += v[u].y;
+                            x.z += v[u].z;
+                            x.w += v[u].w;
+                        }
                     }
                     sums[col] = x;
                 }
@@ -481,8 +498,11 @@ hipError_t launch_split_model_select(const EvoArgs &a, int g, int init, const fl
 {
     const size_t window = static_cast<size_t>(std::min(a.T, kSelectLds));
     const size_t lds = (window + 1) / 2 * 2 * sizeof(double) + (window + 3) / 4 * sizeof(float4);
-    hipLaunchKernelGGL(split_select_kernel<true>, dim3(a.P), dim3(1024), lds, s, a, g, init, part, slices, Npad, Mpad,
-                       ex);
+    const int cols = (static_cast<int>(window) + 3) / 4;
+    // the wavefronts that have slices to add, and one per 64 residuals
+    const int used = std::max(cols * slice_runs(cols, slices, kSelectThreads), std::min(a.T, kSelectThreads));
+    hipLaunchKernelGGL(split_select_kernel<true>, dim3(a.P), dim3(static_cast<unsigned>((used + kWave - 1) / kWave * kWave)),
+                       lds, s, a, g, init, part, slices, Npad, Mpad, ex);
     return hipGetLastError();
 }
 
