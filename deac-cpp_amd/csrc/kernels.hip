@@ -583,14 +583,20 @@ struct KUnits {
     __device__ __forceinline__ void advance() { base += kChunkUnits * 1024; }
 };
 
+// Positions in front of a chunk: rows may be longer than the 4 GiB that a buffer
+// load's own offset reaches, so that the base moves.
+__host__ __device__ constexpr size_t chunk_offset(int chunk) { return static_cast<size_t>(chunk) * kChunk; }
+static_assert(chunk_offset((1 << 30) / kChunk) * sizeof(double) == size_t(8) << 30, "rows of 2^30 positions");
+
 // A member group's four genome rows, read the same way, 128 positions a load.
 struct GenomeRows {
     const double *row[kChainRows];
     int vo;  // this lane's two positions, bytes
     __device__ __forceinline__ dvec2 load(int m, int chunk) const
     {
-        const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(row[m]), 0, -1, 0x00020000);
-        return __builtin_bit_cast(dvec2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, static_cast<unsigned>(chunk) * (kChunk * 8), 0));
+        const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(row[m] + chunk_offset(chunk)), 0, kChunk * 8,
+                                                         0x00020000);
+        return __builtin_bit_cast(dvec2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, 0, 0));
     }
 };
 
