@@ -68,13 +68,17 @@ struct GridBarrier {
     {
     }
 
-    // Each wave drains its own memory operations; then one thread per
+    // Each wave drains its own memory operations (the wait alone is no memory
+    // fence to the compiler: the one in front holds the stores there; where
+    // an XCD's workgroups arrive together, nothing else stands between the
+    // stores of all but the last and their arrival); then one thread per
     // workgroup publishes the workgroup's stores at agent scope (L2 write-back,
     // visible to the other XCDs), arrives, waits, and invalidates this CU's
     // caches for what the other workgroups wrote.
     __device__ __forceinline__ bool wait()
     {
         __shared__ int timed_out;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         target += arrivals;
