@@ -216,20 +216,24 @@ __device__ __forceinline__ bool stopped(const int *halt)
     return halt && __hip_atomic_load(halt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
-// Which draws of a sequence are values: bit i+1 where bit i is a test (not a
-// value) whose limit the draw passed.  carry: whether draw 0 is a value; set
-// to whether draw 64 is.  Runs of passed draws alternate test, value, test,
-// ..., which an addition resolves for all runs at once: a run's values are
-// its positions of the parity opposite to its first.
+// Which of a window's 64 draws are values: bit i where draw i belongs to a test
+// before it that passed its limit (bit i of passed: draw i is under the limit).
+// Among draws under the limit tests and values alternate, a test first, so a
+// draw is a value where the run of them that ends in front of it is odd; every
+// lane measures its own.  carry: whether draw 0 is a value (which ends a run,
+// whatever its size); set to whether the draw behind the window is.  By the whole
+// wavefront.
 __device__ __forceinline__ uint64_t value_bits(uint64_t passed, bool &carry)
 {
-    const uint64_t kEven = UINT64_C(0x5555555555555555);
-    passed &= ~static_cast<uint64_t>(carry ? 1 : 0);
-    const uint64_t follows = (passed << 1) | (carry ? 1 : 0);
-    const uint64_t odd_starts = passed & ~kEven & ~follows;
-    const uint64_t sum = odd_starts + passed;
-    carry = sum < passed;
-    return (kEven ^ (sum << 1)) & follows;
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint64_t failed = ~(carry ? passed & ~UINT64_C(1) : passed);
+    auto run_before = [&](int i) {  // i > 0
+        const uint64_t f = failed << (64 - i);
+        return f ? __builtin_clzll(f) : i;
+    };
+    const bool value = lane ? run_before(lane) & 1 : carry;
+    carry = run_before(64) & 1;
+    return __ballot(value);
 }
 
 // Walk of a.ngen generations by one wavefront (deac.cpp:1180-1240): the
