@@ -125,7 +125,7 @@ struct deac_batch {
     double *best_rows = nullptr;               // [genomes of all instances]: best members, gathered for the readback
     long *best_off = nullptr;                  // per instance: offset in best_rows, of its population, P, Kc, Lpad
     std::vector<size_t> best_at;               // offset in best_rows, host side
-    double *stats_ws = nullptr;                // statistics histories, kept between runs and grown on demand
+    double *stats_ws = nullptr;                // statistics histories, kept between runs up to kStatsKept
     size_t stats_cap = 0;
     double *scratch = nullptr;                 // this device's statistics scratch (deac_batch_run_noalloc)
     std::vector<long> reached;                 // per instance: generation reached by the last run (absolute)
@@ -277,6 +277,38 @@ struct TempRows {
             return true;
         (void)hipGetLastError();
         return false;
+    }
+};
+
+// Packed device memory read back in pieces of kPiece doubles (32 MiB) or one
+// item, items in ascending order.
+constexpr size_t kPiece = size_t(4) << 20;
+// A history of more doubles than this (1 MiB) is copied by itself, as far as it
+// was written.
+constexpr size_t kLongHistory = size_t(1) << 17;
+class Pieces {
+    const double *from_;
+    size_t total_, at_ = 0, size_ = 0, cap_ = 0;
+    std::unique_ptr<double[]> buf_;
+
+public:
+    Pieces(const double *from, size_t total) : from_(from), total_(total) {}
+    hipError_t get(size_t offset, size_t count, const double *&item)
+    {
+        if (offset < at_ || offset + count > at_ + size_) {
+            const size_t size = std::min(total_ - offset, std::max(count, kPiece));
+            if (size > cap_) {
+                buf_.reset(new double[size]);
+                cap_ = size;
+            }
+            size_ = 0;
+            const hipError_t e = hipMemcpy(buf_.get(), from_ + offset, size * sizeof(double), hipMemcpyDeviceToHost);
+            if (e != hipSuccess) return e;
+            at_ = offset;
+            size_ = size;
+        }
+        item = buf_.get() + (offset - at_);
+        return hipSuccess;
     }
 };
 
@@ -719,10 +751,22 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
     size_t stats_n = 0;
     for (size_t i = 0; i < n; i++)
         if (options[i].track_stats) stats_n += 3 * options[i].number_of_generations;
-    if (!stats_pool && stats_n > h->stats_cap) {
+    auto release_stats = [&]() {
         h->release(h->stats_ws);
         h->stats_ws = nullptr;
         h->stats_cap = 0;
+    };
+    // (frees the histories of a long run behind it, whatever its outcome)
+    struct AtReturn {
+        decltype(release_stats) &release;
+        const size_t &cap;
+        ~AtReturn()
+        {
+            if (cap > deac::kStatsKept) release();
+        }
+    } at_return{release_stats, h->stats_cap};
+    if (!stats_pool && stats_n > h->stats_cap) {
+        release_stats();
         if (h->alloc(h->stats_ws, stats_n) != DEAC_OK) return DEAC_ERR_OUT_OF_MEMORY;
         h->stats_cap = stats_n;
     }
@@ -1056,15 +1100,12 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
     h->last = prof;
 
     // Epilogue per instance (deac.cpp:1576-1685), as deac_run.
-    // The best members' rows are gathered on the device: one copy each for the
-    // fitnesses, the random states, the rows and the statistics.
-    const size_t last = n - 1;
-    std::vector<double> rows(h->best_at[last] + h->models[h->model_of[last]]->m.Kc), stats_host(stats_n);
+    // The best members' rows are gathered on the device; rows and statistics come
+    // back in pieces that hold many instances (a copy each took 25 us).
     BATCH_HIP(deac::launch_gather_best(h->best_off, n, h->fitness, deac::kBatchMaxP, h->pop, h->best_rows, s));
     BATCH_HIP(hipStreamSynchronize(s));
-    BATCH_HIP(hipMemcpy(rows.data(), h->best_rows, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
-    if (stats_n)
-        BATCH_HIP(hipMemcpy(stats_host.data(), stats_base_ptr, stats_n * sizeof(double), hipMemcpyDeviceToHost));
+    const BatchModel &last = *h->models[h->model_of[n - 1]];
+    Pieces rows(h->best_rows, h->best_at[n - 1] + last.m.Kc), histories(stats_base_ptr, stats_n);
     std::vector<double> fit_all(n * deac::kBatchMaxP);
     BATCH_HIP(hipMemcpy(fit_all.data(), h->fitness, fit_all.size() * sizeof(double), hipMemcpyDeviceToHost));
     BATCH_HIP(hipMemcpy(rng_host.data(), h->rng, rng_host.size() * sizeof(uint64_t), hipMemcpyDeviceToHost));
@@ -1081,14 +1122,22 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
                 minimum = fit[k];
                 best = k;
             }
-        deac::output_transform(m, &rows[h->best_at[i]], r->dsf, r->frequency);
+        const double *row = nullptr;
+        BATCH_HIP(rows.get(h->best_at[i], m.Kc, row));
+        deac::output_transform(m, row, r->dsf, r->frequency);
         size_t generation = stopped_at[i] >= 0 ? static_cast<size_t>(stopped_at[i] - base[i]) : N - 2;
         if (stats[i]) {
-            const double *hs = &stats_host[static_cast<size_t>(stats[i] - stats_base_ptr)];
-            const size_t k = generation + 1;
-            if (r->stats_mean) std::memcpy(r->stats_mean, hs, k * sizeof(double));
-            if (r->stats_minimum) std::memcpy(r->stats_minimum, hs + N, k * sizeof(double));
-            if (r->stats_squared_mean) std::memcpy(r->stats_squared_mean, hs + 2 * N, k * sizeof(double));
+            const size_t k = generation + 1;  // entries written
+            double *const to[3] = {r->stats_mean, r->stats_minimum, r->stats_squared_mean};
+            if (3 * N <= kLongHistory) {
+                const double *hs = nullptr;
+                BATCH_HIP(histories.get(static_cast<size_t>(stats[i] - stats_base_ptr), 3 * N, hs));
+                for (int q = 0; q < 3; q++)
+                    if (to[q]) std::memcpy(to[q], hs + q * N, k * sizeof(double));
+            } else {
+                for (int q = 0; q < 3; q++)
+                    if (to[q]) BATCH_HIP(hipMemcpy(to[q], stats[i] + q * N, k * sizeof(double), hipMemcpyDeviceToHost));
+            }
         }
         if (generation + 2 == N) {  // deac.cpp:1677-1685
             generation += 1;

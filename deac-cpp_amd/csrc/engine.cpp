@@ -58,7 +58,7 @@ struct deac_handle {
     bool wide = false;
     uint64_t *init_start = nullptr;     // [P][4]: random state at each member's first initial draw
     std::vector<uint64_t> skip_tab;     // nibble table of T^Kc, host side
-    double *stats = nullptr;            // statistics histories, kept between runs and grown on demand
+    double *stats = nullptr;            // statistics histories, kept between runs up to kStatsKept
     size_t stats_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // per set: walk start, walk end, mask end (fused path: the first batch's
@@ -449,14 +449,26 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     std::vector<double> cr(P * nsign, m.cr0), fw(P * nsign, m.f0);  // deac.cpp:990-1032
 
     const bool track = o->track_stats != 0;
-    if (track && h->stats_cap < 3 * N) {
+    auto release_stats = [&]() {
         void *old = h->stats;
-        h->release(old);
         h->stats = nullptr;
         h->stats_cap = 0;
+        h->release(old);
+    };
+    if (track && h->stats_cap < 3 * N) {
+        release_stats();
         DEAC_TRY(h->alloc(h->stats, 3 * N));
         h->stats_cap = 3 * N;
     }
+    // (frees the histories of a long run behind it, whatever its outcome)
+    struct AtReturn {
+        decltype(release_stats) &release;
+        const size_t &cap;
+        ~AtReturn()
+        {
+            if (cap > deac::kStatsKept) release();
+        }
+    } at_return{release_stats, h->stats_cap};
     double *const stats = track ? h->stats : nullptr;
 
     DEAC_HIP(hipMemcpyAsync(h->init_start, starts.data(), starts.size() * sizeof(uint64_t), hipMemcpyHostToDevice, s));
@@ -880,12 +892,10 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     deac::output_transform(m, row.data(), r->dsf, r->frequency);
 
     if (track) {
-        std::vector<double> host_stats(3 * N, 0.0);
-        const size_t n = generation + 1;
-        DEAC_HIP(hipMemcpy(host_stats.data(), stats, 3 * N * sizeof(double), hipMemcpyDeviceToHost));
-        if (r->stats_mean) std::memcpy(r->stats_mean, host_stats.data(), n * sizeof(double));
-        if (r->stats_minimum) std::memcpy(r->stats_minimum, host_stats.data() + N, n * sizeof(double));
-        if (r->stats_squared_mean) std::memcpy(r->stats_squared_mean, host_stats.data() + 2 * N, n * sizeof(double));
+        const size_t n = generation + 1;  // entries written
+        double *const to[3] = {r->stats_mean, r->stats_minimum, r->stats_squared_mean};
+        for (int k = 0; k < 3; k++)
+            if (to[k]) DEAC_HIP(hipMemcpy(to[k], stats + k * N, n * sizeof(double), hipMemcpyDeviceToHost));
     }
     if (generation + 2 == N) {  // deac.cpp:1677-1685
         generation += 1;

@@ -72,6 +72,10 @@ deac_status validate(const deac_problem &p, std::string &message);
 // Builds K (deac.cpp:310-401) and the moment vectors (deac.cpp:489-827).
 Model build_model(const deac_problem &p);
 
+// Device memory for statistics histories that a handle keeps from run to run, in
+// doubles (64 MiB); a longer run's is given back behind it.
+constexpr size_t kStatsKept = size_t(8) << 20;
+
 // In-order reductions of the reference build (see host_model.cpp).
 double mean_of(const double *a, size_t n);
 double squared_mean_of(const double *a, size_t n);

@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <new>
 #include <set>
 #include <string>
 #include <vector>
@@ -43,6 +44,7 @@ long fail_malloc = 0;            // the n-th allocation from now on fails (1: th
 long fail_launch = 0;            // likewise the launches
 std::map<void *, unsigned> pinned;
 std::set<Stream *> streams;
+size_t host_largest = 0;         // largest single host allocation so far
 
 Stream *stream_of(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
 Event *event_of(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
@@ -62,6 +64,15 @@ bool anything_in_flight()
 }
 
 }  // namespace
+
+void *operator new(size_t n)
+{
+    if (n > host_largest) host_largest = n;
+    if (void *p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
@@ -302,12 +313,82 @@ void status_memory()
     expect(live.empty(), "device memory left after deac_destroy");
 }
 
+// A batch of n instances of one problem, and their outputs.
+struct Batch {
+    Problem q;
+    deac_batch *h = nullptr;
+    std::vector<uint64_t> rng;
+    std::vector<deac_run_options> o;
+    std::vector<deac_result> r;
+    std::vector<std::vector<double>> out;
+    Batch(size_t n, size_t T, size_t G, size_t generations) : q(T, G), rng(4 * n), o(n), r(n), out(5 * n)
+    {
+        const std::vector<deac_problem> p(n, q.p);
+        expect(deac_batch_create(p.data(), n, &h, nullptr) == DEAC_OK, "deac_batch_create failed");
+        const size_t len = deac_output_length(&q.p);
+        for (size_t i = 0; i < n; i++) {
+            deac_seed_state(i, &rng[4 * i]);
+            o[i].number_of_generations = generations;
+            o[i].track_stats = 1;
+            for (int k = 0; k < 5; k++) out[5 * i + k].resize(k < 2 ? len : generations);
+            r[i].dsf = out[5 * i].data();
+            r[i].frequency = out[5 * i + 1].data();
+            r[i].stats_mean = out[5 * i + 2].data();
+            r[i].stats_minimum = out[5 * i + 3].data();
+            r[i].stats_squared_mean = out[5 * i + 4].data();
+        }
+    }
+    ~Batch() { deac_batch_destroy(h); }
+    deac_status run() { return deac_batch_run(h, rng.data(), o.data(), r.data()); }
+};
+
+// Long histories: neither the host nor the device keeps all instances' at once
+// behind a run, and a long genome's best rows come back in pieces.
+void long_histories()
+{
+    constexpr size_t kMuch = size_t(48) << 20;
+    {
+        Batch b(24, 9, 32, 1000000);  // 24 MB each, three histories
+        const size_t before = live_bytes;
+        host_largest = 0;
+        expect(b.run() == DEAC_OK, "deac_batch_run failed");
+        expect(host_largest < kMuch, "batch: one host allocation of " + std::to_string(host_largest) + " bytes");
+        expect(live_bytes == before, "batch: " + std::to_string(live_bytes - before) + " bytes of device memory kept");
+    }
+    {
+        Batch b(400, 3, 16384, 10);  // 105 MB of best rows
+        host_largest = 0;
+        expect(b.run() == DEAC_OK, "deac_batch_run failed");
+        expect(host_largest < kMuch, "rows: one host allocation of " + std::to_string(host_largest) + " bytes");
+    }
+    Problem q(9, 32);
+    deac_handle *h = nullptr;
+    expect(deac_create(&q.p, &h, nullptr) == DEAC_OK, "deac_create failed");
+    const size_t before = live_bytes, len = deac_output_length(&q.p), N = 4000000;
+    std::vector<double> dsf(len), freq(len), mean(N);
+    deac_run_options o{};
+    o.number_of_generations = N;
+    o.track_stats = 1;
+    deac_result r{};
+    r.dsf = dsf.data();
+    r.frequency = freq.data();
+    r.stats_mean = mean.data();
+    uint64_t rng[4];
+    deac_seed_state(1, rng);
+    host_largest = 0;
+    expect(deac_run(h, rng, &o, &r) == DEAC_OK, "deac_run failed");
+    expect(host_largest < kMuch, "engine: one host allocation of " + std::to_string(host_largest) + " bytes");
+    expect(live_bytes == before, "engine: " + std::to_string(live_bytes - before) + " bytes of device memory kept");
+    deac_destroy(h);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> scenarios = {
         {"status_memory", status_memory},
+        {"long_histories", long_histories},
     };
     auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return std::printf("no such scenario\n"), 2;
