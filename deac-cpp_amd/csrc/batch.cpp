@@ -155,11 +155,13 @@ struct deac_batch {
     deac_status alloc(T *&out, size_t count)
     {
         void *p = nullptr;
+        allocations.push_back(nullptr);  // its place, before there is anything to lose
         if (hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) {
             (void)hipGetLastError();
+            allocations.pop_back();
             return DEAC_ERR_OUT_OF_MEMORY;
         }
-        allocations.push_back(p);
+        allocations.back() = p;
         out = static_cast<T *>(p);
         return DEAC_OK;
     }
@@ -454,7 +456,7 @@ deac_status upload_model(deac_batch *h, BatchModel &b)
 extern "C" {
 
 deac_status deac_batch_create(const deac_problem *problems, size_t count, deac_batch **out, const char **message)
-{
+try {
     if (message) *message = nullptr;
     if (!out) return DEAC_ERR_INVALID_ARGUMENT;
     *out = nullptr;
@@ -594,6 +596,8 @@ deac_status deac_batch_create(const deac_problem *problems, size_t count, deac_b
     }
     *out = h.release();
     return DEAC_OK;
+} catch (...) {
+    return deac::caught();
 }
 
 void deac_batch_destroy(deac_batch *h) { delete h; }
@@ -616,7 +620,7 @@ namespace {
 // tracking instance, packed), or null to allocate them here.
 deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_options *options,
                            deac_result *results, bool resume, double *stats_pool)
-{
+try {
     if (!h || !rng_states || !options || !results) return DEAC_ERR_INVALID_ARGUMENT;
     const size_t n = h->model_of.size();
     if (resume && h->reached.size() != n) {
@@ -1158,6 +1162,8 @@ deac_status batch_run_impl(deac_batch *h, uint64_t *rng_states, const deac_run_o
     h->epar_valid.assign(n, 0);
     for (size_t i = 0; i < n; i++) h->epar_valid[i] = options[i].ks_precision != DEAC_PRECISION_FP64;
     return DEAC_OK;
+} catch (...) {
+    return deac::caught();
 }
 
 }  // namespace
@@ -1177,7 +1183,7 @@ deac_status deac_batch_continue(deac_batch *h, uint64_t *rng_states, const deac_
 
 deac_status deac_batch_run_noalloc(deac_batch *h, uint64_t *rng_states, const deac_run_options *options,
                                    deac_result *results)
-{
+try {
     if (!h || !rng_states || !options || !results) return DEAC_ERR_INVALID_ARGUMENT;
     const size_t n = h->model_of.size();
     size_t need = 0;
@@ -1197,6 +1203,8 @@ deac_status deac_batch_run_noalloc(deac_batch *h, uint64_t *rng_states, const de
         return DEAC_ERR_INVALID_ARGUMENT;
     }
     return batch_run_impl(h, rng_states, options, results, false, h->scratch);
+} catch (...) {
+    return deac::caught();
 }
 
 deac_status deac_batch_role_cycles(int precision, unsigned long long *cycles, int reset)
@@ -1235,7 +1243,7 @@ deac_status deac_batch_get_schedule(const deac_batch *h, deac_batch_schedule *sc
 
 deac_status deac_batch_tune(deac_batch *h, const uint64_t *rng_states, const deac_run_options *options,
                             size_t generations, deac_batch_schedule *chosen)
-{
+try {
     if (!h || !rng_states || !options || generations < 1) return DEAC_ERR_INVALID_ARGUMENT;
     const size_t n = h->model_of.size();
     // scratch outputs and a bounded run of every instance
@@ -1304,6 +1312,8 @@ deac_status deac_batch_tune(deac_batch *h, const uint64_t *rng_states, const dea
     }
     if (chosen) *chosen = best;
     return DEAC_OK;
+} catch (...) {
+    return deac::caught();
 }
 
 

@@ -7,6 +7,7 @@
 #include <cstdlib>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -95,8 +96,12 @@ struct deac_handle {
     deac_status alloc(T *&out, size_t count)
     {
         void *p = nullptr;
-        if (hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return DEAC_ERR_OUT_OF_MEMORY;
-        allocations.push_back(p);
+        allocations.push_back(nullptr);  // its place, before there is anything to lose
+        if (hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) {
+            allocations.pop_back();
+            return DEAC_ERR_OUT_OF_MEMORY;
+        }
+        allocations.back() = p;
         out = static_cast<T *>(p);
         return DEAC_OK;
     }
@@ -223,7 +228,7 @@ deac_status deac_frequency_grid(size_t G, double omega_max, double *f)
 }
 
 deac_status deac_create(const deac_problem *p, deac_handle **out, const char **message)
-{
+try {
     if (message) *message = nullptr;
     if (!p || !out) return DEAC_ERR_INVALID_ARGUMENT;
     *out = nullptr;
@@ -243,26 +248,23 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     DEAC_HIP(hipGetDeviceProperties(&prop, device));
     if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0) return DEAC_ERR_NO_DEVICE;
 
-    deac_handle *h = new deac_handle();
+    std::unique_ptr<deac_handle> own(new deac_handle());
+    deac_handle *const h = own.get();
     h->m = deac::build_model(*p);
     h->device = device;
     const deac::Model &m = h->m;
-    auto fail = [&](deac_status s) {
-        delete h;
-        return s;
-    };
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&h->draw_stream, hipStreamNonBlocking) != hipSuccess)
-        return fail(DEAC_ERR_DEVICE);
-    if (hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess) return fail(DEAC_ERR_DEVICE);
+        return DEAC_ERR_DEVICE;
+    if (hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess) return DEAC_ERR_DEVICE;
     for (auto &set : h->kev)
         for (hipEvent_t &e : set)
-            if (hipEventCreate(&e) != hipSuccess) return fail(DEAC_ERR_DEVICE);
+            if (hipEventCreate(&e) != hipSuccess) return DEAC_ERR_DEVICE;
     // coherent: kernels write it (EvoArgs::host_status), the host reads it after a dispatch's own event
     if (hipHostMalloc(reinterpret_cast<void **>(&h->host_status), 12 * sizeof(int), hipHostMallocCoherent) !=
         hipSuccess) {
         h->host_status = nullptr;
-        return fail(DEAC_ERR_OUT_OF_MEMORY);
+        return DEAC_ERR_OUT_OF_MEMORY;
     }
 
     const int T = static_cast<int>(m.T), P = static_cast<int>(m.P), Kc = static_cast<int>(m.Kc);
@@ -283,7 +285,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     h->batch = static_cast<int>(std::clamp<size_t>(std::max((size_t(64) << 20) / per_gen, std::min<size_t>(16, most)), 1, 1024));
 
     const int maxwg = deac::evolve_max_workgroups(device);
-    if (maxwg <= 0) return fail(DEAC_ERR_DEVICE);
+    if (maxwg <= 0) return DEAC_ERR_DEVICE;
     h->maxwg = maxwg;
     // One workgroup per chain task or moment fold (a chain wavefront alone on its CU takes
     // 28 us at 8192 positions, three together 33), more where there is a trial
@@ -348,7 +350,7 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
     if (!m.fterm.empty()) A(h->fterm, Kc + 1);
     if (!m.tterm.empty()) A(h->tterm, Kc + 1);
     if (m.use_nfm) A(h->nfm_dt, T);
-    if (st != DEAC_OK) return fail(st);
+    if (st != DEAC_OK) return st;
 
     // Jump tables: T^(nsign*G) by rows for the serial walk and by nibbles for
     // the wide one, T^(l*chunk) by lanes for the mask generator, T^(l*c1) and
@@ -396,9 +398,11 @@ deac_status deac_create(const deac_problem *p, deac_handle **out, const char **m
         if (st == DEAC_OK &&
             hipMemsetAsync(p, 0, static_cast<size_t>(h->batch) * P * sizeof(deac::MemberCtl), h->stream) != hipSuccess)
             st = DEAC_ERR_DEVICE;
-    if (st != DEAC_OK) return fail(st);
-    *out = h;
+    if (st != DEAC_OK) return st;
+    *out = own.release();
     return DEAC_OK;
+} catch (...) {
+    return deac::caught();
 }
 
 void deac_destroy(deac_handle *h) { delete h; }
@@ -411,7 +415,7 @@ deac_status deac_last_run_profile(const deac_handle *h, deac_run_profile *profil
 }
 
 deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_options *o, deac_result *r)
-{
+try {
     if (!h || !rng_state || !o || !r || !r->dsf || !r->frequency) return DEAC_ERR_INVALID_ARGUMENT;
     if (o->number_of_generations < 2) {
         deac::last_message() = "number_of_generations must be at least 2";
@@ -447,6 +451,7 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     }
     std::vector<int> cur(P, 0);
     std::vector<double> cr(P * nsign, m.cr0), fw(P * nsign, m.f0);  // deac.cpp:990-1032
+    std::vector<double> fit(P), row(Kc);                            // for the results
 
     const bool track = o->track_stats != 0;
     auto release_stats = [&]() {
@@ -876,7 +881,6 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     std::memcpy(rng_state, rng.s, sizeof rng.s);
 
     // Epilogue on the host (deac.cpp:1576-1685).
-    std::vector<double> fit(P), row(Kc);
     DEAC_HIP(hipMemcpy(fit.data(), h->fitness, P * sizeof(double), hipMemcpyDeviceToHost));
     DEAC_HIP(hipMemcpy(cur.data(), h->cur, P * sizeof(int), hipMemcpyDeviceToHost));
     size_t generation = stopped_at >= 0 ? static_cast<size_t>(stopped_at) : N - 2;
@@ -910,6 +914,8 @@ deac_status deac_run(deac_handle *h, uint64_t rng_state[4], const deac_run_optio
     r->best_index = best;
     if (r->final_fitness) std::memcpy(r->final_fitness, fit.data(), P * sizeof(double));
     return DEAC_OK;
+} catch (...) {
+    return deac::caught();
 }
 
 }  // extern "C"

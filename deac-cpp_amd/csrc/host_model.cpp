@@ -9,7 +9,8 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
-#include <system_error>
+#include <new>
+#include <stdexcept>
 #include <thread>
 
 namespace deac {
@@ -252,6 +253,7 @@ static void parallel_rows(size_t rows, size_t values, F fn)
     const size_t most = std::clamp<size_t>(std::thread::hardware_concurrency(), 1, 16);
     const size_t nt = std::min({rows, most, values >> 15});
     std::vector<std::thread> th;
+    th.reserve(nt);  // (nothing may be thrown past a thread that has started)
     std::atomic<size_t> next{0};
     auto work = [&] {
         for (size_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < rows;) fn(i);
@@ -259,12 +261,25 @@ static void parallel_rows(size_t rows, size_t values, F fn)
     for (size_t t = 1; t < nt; t++) {
         try {
             th.emplace_back(work);
-        } catch (const std::system_error &) {  // no more threads: the ones there are do it
+        } catch (const std::exception &) {  // no more threads: the ones there are do it
             break;
         }
     }
     work();
     for (auto &x : th) x.join();
+}
+
+deac_status caught() noexcept
+{
+    try {
+        throw;
+    } catch (const std::bad_alloc &) {
+        return DEAC_ERR_OUT_OF_MEMORY;
+    } catch (const std::length_error &) {  // more than a vector can hold
+        return DEAC_ERR_OUT_OF_MEMORY;
+    } catch (...) {
+        return DEAC_ERR_DEVICE;
+    }
 }
 
 Model build_model(const deac_problem &p)

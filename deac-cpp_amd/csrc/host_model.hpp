@@ -72,6 +72,10 @@ deac_status validate(const deac_problem &p, std::string &message);
 // Builds K (deac.cpp:310-401) and the moment vectors (deac.cpp:489-827).
 Model build_model(const deac_problem &p);
 
+// The status of the exception being handled: each entry point that allocates ends
+// with it, since its callers may be C.
+deac_status caught() noexcept;
+
 // Device memory for statistics histories that a handle keeps from run to run, in
 // doubles (64 MiB); a longer run's is given back behind it.
 constexpr size_t kStatsKept = size_t(8) << 20;

@@ -34,11 +34,13 @@ struct Buffers {
     bool alloc(T *&out, size_t count)
     {
         void *p = nullptr;
+        ptrs.push_back(nullptr);  // its place, before there is anything to lose
         if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) {
             (void)hipGetLastError();
+            ptrs.pop_back();
             return false;
         }
-        ptrs.push_back(p);
+        ptrs.back() = p;
         out = static_cast<T *>(p);
         return true;
     }
@@ -75,7 +77,7 @@ extern "C" size_t deac_genome_length(const deac_problem *p)
 
 extern "C" deac_status deac_model_isf(const deac_problem *p, const double *genomes, size_t count, int precision,
                                       double *model_isf, double *chi2, double *kernel_ms, const char **message)
-{
+try {
     if (message) *message = nullptr;
     if (!p || !genomes || count == 0) return DEAC_ERR_INVALID_ARGUMENT;
     if (precision != DEAC_PRECISION_FP64 && precision != DEAC_PRECISION_FP32 && precision != DEAC_PRECISION_BF16X3) {
@@ -209,4 +211,6 @@ extern "C" deac_status deac_model_isf(const deac_problem *p, const double *genom
     if (chi2)
         for (int n = 0; n < N; n++) chi2[n] = reduced_chi2(m, &E[static_cast<size_t>(n) * T]);
     return DEAC_OK;
+} catch (...) {
+    return deac::caught();
 }

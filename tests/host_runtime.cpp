@@ -45,6 +45,12 @@ long fail_launch = 0;            // likewise the launches
 std::map<void *, unsigned> pinned;
 std::set<Stream *> streams;
 size_t host_largest = 0;         // largest single host allocation so far
+long fail_new = 0;               // the n-th host allocation of the code under test fails, 0: none
+thread_local int inside = 0;     // in the stand-in, whose own allocations do not count
+struct Inside {
+    Inside() { inside++; }
+    ~Inside() { inside--; }
+};
 
 Stream *stream_of(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
 Event *event_of(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
@@ -67,7 +73,10 @@ bool anything_in_flight()
 
 void *operator new(size_t n)
 {
-    if (n > host_largest) host_largest = n;
+    if (!inside) {
+        if (n > host_largest) host_largest = n;
+        if (fail_new > 0 && --fail_new == 0) throw std::bad_alloc();
+    }
     if (void *p = std::malloc(n ? n : 1)) return p;
     throw std::bad_alloc();
 }
@@ -88,6 +97,7 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int)
 }
 hipError_t hipMalloc(void **p, size_t n)
 {
+    const Inside own;
     if (fail_malloc > 0 && --fail_malloc == 0) return hipErrorOutOfMemory;
     if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
     live[*p] = n;
@@ -106,6 +116,7 @@ hipError_t hipFree(void *p)
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned flags)
 {
+    const Inside own;
     *p = std::calloc(n, 1);
     pinned[*p] = flags;
     return hipSuccess;
@@ -124,6 +135,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
 {
+    const Inside own;
     Stream *n = new Stream;
     streams.insert(n);
     *s = reinterpret_cast<hipStream_t>(n);
@@ -143,11 +155,13 @@ hipError_t hipStreamSynchronize(hipStream_t s)
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
 {
+    const Inside own;
     for (Stream *b : event_of(e)->covers) stream_of(s)->behind.insert(b);
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
 {
+    const Inside own;
     *e = reinterpret_cast<hipEvent_t>(new Event);
     return hipSuccess;
 }
@@ -155,6 +169,7 @@ hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0);
 hipError_t hipEventDestroy(hipEvent_t e) { return delete event_of(e), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 {
+    const Inside own;
     event_of(e)->covers = stream_of(s)->behind;
     event_of(e)->covers.insert(stream_of(s));
     return hipSuccess;
@@ -235,6 +250,11 @@ hipError_t launch_ks_bf16x3(const void *, const void *, const void *, const void
     return launch(s);
 }
 
+hipError_t launch_reduce_slices(const float *, float *, int, size_t, hipStream_t s, hipEvent_t, hipEvent_t)
+{
+    return launch(s);
+}
+
 static hipError_t batch_launch(const BatchDesc *d, int count, hipStream_t s)
 {
     for (int i = 0; i < count; i++)
@@ -253,6 +273,7 @@ hipError_t launch_batch_mixed(const BatchDesc *d, int n, int, int, int, int, hip
 int batch_mixed_nq(int ntm, int) { return ntm <= 9 ? 9 : 0; }
 hipError_t batch_scratch(int, double **p)
 {
+    const Inside own;
     static std::vector<double> scratch(kBatchScratchDoubles);
     return *p = scratch.data(), hipSuccess;
 }
@@ -342,6 +363,101 @@ struct Batch {
     deac_status run() { return deac_batch_run(h, rng.data(), o.data(), r.data()); }
 };
 
+// Calls f with its first, second, ... host allocation failing until it gets by:
+// every failure is a status, and leaves no more device memory than before.
+template <class F>
+void each_host_allocation(const char *what, F f)
+{
+    const size_t before = live_bytes;
+    for (long k = 1; k < 100000; k++) {
+        fail_new = k;
+        deac_status st = DEAC_OK;
+        bool thrown = false;
+        try {
+            st = f();
+        } catch (...) {
+            thrown = true;
+        }
+        const bool failed = fail_new == 0;
+        fail_new = 0;
+        expect(!thrown, std::string(what) + ": an exception left the entry point at allocation " + std::to_string(k));
+        if (!failed) return expect(st == DEAC_OK, std::string(what) + ": fails by itself");
+        // (a thread that cannot be started is done without)
+        expect(st == DEAC_OK || st == DEAC_ERR_OUT_OF_MEMORY, std::string(what) + ": another status");
+        if (st != DEAC_OK) expect(live_bytes <= before, std::string(what) + ": device memory left behind");
+        if (wrong) return;
+    }
+    expect(false, std::string(what) + ": never got by");
+}
+
+void host_memory_runs_out()
+{
+    Problem q(20, 2048);  // its kernel matrix is built on two threads
+    {
+        deac_handle *h = nullptr;
+        each_host_allocation("deac_create", [&] {
+            deac_destroy(h);
+            h = nullptr;
+            return deac_create(&q.p, &h, nullptr);
+        });
+        const size_t len = deac_output_length(&q.p);
+        std::vector<double> dsf(len), freq(len), mean(100);
+        deac_result r{};
+        r.dsf = dsf.data();
+        r.frequency = freq.data();
+        r.stats_mean = mean.data();
+        for (int precision : {DEAC_PRECISION_FP64, DEAC_PRECISION_FP32}) {
+            deac_run_options o{};
+            o.number_of_generations = 100;
+            o.track_stats = 1;
+            o.ks_precision = precision;
+            uint64_t first[4], rng[4];
+            deac_seed_state(1, first);
+            // (what a handle keeps is there before)
+            std::memcpy(rng, first, sizeof rng);
+            expect(deac_run(h, rng, &o, &r) == DEAC_OK, "deac_run failed");
+            bool moved = false;
+            each_host_allocation("deac_run", [&] {
+                std::memcpy(rng, first, sizeof rng);
+                const deac_status st = deac_run(h, rng, &o, &r);
+                moved |= st != DEAC_OK && std::memcmp(rng, first, sizeof rng) != 0;
+                return st;
+            });
+            expect(!moved, "deac_run: the random state of a run that failed has moved on");
+        }
+        deac_destroy(h);
+    }
+    each_host_allocation("deac_batch_create", [&] {
+        deac_batch *h = nullptr;
+        const deac_status st = deac_batch_create(&q.p, 1, &h, nullptr);
+        deac_batch_destroy(h);
+        return st;
+    });
+    {
+        Batch b(3, 9, 64, 50);
+        expect(b.run() == DEAC_OK, "deac_batch_run failed");
+        each_host_allocation("deac_batch_run", [&] { return b.run(); });
+        each_host_allocation("deac_batch_continue",
+                             [&] {
+                                 const long k = fail_new;
+                                 fail_new = 0;
+                                 (void)b.run();
+                                 fail_new = k;
+                                 return deac_batch_continue(b.h, b.rng.data(), b.o.data(), b.r.data());
+                             });
+        each_host_allocation("deac_batch_run_noalloc",
+                             [&] { return deac_batch_run_noalloc(b.h, b.rng.data(), b.o.data(), b.r.data()); });
+        each_host_allocation("deac_batch_tune",
+                             [&] { return deac_batch_tune(b.h, b.rng.data(), b.o.data(), 10, nullptr); });
+    }
+    std::vector<double> genomes(5 * deac_genome_length(&q.p)), chi2(5);
+    for (int precision : {DEAC_PRECISION_FP64, DEAC_PRECISION_FP32, DEAC_PRECISION_BF16X3})
+        each_host_allocation("deac_model_isf", [&] {
+            return deac_model_isf(&q.p, genomes.data(), 5, precision, nullptr, chi2.data(), nullptr, nullptr);
+        });
+    expect(live.empty(), "device memory left");
+}
+
 // Long histories: neither the host nor the device keeps all instances' at once
 // behind a run, and a long genome's best rows come back in pieces.
 void long_histories()
@@ -389,6 +505,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> scenarios = {
         {"status_memory", status_memory},
         {"long_histories", long_histories},
+        {"host_memory_runs_out", host_memory_runs_out},
     };
     auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return std::printf("no such scenario\n"), 2;
