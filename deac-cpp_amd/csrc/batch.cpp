@@ -173,6 +173,12 @@ struct deac_batch {
             (void)hipFree(p);
         }
     }
+    void release_stats()
+    {
+        release(stats_ws);
+        stats_ws = nullptr;
+        stats_cap = 0;
+    }
 };
 
 namespace {
@@ -655,6 +661,22 @@ try {
         }
     }
     BATCH_HIP(hipSetDevice(h->device));
+    // Whatever the outcome, nothing stays in flight past this call (a run that
+    // fails between the group streams' fork and join would leave work that s does
+    // not wait for), and the histories of a long run are given back.
+    struct AtReturn {
+        deac_batch *h;
+        bool completed = false;
+        ~AtReturn()
+        {
+            if (!completed) {
+                (void)hipStreamSynchronize(h->stream);
+                for (hipStream_t g : h->gstream) (void)hipStreamSynchronize(g);
+                (void)hipGetLastError();
+            }
+            if (h->stats_cap > deac::kStatsKept) h->release_stats();
+        }
+    } at_return{h};
     hipStream_t s = h->stream;
     // n launches side by side on `lanes` streams (the group streams, then s
     // itself), s behind all of them: f(k, stream) issues the k-th.
@@ -755,22 +777,8 @@ try {
     size_t stats_n = 0;
     for (size_t i = 0; i < n; i++)
         if (options[i].track_stats) stats_n += 3 * options[i].number_of_generations;
-    auto release_stats = [&]() {
-        h->release(h->stats_ws);
-        h->stats_ws = nullptr;
-        h->stats_cap = 0;
-    };
-    // (frees the histories of a long run behind it, whatever its outcome)
-    struct AtReturn {
-        decltype(release_stats) &release;
-        const size_t &cap;
-        ~AtReturn()
-        {
-            if (cap > deac::kStatsKept) release();
-        }
-    } at_return{release_stats, h->stats_cap};
     if (!stats_pool && stats_n > h->stats_cap) {
-        release_stats();
+        h->release_stats();
         if (h->alloc(h->stats_ws, stats_n) != DEAC_OK) return DEAC_ERR_OUT_OF_MEMORY;
         h->stats_cap = stats_n;
     }
@@ -1161,6 +1169,7 @@ try {
     h->masks_at = masks_at;
     h->epar_valid.assign(n, 0);
     for (size_t i = 0; i < n; i++) h->epar_valid[i] = options[i].ks_precision != DEAC_PRECISION_FP64;
+    at_return.completed = true;
     return DEAC_OK;
 } catch (...) {
     return deac::caught();

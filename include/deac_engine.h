@@ -245,7 +245,9 @@ deac_status deac_batch_continue(deac_batch *batch, uint64_t *rng_states, const d
  * batches of the same shapes (T, G, P, signs, precision of every instance),
  * by the process. */
 typedef struct deac_batch_schedule {
-    int group_streams;         /* 1..3: kernel-shape groups launched side by side on this many streams */
+    int group_streams;         /* kernel-shape groups side by side: 1 one after the other; 2 that many at once; 3
+                                  (the default) three, or four where the workgroups of all groups fit on the compute
+                                  units.  With 2 and 3, initial populations and evaluations take up to four. */
     int group_order;           /* 0: most expensive group first, 1: least expensive first, 2: by kernel shape */
     int instance_order;        /* 0: longest instances first, 1: round robin over distinct problems */
     double ms_per_generation;  /* deac_batch_tune: the chosen schedule's time per generation of the batch */

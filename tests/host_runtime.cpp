@@ -458,6 +458,44 @@ void host_memory_runs_out()
     expect(live.empty(), "device memory left");
 }
 
+// A launch that fails in the middle of a run: nothing of the run is in flight when
+// its status comes back, on whichever stream, and the next run is sound.
+void launches_fail()
+{
+    Problem q[4] = {{9, 64}, {20, 64}, {40, 64}, {70, 64}};  // four kernel shapes
+    std::vector<deac_problem> p;
+    for (Problem &x : q) p.push_back(x.p);
+    deac_batch *h = nullptr;
+    expect(deac_batch_create(p.data(), p.size(), &h, nullptr) == DEAC_OK, "deac_batch_create failed");
+    std::vector<double> out(8 * 127);
+    std::vector<deac_run_options> o(4);
+    std::vector<deac_result> r(4);
+    std::vector<uint64_t> rng(16);
+    for (size_t i = 0; i < 4; i++) {
+        o[i].number_of_generations = 20;
+        r[i].dsf = &out[2 * i * 127];
+        r[i].frequency = r[i].dsf + 127;
+    }
+    for (int precision : {DEAC_PRECISION_FP64, DEAC_PRECISION_FP32})
+        for (long k = 1;; k++) {
+            for (size_t i = 0; i < 4; i++) {
+                o[i].ks_precision = precision;
+                deac_seed_state(i, &rng[4 * i]);
+            }
+            fail_launch = k;
+            const deac_status st = deac_batch_run(h, rng.data(), o.data(), r.data());
+            const bool failed = fail_launch == 0;
+            fail_launch = 0;
+            expect(!anything_in_flight(), "launch " + std::to_string(k) + " fails: work is left in flight");
+            expect(st == (failed ? DEAC_ERR_DEVICE : DEAC_OK), "launch " + std::to_string(k) + ": another status");
+            if (!failed) {
+                expect(k > 8, "fewer launches than shapes");
+                break;
+            }
+        }
+    deac_batch_destroy(h);
+}
+
 // Long histories: neither the host nor the device keeps all instances' at once
 // behind a run, and a long genome's best rows come back in pieces.
 void long_histories()
@@ -506,6 +544,7 @@ int main(int argc, char **argv)
         {"status_memory", status_memory},
         {"long_histories", long_histories},
         {"host_memory_runs_out", host_memory_runs_out},
+        {"launches_fail", launches_fail},
     };
     auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return std::printf("no such scenario\n"), 2;
