@@ -20,6 +20,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "batch_kernels.hpp"
@@ -337,30 +338,40 @@ deac_status upload_mixed(deac_batch *h, BatchModel &b, int precision)
     // rows up as they are, packed on the device: FP32 [tile][unit of 16
     // positions][lane][4], BF16X3 [tile][32-position block][lane][8 hi, 8 lo]
     const bool f32 = precision == DEAC_PRECISION_FP32;
-    uint32_t *dk = nullptr;
-    deac_status st = h->alloc(dk, static_cast<size_t>(b.ntm) * b.Lpad * 16);  // 4 bytes per value either way
-    if (st != DEAC_OK) return st;
     TempRows rows;
-    int *dex = nullptr;
     if (!rows.alloc(T * L, T)) return DEAC_ERR_OUT_OF_MEMORY;
-    dex = rows.ex;
+    // the tiles and scales, the batch's once they are whole
+    struct Made {
+        deac_batch *h;
+        uint32_t *tiles = nullptr;
+        double *scale = nullptr;
+        ~Made()
+        {
+            if (tiles) h->release(tiles);
+            if (scale) h->release(scale);
+        }
+    } made{h};
+    deac_status st = h->alloc(made.tiles, static_cast<size_t>(b.ntm) * b.Lpad * 16);  // 4 bytes per value either way
+    if (st == DEAC_OK && !b.kscale) st = h->alloc(made.scale, T);
+    if (st != DEAC_OK) return st;
     if (hipMemcpyAsync(rows.rows, m.kernel.data(), T * L * sizeof(double), hipMemcpyHostToDevice, h->stream) !=
             hipSuccess ||
-        hipMemcpyAsync(dex, ex.data(), T * sizeof(int), hipMemcpyHostToDevice, h->stream) != hipSuccess)
+        hipMemcpyAsync(rows.ex, ex.data(), T * sizeof(int), hipMemcpyHostToDevice, h->stream) != hipSuccess)
         return DEAC_ERR_DEVICE;
-    const deac::PackArgs pk{rows.rows, dex, static_cast<int>(T), static_cast<int>(L), b.ntm, b.Lpad / (f32 ? 16 : 32)};
-    if ((f32 ? deac::launch_pack_fp32_units(pk, reinterpret_cast<float *>(dk), h->stream)
-             : deac::launch_pack_bf16x3(pk, dk, nullptr, h->stream)) != hipSuccess ||
+    const deac::PackArgs pk{rows.rows, rows.ex, static_cast<int>(T), static_cast<int>(L), b.ntm,
+                            b.Lpad / (f32 ? 16 : 32)};
+    if ((f32 ? deac::launch_pack_fp32_units(pk, reinterpret_cast<float *>(made.tiles), h->stream)
+             : deac::launch_pack_bf16x3(pk, made.tiles, nullptr, h->stream)) != hipSuccess ||
         hipStreamSynchronize(h->stream) != hipSuccess)
         return DEAC_ERR_DEVICE;
-    if (!b.kscale) {
+    if (made.scale) {
         std::vector<double> sc(T);
         for (size_t t = 0; t < T; t++) sc[t] = std::ldexp(1.0, ex[t]);
-        if ((st = h->alloc(b.kscale, T)) != DEAC_OK) return st;
-        if (hipMemcpy(b.kscale, sc.data(), T * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+        if (hipMemcpy(made.scale, sc.data(), T * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
             return DEAC_ERR_DEVICE;
+        b.kscale = std::exchange(made.scale, nullptr);
     }
-    b.kmix[precision] = dk;
+    b.kmix[precision] = std::exchange(made.tiles, nullptr);
     return DEAC_OK;
 }
 

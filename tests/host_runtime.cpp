@@ -496,6 +496,36 @@ void launches_fail()
     deac_batch_destroy(h);
 }
 
+// A first mixed-precision run for whose tiles the device memory does not last, or
+// whose packing fails: each retry leaves as much as there was before.
+void device_memory_runs_out()
+{
+    for (int precision : {DEAC_PRECISION_FP32, DEAC_PRECISION_BF16X3})
+        for (long *fail : {&fail_malloc, &fail_launch})
+            for (long k = 1;; k++) {
+                Batch b(1, 9, 64, 20);
+                b.o[0].ks_precision = precision;
+                const size_t before = live_bytes;
+                bool failed = true;
+                for (int retry = 0; retry < 3 && failed; retry++) {
+                    *fail = k;
+                    const deac_status st = b.run();
+                    failed = *fail == 0;
+                    *fail = 0;
+                    expect(st == (!failed ? DEAC_OK : fail == &fail_malloc ? DEAC_ERR_OUT_OF_MEMORY : DEAC_ERR_DEVICE),
+                           "failure " + std::to_string(k) + ": another status");
+                    // (the run's own workspaces may come after its tiles)
+                    if (failed && k == 1) expect(live_bytes == before, "a retry leaves device memory behind");
+                    if (failed && fail == &fail_malloc && k <= 3)
+                        expect(live_bytes == before, "a retry at allocation " + std::to_string(k) + " leaves " +
+                                                         std::to_string(live_bytes - before) + " bytes behind");
+                }
+                expect(b.run() == DEAC_OK, "no run behind the failures");
+                if (!failed) break;
+            }
+    expect(live.empty(), "device memory left");
+}
+
 // Long histories: neither the host nor the device keeps all instances' at once
 // behind a run, and a long genome's best rows come back in pieces.
 void long_histories()
@@ -545,6 +575,7 @@ int main(int argc, char **argv)
         {"long_histories", long_histories},
         {"host_memory_runs_out", host_memory_runs_out},
         {"launches_fail", launches_fail},
+        {"device_memory_runs_out", device_memory_runs_out},
     };
     auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return std::printf("no such scenario\n"), 2;

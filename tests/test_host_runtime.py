@@ -22,7 +22,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["status_memory", "long_histories", "host_memory_runs_out", "launches_fail"])
+@pytest.mark.parametrize("scenario", ["status_memory", "long_histories", "host_memory_runs_out", "launches_fail",
+                                      "device_memory_runs_out"])
 def test_host_runtime(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
