@@ -98,6 +98,7 @@ struct deac_handle {
         void *p = nullptr;
         allocations.push_back(nullptr);  // its place, before there is anything to lose
         if (hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) {
+            (void)hipGetLastError();
             allocations.pop_back();
             return DEAC_ERR_OUT_OF_MEMORY;
         }

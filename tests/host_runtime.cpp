@@ -55,8 +55,19 @@ struct Inside {
 Stream *stream_of(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
 Event *event_of(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
 
+hipError_t last_error = hipSuccess;
+
+hipError_t take_last_error()
+{
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
+
+// The launchers return the runtime's last error, whichever call left it.
 hipError_t launch(hipStream_t s)
 {
+    if (last_error != hipSuccess) return take_last_error();
     if (fail_launch > 0 && --fail_launch == 0) return hipErrorLaunchFailure;
     if (s) stream_of(s)->pending = true;
     return hipSuccess;
@@ -87,7 +98,7 @@ extern "C" {
 hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
 hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return take_last_error(); }
 hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int)
 {
     *p = hipDeviceProp_t{};
@@ -98,7 +109,7 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int)
 hipError_t hipMalloc(void **p, size_t n)
 {
     const Inside own;
-    if (fail_malloc > 0 && --fail_malloc == 0) return hipErrorOutOfMemory;
+    if (fail_malloc > 0 && --fail_malloc == 0) return last_error = hipErrorOutOfMemory;
     if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
     live[*p] = n;
     live_bytes += n;
@@ -500,6 +511,53 @@ void launches_fail()
 // whose packing fails: each retry leaves as much as there was before.
 void device_memory_runs_out()
 {
+    {
+        Problem q(9, 64);
+        for (long k = 1;; k++) {
+            deac_handle *h = nullptr;
+            fail_malloc = k;
+            const deac_status st = deac_create(&q.p, &h, nullptr);
+            const bool failed = fail_malloc == 0;
+            fail_malloc = 0;
+            expect(st == (failed ? DEAC_ERR_OUT_OF_MEMORY : DEAC_OK), "deac_create: another status");
+            deac_destroy(h);
+            expect(live.empty(), "deac_create: device memory left");
+            h = nullptr;
+            expect(deac_create(&q.p, &h, nullptr) == DEAC_OK, "no deac_create behind a failed allocation");
+            deac_destroy(h);
+            if (!failed) break;
+        }
+        deac_handle *h = nullptr;
+        expect(deac_create(&q.p, &h, nullptr) == DEAC_OK, "deac_create failed");
+        std::vector<double> out(2 * deac_output_length(&q.p));
+        deac_run_options o{};
+        o.number_of_generations = 50;
+        o.track_stats = 1;
+        deac_result r{};
+        r.dsf = out.data();
+        r.frequency = out.data() + out.size() / 2;
+        for (int precision : {DEAC_PRECISION_FP64, DEAC_PRECISION_FP32, DEAC_PRECISION_BF16X3})
+            for (long k = 1;; k++) {
+                uint64_t rng[4];
+                deac_seed_state(1, rng);
+                o.ks_precision = precision;
+                o.number_of_generations += 1;  // (longer statistics than there are)
+                fail_malloc = k;
+                const deac_status st = deac_run(h, rng, &o, &r);
+                const bool failed = fail_malloc == 0;
+                fail_malloc = 0;
+                expect(st == (failed ? DEAC_ERR_OUT_OF_MEMORY : DEAC_OK), "deac_run: another status");
+                deac_seed_state(1, rng);
+                expect(deac_run(h, rng, &o, &r) == DEAC_OK, "no deac_run behind a failed allocation");
+                if (!failed) break;
+                if (precision != DEAC_PRECISION_FP64) {  // another precision's operands again
+                    o.ks_precision = precision ^ 3;
+                    deac_seed_state(1, rng);
+                    expect(deac_run(h, rng, &o, &r) == DEAC_OK, "deac_run failed");
+                }
+            }
+        deac_destroy(h);
+    }
     for (int precision : {DEAC_PRECISION_FP32, DEAC_PRECISION_BF16X3})
         for (long *fail : {&fail_malloc, &fail_launch})
             for (long k = 1;; k++) {
