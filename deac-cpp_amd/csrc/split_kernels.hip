@@ -258,11 +258,12 @@ __global__ __launch_bounds__(kThreads) void split_pack_bf16x3_kernel(EvoArgs a, 
 
 // The trials' model ISF as the detailed-balance (bdsf) reference build sums
 // it, straight into emod: one wavefront per member and 16 timeslices.
-__global__ __launch_bounds__(kWave) void split_fold_kernel(EvoArgs a)
+__global__ __launch_bounds__(kWave) void split_fold_kernel(EvoArgs a, int first)
 {
     if (stopped(a)) return;
     __shared__ __attribute__((aligned(16))) double buf[kFoldTaskLds];
-    const int lane = threadIdx.x, tb = blockIdx.x % a.TB, i = blockIdx.x / a.TB;
+    const int task = first + static_cast<int>(blockIdx.x), tb = task % a.TB, i = task / a.TB;
+    const int lane = threadIdx.x;
     const double e = fold_task(a.ktile + static_cast<size_t>(tb) * a.stride * kChainTau, chain_row(a, i, false),
                                a.stride / kFoldBlock, a.Kc, (a.G & 1) != 0, buf);
     const int t = tb * kChainTau + 4 * ((lane >> 2) & 3) + (lane >> 4);
@@ -313,16 +314,17 @@ __host__ __device__ __forceinline__ int slice_runs(int cols, int slices, int thr
 template <bool MODEL>
 __global__ __launch_bounds__(MODEL ? kSelectThreads : kWave) void split_select_kernel(EvoArgs a, int g, int init,
                                                                                       const float *part, int slices,
-                                                                                      int Npad, int Mpad, const int *ex)
+                                                                                      int Npad, int Mpad, const int *ex,
+                                                                                      int first)
 {
     constexpr int kTauEach = 4;
+    const int i = first + static_cast<int>(blockIdx.x);
     if (stopped(a)) return;
     if (a.iter && !init) {
         g = static_cast<int>(a.iter[2]);
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.iter[1] = g + 1;
+        if (i == 0 && threadIdx.x == 0) a.iter[1] = g + 1;
     }
     extern __shared__ __attribute__((aligned(16))) double dsh[];  // a window of residuals, and MODEL their sums
-    const int i = blockIdx.x;
     const Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
     Controls next;  // loaded ahead of their use
     double old = 0.0;
@@ -426,6 +428,17 @@ unsigned grid_for(size_t work, unsigned threads)
     return static_cast<unsigned>(std::max<size_t>(1, std::min<size_t>(blocks, 4096)));
 }
 
+// go(first, grid) for all items, a workgroup each: a dispatch holds fewer than
+// 2^32 threads, which a selection of 4 million members or a fold of 67 million
+// tasks exceeds.
+template <class F>
+void in_dispatches(size_t items, unsigned threads, F go)
+{
+    const size_t most = UINT32_MAX / threads;
+    for (size_t first = 0; first < items; first += most)
+        go(static_cast<int>(first), static_cast<unsigned>(std::min(most, items - first)));
+}
+
 }  // namespace
 
 hipError_t launch_split_trial(const EvoArgs &a, int g, int pack, void *B, void *Bl, int Kb, hipStream_t s)
@@ -475,7 +488,9 @@ hipError_t launch_split_pack_bf16x3(const EvoArgs &a, int init, void *Bh, void *
 
 hipError_t launch_split_fold(const EvoArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(split_fold_kernel, dim3(a.P * a.TB), dim3(kWave), 0, s, a);
+    in_dispatches(static_cast<size_t>(a.P) * a.TB, kWave, [&](int first, unsigned grid) {
+        hipLaunchKernelGGL(split_fold_kernel, dim3(grid), dim3(kWave), 0, s, a, first);
+    });
     return hipGetLastError();
 }
 
@@ -489,7 +504,10 @@ hipError_t launch_split_moments(const EvoArgs &a, int init, hipStream_t s)
 hipError_t launch_split_select(const EvoArgs &a, int g, int init, hipStream_t s)
 {
     const size_t lds = static_cast<size_t>(std::min(a.T, kSelectLds)) * sizeof(double);
-    hipLaunchKernelGGL(split_select_kernel<false>, dim3(a.P), dim3(kWave), lds, s, a, g, init, nullptr, 0, 0, 0, nullptr);
+    in_dispatches(a.P, kWave, [&](int first, unsigned grid) {
+        hipLaunchKernelGGL(split_select_kernel<false>, dim3(grid), dim3(kWave), lds, s, a, g, init, nullptr, 0, 0, 0,
+                           nullptr, first);
+    });
     return hipGetLastError();
 }
 
@@ -501,8 +519,11 @@ hipError_t launch_split_model_select(const EvoArgs &a, int g, int init, const fl
     const int cols = (static_cast<int>(window) + 3) / 4;
     // the wavefronts that have slices to add, and one per 64 residuals
     const int used = std::max(cols * slice_runs(cols, slices, kSelectThreads), std::min(a.T, kSelectThreads));
-    hipLaunchKernelGGL(split_select_kernel<true>, dim3(a.P), dim3(static_cast<unsigned>((used + kWave - 1) / kWave * kWave)),
-                       lds, s, a, g, init, part, slices, Npad, Mpad, ex);
+    const unsigned threads = static_cast<unsigned>((used + kWave - 1) / kWave * kWave);
+    in_dispatches(a.P, threads, [&](int first, unsigned grid) {
+        hipLaunchKernelGGL(split_select_kernel<true>, dim3(grid), dim3(threads), lds, s, a, g, init, part, slices, Npad,
+                           Mpad, ex, first);
+    });
     return hipGetLastError();
 }
 
