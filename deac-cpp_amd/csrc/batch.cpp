@@ -292,9 +292,6 @@ struct TempRows {
 // Packed device memory read back in pieces of kPiece doubles (32 MiB) or one
 // item, items in ascending order.
 constexpr size_t kPiece = size_t(4) << 20;
-// A history of more doubles than this (1 MiB) is copied by itself, as far as it
-// was written.
-constexpr size_t kLongHistory = size_t(1) << 17;
 class Pieces {
     const double *from_;
     size_t total_, at_ = 0, size_ = 0, cap_ = 0;
@@ -1152,7 +1149,7 @@ try {
         if (stats[i]) {
             const size_t k = generation + 1;  // entries written
             double *const to[3] = {r->stats_mean, r->stats_minimum, r->stats_squared_mean};
-            if (3 * N <= kLongHistory) {
+            if (3 * N <= deac::kLongHistory) {
                 const double *hs = nullptr;
                 BATCH_HIP(histories.get(static_cast<size_t>(stats[i] - stats_base_ptr), 3 * N, hs));
                 for (int q = 0; q < 3; q++)

@@ -455,6 +455,7 @@ try {
     std::vector<double> fit(P), row(Kc);                            // for the results
 
     const bool track = o->track_stats != 0;
+    std::vector<double> histories(track && 3 * N <= deac::kLongHistory ? 3 * N : 0);
     auto release_stats = [&]() {
         void *old = h->stats;
         h->stats = nullptr;
@@ -899,8 +900,14 @@ try {
     if (track) {
         const size_t n = generation + 1;  // entries written
         double *const to[3] = {r->stats_mean, r->stats_minimum, r->stats_squared_mean};
-        for (int k = 0; k < 3; k++)
-            if (to[k]) DEAC_HIP(hipMemcpy(to[k], stats + k * N, n * sizeof(double), hipMemcpyDeviceToHost));
+        if (!histories.empty()) {
+            DEAC_HIP(hipMemcpy(histories.data(), stats, 3 * N * sizeof(double), hipMemcpyDeviceToHost));
+            for (int k = 0; k < 3; k++)
+                if (to[k]) std::memcpy(to[k], &histories[k * N], n * sizeof(double));
+        } else {
+            for (int k = 0; k < 3; k++)
+                if (to[k]) DEAC_HIP(hipMemcpy(to[k], stats + k * N, n * sizeof(double), hipMemcpyDeviceToHost));
+        }
     }
     if (generation + 2 == N) {  // deac.cpp:1677-1685
         generation += 1;

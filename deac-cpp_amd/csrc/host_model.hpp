@@ -79,6 +79,10 @@ deac_status caught() noexcept;
 // Device memory for statistics histories that a handle keeps from run to run, in
 // doubles (64 MiB); a longer run's is given back behind it.
 constexpr size_t kStatsKept = size_t(8) << 20;
+// Three histories of more doubles than this (1 MiB) together are copied straight to
+// the caller's arrays, as far as they were written; shorter ones in one copy (a
+// copy costs 15 us).
+constexpr size_t kLongHistory = size_t(1) << 17;
 
 // In-order reductions of the reference build (see host_model.cpp).
 double mean_of(const double *a, size_t n);
