@@ -226,14 +226,11 @@ __device__ __forceinline__ bool stopped(const int *halt)
 __device__ __forceinline__ uint64_t value_bits(uint64_t passed, bool &carry)
 {
     const int lane = threadIdx.x & (kWave - 1);
-    const uint64_t failed = ~(carry ? passed & ~UINT64_C(1) : passed);
-    auto run_before = [&](int i) {  // i > 0
-        const uint64_t f = failed << (64 - i);
-        return f ? __builtin_clzll(f) : i;
-    };
-    const bool value = lane ? run_before(lane) & 1 : carry;
-    carry = run_before(64) & 1;
-    return __ballot(value);
+    const uint64_t first = carry ? 1 : 0, failed = ~passed | first;
+    // the failed draws in front of the lane's, the nearest at the top
+    const int zeros = lane ? __clzll(failed << (kWave - lane)) : 0;
+    carry = __clzll(failed) & 1;
+    return __ballot(min(zeros, lane) & 1) | first;
 }
 
 // Walk of a.ngen generations by one wavefront (deac.cpp:1180-1240): the
