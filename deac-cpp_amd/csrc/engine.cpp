@@ -288,11 +288,13 @@ try {
     const int maxwg = deac::evolve_max_workgroups(device);
     if (maxwg <= 0) return DEAC_ERR_DEVICE;
     h->maxwg = maxwg;
-    // One workgroup per chain task or moment fold (a chain wavefront alone on its CU takes
-    // 28 us at 8192 positions, three together 33), more where there is a trial
-    // phase (not EvoArgs::fed) with over 1024 pairs of positions for each (P = 8
-    // at 8192 positions: 39.6 us per generation with 32 workgroups, 42.2 with 16,
-    // 40.0 with 64).
+    // One workgroup per chain task or moment fold, which share a CU's L1 and
+    // matrix cores otherwise, more where there is a trial phase (not
+    // EvoArgs::fed) with over 1024 pairs of positions for each.  With a first
+    // moment, 17 timeslices, us per generation: 16 members of 16384 positions 68.1
+    // with the rule's 128 workgroups, 68.1 with 64, 72.0 with 32, 69.7 with 248; 40
+    // members of 8192 43.9 with its 160, 47.4 with 48, 45.9 with 248; 8 members 37.7
+    // with its 32, 38.9 with 12, 40.2 with 248.
     // One CU per XCD stays free for the walk: workgroups go to the XCDs in
     // turn, and one that found its XCD full would hold up the grid barriers
     // until the walk ends.

@@ -566,7 +566,8 @@ static_assert((kEvoWaves * kChainLds + kResidLds) * sizeof(double) <= kEvoLds, "
 // A tau block's K units from a moving chunk on, as buffer loads: the base is
 // scalar and the unit an immediate offset from one of four lane offsets, so a
 // load is one instruction with one address register (with 64-bit lane
-// addresses a unit took 28 ns, 24.5 this way).
+// addresses a unit took 28 ns, 24.5 this way, with the genome's loads still in
+// front of the MFMAs; 17.6 now).
 struct KUnits {
     static_assert(kChunkUnits == 16, "four lane offsets, four units each");
     const char *base;

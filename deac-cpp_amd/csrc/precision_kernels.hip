@@ -12,7 +12,7 @@
 //           Kl.Sh + Kh.Sl + Kh.Sh per 32 positions on v_mfma_f32_16x16x32_bf16,
 //           FP32 accumulation as above.
 //
-// Operands arrive in MFMA lane order (prepared on the host), one coalesced
+// Operands arrive in MFMA lane order (pack_kernels.hip), one coalesced
 // load per wave and k-block:
 //   16x16x4  (FP64, FP32): A[mt][kb][lane] = K[16 mt + lane%16][4 kb + lane/16],
 //                          B[nt][kb][lane] = S[16 nt + lane%16][4 kb + lane/16];

@@ -295,8 +295,9 @@ __global__ __launch_bounds__(kWave) void split_moment_kernel(EvoArgs a, int init
 // runs then take over each other's sums in order.
 //
 // Bound: latency: loads, one barrier per run, thread 0's sum.  257 timeslices,
-// 114 slices, 64 members: 13.3 us; as two kernels, with a part of each
-// sum's loads in flight, 9.2 and 7.5.
+// 114 slices, 64 members: 11.6 us in a kernel trace (15.0 with a test around each
+// load); as two kernels, with a part of each sum's loads in flight, 9.2 and 7.5
+// by themselves and the gap between them.
 constexpr int kSliceRun = 8;  // slices a thread loads at once
 constexpr int kSelectThreads = 1024;
 
