@@ -118,17 +118,23 @@ __device__ __forceinline__ void bf16_split(float x, int e, uint32_t (&hi)[4], ui
 // reach, once, for the initial fitness).  Workgroup 0 runs the top of the
 // generation: it reads only the fitnesses, which no trial writes, and if its
 // stop test fires the trials are never selected (every later kernel of the
-// generation returns).  The others take 16 members x 128 positions each, a
-// member's 128 per wavefront, so that rows and operand are both whole lines.
+// generation returns).  The others take 128 positions of a member per wavefront:
+// with an operand 16 members each, four per wavefront, so that rows and operand
+// are both whole lines; without one a member per wavefront, whose records and
+// rows are waited for one after the other.
 //
 // Bound: memory (40 bytes read, 12 written per position).  64 members of 32768
 // positions: 19.3 us; with a kernel of its own for the operand 17.4 and 9.7.
+// Without an operand, one member per wavefront and four: 4 members of 600
+// positions 3.8 us and 5.5, 20 members 4.2 and 8.7, 64 members of 32768 13.2 and
+// 16.7, 300 members of 16384 27.3 and 32.0.
 constexpr int kTileMembers = 16;
+constexpr int trial_members(int pack) { return pack == DEAC_PRECISION_FP64 ? kThreads / kWave : kTileMembers; }
 constexpr int kTileRow = kChunk + 4;  // floats: the operand's readers meet no bank twice
 template <int PACK>
 __global__ __launch_bounds__(kThreads) void split_trial_kernel(EvoArgs a, int g, void *B, void *Bl, int Kb)
 {
-    constexpr int kWaves = kThreads / kWave, kEach = kTileMembers / kWaves;
+    constexpr int kWaves = kThreads / kWave, kMembers = trial_members(PACK), kEach = kMembers / kWaves;
     __shared__ __attribute__((aligned(16))) float tile[PACK == DEAC_PRECISION_FP64 ? 1 : kTileMembers][kTileRow];
     if (stopped(a)) return;
     if (a.iter) g = static_cast<int>(a.iter[1]);
@@ -144,12 +150,13 @@ __global__ __launch_bounds__(kThreads) void split_trial_kernel(EvoArgs a, int g,
     const Members s = {a.fitness, a.cr_old, a.f_old, a.cur};
     const MemberCtl *ctlg = a.ctl + static_cast<size_t>(g) * a.P;
     const uint64_t *rawg = a.raw + static_cast<size_t>(g) * a.P * a.rstride;
-    auto member = [&](int j) { return nt * kTileMembers + wid + j * kWaves; };
+    auto member = [&](int j) { return nt * kMembers + wid + j * kWaves; };
     auto trial = [&](int j) {
         const int i = min(member(j), a.P - 1);
         return Trial(a, s, a.cur, ctlg[i], rawg + static_cast<size_t>(i) * a.rstride, i);
     };
-    const Trial t[kEach] = {trial(0), trial(1), trial(2), trial(3)};
+    static_assert(kEach == 1 || kEach == 4);
+    const Trial t[4] = {trial(0), trial(1 % kEach), trial(2 % kEach), trial(3 % kEach)};
     Trial::Load v[kEach] = {};
 #pragma unroll
     for (int j = 0; j < kEach; j++) t[j].load(b, v[j]);
@@ -444,7 +451,8 @@ void in_dispatches(size_t items, unsigned threads, F go)
 
 hipError_t launch_split_trial(const EvoArgs &a, int g, int pack, void *B, void *Bl, int Kb, hipStream_t s)
 {
-    const size_t tiles = static_cast<size_t>((a.P + kTileMembers - 1) / kTileMembers) * (a.stride / kChunk);
+    const int members = trial_members(pack);
+    const size_t tiles = static_cast<size_t>((a.P + members - 1) / members) * (a.stride / kChunk);
     const dim3 grid(static_cast<unsigned>(tiles) + 1), threads(kThreads);
     if (pack == DEAC_PRECISION_FP32)
         hipLaunchKernelGGL(split_trial_kernel<DEAC_PRECISION_FP32>, grid, threads, 0, s, a, g, B, Bl, Kb);
