@@ -253,7 +253,6 @@ static void parallel_rows(size_t rows, size_t values, F fn)
     const size_t most = std::clamp<size_t>(std::thread::hardware_concurrency(), 1, 16);
     const size_t nt = std::min({rows, most, values >> 15});
     std::vector<std::thread> th;
-    th.reserve(nt);  // (nothing may be thrown past a thread that has started)
     std::atomic<size_t> next{0};
     auto work = [&] {
         for (size_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < rows;) fn(i);
@@ -261,7 +260,7 @@ static void parallel_rows(size_t rows, size_t values, F fn)
     for (size_t t = 1; t < nt; t++) {
         try {
             th.emplace_back(work);
-        } catch (const std::exception &) {  // no more threads: the ones there are do it
+        } catch (const std::exception &) {  // no more threads, or no room for one more: those there are do it
             break;
         }
     }
